@@ -395,10 +395,8 @@ void Net::fuse_binconv_epilogues() {
     for (size_t i = 0; i < layers.size(); ++i) {
         auto producer = std::dynamic_pointer_cast<BinConv>(layers[i]);
         if (!producer || !producer->fused_a || producer->output_mat->c % 64 != 0) continue;
-        // not with 512 input channels: sign bits need work items of 8 output channels, four units there, and the
-        // coarser split costs more than the separate pack_mat it saves (measured at batch 64 and 256) -- unless the
-        // problem is small enough for the kernel whose work items are 8 channels anyway, or of the size that the
-        // row-split kernel takes (its store pass writes the bits at no extra pass)
+        // with 512 input channels only in the size classes 0 and 3 (dabnn_hip_tuning.h): large problems there leave the
+        // packing to the layer that reads the blob
         if (producer->input_mat->elem_c >= 512) {
             const int64_t pixels = (int64_t)producer->output_mat->n * producer->output_mat->h * producer->output_mat->w;
             if (!dab_bconv3x3_splits_depth(pixels, producer->input_mat->elem_c, producer->output_mat->c) &&
