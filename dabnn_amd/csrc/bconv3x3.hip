@@ -32,6 +32,7 @@ struct BconvArgs {
     int cols;         // channel tiles
     int px_tiles;     // pixel tiles
     int window;       // window kernel: pixels of input that a tile's windows reach at most
+    int buffers;      // and how many such windows fit LDS, one or two
     uint32_t x_bytes, w_bytes;
     FastDiv div_ow, div_oh, div_cols;
     // fused epilogue (MODE >= 1 kernels only): out = a*cnt + b (+ shortcut); MODE 2 also writes sign bits of out
@@ -341,8 +342,9 @@ __global__ __launch_bounds__(256, MT == 2 ? 2 : NT == 2 ? 3 : 4) void bconv3x3_s
 // kernels before took 50 and 56), four pixel groups per wave (spills with an epilogue).
 template <int CW>
 struct WindowRow {
-    static constexpr int bytes = CW * 8 + (CW == 2 ? 8 : 16);  // of a pixel in LDS: an odd number of load-sized slots
+    static constexpr int bytes = CW * 32 + 16;  // of a pixel in LDS, expanded: an odd number of 16-byte slots
 };
+constexpr long long kWindowLdsBytes = 78 * 1024;  // of a block: two blocks of a CU
 constexpr int kWindowPieces = 4;  // 16-byte pieces of the next window a thread holds in registers
 template <int CW>
 struct WindowTile {
@@ -364,7 +366,7 @@ __global__ __launch_bounds__(256, CW == 2 ? 3 : 2) void bconv3x3_window_kernel(c
 #pragma unroll
     for (int t = 0; t < 9; ++t) load_dwords<CW>(w[t], rw, ch_ok ? ch * (CW * 72) + t * (CW * 8) + half * (CW * 4) : kOutside);
     const int wbytes = p.window * RS, pieces = p.window * PP;
-    if (tid < RS / 8) reinterpret_cast<uint64_t *>(win + 2 * wbytes)[tid] = 0;
+    if (tid < RS / 16) reinterpret_cast<u32x4 *>(win + p.buffers * wbytes)[tid] = u32x4{0u, 0u, 0u, 0u};
 
     u32x4 next[kWindowPieces];
     auto fetch = [&](int tile) {
@@ -382,13 +384,9 @@ __global__ __launch_bounds__(256, CW == 2 ? 3 : 2) void bconv3x3_window_kernel(c
         for (int i = 0; i < kWindowPieces; ++i) {
             const int c = tid + i * 256;
             if (c < pieces) {
-                unsigned char *d = win + buf * wbytes + (c / PP) * RS + (c % PP) * 16;
-                if constexpr (RS % 16 == 0) {
-                    *reinterpret_cast<u32x4 *>(d) = next[i];
-                } else {
-                    *reinterpret_cast<u32x2 *>(d) = u32x2{next[i].x, next[i].y};
-                    *reinterpret_cast<u32x2 *>(d + 8) = u32x2{next[i].z, next[i].w};
-                }
+                i32x4 *d = reinterpret_cast<i32x4 *>(win + buf * wbytes + (c / PP) * RS + (c % PP) * 64);
+                d[0] = lower_half(bits01(next[i].x)), d[1] = lower_half(bits01(next[i].y));
+                d[2] = lower_half(bits01(next[i].z)), d[3] = lower_half(bits01(next[i].w));
             }
         }
     };
@@ -408,18 +406,19 @@ __global__ __launch_bounds__(256, CW == 2 ? 3 : 2) void bconv3x3_window_kernel(c
     put(0);
     __syncthreads();
 
-    for (int buf = 0; tile < p.px_tiles; tile += groups, buf ^= 1) {
+    for (int buf = 0, next_buf; tile < p.px_tiles; tile += groups, buf = next_buf) {
+        next_buf = p.buffers == 1 ? 0 : buf ^ 1;
         const bool more = tile + groups < p.px_tiles;
         int tap[MT][9];  // LDS addresses
         {
             int y, x;
-            const int lo = window_origin(p, tile * PX, y, x), zero = 2 * wbytes;
+            const int lo = window_origin(p, tile * PX, y, x), zero = p.buffers * wbytes;
 #pragma unroll
             for (int m = 0; m < MT; ++m) {
                 int pix = tile * PX + m * 32 + l32;
                 pix = pix < p.total ? pix : p.total - 1;
                 int y0, x0;
-                const int base = buf * wbytes + (window_origin(p, pix, y0, x0) - lo) * RS + half * (CW * 4);
+                const int base = buf * wbytes + (window_origin(p, pix, y0, x0) - lo) * RS + half * (CW * 16);
 #pragma unroll
                 for (int t = 0; t < 9; ++t) {
                     const int kh = t / 3, kw = t % 3;
@@ -445,19 +444,18 @@ __global__ __launch_bounds__(256, CW == 2 ? 3 : 2) void bconv3x3_window_kernel(c
             for (int v = 0; v < 16; ++v) acc[m][v] = init;
 #pragma unroll
         for (int t = 0; t < 9; ++t) {
-            uint32_t a[MT][CW];
-#pragma unroll
-            for (int m = 0; m < MT; ++m) lds_dwords<CW>(a[m], win + tap[m][t]);
 #pragma unroll
             for (int c = 0; c < CW; ++c) {
                 // expanded here, not ahead of the loop: only the 72 registers of 128 channels would fit
                 if constexpr (CW >= 4) asm volatile("" : "+v"(w[t][c]));
                 const i32x8 b = bitspm(w[t][c]);
 #pragma unroll
-                for (int m = 0; m < MT; ++m) mfma_fp4<32>(acc[m], bits01(a[m][c]), b);
+                for (int m = 0; m < MT; ++m)
+                    mfma_fp4<32>(acc[m], upper_zero(*reinterpret_cast<const i32x4 *>(win + tap[m][t] + c * 16)), b);
             }
         }
-        if (more) put(buf ^ 1);
+        if (p.buffers == 1) __syncthreads();  // every wave has read this window
+        if (more) put(next_buf);
         const __amdgpu_buffer_rsrc_t ro = make_rsrc(p.out + view.base, view.bytes);
 #pragma unroll
         for (int m = 0; m < MT; ++m) {
@@ -516,7 +514,7 @@ static int launch_stream(BconvArgs &a, hipStream_t stream) {
 template <int CW, int MODE>
 static bool window_fits(BconvArgs &a) {
     a.window = window_pixels(a, 32 * WindowTile<CW>::groups32);
-    return a.window > 0 && a.window * (CW / 2) <= 256 * kWindowPieces;
+    return a.window > 0 && a.window * (CW / 2) <= 256 * kWindowPieces && (a.window + 1ll) * WindowRow<CW>::bytes <= kWindowLdsBytes;
 }
 
 template <int CW, int MODE>
@@ -525,10 +523,14 @@ static int launch_window(BconvArgs &a, hipStream_t stream) {
     a.cols = (a.cout + 127) / 128;
     a.px_tiles = (int)(((long long)a.total + PX - 1) / PX);
     a.div_cols = FastDiv((uint32_t)a.cols);
-    const size_t lds = (size_t)(2 * a.window + 1) * WindowRow<CW>::bytes;  // 49 KB at most, of the CU's 160
+    a.buffers = (2ll * a.window + 1) * WindowRow<CW>::bytes <= kWindowLdsBytes ? 2 : 1;
+    const size_t lds = (size_t)(a.buffers * a.window + 1) * WindowRow<CW>::bytes;
     static const int by_registers = resident_blocks_per_cu(bconv3x3_window_kernel<CW, MODE>, 256);
     const int by_lds = (int)(160 * 1024 / (lds + 512));
     const int groups = resident_groups(a, by_registers < by_lds ? by_registers : by_lds, 1);
+    static const bool whole_lds = hipFuncSetAttribute(reinterpret_cast<const void *>(bconv3x3_window_kernel<CW, MODE>),
+                                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)kWindowLdsBytes) == hipSuccess;
+    (void)whole_lds;
     hipLaunchKernelGGL((bconv3x3_window_kernel<CW, MODE>), dim3((unsigned)(groups * a.cols)), dim3(256), lds, stream, a);
     DAB_LAUNCH_CHECK();
     return DAB_OK;

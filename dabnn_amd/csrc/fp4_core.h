@@ -12,8 +12,8 @@
 // A single bit at position 0, 1 or 2 of its nibble is the value 0.5, 1 or 2; position 3 is the sign, so that dword is
 // shifted down.
 //   bits01:  bit -> {0, m}, m = 0.5, 1, 2, 0.5 in the four dwords.  5 vector instructions.
-//   bitspm:  bit -> {+m', -m'}, m' = 2, 1, 0.5, 2: every product with a bits01 value is 0 or +-1.  11 instructions.
-//   bitspm1: bit -> {+1, -1} in all dwords, for products of two such operands.  11 instructions.
+//   bitspm:  bit -> {+m', -m'}, m' = 2, 1, 0.5, 2: every product with a bits01 value is 0 or +-1.  7 instructions.
+//   bitspm1: bit -> {+1, -1} in all dwords, for products of two such operands.  7 instructions.
 // With x as bits01 and w as bitspm, popcount(w) + sum x * (+-1 for w = 0 / 1) is the number of places where x and w
 // differ; with both as bitspm1 it is (K - sum) / 2.  A zero word in both operands (the reference's padding word,
 // dabnn/pad.h:12) counts no difference either way.
@@ -24,6 +24,7 @@
 namespace dab {
 
 typedef int i32x8 __attribute__((ext_vector_type(8)));  // the instruction's operand; 4-bit floats use the first four
+typedef int i32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x4m __attribute__((ext_vector_type(4)));
 typedef float f32x16m __attribute__((ext_vector_type(16)));
 
@@ -32,18 +33,25 @@ __device__ __forceinline__ i32x8 bits01(uint32_t x) {
     r[0] = x & 0x11111111u, r[1] = x & 0x22222222u, r[2] = x & 0x44444444u, r[3] = (x >> 3) & 0x11111111u;
     return r;
 }
+// (x & y) | z in one instruction.  These expansions are what bounds the deep convolutions: vector instructions and
+// fp4 matrix instructions of a SIMD do not overlap here, and each of the former costs 4 to 5 cycles with 2 or 3 waves.
+__device__ __forceinline__ uint32_t and_or(uint32_t x, uint32_t y, uint32_t z) { return __builtin_amdgcn_bitop3_b32(x, y, z, 0xEA); }
 __device__ __forceinline__ i32x8 bitspm(uint32_t w) {
     i32x8 r = {0, 0, 0, 0, 0, 0, 0, 0};
-    r[0] = ((w << 3) & 0x88888888u) | 0x44444444u, r[1] = ((w << 2) & 0x88888888u) | 0x22222222u;
-    r[2] = ((w << 1) & 0x88888888u) | 0x11111111u, r[3] = (w & 0x88888888u) | 0x44444444u;
+    r[0] = and_or(w << 3, 0x88888888u, 0x44444444u), r[1] = and_or(w << 2, 0x88888888u, 0x22222222u);
+    r[2] = and_or(w << 1, 0x88888888u, 0x11111111u), r[3] = and_or(w, 0x88888888u, 0x44444444u);
     return r;
 }
 __device__ __forceinline__ i32x8 bitspm1(uint32_t w) {
     i32x8 r = {0, 0, 0, 0, 0, 0, 0, 0};
-    r[0] = ((w << 3) & 0x88888888u) | 0x22222222u, r[1] = ((w << 2) & 0x88888888u) | 0x22222222u;
-    r[2] = ((w << 1) & 0x88888888u) | 0x22222222u, r[3] = (w & 0x88888888u) | 0x22222222u;
+    r[0] = and_or(w << 3, 0x88888888u, 0x22222222u), r[1] = and_or(w << 2, 0x88888888u, 0x22222222u);
+    r[2] = and_or(w << 1, 0x88888888u, 0x22222222u), r[3] = and_or(w, 0x88888888u, 0x22222222u);
     return r;
 }
+
+// Expanded dwords in memory hold only the four that 4-bit floats use.
+__device__ __forceinline__ i32x4 lower_half(const i32x8 &v) { return i32x4{v[0], v[1], v[2], v[3]}; }
+__device__ __forceinline__ i32x8 upper_zero(const i32x4 &v) { return i32x8{v[0], v[1], v[2], v[3], 0, 0, 0, 0}; }
 
 // acc += A * B.  T = 32: 32 x 32 outputs over 64 depths, lane l holds row / column l % 32, depths 32 * (l / 32) ..;
 // T = 16: 16 x 16 over 128 depths, row / column l % 16, depths 32 * (l / 16) ...
