@@ -15,6 +15,7 @@ from .ops import (  # noqa: F401
     ave_pool2_fconv1x1,
     global_ave_pool_fconv1x1,
     global_ave_pool_fconv1x1_takes,
+    bconv,
     bconv_3x3,
     bconv_3x3_affine_add,
     bconv_3x3_affine_add_sign,

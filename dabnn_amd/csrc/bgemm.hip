@@ -3,260 +3,457 @@
 //   A(i,h) = a[h*lda + i]   m x k words, the transposed filter bank
 //   B(h,j) = b[j*ldb + h]   k x n words, one contiguous K-row per output pixel
 //   C(i,j) = c[j*ldc + i]   m x n floats, i.e. NHWC output
+// and the convolution over any window that shares its kernels (bgemm_core.h).
 //
-// Mapping: a lane owns one ROW i of A (an output channel).  For a fixed K word
-// the 64 rows of a tile are 512 contiguous bytes of A, so the lane-resident
-// operand is fetched with fully coalesced loads; the K-row of a column j is
-// contiguous in B and wave-uniform, so it comes through scalar loads and
-// enters v_xor_b32 as SGPR operands; and for a fixed column the 64 results are
-// 256 contiguous bytes of C, so the read-modify-write of C is coalesced
-// without any transposition.
-//
-// A unit is 64 rows x Q columns.  Waves own contiguous ranges of units ordered
-// row-tile major, so the A operand is reloaded only when a range crosses into
-// the next row tile.
-//   K64R > 0  k == K64R and ldb == k: the lane keeps its whole A row resident
-//             (the network shapes: 18, 36, 72 words with Q = 8, 4, 2) and the
-//             Q*k words of B of a unit are one contiguous run
-//   K64R == 0 any k, any ldb: K is walked in chunks of 8 words; per chunk the
-//             lane reloads 8 words of A (coalesced, L1/L2 resident)
-#include "xnor_core.h"
+// Rows of the matrix instruction are pixels (columns j of C), columns are channels (rows i of C), so an accumulator
+// register is 32 consecutive floats of two pixels and the output needs no transposition.
+#include "bgemm_core.h"
 
 namespace dab {
 
-struct BgemmArgs {
-    const uint64_t *a;
-    const uint64_t *b;
-    float *c;
-    int m, n, k;
-    int lda, ldb, ldc;
-    int n_runs;  // ceil(n / Q) column runs per row tile
-    int items_per_wave, items_extra;
-    FastDiv div_runs;
-    int overwrite;  // C = counts instead of C += counts: what the reference's fill(0) + bgemm pair leaves in C
+struct BitGemmArgs {
+    BitGemm g;
+    int units, chunks;  // units of 2 * CC dwords; of one tap
+    uint32_t x_bytes;   // window form: the packed images
+    uint32_t w_bytes;   // kFilterRows: the filters
+    int col_tiles;
+    long long row_tiles;
+    FastDiv div_ow, div_oh, div_chunks, div_kw, div_col_tiles, div_row_pieces;
 };
 
-constexpr int kGemmWavesPerBlock = 4;
-constexpr int kChunk = 8;  // K words per chunk of the generic variant
+// four dwords that start at any word
+typedef uint32_t u32x4u __attribute__((ext_vector_type(4), aligned(8)));
 
-// C(row, j) += counts of a unit.  Columns below j_first belong to the previous
-// (shifted) run and are skipped; the test is wave-uniform.
-template <int Q>
-__device__ __forceinline__ void add_to_c(float *__restrict__ c, int ldc, int row, bool row_ok, int j0, int j_first,
-                                         const uint32_t (&acc)[Q], bool overwrite) {
+constexpr int kBeyond = (int)0x80000000;  // an offset outside every descriptor: loads return zero
+
+// kFilterColumns goes with a plain matrix (rows of x in memory order), kFilterRows with windows of images.
+template <FilterLayout L>
+struct PixelRows {
+    __amdgpu_buffer_rsrc_t rsrc;  // windows: the packed images
+    int base, y0, x0;
+    const uint64_t *row;          // plain matrix
+    __device__ __forceinline__ void start(const BitGemmArgs &p, long long tile_row, int l32) {
+        long long r = tile_row + l32;
+        r = r < p.g.rows ? r : p.g.rows - 1;
+        if constexpr (L == kFilterColumns) {
+            row = p.g.x + r * p.g.x_ld;
+        } else {
+            rsrc = make_rsrc(p.g.x, p.x_bytes);
+            const uint32_t t = p.div_ow.div((uint32_t)r);
+            const int ox = (int)r - (int)t * p.g.OW;
+            const uint32_t n = p.div_oh.div(t);
+            const int oy = (int)t - (int)n * p.g.OH;
+            y0 = oy * p.g.stride_h - p.g.pad_h, x0 = ox * p.g.stride_w - p.g.pad_w;
+            base = (((int)n * p.g.H + y0) * p.g.W + x0) * (int)(p.g.x_ld * 8);
+        }
+    }
+    // the lane's CC dwords of unit u (wave-uniform); zero outside the image and past the last word
+    template <int CC>
+    __device__ __forceinline__ void load(uint32_t (&d)[CC], const BitGemmArgs &p, int u, int half) const {
+        if constexpr (L == kFilterColumns) {
+            static_assert(CC == 4, "a plain matrix is walked four words at a time");
+            const int word = u * 4 + half * 2;
+            d[0] = d[1] = d[2] = d[3] = 0u;
+            if (word + 1 < p.g.words) {
+                const u32x4u v = *reinterpret_cast<const u32x4u *>(row + word);
+                d[0] = v.x, d[1] = v.y, d[2] = v.z, d[3] = v.w;
+            } else if (word < p.g.words) {
+                const u32x2 v = *reinterpret_cast<const u32x2 *>(row + word);
+                d[0] = v.x, d[1] = v.y;
+            }
+        } else {
+            const int tap = (int)p.div_chunks.div((uint32_t)u), chunk = u - tap * p.chunks;
+            const int kh = (int)p.div_kw.div((uint32_t)tap), kw = tap - kh * p.g.kw;
+            const bool ok = (unsigned)(y0 + kh) < (unsigned)p.g.H && (unsigned)(x0 + kw) < (unsigned)p.g.W;
+            const int off = ok ? base + (kh * p.g.W + kw) * (int)(p.g.x_ld * 8) + (chunk * 2 + half) * (CC * 4) : kBeyond;
+            if constexpr (CC == 3) {
+                const u32x3 v = __builtin_amdgcn_raw_buffer_load_b96(rsrc, off, 0, 0);
+                d[0] = v.x, d[1] = v.y, d[2] = v.z;
+            } else {
+                load_dwords<CC>(d, rsrc, off);
+            }
+        }
+    }
+};
+
+// CC dwords of unit u of filter `col` for one half of the lanes
+template <int CC, FilterLayout L>
+__device__ __forceinline__ void load_filter(uint32_t (&d)[CC], const BitGemmArgs &p, __amdgpu_buffer_rsrc_t rw, int col, int u, int half) {
+    if constexpr (L == kFilterColumns) {
+        const int word = u * 4 + half * 2;
+        const uint64_t *src = p.g.w + (long long)word * p.g.w_ld + col;
+        const bool ok = col < p.g.cols;
+        const uint64_t v0 = ok && word < p.g.words ? src[0] : 0ull, v1 = ok && word + 1 < p.g.words ? src[p.g.w_ld] : 0ull;
+        d[0] = (uint32_t)v0, d[1] = (uint32_t)(v0 >> 32), d[2] = (uint32_t)v1, d[3] = (uint32_t)(v1 >> 32);
+    } else {
+        const int off = col < p.g.cols && u < p.units ? col * (int)(p.g.w_ld * 8) + (u * 2 + half) * (CC * 4) : kBeyond;
+        if constexpr (CC == 3) {
+            const u32x3 v = __builtin_amdgcn_raw_buffer_load_b96(rw, off, 0, 0);
+            d[0] = v.x, d[1] = v.y, d[2] = v.z;
+        } else {
+            load_dwords<CC>(d, rw, off);
+        }
+    }
+}
+// Set bits of the word that pads filter `col` to 128 bits
+__device__ __forceinline__ uint32_t extra_bits(const BitGemmArgs &p, __amdgpu_buffer_rsrc_t rw, int col) {
+    const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(rw, col < p.g.cols ? (col * (int)p.g.w_ld + p.g.words) * 8 : kBeyond, 0, 0);
+    return __popc(v.x) + __popc(v.y);
+}
+
+// The output (or a tensor laid out like it) from a tile's first pixel to the tensor's end: offsets past it load zero and
+// store nothing.  Rows are below 64 MB (bit_gemm).
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t tile_rsrc(const float *t, const BitGemmArgs &p, long long row0) {
+    const long long left = ((p.g.rows - 1 - row0) * p.g.out_ld + p.g.cols) * 4;
+    return make_rsrc(t + row0 * p.g.out_ld, left < 0x7fffffff ? (uint32_t)left : 0x7fffffffu);
+}
+
+enum Epilogue { kStoreCounts, kAddCounts, kAffine, kAffineSign };
+
+// Few tiles, or a depth that does not fit LDS as filters: a block is one tile of 32 pixels x 32 * NT channels, its four
+// waves take every fourth unit of the depth each and load their operands straight from memory, five units at a time; the
+// partial sums meet in LDS.  Both operands +-1 (fp4_core.h).  m512 k72 n3136, accumulating: 7.8 us against 16.2 for the
+// xor/popcount kernel before.
+constexpr int kUnitsAhead = 3;
+template <int CC, FilterLayout L, int E, int NT>
+__global__ __launch_bounds__(256, 4) void bit_gemm_split_kernel(const BitGemmArgs p) {
+    constexpr int CH = 32 * NT, LD = CH + 1;
+    __shared__ float part[4][32 * LD];
+    const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5, l32 = lane & 31;
+    const int wib = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t row_tile = p.div_col_tiles.div(blockIdx.x);
+    const int ch0 = (int)(blockIdx.x - row_tile * p.col_tiles) * CH;
+    const long long row0 = (long long)row_tile * 32;
+    const __amdgpu_buffer_rsrc_t rw = make_rsrc(p.g.w, L == kFilterRows ? p.w_bytes : 0u);
+    PixelRows<L> px;
+    px.start(p, row0, l32);
+
+    // this thread's outputs: channel tid % CH of pixels tid / CH + i * (256 / CH)
+    constexpr int RPI = 256 / CH, ROWS = 32 / RPI;
+    const int ch = ch0 + tid % CH, r0 = tid / CH;
+    const bool ch_ok = ch < p.g.cols;
+    float old[ROWS], ea = 0.f, eb = 0.f;
+    uint32_t extra = 0;
+    if (L == kFilterRows && p.g.extra_word) extra = extra_bits(p, rw, ch);
+    if (E == kAffine || E == kAffineSign)
+        if (ch_ok) ea = p.g.a[ch], eb = p.g.b[ch];
+    const int out_off = ch_ok ? (r0 * (int)p.g.out_ld + ch) * 4 : kBeyond, out_step = RPI * (int)p.g.out_ld * 4;
+    const float *second = E == kAddCounts ? p.g.out : p.g.shortcut;
+    if (E != kStoreCounts && second != nullptr) {
+        const __amdgpu_buffer_rsrc_t rs = tile_rsrc(second, p, row0);
 #pragma unroll
-    for (int q = 0; q < Q; ++q) {
-        const int j = j0 + q;
-        if (j >= j_first && row_ok) {
-            float *d = c + (size_t)j * ldc + row;
-            const float cnt = __uint_as_float(acc[q]) - kAccBias;
-            // 0.f + cnt == cnt: the store alone is the fill + accumulate pair.  The accumulating form reads C when
-            // the count is done and wants it in the L2, where ordinary stores of an earlier launch leave it
-            if (overwrite)
-                store_through(d, cnt);
+        for (int i = 0; i < ROWS; ++i) old[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, out_off, i * out_step, 0));
+    }
+
+    f32x16m acc[NT];
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[n][v] = 0.f;
+    for (int u0 = wib; u0 < p.units; u0 += 4 * kUnitsAhead) {
+        uint32_t a[kUnitsAhead][CC], w[kUnitsAhead][NT][CC];
+#pragma unroll
+        for (int i = 0; i < kUnitsAhead; ++i)
+            if (u0 + 4 * i < p.units) {
+                px.load(a[i], p, u0 + 4 * i, half);
+#pragma unroll
+                for (int n = 0; n < NT; ++n) load_filter<CC, L>(w[i][n], p, rw, ch0 + n * 32 + l32, u0 + 4 * i, half);
+            }
+#pragma unroll
+        for (int i = 0; i < kUnitsAhead; ++i)
+            if (u0 + 4 * i < p.units) {
+#pragma unroll
+                for (int c = 0; c < CC; ++c) {
+                    const i32x8 av = bitspm1(a[i][c]);
+#pragma unroll
+                    for (int n = 0; n < NT; ++n) mfma_fp4<32>(acc[n], av, bitspm1(w[i][n][c]));
+                }
+            }
+    }
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) part[wib][fp4_row<32>(half, v) * LD + n * 32 + l32] = acc[n][v];
+    __syncthreads();
+
+    const __amdgpu_buffer_rsrc_t ro = tile_rsrc(p.g.out, p, row0);
+    const float half_depth = (float)(p.units * CC) * 32.f;  // of the units; words past the last are zero on both sides and equal
+#pragma unroll
+    for (int i = 0; i < ROWS; ++i) {
+        const int row = r0 + i * RPI;
+        const long long r = row0 + row;
+        const int o = row * LD + tid % CH;
+        float v = half_depth - 0.5f * ((part[0][o] + part[1][o]) + (part[2][o] + part[3][o])) + (float)extra;
+        if constexpr (E == kAddCounts) v = old[i] + v;
+        if constexpr (E == kAffine || E == kAffineSign) {
+#pragma clang fp contract(off)
+            v = ea * v;
+            v = v + eb;
+            if (p.g.shortcut) v = v + old[i];
+        }
+        const bool ok = ch_ok && r < p.g.rows;
+        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), ro, out_off, i * out_step, kStoreThrough);
+        if constexpr (E == kAffineSign) {
+            const uint64_t mask = __ballot(v > 0.f);
+            if (ok && (tid & 31) == 0)
+                p.g.bits[r * p.g.bits_ld + (ch >> 5)] = (lane & 32) ? (uint32_t)(mask >> 32) : (uint32_t)mask;
+        }
+    }
+}
+
+// Many tiles: a block keeps the filters of 32 * NT channels in LDS as bits, in the order its lanes read them, and its
+// four waves walk over tiles of 32 pixels, four units of their pixels ahead of the multiplication.
+template <int CC, FilterLayout L, int E, int NT>
+__global__ __launch_bounds__(256, NT == 2 ? 3 : 4) void bit_gemm_stream_kernel(const BitGemmArgs p) {
+    constexpr int CH = 32 * NT, SLOT = CC == 3 ? 16 : CC * 4;  // bytes of a (unit, channel, half)
+    extern __shared__ __attribute__((aligned(16))) unsigned char filters[];
+    __shared__ uint32_t pop[CH];  // set bits per filter
+    const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5, l32 = lane & 31;
+    const int wib = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int group = (int)p.div_col_tiles.div(blockIdx.x), groups = (int)p.div_col_tiles.div(gridDim.x);
+    const int ch0 = ((int)blockIdx.x - group * p.col_tiles) * CH;
+    const __amdgpu_buffer_rsrc_t rw = make_rsrc(p.g.w, L == kFilterRows ? p.w_bytes : 0u);
+    if (tid < CH) pop[tid] = L == kFilterRows && p.g.extra_word ? extra_bits(p, rw, ch0 + tid) : 0u;
+    __syncthreads();
+    constexpr int kBatch = 3;  // pieces a thread asks for before it puts the first of them away
+    const int n_pieces = p.units * CH * 2;
+    for (int s0 = tid; s0 < n_pieces; s0 += 256 * kBatch) {
+        uint32_t d[kBatch][CC];
+        int slot[kBatch], chan[kBatch];
+#pragma unroll
+        for (int j = 0; j < kBatch; ++j) {
+            // consecutive threads take consecutive channels of column-major filters, consecutive units of filter rows
+            const int s = s0 + j * 256;
+            int u, c, h;
+            if constexpr (L == kFilterColumns) {
+                c = s % CH, h = (s / CH) & 1, u = s / (2 * CH);
+            } else {
+                c = (int)p.div_row_pieces.div((uint32_t)s);
+                const int r = s - c * p.units * 2;
+                u = r >> 1, h = r & 1;
+            }
+            chan[j] = c, slot[j] = (u * CH + c) * 2 + h;
+            if (s < n_pieces) load_filter<CC, L>(d[j], p, rw, ch0 + c, u, h);
+        }
+#pragma unroll
+        for (int j = 0; j < kBatch; ++j) {
+            if (s0 + j * 256 < n_pieces) {
+                uint32_t *dst = reinterpret_cast<uint32_t *>(filters + slot[j] * SLOT);
+                uint32_t set = 0;
+#pragma unroll
+                for (int i = 0; i < CC; ++i) dst[i] = d[j][i], set += __popc(d[j][i]);
+                atomicAdd(&pop[chan[j]], set);
+            }
+        }
+    }
+    __syncthreads();
+    float init[NT], ea[NT], eb[NT];
+    int out_off[NT];
+    const int row_bytes = (int)p.g.out_ld * 4;
+#pragma unroll
+    for (int n = 0; n < NT; ++n) {
+        const int ch = ch0 + n * 32 + l32;
+        out_off[n] = ch < p.g.cols ? half * 4 * row_bytes + ch * 4 : kBeyond;
+        init[n] = (float)pop[n * 32 + l32];
+        ea[n] = 0.f, eb[n] = 0.f;
+        if (E == kAffine || E == kAffineSign)
+            if (ch < p.g.cols) ea[n] = p.g.a[ch], eb[n] = p.g.b[ch];
+    }
+    const unsigned char *mine = filters + (l32 * 2 + half) * SLOT;
+
+    for (long long tile = (long long)group * 4 + wib; tile < p.row_tiles; tile += (long long)groups * 4) {
+        const long long row0 = tile * 32;
+        PixelRows<L> px;
+        px.start(p, row0, l32);
+        uint32_t a[4][CC];
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (i < p.units) px.load(a[i], p, i, half);
+        float old[NT][16];
+        if constexpr (E != kStoreCounts) {
+            const float *second = E == kAddCounts ? p.g.out : p.g.shortcut;
+            if (second != nullptr) {
+                const __amdgpu_buffer_rsrc_t rs = tile_rsrc(second, p, row0);
+#pragma unroll
+                for (int v = 0; v < 16; ++v)
+#pragma unroll
+                    for (int n = 0; n < NT; ++n)
+                        old[n][v] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, out_off[n], fp4_row<32>(0, v) * row_bytes, 0));
+            }
+        }
+        f32x16m acc[NT];
+#pragma unroll
+        for (int n = 0; n < NT; ++n)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) acc[n][v] = init[n];
+        for (int u0 = 0; u0 < p.units; u0 += 4) {
+            uint32_t next[4][CC];
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (u0 + 4 + i < p.units) px.load(next[i], p, u0 + 4 + i, half);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                if (u0 + i < p.units) {
+                    const unsigned char *fu = mine + (u0 + i) * (CH * 2 * SLOT);
+                    uint32_t w[NT][CC];
+#pragma unroll
+                    for (int n = 0; n < NT; ++n) {
+                        if constexpr (CC == 3) {
+                            const u32x4 v = *reinterpret_cast<const u32x4 *>(fu + n * 64 * SLOT);
+                            w[n][0] = v.x, w[n][1] = v.y, w[n][2] = v.z;
+                        } else {
+                            lds_dwords<CC>(w[n], fu + n * 64 * SLOT);
+                        }
+                    }
+#pragma unroll
+                    for (int c = 0; c < CC; ++c) {
+                        const i32x8 av = bits01(a[i][c]);
+#pragma unroll
+                        for (int n = 0; n < NT; ++n) mfma_fp4<32>(acc[n], av, bitspm(w[n][c]));
+                    }
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int c = 0; c < CC; ++c) a[i][c] = next[i][c];
+        }
+        const __amdgpu_buffer_rsrc_t ro = tile_rsrc(p.g.out, p, row0);
+        uint32_t word[NT];
+#pragma unroll
+        for (int n = 0; n < NT; ++n) word[n] = 0;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+#pragma unroll
+            for (int n = 0; n < NT; ++n) {
+                float res = acc[n][v];
+                if constexpr (E == kAddCounts) res = old[n][v] + res;
+                if constexpr (E == kAffine || E == kAffineSign) {
+#pragma clang fp contract(off)
+                    res = ea[n] * res;
+                    res = res + eb[n];
+                    if (p.g.shortcut) res = res + old[n][v];
+                }
+                __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, res), ro, out_off[n], fp4_row<32>(0, v) * row_bytes, kStoreThrough);
+                if constexpr (E == kAffineSign) {
+                    const uint64_t mask = __ballot(res > 0.f);
+                    word[n] = dab_writelane((uint32_t)mask, fp4_row<32>(0, v), word[n]);
+                    word[n] = dab_writelane((uint32_t)(mask >> 32), fp4_row<32>(1, v), word[n]);
+                }
+            }
+        }
+        if constexpr (E == kAffineSign) {
+            const long long r = row0 + l32;
+            if (half == 0 && r < p.g.rows) {
+#pragma unroll
+                for (int n = 0; n < NT; ++n)
+                    if (ch0 + n * 32 < p.g.cols) p.g.bits[r * p.g.bits_ld + ch0 / 32 + n] = word[n];
+            }
+        }
+    }
+}
+
+// LDS that a block's filters may take: two blocks of a CU
+constexpr long long kFilterLdsBytes = 72 * 1024;
+
+template <int CC, FilterLayout L, int E>
+static int launch_bit_gemm(const char *fn, BitGemmArgs &p, hipStream_t s) {
+    p.row_tiles = (p.g.rows + 31) / 32;
+    const int tiles32 = (p.g.cols + 31) / 32;
+    const long long pieces = p.row_tiles * tiles32;
+    const long long per_channel = (long long)p.units * 2 * (CC == 3 ? 16 : CC * 4);
+    // The walking kernel where its filters fit and its waves find tiles for every SIMD; also for one to three units of
+    // depth, which are no work for four waves.
+    // 64 channels a wave for plain matrices (m128 k18 n50176: 12.6 us against 16.4), 32 for windows, whose lanes spend
+    // more on addresses than on filters (100 x 25 x 25 x 192 -> 472, 5 x 5, stride 2: 34 us against 43).
+    const bool two = L == kFilterColumns && p.g.cols > 32 && pieces >= 2048;
+    const int ch = two ? 64 : 32;
+    if ((pieces >= 2048 || p.units < 4) && per_channel * ch <= kFilterLdsBytes) {
+        p.col_tiles = (p.g.cols + ch - 1) / ch;
+        p.div_col_tiles = FastDiv((uint32_t)p.col_tiles);
+        const size_t lds = (size_t)(per_channel * ch);
+        int per_cu = (int)(160 * 1024 / (lds + 1024));
+        const int by_registers = two ? 3 : 4;
+        per_cu = per_cu > by_registers ? by_registers : per_cu;
+        const long long most = (long long)(simd_count() / 4) * per_cu / p.col_tiles, want = (p.row_tiles + 3) / 4;
+        long long groups = want < most ? want : most < 1 ? 1 : most;
+        const long long per_wave = (p.row_tiles + groups * 4 - 1) / (groups * 4);
+        groups = (p.row_tiles + 4 * per_wave - 1) / (4 * per_wave);
+        auto launch = [&](auto kernel) {
+            static const bool whole_lds = hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                              (int)kFilterLdsBytes) == hipSuccess;
+            (void)whole_lds;
+            hipLaunchKernelGGL(kernel, dim3((unsigned)(groups * p.col_tiles)), dim3(256), lds, s, p);
+        };
+        if constexpr (L == kFilterColumns) {
+            if (two)
+                launch(bit_gemm_stream_kernel<CC, L, E, 2>);
             else
-                *d = *d + cnt;
-        }
-    }
-}
-
-// The same with the old values of C fetched by the caller before it counted (fetch_c), so that the round trip to
-// memory lies behind the unit's arithmetic instead of after it.
-template <int Q>
-__device__ __forceinline__ void fetch_c(const float *__restrict__ c, int ldc, int row, bool row_ok, int j0, int j_first,
-                                        float (&old)[Q], bool overwrite) {
-#pragma unroll
-    for (int q = 0; q < Q; ++q) {
-        const int j = j0 + q;
-        old[q] = (!overwrite && j >= j_first && row_ok) ? c[(size_t)j * ldc + row] : 0.f;
-    }
-}
-template <int Q>
-__device__ __forceinline__ void store_c(float *__restrict__ c, int ldc, int row, bool row_ok, int j0, int j_first,
-                                        const uint32_t (&acc)[Q], const float (&old)[Q]) {
-#pragma unroll
-    for (int q = 0; q < Q; ++q) {
-        const int j = j0 + q;
-        if (j >= j_first && row_ok) {
-            const float cnt = __uint_as_float(acc[q]) - kAccBias;
-            store_through(c + (size_t)j * ldc + row, old[q] + cnt);  // 0.f + cnt == cnt: the overwriting form never read C
-        }
-    }
-}
-
-template <int K64R, int Q>
-__global__ __launch_bounds__(64 * kGemmWavesPerBlock, K64R >= 72 ? 3 : (K64R >= 36 ? 5 : 6)) void bgemm_resident_kernel(const BgemmArgs p) {
-    constexpr int K32 = 2 * K64R;
-    const int lane = threadIdx.x & 63;
-    const int wib = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int wv = blockIdx.x * kGemmWavesPerBlock + wib;
-    int i0, i1;
-    item_range(wv, p.items_per_wave, p.items_extra, i0, i1);
-    if (i0 >= i1) return;
-
-    int mt = (int)p.div_runs.div((uint32_t)i0);
-    int run = i0 - mt * p.n_runs;
-    bool need_load = true;
-    uint32_t w[K32];
-    int row = 0;
-    bool row_ok = false;
-    for (int it = i0; it < i1; ++it) {
-        if (need_load) {
-            need_load = false;
-            row = mt * 64 + lane;
-            row_ok = row < p.m;
-            const uint64_t *col = p.a + (row_ok ? row : p.m - 1);
-#pragma unroll
-            for (int h = 0; h < K64R; ++h) {
-                const uint64_t v = col[(size_t)h * p.lda];
-                w[2 * h] = (uint32_t)v, w[2 * h + 1] = (uint32_t)(v >> 32);
-            }
-        }
-        // Priority by remaining work: the SIMD issues from its oldest wave first, so with equal priorities its few
-        // resident waves finish one after the other and the last one runs alone at the single-wave issue rate.
-        const int left = K64R >= 36 ? i1 - it - 1 : 0;  // 3-5 resident waves per SIMD; no effect measured with 6
-        if (left >= 3) {
-            __builtin_amdgcn_s_setprio(3);
-        } else if (left == 2) {
-            __builtin_amdgcn_s_setprio(2);
-        } else if (left == 1) {
-            __builtin_amdgcn_s_setprio(1);
+                launch(bit_gemm_stream_kernel<CC, L, E, 1>);
         } else {
-            __builtin_amdgcn_s_setprio(0);
+            launch(bit_gemm_stream_kernel<CC, L, E, 1>);
         }
-        // the last run of a ragged n is shifted back so its scalar loads stay inside B
-        const int j_first = run * Q;
-        const int j0 = j_first + Q <= p.n ? j_first : p.n - Q;
-        uint32_t acc[Q];
-        // B streams through the scalar cache: two vectors per wait.  The accumulating form asks for the old values of
-        // C before it counts (cfg m512 k72 n3136: 16.8 instead of 17.2 us, four times the columns 59.7 instead of 65);
-        // the overwriting form keeps the registers (two code paths, the test is wave-uniform).
-        if (p.overwrite) {
-            unit_rowmajor<K32, Q, 2, (K64R >= 72)>(p.b + (size_t)j0 * K64R, w, acc);
-            add_to_c<Q>(p.c, p.ldc, row, row_ok, j0, j_first, acc, true);
-        } else {
-            float old[Q];
-            fetch_c<Q>(p.c, p.ldc, row, row_ok, j0, j_first, old, false);
-            unit_rowmajor<K32, Q, 2, (K64R >= 72)>(p.b + (size_t)j0 * K64R, w, acc);
-            store_c<Q>(p.c, p.ldc, row, row_ok, j0, j_first, acc, old);
-        }
-        if (++run == p.n_runs) {
-            run = 0;
-            ++mt;
-            need_load = true;
-        }
+    } else {
+        const int split_ch = p.g.cols > 32 && pieces >= 1024 ? 64 : 32;
+        p.col_tiles = (p.g.cols + split_ch - 1) / split_ch;
+        p.div_col_tiles = FastDiv((uint32_t)p.col_tiles);
+        const long long blocks = p.row_tiles * p.col_tiles;
+        if (blocks >= (1ll << 31)) return fail(DAB_EUNSUPPORTED, "%s: too many work units", fn);
+        if (split_ch == 64)
+            hipLaunchKernelGGL((bit_gemm_split_kernel<CC, L, E, 2>), dim3((unsigned)blocks), dim3(256), 0, s, p);
+        else
+            hipLaunchKernelGGL((bit_gemm_split_kernel<CC, L, E, 1>), dim3((unsigned)blocks), dim3(256), 0, s, p);
     }
-}
-
-// Any k and ldb; Q = 8 columns per unit, two columns per scalar-load batch.
-__global__ __launch_bounds__(64 * kGemmWavesPerBlock) void bgemm_chunked_kernel(const BgemmArgs p) {
-    constexpr int Q = 8;
-    const int lane = threadIdx.x & 63;
-    const int wib = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int wv = blockIdx.x * kGemmWavesPerBlock + wib;
-    int i0, i1;
-    item_range(wv, p.items_per_wave, p.items_extra, i0, i1);
-    if (i0 >= i1) return;
-
-    int mt = (int)p.div_runs.div((uint32_t)i0);
-    int run = i0 - mt * p.n_runs;
-    for (int it = i0; it < i1; ++it) {
-        const int row = mt * 64 + lane;
-        const bool row_ok = row < p.m;
-        const uint64_t *acol = p.a + (row_ok ? row : p.m - 1);
-        const int j_first = run * Q;
-        const int j0 = j_first + Q <= p.n ? j_first : p.n - Q;
-        uint32_t acc[Q];
-#pragma unroll
-        for (int q = 0; q < Q; ++q) acc[q] = kAccInit;
-
-        int h0 = 0;
-        for (; h0 + kChunk <= p.k; h0 += kChunk) {
-            uint32_t w[2 * kChunk];
-#pragma unroll
-            for (int h = 0; h < kChunk; ++h) {
-                const uint64_t v = acol[(size_t)(h0 + h) * p.lda];
-                w[2 * h] = (uint32_t)v, w[2 * h + 1] = (uint32_t)(v >> 32);
-            }
-            // column j0+q contributes the 16 dwords b[(j0+q)*ldb + h0 .. +8)
-            const uint64_t *bbase = p.b + (size_t)j0 * p.ldb + h0;
-            const uint32_t bstride = (uint32_t)p.ldb * 8u;
-            u32x16 buf[2][2];
-            sload_off<16>(buf[0][0], bbase, 0u);
-            sload_off<16>(buf[0][1], bbase, bstride);
-            swait(buf[0][0]);
-            swait(buf[0][1]);
-            uint32_t off = bstride;
-            static_for<Q / 2>([&](auto s_) {
-                constexpr int s = s_;
-                if constexpr (s + 1 < Q / 2) {
-                    off += bstride;
-                    sload_off<16>(buf[(s + 1) & 1][0], bbase, off);
-                    off += bstride;
-                    sload_off<16>(buf[(s + 1) & 1][1], bbase, off);
-                }
-                static_for<2>([&](auto c_) {
-                    static_for<kChunk>([&](auto h_) {
-                        xp2(acc[2 * s + c_], buf[s & 1][c_][2 * h_], buf[s & 1][c_][2 * h_ + 1], w[2 * h_], w[2 * h_ + 1]);
-                    });
-                });
-                if constexpr (s + 1 < Q / 2) {
-                    swait(buf[(s + 1) & 1][0]);
-                    swait(buf[(s + 1) & 1][1]);
-                }
-            });
-        }
-        for (; h0 < p.k; ++h0) {  // K tail, one word at a time
-            const uint64_t v = acol[(size_t)h0 * p.lda];
-            const uint32_t wlo = (uint32_t)v, whi = (uint32_t)(v >> 32);
-#pragma unroll
-            for (int q = 0; q < Q; ++q) {
-                const uint64_t bw = p.b[(size_t)(j0 + q) * p.ldb + h0];  // wave-uniform address
-                acc[q] += __builtin_popcount(wlo ^ (uint32_t)bw) + __builtin_popcount(whi ^ (uint32_t)(bw >> 32));
-            }
-        }
-        add_to_c<Q>(p.c, p.ldc, row, row_ok, j0, j_first, acc, p.overwrite != 0);
-        if (++run == p.n_runs) {
-            run = 0;
-            ++mt;
-        }
-    }
-}
-
-// One thread per output element; for n < 8, where the column runs do not apply.
-__global__ void bgemm_small_n_kernel(const BgemmArgs p) {
-    const long long idx = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= (long long)p.m * p.n) return;
-    const int i = (int)(idx % p.m);
-    const long long j = idx / p.m;
-    uint32_t cnt = 0;
-    for (int h = 0; h < p.k; ++h) cnt += __popcll(p.a[(size_t)h * p.lda + i] ^ p.b[(size_t)j * p.ldb + h]);
-    float *d = p.c + (size_t)j * p.ldc + i;
-    *d = p.overwrite ? (float)cnt : *d + (float)cnt;
-}
-
-template <int Q, class Kernel>
-static bool plan_items(BgemmArgs &g, Kernel kernel, int &n_waves) {
-    static const int blocks_per_cu = resident_blocks_per_cu(kernel, 64 * kGemmWavesPerBlock);
-    g.n_runs = (g.n + Q - 1) / Q;
-    const long long items = (((long long)g.m + 63) / 64) * g.n_runs;
-    if (items >= (1ll << 31)) return false;
-    n_waves = pick_wave_count((int)items, blocks_per_cu, kGemmWavesPerBlock);
-    g.items_per_wave = (int)(items / n_waves);
-    g.items_extra = (int)(items % n_waves);
-    g.div_runs = FastDiv((uint32_t)g.n_runs);
-    return true;
-}
-
-template <int K64R, int Q>
-static int launch_resident(BgemmArgs &g, hipStream_t stream) {
-    int n_waves = 0;
-    if (!plan_items<Q>(g, bgemm_resident_kernel<K64R, Q>, n_waves)) return fail(DAB_EUNSUPPORTED, "dab_bgemm: too many work units");
-    hipLaunchKernelGGL((bgemm_resident_kernel<K64R, Q>), dim3(n_waves / kGemmWavesPerBlock), dim3(64 * kGemmWavesPerBlock), 0,
-                       stream, g);
     DAB_LAUNCH_CHECK();
     return DAB_OK;
 }
+
+bool bit_gemm_takes_images(long long image_words, long long filter_words, long long rows, int cols) {
+    return image_words * 8 < (1ll << 31) && filter_words * 8 < (1ll << 31) && rows < (1ll << 31) - 64 && cols < (1 << 22);
+}
+
+int bit_gemm(const char *fn, const BitGemm &g, FilterLayout layout, hipStream_t stream) {
+    if (g.out_ld >= (1 << 24) && g.rows > 1) {
+        // rows of 64 MB and more (plain matrices only): tile offsets would not fit, one launch per row
+        if (layout != kFilterColumns) return fail(DAB_EUNSUPPORTED, "%s: output rows too long", fn);
+        BitGemm one = g;
+        one.rows = 1;
+        for (long long r = 0; r < g.rows; ++r, one.x += g.x_ld, one.out += g.out_ld) {
+            const int rc = bit_gemm(fn, one, layout, stream);
+            if (rc != DAB_OK) return rc;
+        }
+        return DAB_OK;
+    }
+    BitGemmArgs p = {};
+    p.g = g;
+    if (layout == kFilterColumns) {
+        p.units = (g.words + 3) / 4, p.chunks = p.units;
+        return g.accumulate ? launch_bit_gemm<4, kFilterColumns, kAddCounts>(fn, p, stream)
+                            : launch_bit_gemm<4, kFilterColumns, kStoreCounts>(fn, p, stream);
+    }
+    const int cw = g.tap_words, cc = cw % 4 == 0 ? 4 : cw % 3 == 0 ? 3 : cw % 2 == 0 ? 2 : 1;
+    p.chunks = cw / cc;
+    p.units = g.words / cc;
+    p.x_bytes = (uint32_t)(((g.rows / ((long long)g.OH * g.OW)) * g.H * g.W) * g.x_ld * 8);
+    p.w_bytes = (uint32_t)(g.cols * g.w_ld * 8);
+    p.div_ow = FastDiv((uint32_t)g.OW), p.div_oh = FastDiv((uint32_t)g.OH);
+    p.div_chunks = FastDiv((uint32_t)p.chunks), p.div_kw = FastDiv((uint32_t)g.kw);
+    p.div_row_pieces = FastDiv((uint32_t)(2 * p.units));
+    auto with_epilogue = [&](auto cc_) {
+        constexpr int CC = decltype(cc_)::value;
+        if (g.bits) return launch_bit_gemm<CC, kFilterRows, kAffineSign>(fn, p, stream);
+        if (g.a) return launch_bit_gemm<CC, kFilterRows, kAffine>(fn, p, stream);
+        return launch_bit_gemm<CC, kFilterRows, kStoreCounts>(fn, p, stream);
+    };
+    switch (cc) {
+        case 4: return with_epilogue(std::integral_constant<int, 4>{});
+        case 3: return with_epilogue(std::integral_constant<int, 3>{});
+        case 2: return with_epilogue(std::integral_constant<int, 2>{});
+        default: return with_epilogue(std::integral_constant<int, 1>{});
+    }
+}
+
+constexpr int kMaxCount = (1 << 23) - 1;  // exact in fp32, twice over
 
 }  // namespace dab
 
@@ -272,32 +469,13 @@ static int bgemm_impl(int m, int n, int k, const uint64_t *a, int lda, const uin
                 "dab_bgemm: misaligned pointer");
     if ((long long)k * 64 > kMaxCount) return fail(DAB_EUNSUPPORTED, "dab_bgemm: k %d words exceeds the exact-count range", k);
     if ((long long)ldb * 8 * 8 >= (1ll << 32)) return fail(DAB_EUNSUPPORTED, "dab_bgemm: ldb too large");
-
-    BgemmArgs g;
-    g.a = a, g.b = b, g.c = c;
-    g.m = m, g.n = n, g.k = k;
-    g.lda = lda, g.ldb = ldb, g.ldc = ldc;
-    g.overwrite = overwrite ? 1 : 0;
-    hipStream_t s = as_stream(stream);
-    if (n < 8) {
-        const long long total = (long long)m * n;
-        hipLaunchKernelGGL(bgemm_small_n_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, g);
-        DAB_LAUNCH_CHECK();
-        return DAB_OK;
-    }
-    if (ldb == k) {
-        switch (k) {
-            case 18: return launch_resident<18, 8>(g, s);
-            case 36: return launch_resident<36, 4>(g, s);
-            case 72: return launch_resident<72, 2>(g, s);
-            default: break;
-        }
-    }
-    int n_waves = 0;
-    if (!plan_items<8>(g, bgemm_chunked_kernel, n_waves)) return fail(DAB_EUNSUPPORTED, "dab_bgemm: too many work units");
-    hipLaunchKernelGGL(bgemm_chunked_kernel, dim3(n_waves / kGemmWavesPerBlock), dim3(64 * kGemmWavesPerBlock), 0, s, g);
-    DAB_LAUNCH_CHECK();
-    return DAB_OK;
+    BitGemm g = {};
+    g.x = b, g.w = a, g.out = c;
+    g.rows = n, g.cols = m;
+    g.x_ld = ldb, g.w_ld = lda, g.out_ld = ldc;
+    g.words = k, g.tap_words = k;
+    g.accumulate = !overwrite;
+    return bit_gemm("dab_bgemm", g, kFilterColumns, as_stream(stream));
 }
 
 extern "C" int dab_bgemm(int m, int n, int k, const uint64_t *a, int lda, const uint64_t *b, int ldb, float *c, int ldc,

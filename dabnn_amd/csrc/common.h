@@ -253,6 +253,7 @@ __device__ __forceinline__ void mfma6_16x16x32(f32x4w &acc0, f32x4w &acc1, const
 
 // ---------------------------------------------------------------- buffer resources
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x3 __attribute__((ext_vector_type(3)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x8 __attribute__((ext_vector_type(8)));
 typedef uint32_t u32x16 __attribute__((ext_vector_type(16)));

@@ -117,6 +117,15 @@ BinConv::Method BinConv::method() const {
     return BGEMM;
 }
 
+bool BinConv::reads_packed() const {
+    if (method() == DIRECT_CONV) return true;
+    // the windows of other shapes on packed input, within dab_bconv's limits; without `optimize` the reference's own
+    // sequence (column matrix and GEMM) runs
+    const long long words = input_mat->elem_c / 64, pixels = (long long)input_mat->n * input_mat->h * input_mat->w;
+    return net_.lock()->optimize && (long long)kernel_h() * kernel_w() * input_mat->elem_c < 60000 && pixels * words * 8 < (1ll << 31) &&
+           (long long)weight_mat->total() * 8 < (1ll << 31);
+}
+
 void BinConv::forward_impl() const {
     void *s = stream();
     const auto *x = static_cast<const float *>(input_mat->dev);
@@ -145,6 +154,18 @@ void BinConv::forward_impl() const {
             break;
         }
         case BGEMM: {
+            if (reads_packed()) {
+                // the column matrix's rows are windows of the packed input: convolved where they lie
+                auto *packed = static_cast<uint64_t *>(binarized_mat->dev);
+                if (!input_prepacked) dab_check(dab_bitpack_nhwc(x, packed, (int64_t)n * h * w, c, s));
+                dab_check(dab_bconv(packed, c / 64, n, h, w, c, static_cast<const uint64_t *>(weight_mat->dev),
+                                    (int)(weight_mat->total() / weight_mat->n), kernel_h(), kernel_w(), pad_h, pad_w, stride_h, stride_w,
+                                    weight_mat->n, fused_a ? static_cast<const float *>(fused_a->dev) : nullptr,
+                                    fused_b ? static_cast<const float *>(fused_b->dev) : nullptr,
+                                    fused_shortcut ? static_cast<const float *>(fused_shortcut->dev) : nullptr, out, output_mat->c,
+                                    fused_sign_out ? static_cast<uint64_t *>(fused_sign_out->dev) : nullptr, (output_mat->c + 63) / 64, s));
+                break;
+            }
             // fill + fused_binarize_im2col + bgemm, dabnn/layers/BinConv.cpp:152-165; the fill and the accumulation
             // into it are one store (0.f + count == count)
             auto *col = static_cast<uint64_t *>(col_mat->dev);

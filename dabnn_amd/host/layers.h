@@ -34,6 +34,7 @@ class BNN_API BinConv : public Layer {
     void forward_impl() const override;
     std::string to_str() const override;
     Method method() const;
+    bool reads_packed() const;  // works on the packed input (a producer may write it), not on the fp32 blob
 
    private:
     int kernel_h() const { return weight_mat->h; }

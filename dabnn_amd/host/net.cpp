@@ -305,9 +305,9 @@ static bool contains(const std::vector<const Mat *> &v, const Mat *m) {
 //  1. In a down-sampling block the converter emits BinConv, Affine, [AvePool, FpConv2D, Affine], Add: the shortcut
 //     branch in brackets neither reads nor writes the BinConv's blobs, so BinConv and Affine move behind it, next to
 //     their Add.
-//  2. BinConv -> Affine (-> Add) on the same blob becomes one pass of the direct kernel, FloatConv -> Affine (-> Relu)
-//     one pass of the float convolution.
-//  3. When the blob such a fused BinConv completes is the input of a later direct BinConv, the pass also writes that
+//  2. BinConv -> Affine (-> Add) on the same blob becomes one pass of its kernel, FloatConv -> Affine (-> Relu) one
+//     pass of the float convolution.
+//  3. When the blob such a fused BinConv completes is the input of a later BinConv, the pass also writes that
 //     layer's packed input and the later layer skips its pack_mat.
 //  4. AvePool 2x2 stride 2 -> 1x1 FloatConv (the shortcut branch of a down-sampling block), the convolution being
 //     the only reader of the pooled blob, becomes one launch that does not write that blob: it leaves the net
@@ -341,9 +341,9 @@ void Net::fuse_binconv_epilogues() {
     for (size_t i = 0; i < layers.size(); ++i) {
         auto bc = std::dynamic_pointer_cast<BinConv>(layers[i]);
         auto af = i + 1 < layers.size() ? std::dynamic_pointer_cast<Affine>(layers[i + 1]) : nullptr;
-        // (1024 input channels: the direct kernel counts them in two passes and has no fused epilogue)
-        if (bc && af && bc->method() == BinConv::DIRECT_CONV && bc->input_mat->elem_c <= 512 && af->data_mat == bc->output_mat &&
-            bc->output_mat->c % 4 == 0) {
+        // (1024 input channels: the direct kernel has no fused epilogue)
+        if (bc && af && bc->reads_packed() && (bc->method() == BinConv::BGEMM || (bc->input_mat->elem_c <= 512 && bc->output_mat->c % 4 == 0)) &&
+            af->data_mat == bc->output_mat) {
             bc->fused_a = af->a_mat;
             bc->fused_b = af->b_mat;
             size_t skip = 1;
@@ -375,14 +375,14 @@ void Net::fuse_binconv_epilogues() {
     }
     layers.swap(out);
 
-    // the same for a MaxPool whose output a direct BinConv packs (the first block of a Bi-Real net)
+    // the same for a MaxPool whose output a BinConv packs (the first block of a Bi-Real net)
     for (size_t i = 0; i < layers.size(); ++i) {
         auto pool = std::dynamic_pointer_cast<MaxPool>(layers[i]);
         if (!pool || pool->output_mat->c % 64 != 0) continue;
         for (size_t j = i + 1; j < layers.size(); ++j) {
             auto consumer = std::dynamic_pointer_cast<BinConv>(layers[j]);
             if (consumer && consumer->input_mat == pool->output_mat) {
-                if (consumer->method() == BinConv::DIRECT_CONV && !consumer->input_prepacked) {
+                if (consumer->reads_packed() && !consumer->input_prepacked) {
                     pool->fused_sign_out = consumer->binarized_mat;
                     consumer->input_prepacked = true;
                 }
@@ -397,7 +397,7 @@ void Net::fuse_binconv_epilogues() {
         if (!producer || !producer->fused_a || producer->output_mat->c % 64 != 0) continue;
         // with 512 input channels only in the size classes 0 and 3 (dabnn_hip_tuning.h): large problems there leave the
         // packing to the layer that reads the blob
-        if (producer->input_mat->elem_c >= 512) {
+        if (producer->method() == BinConv::DIRECT_CONV && producer->input_mat->elem_c >= 512) {
             const int64_t pixels = (int64_t)producer->output_mat->n * producer->output_mat->h * producer->output_mat->w;
             if (!dab_bconv3x3_splits_depth(pixels, producer->input_mat->elem_c, producer->output_mat->c) &&
                 dab_bconv3x3_epilogue_build(pixels, producer->input_mat->elem_c, producer->output_mat->c, producer->stride_h, 1) != 3)
@@ -406,7 +406,7 @@ void Net::fuse_binconv_epilogues() {
         for (size_t j = i + 1; j < layers.size(); ++j) {
             auto consumer = std::dynamic_pointer_cast<BinConv>(layers[j]);
             if (consumer && consumer->input_mat == producer->output_mat) {
-                if (consumer->method() == BinConv::DIRECT_CONV) {
+                if (consumer->reads_packed()) {
                     producer->fused_sign_out = consumer->binarized_mat;
                     consumer->input_prepacked = true;
                 }

@@ -192,6 +192,27 @@ def bconv_3x3_affine_add_sign(x, weight, a, b, shortcut=None, stride=1, pad=1):
     return out, packed
 
 
+def bconv(x, weight, kh, kw, pad_h, pad_w, stride_h, stride_w, a=None, b=None, shortcut=None, want_sign=False):
+    """A binary convolution over any window on packed input [N,H,W,CW], weight int64 [Cout, words]: counts, or with a and
+    b a*cnt + b (+ shortcut); with want_sign (result, pack_mat of it)."""
+    _need(x, torch.int64, "x")
+    _need(weight, torch.int64, "weight")
+    n, h, w, cw = x.shape
+    cout, words = weight.shape
+    oh, ow = out_dim(h, pad_h, kh, stride_h), out_dim(w, pad_w, kw, stride_w)
+    out = _empty((n, max(oh, 0), max(ow, 0), cout), torch.float32, x.device)
+    packed = _empty((n, max(oh, 0), max(ow, 0), max(cout // 64, 1)), torch.int64, x.device) if want_sign else None
+    for name, t, shape in (("a", a, (cout,)), ("b", b, (cout,)), ("shortcut", shortcut, out.shape)):
+        if t is not None:
+            _need(t, torch.float32, name)
+            if tuple(t.shape) != tuple(shape):
+                raise capi.DabError(capi.DAB_EINVAL, "bconv: %s does not match the output" % name)
+    opt = lambda t: _ptr(t) if t is not None else None
+    check(lib.dab_bconv(_ptr(x), cw, n, h, w, cw * 64, _ptr(weight), words, kh, kw, pad_h, pad_w, stride_h, stride_w, cout,
+                        opt(a), opt(b), opt(shortcut), _ptr(out), cout, opt(packed), max(cout // 64, 1), _stream()))
+    return (out, packed) if want_sign else out
+
+
 class BinConv:
     """The BinConv layer (dabnn/layers/BinConv.h:9-38, BinConv.cpp:17-191) over a batch.
 

@@ -123,6 +123,21 @@ DAB_API int dab_bgemm_overwrite(int m, int n, int k, const uint64_t *a, int lda,
 DAB_API int dab_weight_transpose(const uint64_t *w, int m, int k, uint64_t *wt, dab_stream_t stream);
 
 /*
+ * A binary convolution over any window, stride and multiple of 64 channels on packed input: what the reference's BGEMM
+ * arm makes of it (fused_binarize_im2col + bgemm on a zero-filled output, dabnn/layers/BinConv.cpp:152-165), without
+ * the column matrix.  x holds c/64 words per pixel, x_ld words from one pixel to the next (x_ld >= c/64: the input may be
+ * a slice of the channels of a wider tensor); wgt is [cout][hwc_words], kh*kw*c/64 words and at most one that pads the
+ * filter to 128 bits (it counts against zeros, as in the column matrix).  out is fp32, out_ld floats from one of the
+ * n*oh*ow pixels to the next.  With a and b (both or neither): out = a[ch]*cnt + b[ch] (+ shortcut, laid out as out), each
+ * operation rounded by itself like the Affine and Add layers; out_packed (cout a multiple of 64, packed_ld words per
+ * pixel) then receives pack_mat of the result.  kh*kw*c must be smaller than 60000, as for dab_fused_binarize_im2col.
+ */
+DAB_API int dab_bconv(const uint64_t *x, int64_t x_ld, int n, int h, int w, int c, const uint64_t *wgt, int hwc_words, int kh,
+                      int kw, int pad_h, int pad_w, int stride_h, int stride_w, int cout, const float *a, const float *b,
+                      const float *shortcut, float *out, int64_t out_ld, uint64_t *out_packed, int64_t packed_ld,
+                      dab_stream_t stream);
+
+/*
  * bconv_3x3 on top of pad (dabnn/bconv.h:855-931 with dabnn/pad.h, i.e. the
  * DIRECT_CONV arm of dabnn/layers/BinConv.cpp:145-150) == baseline_bconv
  * (common/baseline.h:77-116) with a 3x3 kernel: x is the UNPADDED packed
@@ -130,10 +145,9 @@ DAB_API int dab_weight_transpose(const uint64_t *w, int m, int k, uint64_t *wt, 
  * wgt is [cout][9*cin/64] words.  out is fp32 [n][oh][ow][cout] holding the
  * mismatch counts, oh = (h + 2*pad - 3)/stride + 1.
  * Implemented for cin in {64, 128, 256, 512, 1024} (the reference's list,
- * dabnn/layers/BinConv.cpp:118; 1024 as two passes over 512 channels each, the
- * second adding to the first) and cout % 8 == 0; other shapes return
- * DAB_EUNSUPPORTED (use dab_fused_binarize_im2col + dab_bgemm, as the
- * reference's BGEMM arm does).
+ * dabnn/layers/BinConv.cpp:118) and cout % 8 == 0; other shapes return
+ * DAB_EUNSUPPORTED (dab_bconv takes them, and dab_fused_binarize_im2col +
+ * dab_bgemm as in the reference's BGEMM arm).
  */
 DAB_API int dab_bconv3x3(const uint64_t *x, int n, int h, int w, int cin, const uint64_t *wgt, int cout, int stride,
                  int pad, float *out, dab_stream_t stream);
