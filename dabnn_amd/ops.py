@@ -14,6 +14,13 @@ import torch
 from . import capi
 from .capi import check, lib
 
+try:
+    # the per-layer operators from tensors to the C ABI without ctypes (binding/ops_module.cpp)
+    from .lib import _ops_native as _native
+except ImportError as e:
+    raise ImportError("dabnn_amd/lib/_ops_native.so does not load (%s): build it with `make -C dabnn_amd/binding` "
+                      "(or __graft_entry__.build())" % e) from e
+
 
 def _stream():
     return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
@@ -26,6 +33,13 @@ def _ptr(t):
 def _need(t, dtype, name):
     if not (isinstance(t, torch.Tensor) and t.is_cuda and t.dtype == dtype and t.is_contiguous()):
         raise capi.DabError(capi.DAB_EINVAL, "%s must be a contiguous CUDA tensor of %s" % (name, dtype))
+
+
+def _done(r):
+    """The result of a native call; an int is an error code of the C ABI."""
+    if r.__class__ is int:
+        check(r)
+    return r
 
 
 def _empty(shape, dtype, device):
@@ -48,6 +62,9 @@ def col_row_words(kh, kw, c):
 
 def pack_mat(x):
     """pack_mat (dabnn/bitpack.h:277-293): fp32 [..., C] -> int64 [..., C/64]."""
+    r = _native.pack_mat(x)
+    if r is not None:
+        return _done(r)
     _need(x, torch.float32, "x")
     c = x.shape[-1]
     out = _empty(x.shape[:-1] + (max(c // 64, 0),), torch.int64, x.device)
@@ -113,6 +130,9 @@ def weight_transpose(w):
 
 def bgemm(m, n, k, a, lda, b, ldb, c, ldc):
     """bgemm (dabnn/bgemm.h:46-66): column-major C += popcount(A ^ B), in place on c."""
+    r = _native.bgemm(m, n, k, a, lda, b, ldb, c, ldc)
+    if r is not None:
+        return _done(r)
     _need(a, torch.int64, "a")
     _need(b, torch.int64, "b")
     _need(c, torch.float32, "c")
@@ -124,6 +144,9 @@ def bgemm(m, n, k, a, lda, b, ldb, c, ldc):
 
 def bgemm_overwrite(m, n, k, a, lda, b, ldb, c, ldc):
     """fill(0) + bgemm (dabnn/layers/BinConv.cpp:153-165) as one launch: C = popcount(A ^ B), C is not read."""
+    r = _native.bgemm_overwrite(m, n, k, a, lda, b, ldb, c, ldc)
+    if r is not None:
+        return _done(r)
     _need(a, torch.int64, "a")
     _need(b, torch.int64, "b")
     _need(c, torch.float32, "c")
@@ -135,6 +158,9 @@ def bgemm_overwrite(m, n, k, a, lda, b, ldb, c, ldc):
 
 def bconv_3x3(x, weight, stride=1, pad=1):
     """pad + bconv_3x3 (dabnn/bconv.h:855-931): packed [N,H,W,CW], weight int64 [Cout, 9*CW] -> fp32 counts."""
+    r = _native.bconv_3x3(x, weight, stride, pad)
+    if r is not None:
+        return _done(r)
     _need(x, torch.int64, "x")
     _need(weight, torch.int64, "weight")
     n, h, w, cw = x.shape
@@ -149,6 +175,9 @@ def bconv_3x3(x, weight, stride=1, pad=1):
 
 def bconv_3x3_affine_add(x, weight, a, b, shortcut=None, stride=1, pad=1):
     """bconv_3x3, affine_inplace and add_inplace of a residual block in one pass: a*cnt + b (+ shortcut)."""
+    r = _native.bconv_3x3_affine_add(x, weight, a, b, shortcut, stride, pad)
+    if r is not None:
+        return _done(r)
     _need(x, torch.int64, "x")
     _need(weight, torch.int64, "weight")
     _need(a, torch.float32, "a")
@@ -171,6 +200,9 @@ def bconv_3x3_affine_add(x, weight, a, b, shortcut=None, stride=1, pad=1):
 def bconv_3x3_affine_add_sign(x, weight, a, b, shortcut=None, stride=1, pad=1):
     """bconv_3x3_affine_add that also returns pack_mat of its result (the next BinConv's packed input):
     (fp32 [N,OH,OW,Cout], int64 [N,OH,OW,Cout/64])."""
+    r = _native.bconv_3x3_affine_add_sign(x, weight, a, b, shortcut, stride, pad)
+    if r is not None:
+        return _done(r)
     _need(x, torch.int64, "x")
     _need(weight, torch.int64, "weight")
     _need(a, torch.float32, "a")
@@ -234,6 +266,11 @@ class BinConv:
         self._ws = None
 
     def forward(self, x):
+        r = _native.binconv(x, self.weight, self.transposed_weight, self._ws, self.kh, self.kw, self.pad_h, self.pad_w,
+                            self.stride_h, self.stride_w)
+        if r is not None:
+            out, self.method, self._ws = _done(r)
+            return out
         _need(x, torch.float32, "x")
         n, h, w, c = x.shape
         need = lib.dab_binconv_workspace_bytes(n, h, w, c, self.kh, self.kw, self.pad_h, self.pad_w, self.stride_h,
