@@ -53,6 +53,7 @@ SIGNATURES = {
     "dab_bgemm": (_i, [_i, _i, _i, _vp, _i, _vp, _i, _vp, _i, _vp]),
     "dab_bgemm_overwrite": (_i, [_i, _i, _i, _vp, _i, _vp, _i, _vp, _i, _vp]),
     "dab_weight_transpose": (_i, [_vp, _i, _i, _vp, _vp]),
+    "dab_fconv_affine_prelu": (_i, [_vp] + [_i] * 4 + [_vp] * 5 + [_i] * 10 + [_vp, _i64, _vp, _i64, _vp]),
     "dab_bconv": (_i, [_vp, _i64] + [_i] * 4 + [_vp] + [_i] * 8 + [_vp, _vp, _vp, _vp, _i64, _vp, _i64, _vp]),
     "dab_bconv3x3": (_i, [_vp, _i, _i, _i, _i, _vp, _i, _i, _i, _vp, _vp]),
     "dab_bconv3x3_affine_add": (_i, [_vp, _i, _i, _i, _i, _vp, _i, _i, _i, _vp, _vp, _vp, _vp, _vp]),

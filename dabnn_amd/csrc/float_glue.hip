@@ -4,7 +4,7 @@
 
 #include <type_traits>
 
-#include "common.h"
+#include "fp4_core.h"
 
 namespace dab {
 
@@ -52,6 +52,12 @@ struct FconvArgs {
     int K;  // kh*kw*c
     int M;  // n*oh*ow
     int relu;
+    // PRelu in the Relu's place (null: none), and with it the sign bits of the result (null: none), bits_ld dwords per
+    // pixel; out_ld floats from one output pixel to the next
+    const float *slope;
+    int slope_n;
+    uint32_t *bits;
+    int out_ld, bits_ld;
     FastDiv div_ow, div_oh, div_c, div_kw;
 };
 
@@ -96,7 +102,7 @@ __global__ __launch_bounds__(256) void fconv_kernel(const FconvArgs p) {
     const auto x_rsrc = make_rsrc(p.x + (size_t)img0 * img_elems, (uint32_t)(x_left < kOobRow ? x_left : kOobRow));
     const int rows_n = p.cout - n0 < BN ? p.cout - n0 : BN, rows_m = p.M - m0 < BM ? p.M - m0 : BM;
     const auto w_rsrc = make_rsrc(p.w + (size_t)n0 * p.K, (uint32_t)rows_n * p.K * 4u);
-    const auto o_rsrc = make_rsrc(p.out + (size_t)m0 * p.cout, (uint32_t)rows_m * p.cout * 4u);
+    const auto o_rsrc = make_rsrc(p.out + (size_t)m0 * p.out_ld, (uint32_t)((rows_m - 1) * p.out_ld + p.cout) * 4u);
 
     // loader: depth l_k of the slice, tile rows l_r + RP*i
     const int l_k = tid % LK, l_r = tid / LK;
@@ -263,22 +269,40 @@ __global__ __launch_bounds__(256) void fconv_kernel(const FconvArgs p) {
     }
 
     // Epilogue.  The three optional steps are decided once per launch, so the per-element code is straight-line:
-    // (+ bias) (a*v + b, two roundings) (relu) and one store.  An element's byte offset is the lane's own part (its
+    // (+ bias) (a*v + b, two roundings) (relu or prelu) and one store.  An element's byte offset is the lane's own part (its
     // column, its share of the row index) plus a wave-uniform multiple of the row pitch; rows past the last pixel are
     // past the end of the output descriptor and a column past the last channel carries kOob.
-    const uint32_t row_bytes = (uint32_t)p.cout * 4u;
-    auto emit = [&](auto has_bias, auto has_affine, auto has_relu, uint32_t off, float v, float bias, float fa, float fb) {
+    const uint32_t row_bytes = (uint32_t)p.out_ld * 4u;
+    using Prelu = std::integral_constant<int, 2>;
+    auto emit = [&](auto has_bias, auto has_affine, auto act, uint32_t off, float v, float bias, float fa, float fb, float slope) {
 #pragma clang fp contract(off)
         if constexpr (decltype(has_bias)::value) v = v + bias;
         if constexpr (decltype(has_affine)::value) {
             const float prod = fa * v;
             v = prod + fb;
         }
-        if constexpr (decltype(has_relu)::value) v = v < 0.f ? 0.f : v;  // std::max(v, 0.f): a NaN stays
+        if constexpr (std::is_same<decltype(act), Prelu>::value)
+            v = v < 0.f ? v * slope : v;
+        else if constexpr (decltype(act)::value)
+            v = v < 0.f ? 0.f : v;  // std::max(v, 0.f): a NaN stays
         __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), o_rsrc, (int)off, 0, 0);
+        return v;
+    };
+    // The sign bits of a 32 x 32 tile: element e of all lanes is channels 0..31 of two rows, a dword of each, which is
+    // kept in the lane of the row's number until the tile's 32 rows leave in one store.
+    auto keep_signs = [&](uint32_t &rows, auto e_, float v) {
+        constexpr int row = 8 * (decltype(e_)::value / 4) + decltype(e_)::value % 4;
+        const uint64_t mask = __ballot(v > 0.f);
+        rows = dab_writelane((uint32_t)mask, row, rows);
+        rows = dab_writelane((uint32_t)(mask >> 32), row + 4, rows);
+    };
+    auto store_signs = [&](uint32_t rows, int first_row, int first_col, bool mine) {
+        const int pix = m0 + first_row + f_i;
+        if (mine && f_k == 0 && first_col < p.cout && pix < p.M) p.bits[(size_t)pix * p.bits_ld + (first_col >> 5)] = rows;
     };
     // accumulator element e of lane l: row 8*(e/4) + 4*(l/32) + e%4, column l % 32
-    auto emit_all = [&](auto has_bias, auto has_affine, auto has_relu) {
+    auto emit_all = [&](auto has_bias, auto has_affine, auto act) {
+        constexpr bool PRELU = std::is_same<decltype(act), Prelu>::value;
         if constexpr (KSPLIT == 1) {
 #pragma unroll
             for (int j = 0; j < TN; ++j) {
@@ -287,13 +311,20 @@ __global__ __launch_bounds__(256) void fconv_kernel(const FconvArgs p) {
                 const float bias = (decltype(has_bias)::value && co_ok) ? p.bias[co] : 0.f;
                 const float fa = (decltype(has_affine)::value && co_ok) ? p.aff_a[co] : 0.f;
                 const float fb = (decltype(has_affine)::value && co_ok) ? p.aff_b[co] : 0.f;
+                const float slope = (PRELU && co_ok) ? p.slope[p.slope_n == 1 ? 0 : co] : 0.f;
                 const uint32_t lane_off = (co_ok ? (uint32_t)co * 4u : kOob) + (uint32_t)(wm * WTM + 4 * f_k) * row_bytes;
 #pragma unroll
-                for (int i = 0; i < TM; ++i)
-#pragma unroll
-                    for (int e = 0; e < 16; ++e)
-                        emit(has_bias, has_affine, has_relu, lane_off + (uint32_t)(i * 32 + 8 * (e / 4) + (e % 4)) * row_bytes,
-                             acc[i][j][e], bias, fa, fb);
+                for (int i = 0; i < TM; ++i) {
+                    uint32_t signs = 0;
+                    static_for<16>([&](auto e_) {
+                        constexpr int e = decltype(e_)::value;
+                        const float v = emit(has_bias, has_affine, act, lane_off + (uint32_t)(i * 32 + 8 * (e / 4) + (e % 4)) * row_bytes,
+                                             acc[i][j][e], bias, fa, fb, slope);
+                        if constexpr (PRELU) keep_signs(signs, e_, v);
+                    });
+                    if constexpr (PRELU)
+                        if (p.bits) store_signs(signs, wm * WTM + i * 32, n0 + wn * WTN + j * 32, true);
+                }
             }
         } else {
             // one 32 x 32 tile: the waves' partial sums are added in wave order, four accumulator elements per thread
@@ -302,15 +333,20 @@ __global__ __launch_bounds__(256) void fconv_kernel(const FconvArgs p) {
             const float bias = (decltype(has_bias)::value && co_ok) ? p.bias[co] : 0.f;
             const float fa = (decltype(has_affine)::value && co_ok) ? p.aff_a[co] : 0.f;
             const float fb = (decltype(has_affine)::value && co_ok) ? p.aff_b[co] : 0.f;
+            const float slope = (PRELU && co_ok) ? p.slope[p.slope_n == 1 ? 0 : co] : 0.f;
             const uint32_t lane_off = (co_ok ? (uint32_t)co * 4u : kOob) + (uint32_t)(4 * f_k) * row_bytes;
-#pragma unroll
-            for (int q = 0; q < 16 / KSPLIT; ++q) {
+            uint32_t signs = 0;
+            static_for<16 / KSPLIT>([&](auto q_) {
+                constexpr int q = decltype(q_)::value;
                 const int e = wave * (16 / KSPLIT) + q;
                 float v = red[e * 64 + lane];
 #pragma unroll
                 for (int s = 1; s < KSPLIT; ++s) v = __fadd_rn(v, red[(s * 16 + e) * 64 + lane]);
-                emit(has_bias, has_affine, has_relu, lane_off + (uint32_t)(8 * (e / 4) + (e % 4)) * row_bytes, v, bias, fa, fb);
-            }
+                v = emit(has_bias, has_affine, act, lane_off + (uint32_t)(8 * (e / 4) + (e % 4)) * row_bytes, v, bias, fa, fb, slope);
+                if constexpr (PRELU) keep_signs(signs, q_, v);  // a wave's four elements are eight consecutive rows
+            });
+            if constexpr (PRELU)
+                if (p.bits) store_signs(signs, 8 * wave, n0, f_i < 8);
         }
     };
     if constexpr (KSPLIT > 1) {
@@ -320,7 +356,19 @@ __global__ __launch_bounds__(256) void fconv_kernel(const FconvArgs p) {
     }
     using T = std::true_type;
     using F = std::false_type;
-    switch ((p.bias ? 4 : 0) | (p.aff_a ? 2 : 0) | (p.relu ? 1 : 0)) {
+    const int steps = (p.bias ? 4 : 0) | (p.aff_a ? 2 : 0) | (p.relu ? 1 : 0);
+    if constexpr (!POOL) {
+        if (p.slope != nullptr) {
+            switch (steps) {
+                case 0: emit_all(F{}, F{}, Prelu{}); break;
+                case 2: emit_all(F{}, T{}, Prelu{}); break;
+                case 4: emit_all(T{}, F{}, Prelu{}); break;
+                default: emit_all(T{}, T{}, Prelu{}); break;
+            }
+            return;
+        }
+    }
+    switch (steps) {
         case 0: emit_all(F{}, F{}, F{}); break;
         case 1: emit_all(F{}, F{}, T{}); break;
         case 2: emit_all(F{}, T{}, F{}); break;
@@ -820,9 +868,18 @@ static int small_1x1_tiles(int taps, long long M, int cout) {
     return 3;
 }
 
+// PRelu and a result that is a slice of a wider tensor (dab_fconv_affine_prelu)
+struct PreluSlice {
+    const float *slope;
+    int slope_n;
+    int64_t out_ld;
+    uint64_t *packed;
+    int64_t packed_ld;
+};
+
 static int fconv_impl(const char *fn, const float *x, int n, int h, int w, int c, const float *wgt, const float *bias,
                       const float *aff_a, const float *aff_b, int relu, int kh, int kw, int pad_h, int pad_w, int stride_h,
-                      int stride_w, int dil_h, int dil_w, int cout, float *out, dab_stream_t stream) {
+                      int stride_w, int dil_h, int dil_w, int cout, float *out, dab_stream_t stream, const PreluSlice *slice = nullptr) {
     using namespace dab;
     DAB_REQUIRE(x && wgt && out, "%s: null pointer", fn);
     DAB_REQUIRE(n > 0 && h > 0 && w > 0 && c > 0 && kh > 0 && kw > 0 && cout > 0, "%s: non-positive dimension", fn);
@@ -832,6 +889,7 @@ static int fconv_impl(const char *fn, const float *x, int n, int h, int w, int c
     FconvArgs a;
     a.x = x, a.w = wgt, a.bias = bias, a.aff_a = aff_a, a.aff_b = aff_b, a.relu = relu, a.out = out;
     a.pooled = nullptr;
+    a.slope = nullptr, a.slope_n = 0, a.bits = nullptr, a.bits_ld = 0, a.out_ld = cout;
     a.n = n, a.h = h, a.wd = w, a.c = c;
     a.pad_h = pad_h, a.pad_w = pad_w, a.stride_h = stride_h, a.stride_w = stride_w;
     a.oh = out_dim(h, pad_h, kh, dil_h, stride_h), a.ow = out_dim(w, pad_w, kw, dil_w, stride_w);
@@ -851,7 +909,17 @@ static int fconv_impl(const char *fn, const float *x, int n, int h, int w, int c
     const long long span_imgs = 128 / ((long long)a.oh * a.ow) + 2;
     if (span_imgs * h * w * c * 4 >= (1ll << 30) || 128ll * a.K * 4 >= (1ll << 30) || 128ll * cout * 4 >= (1ll << 30))
         return fail(DAB_EUNSUPPORTED, "%s: image, filter or channel count too large for 32-bit tile offsets", fn);
-    {
+    if (slice != nullptr) {
+        DAB_REQUIRE(slice->slope, "%s: null slopes", fn);
+        DAB_REQUIRE(slice->slope_n == 1 || slice->slope_n == cout, "%s: slope must have size 1 or cout (%d), got %d", fn, cout, slice->slope_n);
+        DAB_REQUIRE(slice->out_ld >= cout && (!slice->packed || slice->packed_ld * 64 >= cout), "%s: leading dimension smaller than the row", fn);
+        DAB_REQUIRE((reinterpret_cast<uintptr_t>(slice->packed) & 7) == 0, "%s: misaligned packed output", fn);
+        if (slice->packed && cout % 64 != 0) return fail(DAB_EUNSUPPORTED, "%s: sign bits need cout %% 64 == 0", fn);
+        if (128 * slice->out_ld * 4 >= (1ll << 30) || slice->packed_ld >= (1 << 24))
+            return fail(DAB_EUNSUPPORTED, "%s: leading dimension too large for 32-bit tile offsets", fn);
+        a.slope = slice->slope, a.slope_n = slice->slope_n, a.out_ld = (int)slice->out_ld;
+        a.bits = reinterpret_cast<uint32_t *>(slice->packed), a.bits_ld = (int)(2 * slice->packed_ld);
+    } else {
         const int rc = fconv_c32_try(x, n, h, w, c, wgt, bias, aff_a, aff_b, relu, kh, kw, pad_h, pad_w, stride_h, stride_w,
                                      dil_h, dil_w, cout, a.oh, a.ow, out, s);
         if (rc != 0) return rc < 0 ? rc : DAB_OK;
@@ -875,7 +943,7 @@ static int fconv_impl(const char *fn, const float *x, int n, int h, int w, int c
     const int taps = kh * kw;
     const bool vec4 = c % 4 == 0 && (reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(wgt)) % 16 == 0;
     const bool vec3 = c == 3 && bn == 64 && (taps + 7) / 8 * 24 * 10 <= (a.K + 15) / 16 * 16 * 11;
-    if (M <= 8 && kh == 1 && kw == 1 && pad_h == 0 && pad_w == 0 && stride_h == 1 && stride_w == 1 && vec4 && cout >= 64) {
+    if (slice == nullptr && M <= 8 && kh == 1 && kw == 1 && pad_h == 0 && pad_w == 0 && stride_h == 1 && stride_w == 1 && vec4 && cout >= 64) {
         // a matrix-vector product (the classifier at small batch): one wave per output channel
         hipLaunchKernelGGL(fconv_gemv_kernel, dim3((unsigned)((cout + 3) / 4)), dim3(256), 0, s, a);
     } else if (big_tiles < simd_count() / 4 && vec3 && (M + 63) / 64 >= simd_count() / 8) {
@@ -975,6 +1043,7 @@ extern "C" int dab_ave_pool2_fconv1x1(const float *x, int n, int h, int w, int c
         return fail(DAB_EUNSUPPORTED, "%s: needs c %% 4 == 0 and 16-byte aligned buffers", fn);
     FconvArgs a;
     a.x = x, a.w = wgt, a.bias = bias, a.aff_a = aff_a, a.aff_b = aff_b, a.relu = relu, a.out = out, a.pooled = pooled;
+    a.slope = nullptr, a.slope_n = 0, a.bits = nullptr, a.bits_ld = 0, a.out_ld = cout;
     a.n = n, a.h = h, a.wd = w, a.c = c;
     a.pad_h = 0, a.pad_w = 0, a.stride_h = 2, a.stride_w = 2;  // a pooled pixel's window starts at twice its coordinates
     a.oh = out_dim(h, 0, 2, 1, 2), a.ow = out_dim(w, 0, 2, 1, 2);
@@ -1058,6 +1127,16 @@ extern "C" int dab_fconv_affine_relu(const float *x, int n, int h, int w, int c,
                                      dab_stream_t stream) {
     return fconv_impl("dab_fconv_affine_relu", x, n, h, w, c, wgt, bias, a, b, relu, kh, kw, pad_h, pad_w, stride_h,
                       stride_w, dil_h, dil_w, cout, out, stream);
+}
+
+extern "C" int dab_fconv_affine_prelu(const float *x, int n, int h, int w, int c, const float *wgt, const float *bias,
+                                      const float *a, const float *b, const float *slope, int slope_n, int kh, int kw,
+                                      int pad_h, int pad_w, int stride_h, int stride_w, int dil_h, int dil_w, int cout,
+                                      float *out, int64_t out_ld, uint64_t *out_packed, int64_t packed_ld,
+                                      dab_stream_t stream) {
+    const PreluSlice slice{slope, slope_n, out_ld, out_packed, packed_ld};
+    return fconv_impl("dab_fconv_affine_prelu", x, n, h, w, c, wgt, bias, a, b, 0, kh, kw, pad_h, pad_w, stride_h, stride_w,
+                      dil_h, dil_w, cout, out, stream, &slice);
 }
 
 extern "C" int dab_affine_inplace(float *x, int64_t n_pix, int c, const float *a, const float *b, dab_stream_t stream) {

@@ -78,8 +78,7 @@ BinConv::BinConv(NetCP net, css name, css input, css weight, css output, int pad
 
     const std::string binarized_name = "binaized_for_" + output + "_cal";
     if (!n->has_blob(binarized_name))
-        n->add_mat(binarized_name, std::make_shared<Mat>(input_mat->n, input_mat->h, input_mat->w, input_mat->elem_c,
-                                                         DataType::Bit, binarized_name));
+        n->add_mat(binarized_name, Mat::planned(input_mat->n, input_mat->h, input_mat->w, input_mat->elem_c, DataType::Bit, binarized_name));
     binarized_mat = mat(binarized_name);
     BNN_ASSERT(binarized_mat->data_type == DataType::Bit &&
                    binarized_mat->total() >= (size_t)input_mat->n * input_mat->h * input_mat->w * (input_mat->elem_c / 64),
@@ -126,11 +125,31 @@ bool BinConv::reads_packed() const {
            (long long)weight_mat->total() * 8 < (1ll << 31);
 }
 
+bool BinConv::has_slices() const { return output_mat->ld || binarized_mat->ld || (fused_sign_out && fused_sign_out->ld); }
+
 void BinConv::forward_impl() const {
     void *s = stream();
     const auto *x = static_cast<const float *>(input_mat->dev);
     auto *out = static_cast<float *>(output_mat->dev);
     const int n = input_mat->n, h = input_mat->h, w = input_mat->w, c = input_mat->elem_c;
+    auto convolve_packed = [&](const uint64_t *packed) {
+        auto pixel_words = [](const Mat &m) { return m.ld ? m.ld : m.c; };
+        dab_check(dab_bconv(packed, pixel_words(*binarized_mat), n, h, w, c, static_cast<const uint64_t *>(weight_mat->dev),
+                            (int)(weight_mat->total() / weight_mat->n), kernel_h(), kernel_w(), pad_h, pad_w, stride_h, stride_w,
+                            weight_mat->n, fused_a ? static_cast<const float *>(fused_a->dev) : nullptr,
+                            fused_b ? static_cast<const float *>(fused_b->dev) : nullptr,
+                            fused_shortcut ? static_cast<const float *>(fused_shortcut->dev) : nullptr, out,
+                            output_mat->ld ? output_mat->ld : output_mat->c,
+                            fused_sign_out ? static_cast<uint64_t *>(fused_sign_out->dev) : nullptr,
+                            fused_sign_out ? pixel_words(*fused_sign_out) : 0, s));
+    };
+    if (has_slices()) {
+        auto *packed = static_cast<uint64_t *>(binarized_mat->dev);
+        // (a layer whose packed input is a slice has it from its producers)
+        if (!input_prepacked) dab_check(dab_bitpack_nhwc(x, packed, (int64_t)n * h * w, c, s));
+        convolve_packed(packed);
+        return;
+    }
     switch (method()) {
         case DIRECT_CONV: {
             // pack_mat + (pad +) bconv_3x3, dabnn/layers/BinConv.cpp:146-150
@@ -158,12 +177,7 @@ void BinConv::forward_impl() const {
                 // the column matrix's rows are windows of the packed input: convolved where they lie
                 auto *packed = static_cast<uint64_t *>(binarized_mat->dev);
                 if (!input_prepacked) dab_check(dab_bitpack_nhwc(x, packed, (int64_t)n * h * w, c, s));
-                dab_check(dab_bconv(packed, c / 64, n, h, w, c, static_cast<const uint64_t *>(weight_mat->dev),
-                                    (int)(weight_mat->total() / weight_mat->n), kernel_h(), kernel_w(), pad_h, pad_w, stride_h, stride_w,
-                                    weight_mat->n, fused_a ? static_cast<const float *>(fused_a->dev) : nullptr,
-                                    fused_b ? static_cast<const float *>(fused_b->dev) : nullptr,
-                                    fused_shortcut ? static_cast<const float *>(fused_shortcut->dev) : nullptr, out, output_mat->c,
-                                    fused_sign_out ? static_cast<uint64_t *>(fused_sign_out->dev) : nullptr, (output_mat->c + 63) / 64, s));
+                convolve_packed(packed);
                 break;
             }
             // fill + fused_binarize_im2col + bgemm, dabnn/layers/BinConv.cpp:152-165; the fill and the accumulation
@@ -259,6 +273,18 @@ void FloatConv::forward_impl() const {
             static_cast<float *>(fused_maxpool_carry->dev), stream()));
         return;
     }
+    if (fused_slope) {
+        const Mat &o = *output_mat;
+        dab_check(dab_fconv_affine_prelu(
+            static_cast<const float *>(input_mat->dev), input_mat->n, input_mat->h, input_mat->w, input_mat->c,
+            static_cast<const float *>(weight_mat->dev), bias_mat ? static_cast<const float *>(bias_mat->dev) : nullptr,
+            fused_a ? static_cast<const float *>(fused_a->dev) : nullptr,
+            fused_b ? static_cast<const float *>(fused_b->dev) : nullptr, static_cast<const float *>(fused_slope->dev),
+            (int)fused_slope->total(), weight_mat->h, weight_mat->w, pad_h, pad_w, stride_h, stride_w, dilation, dilation, o.c,
+            static_cast<float *>(o.dev), o.ld ? o.ld : o.c, fused_sign_out ? static_cast<uint64_t *>(fused_sign_out->dev) : nullptr,
+            fused_sign_out ? (fused_sign_out->ld ? fused_sign_out->ld : fused_sign_out->c) : 0, stream()));
+        return;
+    }
     dab_check(dab_fconv_affine_relu(
         static_cast<const float *>(input_mat->dev), input_mat->n, input_mat->h, input_mat->w, input_mat->c,
         static_cast<const float *>(weight_mat->dev), bias_mat ? static_cast<const float *>(bias_mat->dev) : nullptr,
@@ -274,6 +300,8 @@ std::string FloatConv::to_str() const {
        << "x" << weight_mat->h << "x" << weight_mat->w;
     if (fused_a) ss << " + Affine";
     if (fused_relu) ss << " + Relu";
+    if (fused_slope) ss << " + PRelu";
+    if (fused_sign_out) ss << " + Sign";
     if (fused_pool_input)
         ss << ", AvePool " << (fused_pool_global ? "over all" : "2x2") << " of " << fused_pool_input->h << "x" << fused_pool_input->w << " inside";
     if (fused_maxpool_out) ss << " + MaxPool 3x3 stride 2" << (fused_maxpool_sign ? " + Sign" : "");
@@ -316,7 +344,10 @@ PRelu::PRelu(NetCP net, css name, css data, css slope)
                "slope must have size 1 or input.channels");
 }
 
+std::string PRelu::to_str() const { return Layer::to_str() + (inside_conv ? ", applied by the convolution" : ""); }
+
 void PRelu::forward_impl() const {
+    if (inside_conv) return;
     dab_check(dab_prelu_inplace(static_cast<float *>(data_mat->dev), (int64_t)data_mat->n * data_mat->h * data_mat->w,
                                 data_mat->c, static_cast<const float *>(slope_mat->dev), (int)slope_mat->total(), stream()));
 }
@@ -329,7 +360,10 @@ Concat::Concat(NetCP net, css name, css input1, css input2, css output)
     BNN_ASSERT(output_mat->c == input1_mat->c + input2_mat->c, "Concat output does not hold both inputs");
 }
 
+std::string Concat::to_str() const { return Layer::to_str() + (in_place ? ", inputs written in place" : ""); }
+
 void Concat::forward_impl() const {
+    if (in_place) return;
     dab_check(dab_concat_channels(static_cast<const float *>(input1_mat->dev), input1_mat->c,
                                   static_cast<const float *>(input2_mat->dev), input2_mat->c,
                                   (int64_t)input1_mat->n * input1_mat->h * input1_mat->w,

@@ -29,6 +29,9 @@ class BNN_API BinConv : public Layer {
     // is made that way skips its own pack_mat (input_prepacked).
     MatP fused_sign_out;
     bool input_prepacked = false;
+    // The packed input, the output or the packed output is a slice of a wider tensor (Mat::ld): dab_bconv runs, which
+    // takes the distance between pixels, whatever the method.
+    bool has_slices() const;
 
     BinConv(NetCP net, css name, css input, css weight, css output, int pad_h, int pad_w, int stride_h, int stride_w);
     void forward_impl() const override;
@@ -48,6 +51,9 @@ class BNN_API FloatConv : public Layer {
     // Affine (and Relu) layers that follow on the output blob, applied in the convolution's epilogue when set
     MatP fused_a, fused_b;
     bool fused_relu = false;
+    // A PRelu that follows instead of the Relu, and the packed copy of the result for the BinConvs that read it: the
+    // convolution's epilogue makes both, and its output may be a slice of a wider tensor.
+    MatP fused_slope, fused_sign_out;
     // Set by Net::prepare for a 1x1 convolution that reads the output of an AvePool 2x2 stride 2: the pool's input.
     // The layer then pools it itself and convolves the result; the pooled blob (input_mat) is written as a side product
     // when it has device memory, and is a shape without memory when the net dropped the blob.
@@ -94,15 +100,19 @@ class BNN_API Relu : public Layer {
 class BNN_API PRelu : public Layer {
    public:
     MatP data_mat, slope_mat;
+    bool inside_conv = false;  // set by Net::prepare: the float convolution before it applies it
     PRelu(NetCP net, css name, css data, css slope);
     void forward_impl() const override;
+    std::string to_str() const override;
 };
 
 class BNN_API Concat : public Layer {
    public:
     MatP input1_mat, input2_mat, output_mat;
+    bool in_place = false;  // set by Net::prepare: both inputs are slices of the output, written there by their producers
     Concat(NetCP net, css name, css input1, css input2, css output);
     void forward_impl() const override;
+    std::string to_str() const override;
 };
 
 // dabnn/layers/Split.{h,cpp}: a Bit blob's words per pixel cut in two halves (first half -> output 1).

@@ -63,7 +63,37 @@ static hipStream_t copy_stream() {
     return s;
 }
 
+std::shared_ptr<Mat> Mat::planned(int n, int h, int w, int c, DataType type, const std::string &name) {
+    if (type == DataType::Bit && c % 64 != 0)
+        throw std::runtime_error("Bit Mat needs a channel count that is a multiple of 64, got " + std::to_string(c));
+    auto m = std::make_shared<Mat>(n, h, w, c, nullptr, type);
+    m->external_memory = false;
+    m->name = name;
+    return m;
+}
+
+void Mat::allocate() {
+    if (!dev && !external_memory && bytes() > 0) hip_check(hipMalloc(&dev, bytes()), "hipMalloc");
+}
+
+void Mat::become_slice(std::shared_ptr<Mat> whole, int first) {
+    whole->allocate();
+    if (dev && !external_memory) hip_check(hipFree(dev), "hipFree");
+    dev = static_cast<unsigned char *>(whole->dev) + (size_t)first * elemsize;
+    ld = whole->c;
+    external_memory = true;
+    storage = std::move(whole);
+    host_valid_ = false;
+}
+
+void Mat::gather_to(void *dst, void *stream) const {
+    const size_t row = (size_t)c * elemsize, pitch = ld ? (size_t)ld * elemsize : row;
+    hip_check(hipMemcpy2DAsync(dst, row, dev, pitch, row, total() / c, hipMemcpyDeviceToDevice, static_cast<hipStream_t>(stream)),
+              "hipMemcpy2DAsync");
+}
+
 void Mat::upload(const void *host, size_t nbytes) {
+    if (ld) throw std::runtime_error("Mat::upload: the tensor is a slice of another one");
     if (nbytes > bytes()) throw std::runtime_error("Mat::upload: source larger than the tensor");
     hip_check(hipMemcpyAsync(dev, host, nbytes, hipMemcpyHostToDevice, copy_stream()), "hipMemcpyAsync H2D");
     hip_check(hipStreamSynchronize(copy_stream()), "hipStreamSynchronize");
@@ -72,6 +102,18 @@ void Mat::upload(const void *host, size_t nbytes) {
 
 void Mat::download(void *host, size_t nbytes) const {
     if (nbytes > bytes()) throw std::runtime_error("Mat::download: destination larger than the tensor");
+    if (ld) {
+        // whole pixels, and what is left of nbytes from the pixel behind them
+        const size_t row = (size_t)c * elemsize, pitch = (size_t)ld * elemsize, rows = nbytes / row, rest = nbytes - rows * row;
+        if (rows)
+            hip_check(hipMemcpy2DAsync(host, row, dev, pitch, row, rows, hipMemcpyDeviceToHost, copy_stream()), "hipMemcpy2DAsync D2H");
+        if (rest)
+            hip_check(hipMemcpyAsync(static_cast<unsigned char *>(host) + rows * row, static_cast<const unsigned char *>(dev) + rows * pitch, rest,
+                                     hipMemcpyDeviceToHost, copy_stream()),
+                      "hipMemcpyAsync D2H");
+        hip_check(hipStreamSynchronize(copy_stream()), "hipStreamSynchronize");
+        return;
+    }
     hip_check(hipMemcpyAsync(host, dev, nbytes, hipMemcpyDeviceToHost, copy_stream()), "hipMemcpyAsync D2H");
     hip_check(hipStreamSynchronize(copy_stream()), "hipStreamSynchronize");
 }
@@ -102,7 +144,7 @@ void Mat::sync_to_host() const {
 }
 
 bool Mat::operator==(const Mat &m) const {
-    if (this == &m || (dev != nullptr && dev == m.dev)) return true;
+    if (this == &m || (dev != nullptr && dev == m.dev && c == m.c && ld == m.ld)) return true;
     if (!(elemsize == m.elemsize && n == m.n && w == m.w && h == m.h && c == m.c && data_type == m.data_type &&
           total() == m.total()))
         return false;

@@ -39,6 +39,10 @@ class BNN_API Mat {
     mutable void *data = nullptr;  // host mirror (null until the first get_blob / accessor); see sync_to_host()
     void *dev = nullptr;           // device memory
     bool external_memory = false;
+    // Channels of a wider tensor, in place: elements (floats or words) from one pixel to the next, 0 for a tensor of its
+    // own.  The Mats that Net::blob hands out are always contiguous; host accessors and downloads gather.
+    int ld = 0;
+    std::shared_ptr<Mat> storage;  // the wider tensor
     std::string name;
 
     Mat() = default;
@@ -57,6 +61,15 @@ class BNN_API Mat {
     size_t total() const { return data_num_ ? data_num_ : (size_t)n * h * w * c; }
     size_t bytes() const { return total() * elemsize; }
     bool empty() const { return dev == nullptr || total() == 0; }
+
+    // An owning Mat whose device memory is taken later, by allocate(): the net plans its blobs, and which of them share
+    // memory or are never written, before it asks for any.
+    static std::shared_ptr<Mat> planned(int n, int h, int w, int c, DataType type, const std::string &name);
+    void allocate();  // nothing if the memory is there or borrowed
+    // Gives up this Mat's own memory and becomes channels [first, first + c) of `whole` (c and first in elements).
+    void become_slice(std::shared_ptr<Mat> whole, int first);
+    // Copies the device data, contiguous, to device memory `dst`; enqueued on `stream`.
+    void gather_to(void *dst, void *stream) const;
 
     void upload(const void *host, size_t nbytes);
     void download(void *host, size_t nbytes) const;

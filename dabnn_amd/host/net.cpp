@@ -65,6 +65,7 @@ Net::~Net() {
     if (graph_exec_) (void)hipGraphExecDestroy(static_cast<hipGraphExec_t>(graph_exec_));
     if (input_own_dev_ && mat_map_.count(input_name_)) mat_map_[input_name_]->dev = input_own_dev_;  // freed by its Mat
     layers.clear();
+    contiguous_.clear();
     mat_map_.clear();
     if (stream_) (void)hipStreamDestroy(static_cast<hipStream_t>(stream_));
 }
@@ -116,6 +117,19 @@ std::shared_ptr<Mat> Net::get_blob(const std::string &name) {
 }
 
 std::shared_ptr<Mat> Net::blob(const std::string &name) {
+    auto m = stored_blob(name);
+    if (!m->ld) return m;
+    auto it = contiguous_.find(m.get());
+    if (it != contiguous_.end()) return it->second;
+    std::lock_guard<std::mutex> lock(capture_mutex());
+    auto copy = std::make_shared<Mat>(m->n, m->h, m->w, m->elem_c, m->data_type, m->name);
+    m->gather_to(copy->dev, stream_);
+    hip_check(hipStreamSynchronize(static_cast<hipStream_t>(stream_)), "hipStreamSynchronize");
+    contiguous_[m.get()] = copy;
+    return copy;
+}
+
+std::shared_ptr<Mat> Net::stored_blob(const std::string &name) {
     auto it = mat_map_.find(name);
     if (it == mat_map_.end()) {
         auto gone = elided_.find(name);
@@ -170,7 +184,7 @@ void Net::prepare(const void *buf, size_t len) {
     auto new_output = [&](const std::string &name, DataType type = DataType::Float, int images = 0) {
         const auto &s = model.shapes.at(name);
         if (!has_blob(name))
-            add_mat(name, std::make_shared<Mat>(images ? images : batch_, (int)s[1], (int)s[2], (int)s[3], type, name));
+            add_mat(name, Mat::planned(images ? images : batch_, (int)s[1], (int)s[2], (int)s[3], type, name));
     };
     auto alias_output = [&](const std::string &output, const std::string &input) {  // ADD_INPLACE_LAYER
         add_mat(output, blob(input));
@@ -239,7 +253,12 @@ void Net::prepare(const void *buf, size_t len) {
                 throw std::runtime_error(std::string("Not supported op ") + layer_type_name(l.type));
         }
     }
-    if (optimize) fuse_binconv_epilogues();
+    if (optimize) {
+        fuse_binconv_epilogues();
+        fuse_prelu();
+        store_concats_in_place();
+    }
+    allocate_blobs();
     // an in-place layer on the input blob would write into a caller's buffer that is read in place
     copy_input_ = layers_write_input();
     hip_check(hipStreamSynchronize(static_cast<hipStream_t>(stream_)), "hipStreamSynchronize");
@@ -256,7 +275,8 @@ static void layer_io(const std::shared_ptr<Layer> &l, std::vector<const Mat *> &
         reads = {fc->fused_pool_input ? fc->fused_pool_input.get() : fc->input_mat.get()};
         writes = {fc->output_mat ? fc->output_mat.get() : fc->fused_maxpool_out.get()};
         if (fc->fused_maxpool_sign) writes.push_back(fc->fused_maxpool_sign.get());
-        if (fc->fused_pool_input && fc->input_mat->dev) writes.push_back(fc->input_mat.get());  // the pooled blob, a side product
+        if (fc->fused_sign_out) writes.push_back(fc->fused_sign_out.get());
+        if (fc->fused_pool_input && !fc->input_mat->external_memory) writes.push_back(fc->input_mat.get());  // the pooled blob, a side product
     } else if (auto af = std::dynamic_pointer_cast<Affine>(l)) {
         reads = writes = {af->data_mat.get()};
     } else if (auto ad = std::dynamic_pointer_cast<Add>(l)) {
@@ -265,7 +285,7 @@ static void layer_io(const std::shared_ptr<Layer> &l, std::vector<const Mat *> &
     } else if (auto re = std::dynamic_pointer_cast<Relu>(l)) {
         reads = writes = {re->data_mat.get()};
     } else if (auto pr = std::dynamic_pointer_cast<PRelu>(l)) {
-        reads = writes = {pr->data_mat.get()};
+        if (!pr->inside_conv) reads = writes = {pr->data_mat.get()};
     } else if (auto cc = std::dynamic_pointer_cast<Concat>(l)) {
         reads = {cc->input1_mat.get(), cc->input2_mat.get()};
         writes = {cc->output_mat.get()};
@@ -280,6 +300,17 @@ static void layer_io(const std::shared_ptr<Layer> &l, std::vector<const Mat *> &
         writes = {sp->output_mat1.get(), sp->output_mat2.get()};
     } else if (auto sh = std::dynamic_pointer_cast<Shuffle>(l)) {
         reads = writes = {sh->data_mat.get()};
+    }
+}
+
+// Memory for the planned blobs that are left.  A blob whose name a later layer took over is only known to its layers.
+void Net::allocate_blobs() {
+    std::vector<const Mat *> rd, wr;
+    for (const auto &kv : mat_map_) kv.second->allocate();
+    for (const auto &l : layers) {
+        layer_io(l, rd, wr);
+        for (const auto *list : {&rd, &wr})
+            for (const Mat *m : *list) const_cast<Mat *>(m)->allocate();
     }
 }
 
@@ -502,6 +533,118 @@ void Net::fuse_binconv_epilogues() {
     }
 }
 
+// FloatConv (-> Affine) -> PRelu on the convolution's blob: the convolution's epilogue applies the slopes.  Convolutions
+// that already run as one pass with a pool, with a Relu, or on the kernel for 32 input channels (3x3, stride 1), which has
+// no such epilogue, keep the layer.
+void Net::fuse_prelu() {
+    for (size_t i = 0; i + 1 < layers.size(); ++i) {
+        auto fc = std::dynamic_pointer_cast<FloatConv>(layers[i]);
+        auto pr = std::dynamic_pointer_cast<PRelu>(layers[i + 1]);
+        if (!fc || !pr || !fc->output_mat || pr->data_mat != fc->output_mat || fc->fused_relu || fc->fused_pool_input || fc->fused_maxpool_out) continue;
+        if (fc->input_mat->c == 32 && fc->weight_mat->h == 3 && fc->weight_mat->w == 3 && fc->stride_h == 1 && fc->stride_w == 1) continue;
+        if (fc->input_mat == fc->output_mat || (long long)fc->output_mat->n * fc->output_mat->h * fc->output_mat->w <= 8) continue;
+        fc->fused_slope = pr->slope_mat;
+        pr->inside_conv = true;
+    }
+}
+
+// A Concat whose inputs are made for it copies nothing: the inputs become slices of the output, their producers write
+// them there, and the BinConvs that read an input, or the output, read its packed copy as a slice of the output's.  The
+// condition on each input: one producer, a BinConv or FloatConv whose epilogue writes slices and sign bits (or a Concat
+// that is itself stored this way), no layer that rewrites it, and no reader but this Concat and BinConvs; on the output:
+// no layer that rewrites it (its inputs keep their values).  DenseNet blocks nest: features, then the concatenation of
+// features and new channels, are slices of the last concatenation of the block.
+void Net::store_concats_in_place() {
+    using MatP = std::shared_ptr<Mat>;
+    std::vector<const Mat *> rd, wr;
+    std::map<const Mat *, std::shared_ptr<Concat>> parent;  // slice -> the Concat whose output holds it
+    // whether a layer may write `m` as a slice, with its sign bits
+    auto writes_slices = [&](const std::shared_ptr<Layer> &l, const MatP &m) {
+        if (auto cc = std::dynamic_pointer_cast<Concat>(l)) return cc->in_place;
+        if (m->c % 64 != 0 || m->data_type != DataType::Float) return false;
+        if (auto bc = std::dynamic_pointer_cast<BinConv>(l)) return bc->output_mat == m && bc->fused_a && !bc->fused_shortcut && bc->reads_packed();
+        if (auto fc = std::dynamic_pointer_cast<FloatConv>(l)) return fc->output_mat == m && fc->fused_slope != nullptr;
+        return false;
+    };
+    for (const auto &layer : layers) {
+        auto cc = std::dynamic_pointer_cast<Concat>(layer);
+        if (!cc || cc->input1_mat == cc->input2_mat) continue;
+        // offsets of dab_bconv and of the float convolution's tiles: 32 bits over the packed and 2^30 bytes over 128 rows
+        const Mat &whole = *cc->output_mat;
+        bool ok = whole.c % 64 == 0 && whole.c < (1 << 20) && (long long)whole.n * whole.h * whole.w * (whole.c / 64) * 8 < (1ll << 31);
+        for (const MatP &m : {cc->input1_mat, cc->input2_mat, cc->output_mat}) {
+            const bool is_output = m == cc->output_mat;
+            if (m == stored_blob(input_name_) || parent.count(m.get())) ok = false;
+            for (const auto &l : layers) {
+                if (!ok) break;
+                layer_io(l, rd, wr);
+                if (contains(wr, m.get()) && l != layer && (is_output || !writes_slices(l, m))) ok = false;
+                auto bc = std::dynamic_pointer_cast<BinConv>(l);
+                if (bc && bc->input_mat == m && !bc->reads_packed()) ok = false;
+                if (!is_output && bc && bc->fused_shortcut == m) ok = false;
+                if (!is_output && contains(rd, m.get()) && l != layer && !bc) ok = false;
+                if (bc && (bc->input_mat == m || bc->output_mat == m) && (long long)bc->weight_mat->total() * 8 >= (1ll << 31)) ok = false;
+            }
+            if (!is_output && ok) {
+                int writers = 0;
+                for (const auto &l : layers) {
+                    layer_io(l, rd, wr);
+                    writers += contains(wr, m.get());
+                }
+                ok = ok && writers == 1;
+            }
+        }
+        if (!ok) continue;
+        cc->in_place = true;
+        parent[cc->input1_mat.get()] = parent[cc->input2_mat.get()] = cc;
+    }
+    if (parent.empty()) return;
+
+    // the outermost Concat output that holds `m`, and where
+    auto locate = [&](MatP m) {
+        int first = 0;
+        for (auto it = parent.find(m.get()); it != parent.end(); it = parent.find(m.get())) {
+            if (m == it->second->input2_mat) first += it->second->input1_mat->c;
+            m = it->second->output_mat;
+        }
+        return std::make_pair(m, first);
+    };
+    auto held = [&](const MatP &m) {  // in the family of an in-place Concat
+        if (parent.count(m.get())) return true;
+        for (const auto &kv : parent)
+            if (kv.second->output_mat == m) return true;
+        return false;
+    };
+    // packed copies: one for each outermost output that a BinConv reads any part of
+    std::map<const Mat *, MatP> packed;
+    for (const auto &l : layers) {
+        auto bc = std::dynamic_pointer_cast<BinConv>(l);
+        if (!bc || !held(bc->input_mat)) continue;
+        const auto at = locate(bc->input_mat);
+        MatP &bits = packed[at.first.get()];
+        if (!bits) bits = Mat::planned(at.first->n, at.first->h, at.first->w, at.first->c, DataType::Bit, "packed_" + at.first->name);
+        bc->binarized_mat->become_slice(bits, at.second / 64);
+        bc->input_prepacked = true;
+    }
+    for (const auto &l : layers) {
+        auto bc = std::dynamic_pointer_cast<BinConv>(l);
+        auto fc = std::dynamic_pointer_cast<FloatConv>(l);
+        MatP out = bc ? bc->output_mat : fc ? fc->output_mat : nullptr;
+        if (!out || !parent.count(out.get())) continue;
+        const auto at = locate(out);
+        MatP sign;
+        if (packed.count(at.first.get())) {
+            sign = std::make_shared<Mat>(out->n, out->h, out->w, out->c, nullptr, DataType::Bit);
+            sign->become_slice(packed[at.first.get()], at.second / 64);
+        }
+        (bc ? bc->fused_sign_out : fc->fused_sign_out) = sign;
+    }
+    for (const auto &kv : mat_map_) {
+        const auto at = locate(kv.second);
+        if (at.first != kv.second && !kv.second->ld) kv.second->become_slice(at.first, at.second);
+    }
+}
+
 void Net::run(const void *host_input) {
     BNN_ASSERT(prepared_, "run before read");
     BNN_ASSERT(host_input != nullptr, "run: null input");
@@ -571,8 +714,10 @@ void Net::launch_layers() {
     } else {
         for (const auto &layer : layers) layer->forward();
     }
+    for (const auto &kv : contiguous_) kv.first->gather_to(kv.second->dev, s);
     ++runs_;
     hip_check(hipStreamSynchronize(s), "hipStreamSynchronize");
+    for (const auto &kv : contiguous_) kv.second->mark_device_written();
     for (const auto &kv : mat_map_) kv.second->mark_device_written();  // host mirrors show the previous run
 }
 

@@ -41,8 +41,11 @@ class BNN_API Net : public std::enable_shared_from_this<Net> {
     // The blob with its host mirror up to date (dabnn/net.cpp:288-290): `data`, operator[] ... read what the last
     // run left on the device.
     std::shared_ptr<Mat> get_blob(const std::string &name);
-    // The same blob without the device-to-host copy (what the layers and the C ABI use).
+    // The same blob without the device-to-host copy (what the layers and the C ABI use).  A blob that the net keeps as
+    // channels of a wider one comes as a contiguous copy, which every later run brings up to date.
     std::shared_ptr<Mat> blob(const std::string &name);
+    // The blob as the layers hold it, slice or not; Mat::download and the host accessors work on both.
+    std::shared_ptr<Mat> stored_blob(const std::string &name);
     bool has_blob(const std::string &name) const { return mat_map_.count(name) != 0; }
     std::vector<std::string> layer_descriptions() const;
 
@@ -73,6 +76,9 @@ class BNN_API Net : public std::enable_shared_from_this<Net> {
     Net();
     void prepare(const void *model_buf, size_t len);
     void fuse_binconv_epilogues();
+    void fuse_prelu();
+    void allocate_blobs();
+    void store_concats_in_place();
     std::weak_ptr<Net> get_weak() { return shared_from_this(); }
     std::vector<std::shared_ptr<Layer>> layers;
     std::map<std::string, std::vector<uint32_t>> shapes_;  // NHWC with N = 1, as stored in the model
@@ -81,6 +87,7 @@ class BNN_API Net : public std::enable_shared_from_this<Net> {
     int batch_ = 1;
     void *stream_ = nullptr;
     bool prepared_ = false;
+    std::map<const Mat *, std::shared_ptr<Mat>> contiguous_;  // slice -> the copy that blob() handed out
     int runs_ = 0;
     void *graph_exec_ = nullptr;
     void *input_own_dev_ = nullptr;       // the input blob's own allocation

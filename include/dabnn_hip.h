@@ -230,6 +230,18 @@ DAB_API int dab_fconv_affine_relu(const float *x, int n, int h, int w, int c, co
                                   dab_stream_t stream);
 
 /*
+ * dab_fconv_affine_relu with a PRelu (dabnn/layers/PRelu.cpp:6-30, slope_n = 1 or cout slopes) in the Relu's place, whose
+ * result may be a slice of the channels of a wider tensor, for a Concat that then copies nothing: out_ld floats from one
+ * output pixel to the next (at least cout).  out_packed, when not null (cout a multiple of 64, packed_ld words per pixel),
+ * receives pack_mat (dabnn/bitpack.h:277-293) of the result.
+ */
+DAB_API int dab_fconv_affine_prelu(const float *x, int n, int h, int w, int c, const float *wgt, const float *bias,
+                                   const float *a, const float *b, const float *slope, int slope_n, int kh, int kw,
+                                   int pad_h, int pad_w, int stride_h, int stride_w, int dil_h, int dil_w, int cout,
+                                   float *out, int64_t out_ld, uint64_t *out_packed, int64_t packed_ld,
+                                   dab_stream_t stream);
+
+/*
  * AvePool 2x2, stride 2, no padding (ave_pool_fallback, dabnn/layers/AvePool.cpp:84-123) followed by a 1x1 FpConv2D
  * (dabnn/fconv.h:14-76) and the optional Affine and Relu of dab_fconv_affine_relu, in one launch: the shortcut branch
  * of a down-sampling block.  pooled [n][(h-2)/2+1][(w-2)/2+1][c] receives the pooled tensor exactly as dab_ave_pool
