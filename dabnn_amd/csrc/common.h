@@ -42,6 +42,7 @@ bool fconv_c32_takes(int n, int h, int w, int c, int kh, int kw, int pad_h, int 
 int fconv_c32_try(const float *x, int n, int h, int w, int c, const float *wgt, const float *bias, const float *aff_a,
                   const float *aff_b, int relu, int kh, int kw, int pad_h, int pad_w, int stride_h, int stride_w, int dil_h,
                   int dil_w, int cout, int oh, int ow, float *out, hipStream_t s);
+bool fconv_c32_many_items(int n, int oh, int ow);  // whether they come to two per wave of the chip
 bool fconv_c32_pool_takes(int n, int h, int w, int c, int kh, int kw, int pad_h, int pad_w, int stride_h, int stride_w, int dil_h,
                           int dil_w, int cout, int oh, int ow);
 long long fconv_c32_pool_workspace_floats(int n, int oh, int ow, int cout);
@@ -248,6 +249,21 @@ __device__ __forceinline__ void mfma6_16x16x32(f32x4w &acc0, f32x4w &acc1, const
     DAB_MFMA2(mid, hif)
     DAB_MFMA2(hif, mid)
     DAB_MFMA2(hi, hi)
+#undef DAB_MFMA2
+}
+// The same with the five cross terms in sums of their own: the caller adds acc and cross at the end.
+__device__ __forceinline__ void mfma6_16x16x32_two_sums(f32x4w &acc0, f32x4w &acc1, f32x4w &cross0, f32x4w &cross1, const SplitFrag8 &a,
+                                                        const SplitFrag8 &b0, const SplitFrag8 &b1) {
+    auto v = [](SplitFrag8::u4 w) { return __builtin_bit_cast(bf16x8, w); };
+#define DAB_MFMA2(S, A, B)                                                           \
+    S##0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v(a.A), v(b0.B), S##0, 0, 0, 0);  \
+    S##1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v(a.A), v(b1.B), S##1, 0, 0, 0);
+    DAB_MFMA2(cross, lo, hif)
+    DAB_MFMA2(cross, hif, lo)
+    DAB_MFMA2(cross, mid, mid)
+    DAB_MFMA2(acc, hi, hi)
+    DAB_MFMA2(cross, mid, hif)
+    DAB_MFMA2(cross, hif, mid)
 #undef DAB_MFMA2
 }
 

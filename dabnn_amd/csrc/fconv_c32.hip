@@ -46,21 +46,27 @@ constexpr uint32_t kC32Oob = 0x80000000u;  // beyond the descriptor (images here
 // (for its first pooled row) and the output pixel left of it (for its first pooled pixel): every column also writes its
 // last output row to p.brow [n][oh / 4][ow][cout] and its last pixel of each row to p.bcol [n][oh / 4][ow / 16][4][cout],
 // and c32_pool_complete_kernel takes the maxima with those afterwards.  oh must be a multiple of 4.
-template <int NT, int KH, int KW, bool POOL = false>  // NT: 16-channel tiles of the output (cout = 16 * NT)
+//
+// NT: 16-channel tiles of the output that a block makes; NY blocks (blockIdx.y) make the cout = 16 * NT * NY channels.
+// TWO_SUMS: the five cross terms are summed by themselves, 2^-8 of the result and less, and added to the sum of the
+// hi * hi products at the end, so that a result takes 9 roundings at its own size instead of 54.  That form has the
+// registers for it because its blocks make 32 channels at most, which small problems want anyway (more work items).
+template <int NT, int NY, int KH, int KW, bool POOL, bool TWO_SUMS>
 __global__ __launch_bounds__(kC32Threads) void fconv_c32_kernel(const FconvC32Args p) {
-    constexpr int TAPS = KH * KW, PT = kC32PixelTiles, COUT = 16 * NT;
+    constexpr int TAPS = KH * KW, PT = kC32PixelTiles, CH = 16 * NT, COUT = CH * NY;
     constexpr int ROW = TAPS * 32 + 8;     // bf16 elements per output channel in a plane
-    constexpr int PLANE = COUT * ROW;      // elements per plane (hi, mid, lo)
+    constexpr int PLANE = CH * ROW;        // elements per plane (hi, mid, lo)
     __shared__ __attribute__((aligned(16))) uint16_t planes[3 * PLANE];
     __shared__ int filter_special;  // a filter value is an infinity or a NaN
     __shared__ int next_item;       // the first item of the block's range that no wave has taken
     // bias, Affine a and b per output channel (zeros where the layer has none): read from here when an item is written,
     // so that no load is outstanding among the stores -- loads and stores share one counter and complete in no fixed
     // order, and a wait for such a load would also wait for every store before it to be acknowledged
-    __shared__ __attribute__((aligned(16))) float per_channel[3][COUT];
+    __shared__ __attribute__((aligned(16))) float per_channel[3][CH];
 
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int g = lane >> 4, f_i = lane & 15;
+    const int ch0 = NY > 1 ? (int)blockIdx.y * CH : 0;
 
     // A block works through a contiguous range of items, its waves side by side: the image rows above and below the
     // ones it is on were fetched by the block itself a moment ago and are still in its L2 (with the items dealt to all
@@ -70,31 +76,6 @@ __global__ __launch_bounds__(kC32Threads) void fconv_c32_kernel(const FconvC32Ar
     // overlapping with anyone's.
     const int per = p.items / (int)gridDim.x, extra = p.items - per * (int)gridDim.x, b = (int)blockIdx.x;
     const int first = b * per + (b < extra ? b : extra), last = first + per + (b < extra ? 1 : 0);
-    if (tid == 0) filter_special = 0, next_item = first + kC32Threads / 64;
-    if (tid < COUT) {
-        per_channel[0][tid] = p.bias ? p.bias[tid] : 0.f;
-        per_channel[1][tid] = p.aff_a ? p.aff_a[tid] : 0.f;
-        per_channel[2][tid] = p.aff_a ? p.aff_b[tid] : 0.f;
-    }
-    __syncthreads();
-    {
-        bool special = false;
-        // pairs of consecutive depths: one dword per plane
-        for (int idx = tid; idx < COUT * TAPS * 16; idx += kC32Threads) {
-            const int co = idx / (TAPS * 16), r = idx - co * (TAPS * 16);  // r: pair index in the channel's 288 depths
-            const float2 v = *reinterpret_cast<const float2 *>(p.w + (size_t)co * (TAPS * 32) + 2 * r);
-            const SplitParts s0 = split_bf16x3(v.x), s1 = split_bf16x3(v.y);
-            special |= s0.hif != s0.hi || s1.hif != s1.hi;
-            uint32_t *d = reinterpret_cast<uint32_t *>(planes + co * ROW + 2 * r);
-            d[0] = pack_upper_halves(s0.hi, s1.hi);
-            d[PLANE / 2] = pack_upper_halves(s0.mid, s1.mid);
-            d[2 * (PLANE / 2)] = pack_upper_halves(s0.lo, s1.lo);
-        }
-        if (special) filter_special = 1;
-    }
-    __syncthreads();
-    const bool w_special = __builtin_amdgcn_readfirstlane(filter_special) != 0;
-
     const __amdgpu_buffer_rsrc_t x_rsrc = make_rsrc(p.x, p.x_bytes);
     typedef float f32x4r __attribute__((ext_vector_type(4)));
     typedef SplitFrag8::u4 u4;
@@ -155,7 +136,33 @@ __global__ __launch_bounds__(kC32Threads) void fconv_c32_kernel(const FconvC32Ar
     for (int j = 0; j < ROWS; ++j) fetch(here, first + wave < last, j, 1, raw[j]);
     fetch_halo(here, first + wave < last, raw_halo);
 
-    f32x4w acc[PT][NT];
+    // the filters, while the first rows are on their way
+    if (tid == 0) filter_special = 0, next_item = first + kC32Threads / 64;
+    if (tid < CH) {
+        per_channel[0][tid] = p.bias ? p.bias[ch0 + tid] : 0.f;
+        per_channel[1][tid] = p.aff_a ? p.aff_a[ch0 + tid] : 0.f;
+        per_channel[2][tid] = p.aff_a ? p.aff_b[ch0 + tid] : 0.f;
+    }
+    __syncthreads();
+    {
+        bool special = false;
+        // pairs of consecutive depths: one dword per plane
+        for (int idx = tid; idx < CH * TAPS * 16; idx += kC32Threads) {
+            const int co = idx / (TAPS * 16), r = idx - co * (TAPS * 16);  // r: pair index in the channel's 288 depths
+            const float2 v = *reinterpret_cast<const float2 *>(p.w + (size_t)(ch0 + co) * (TAPS * 32) + 2 * r);
+            const SplitParts s0 = split_bf16x3(v.x), s1 = split_bf16x3(v.y);
+            special |= s0.hif != s0.hi || s1.hif != s1.hi;
+            uint32_t *d = reinterpret_cast<uint32_t *>(planes + co * ROW + 2 * r);
+            d[0] = pack_upper_halves(s0.hi, s1.hi);
+            d[PLANE / 2] = pack_upper_halves(s0.mid, s1.mid);
+            d[2 * (PLANE / 2)] = pack_upper_halves(s0.lo, s1.lo);
+        }
+        if (special) filter_special = 1;
+    }
+    __syncthreads();
+    const bool w_special = __builtin_amdgcn_readfirstlane(filter_special) != 0;
+
+    f32x4w acc[PT][NT], cross[TWO_SUMS ? PT : 1][TWO_SUMS ? NT : 1];
     // max_pool's step, `v > m ? v : m` from -FLT_MAX on, as the hardware's maximum: a NaN is passed over either way (the
     // running maximum never is one); where +0 and -0 tie the hardware gives +0 and max_pool the earlier tap, which no
     // comparison and no sign bit of the result can tell apart
@@ -194,12 +201,18 @@ __global__ __launch_bounds__(kC32Threads) void fconv_c32_kernel(const FconvC32Ar
             out[e] = (f_i & 1) ? second : h[0][e];
         }
         const size_t cell = ((size_t)at.img * (p.oh >> 1) + (at.oy0 >> 1) + (f_i & 1)) * (p.ow >> 1) + at.xt * 8 + (f_i >> 1);
-        *reinterpret_cast<float4 *>(p.out + cell * COUT + nt * 16 + 4 * g_now) = make_float4(out[0], out[1], out[2], out[3]);
+        *reinterpret_cast<float4 *>(p.out + cell * COUT + ch0 + nt * 16 + 4 * g_now) = make_float4(out[0], out[1], out[2], out[3]);
     };
     // Writes the item at `at`, whose sums are in acc (special: an infinity or a NaN among its pixels or in the filters).
     auto write_item = [&](const Place &at, bool special) __attribute__((always_inline)) {
         int g_now = g;
         asm volatile("" : "+v"(g_now));  // what follows is read per item: hoisted out of the item loop it would be spilled
+        if constexpr (TWO_SUMS) {
+#pragma unroll
+            for (int t = 0; t < PT; ++t)
+#pragma unroll
+                for (int nt = 0; nt < NT; ++nt) acc[t][nt] = acc[t][nt] + cross[t][nt];
+        }
         if (!special) {
             float bs[NT][4], as[NT][4], bb[NT][4];
 #pragma unroll
@@ -255,7 +268,7 @@ __global__ __launch_bounds__(kC32Threads) void fconv_c32_kernel(const FconvC32Ar
                     }
                     pool_store(at, nt, g_now, v0, v1);
                     // the last row as it is; the last pixel of the four rows gathered into lanes 12..15 of each group
-                    float *row = p.brow + ((((size_t)at.img * p.row_groups + (at.oy0 >> 2)) * p.ow + at.xt * 16 + f_i) * COUT + nt * 16 + 4 * g_now);
+                    float *row = p.brow + ((((size_t)at.img * p.row_groups + (at.oy0 >> 2)) * p.ow + at.xt * 16 + f_i) * COUT + ch0 + nt * 16 + 4 * g_now);
                     *reinterpret_cast<float4 *>(row) = make_float4(acc[3][nt][0], acc[3][nt][1], acc[3][nt][2], acc[3][nt][3]);
                     float w[4];
 #pragma unroll
@@ -266,7 +279,7 @@ __global__ __launch_bounds__(kC32Threads) void fconv_c32_kernel(const FconvC32Ar
                         w[e] = f_i == 15 ? acc[3][nt][e] : __int_as_float(f_i == 14 ? r2 : f_i == 13 ? r1 : r0);
                     }
                     if (f_i >= 12) {
-                        float *col = p.bcol + (((((size_t)at.img * p.row_groups + (at.oy0 >> 2)) * p.tiles_per_row + at.xt) * 4 + (f_i - 12)) * COUT + nt * 16 + 4 * g_now);
+                        float *col = p.bcol + (((((size_t)at.img * p.row_groups + (at.oy0 >> 2)) * p.tiles_per_row + at.xt) * 4 + (f_i - 12)) * COUT + ch0 + nt * 16 + 4 * g_now);
                         *reinterpret_cast<float4 *>(col) = make_float4(w[0], w[1], w[2], w[3]);
                     }
                 }
@@ -279,7 +292,7 @@ __global__ __launch_bounds__(kC32Threads) void fconv_c32_kernel(const FconvC32Ar
                 const size_t m = ((size_t)at.img * p.oh + at.oy0 + t) * p.ow + at.xt * 16 + f_i;
 #pragma unroll
                 for (int nt = 0; nt < NT; ++nt)
-                    *reinterpret_cast<float4 *>(p.out + m * COUT + 4 * g_now + nt * 16) =
+                    *reinterpret_cast<float4 *>(p.out + m * COUT + ch0 + 4 * g_now + nt * 16) =
                         make_float4(acc[t][nt][0], acc[t][nt][1], acc[t][nt][2], acc[t][nt][3]);
             }
             }
@@ -297,7 +310,7 @@ __global__ __launch_bounds__(kC32Threads) void fconv_c32_kernel(const FconvC32Ar
 #pragma unroll 1
                 for (int t = 0; t < PT; ++t) {
                     if (at.oy0 + t >= p.oh) break;
-                    f32x4w one = f32x4w{0.f, 0.f, 0.f, 0.f}, none = one;
+                    f32x4w one = f32x4w{0.f, 0.f, 0.f, 0.f}, none = one, one_cross = one, none_cross = one;
 #pragma unroll 1
                     for (int tap = 0; tap < TAPS; ++tap) {
                         const int ty = tap / KW, tx = tap - ty * KW;
@@ -311,8 +324,12 @@ __global__ __launch_bounds__(kC32Threads) void fconv_c32_kernel(const FconvC32Ar
                         f.lo = *reinterpret_cast<const u4 *>(src + 2 * PLANE);
 #pragma unroll
                         for (int e = 0; e < 4; ++e) f.hif[e] = finite_bf16_pair(f.hi[e]);
-                        mfma6_16x16x32(one, none, f, px, px);
+                        if constexpr (TWO_SUMS)
+                            mfma6_16x16x32_two_sums(one, none, one_cross, none_cross, f, px, px);
+                        else
+                            mfma6_16x16x32(one, none, f, px, px);
                     }
+                    if constexpr (TWO_SUMS) one = one + one_cross;
                     const float4 fin = make_float4(finish(one[0], bias.x, fa.x, fb.x), finish(one[1], bias.y, fa.y, fb.y),
                                                    finish(one[2], bias.z, fa.z, fb.z), finish(one[3], bias.w, fa.w, fb.w));
                     if constexpr (POOL) {
@@ -323,11 +340,11 @@ __global__ __launch_bounds__(kC32Threads) void fconv_c32_kernel(const FconvC32Ar
                             if (t >= 1) v1[e] = later_max(v1[e], fv[e]);
                         }
                         const size_t group = (size_t)at.img * p.row_groups + (at.oy0 >> 2);
-                        if (t == PT - 1) *reinterpret_cast<float4 *>(p.brow + ((group * p.ow + at.xt * 16 + f_i) * COUT + co)) = fin;
-                        if (f_i == 15) *reinterpret_cast<float4 *>(p.bcol + (((group * p.tiles_per_row + at.xt) * 4 + t) * COUT + co)) = fin;
+                        if (t == PT - 1) *reinterpret_cast<float4 *>(p.brow + ((group * p.ow + at.xt * 16 + f_i) * COUT + ch0 + co)) = fin;
+                        if (f_i == 15) *reinterpret_cast<float4 *>(p.bcol + (((group * p.tiles_per_row + at.xt) * 4 + t) * COUT + ch0 + co)) = fin;
                     } else {
                         const size_t m = ((size_t)at.img * p.oh + at.oy0 + t) * p.ow + at.xt * 16 + f_i;
-                        *reinterpret_cast<float4 *>(p.out + m * COUT + co) = fin;
+                        *reinterpret_cast<float4 *>(p.out + m * COUT + ch0 + co) = fin;
                     }
                 }
                 if constexpr (POOL) pool_store(at, nt, g_now, v0, v1);
@@ -373,7 +390,10 @@ __global__ __launch_bounds__(kC32Threads) void fconv_c32_kernel(const FconvC32Ar
 #pragma unroll
         for (int t = 0; t < PT; ++t)
 #pragma unroll
-            for (int nt = 0; nt < NT; ++nt) acc[t][nt] = f32x4w{0.f, 0.f, 0.f, 0.f};
+            for (int nt = 0; nt < NT; ++nt) {
+                acc[t][nt] = f32x4w{0.f, 0.f, 0.f, 0.f};
+                if constexpr (TWO_SUMS) cross[t][nt] = acc[t][nt];
+            }
 
         // input row j as horizontal tap TX sees it
         auto shifted = [&](auto tx_c, auto j_c) __attribute__((always_inline)) {
@@ -420,8 +440,13 @@ __global__ __launch_bounds__(kC32Threads) void fconv_c32_kernel(const FconvC32Ar
                     const uint16_t *src = filter_at(nt, ty, TX);
                     const SplitFrag8 f = frag(*reinterpret_cast<const u4 *>(src), *reinterpret_cast<const u4 *>(src + PLANE),
                                               *reinterpret_cast<const u4 *>(src + 2 * PLANE));
-                    mfma6_16x16x32(acc[0][nt], acc[1][nt], f, of_row(a), of_row(b));
-                    mfma6_16x16x32(acc[2][nt], acc[3][nt], f, of_row(c), of_row(d));
+                    if constexpr (TWO_SUMS) {
+                        mfma6_16x16x32_two_sums(acc[0][nt], acc[1][nt], cross[0][nt], cross[1][nt], f, of_row(a), of_row(b));
+                        mfma6_16x16x32_two_sums(acc[2][nt], acc[3][nt], cross[2][nt], cross[3][nt], f, of_row(c), of_row(d));
+                    } else {
+                        mfma6_16x16x32(acc[0][nt], acc[1][nt], f, of_row(a), of_row(b));
+                        mfma6_16x16x32(acc[2][nt], acc[3][nt], f, of_row(c), of_row(d));
+                    }
                 }
                 __builtin_amdgcn_sched_barrier(0);  // rows and filter fragments are made as they are needed, not up front
             };
@@ -507,7 +532,7 @@ __global__ __launch_bounds__(256) void c32_pool_complete_kernel(const C32PoolCom
     }
 }
 
-// Whether the shapes are this kernel's and the problem is large enough to fill its persistent waves (buffer alignment
+// Whether the shapes are this kernel's and the problem is large enough for it (buffer alignment
 // aside, which only the call itself can check).
 bool fconv_c32_takes(int n, int h, int w, int c, int kh, int kw, int pad_h, int pad_w, int stride_h, int stride_w, int dil_h,
                      int dil_w, int cout, int oh, int ow) {
@@ -515,9 +540,38 @@ bool fconv_c32_takes(int n, int h, int w, int c, int kh, int kw, int pad_h, int 
     if ((cout != 32 && cout != 64) || oh <= 0 || ow <= 0 || ow % 16 != 0 || pad_h > 2 || pad_w > 2) return false;
     const long long in_bytes = (long long)n * h * w * 128, tiles = (long long)n * oh * ow / 16;
     if (in_bytes >= (1ll << 31) || tiles >= (1ll << 30)) return false;
-    const long long waves = (long long)(simd_count() / 4) * (kC32Threads / 64);
-    // smaller problems: the general kernel's tiles fill the chip better
-    return (long long)n * ((oh + kC32PixelTiles - 1) / kC32PixelTiles) * (ow / 16) >= 2 * waves;
+    // One image of 48 x 48 is 36 items: 8.9 us against the general kernel's 8.7; everything smaller is left to that.
+    return 8 * (long long)n * ((oh + kC32PixelTiles - 1) / kC32PixelTiles) * (ow / 16) >= simd_count() / 4;
+}
+
+bool fconv_c32_many_items(int n, int oh, int ow) {
+    return (long long)n * ((oh + kC32PixelTiles - 1) / kC32PixelTiles) * (ow / 16) >= 2ll * (simd_count() / 4) * (kC32Threads / 64);
+}
+
+// From two items per wave of the chip on, a block makes all channels: every pixel is split once.  With fewer, the
+// channels go over several blocks -- more items to share out, fewer filters to split first -- and the sums are two.
+// 112 x 112 images, + Affine + Relu (+ MaxPool), the fp32 kernels before / two sums: 32 channels, 1 image 11.6 / 9.1 us
+// (17.1 / 12.7), 6 images 23.1 / 15.6 (29.1 / 20.9), 20 images 49 / 31 (61 / 37); 64 channels, 1 image 11.8 / 9.9
+// (16.9 / 13.8), 6 images 36.1 / 22.7 (44.8 / 30.1), 20 images 83 / 48 (102 / 59).  Blocks of 16 against 32 of the 64
+// channels: 25.4 / 24.8 at 4 images, 35.8 / 38.1 at 8, 44.4 / 42.4 at 12, 62 / 59 at 20: the line is at one item per wave.
+// Distance from 64-bit sums, relative: 8.3e-8, the fp32 kernels 2.2e-7 and one sum 2.4e-7.
+template <bool POOL>
+static int launch_c32(const FconvC32Args &a, hipStream_t s, const char *what) {
+    const int cus = simd_count() / 4;  // one block of eight waves per CU (the filter planes of 64 channels take most of its LDS)
+    const int waves = cus * (kC32Threads / 64);
+    const dim3 threads(kC32Threads);
+    auto grid = [&](int ny) { return dim3(a.items < cus / ny ? a.items : cus / ny, ny); };
+    if (a.items < 2 * waves && a.cout == 32)
+        hipLaunchKernelGGL((fconv_c32_kernel<1, 2, 3, 3, POOL, true>), grid(2), threads, 0, s, a);
+    else if (a.items < waves)
+        hipLaunchKernelGGL((fconv_c32_kernel<1, 4, 3, 3, POOL, true>), grid(4), threads, 0, s, a);
+    else if (a.items < 2 * waves)
+        hipLaunchKernelGGL((fconv_c32_kernel<2, 2, 3, 3, POOL, true>), grid(2), threads, 0, s, a);
+    else if (a.cout == 32)
+        hipLaunchKernelGGL((fconv_c32_kernel<2, 1, 3, 3, POOL, false>), dim3(cus), threads, 0, s, a);
+    else
+        hipLaunchKernelGGL((fconv_c32_kernel<4, 1, 3, 3, POOL, false>), dim3(cus), threads, 0, s, a);
+    return hipGetLastError() == hipSuccess ? 1 : fail(DAB_EHIP, "%s: launch failed", what);
 }
 
 // Runs the convolution if fconv_c32_takes says so and the buffers are 16-byte aligned; returns 1 when it did, 0 when
@@ -530,7 +584,6 @@ int fconv_c32_try(const float *x, int n, int h, int w, int c, const float *wgt, 
     if (bias) align |= reinterpret_cast<uintptr_t>(bias);
     if (aff_a) align |= reinterpret_cast<uintptr_t>(aff_a) | reinterpret_cast<uintptr_t>(aff_b);
     if (align % 16 != 0) return 0;
-    const int blocks = simd_count() / 4;  // one block of eight waves per CU (the filter planes take most of its LDS)
     FconvC32Args a;
     a.x = x, a.w = wgt, a.bias = bias, a.aff_a = aff_a, a.aff_b = aff_b, a.out = out, a.relu = relu;
     a.brow = nullptr, a.bcol = nullptr, a.bits = nullptr;
@@ -539,11 +592,7 @@ int fconv_c32_try(const float *x, int n, int h, int w, int c, const float *wgt, 
     a.row_groups = (oh + kC32PixelTiles - 1) / kC32PixelTiles, a.tiles_per_row = ow / 16;
     a.items = n * a.row_groups * a.tiles_per_row;
     a.div_tiles_per_row = FastDiv((uint32_t)a.tiles_per_row), a.div_row_groups = FastDiv((uint32_t)a.row_groups);
-    if (cout == 32)
-        hipLaunchKernelGGL((fconv_c32_kernel<2, 3, 3>), dim3(blocks), dim3(kC32Threads), 0, s, a);
-    else
-        hipLaunchKernelGGL((fconv_c32_kernel<4, 3, 3>), dim3(blocks), dim3(kC32Threads), 0, s, a);
-    return hipGetLastError() == hipSuccess ? 1 : fail(DAB_EHIP, "fconv_c32: launch failed");
+    return launch_c32<false>(a, s, "fconv_c32");
 }
 
 // The convolution with the MaxPool 3x3, stride 2, pad 1 behind it (fconv_c32_kernel<..., POOL> and the completing pass):
@@ -567,7 +616,6 @@ int fconv_c32_pool_run(const float *x, int n, int h, int w, const float *wgt, co
     if (bias) align |= reinterpret_cast<uintptr_t>(bias);
     if (aff_a) align |= reinterpret_cast<uintptr_t>(aff_a) | reinterpret_cast<uintptr_t>(aff_b);
     if (align % 16 != 0) return 0;
-    const int blocks = simd_count() / 4;
     FconvC32Args a;
     a.x = x, a.w = wgt, a.bias = bias, a.aff_a = aff_a, a.aff_b = aff_b, a.out = pooled, a.relu = relu;
     a.brow = work, a.bcol = work + (size_t)n * (oh / 4) * ow * cout, a.bits = nullptr;
@@ -576,11 +624,8 @@ int fconv_c32_pool_run(const float *x, int n, int h, int w, const float *wgt, co
     a.row_groups = oh / kC32PixelTiles, a.tiles_per_row = ow / 16;
     a.items = n * a.row_groups * a.tiles_per_row;
     a.div_tiles_per_row = FastDiv((uint32_t)a.tiles_per_row), a.div_row_groups = FastDiv((uint32_t)a.row_groups);
-    if (cout == 32)
-        hipLaunchKernelGGL((fconv_c32_kernel<2, 3, 3, true>), dim3(blocks), dim3(kC32Threads), 0, s, a);
-    else
-        hipLaunchKernelGGL((fconv_c32_kernel<4, 3, 3, true>), dim3(blocks), dim3(kC32Threads), 0, s, a);
-    if (hipGetLastError() != hipSuccess) return fail(DAB_EHIP, "fconv_c32 (pooled): launch failed");
+    const int rc = launch_c32<true>(a, s, "fconv_c32 (pooled)");
+    if (rc < 0) return rc;
     C32PoolCompleteArgs f;
     f.pooled = reinterpret_cast<float4 *>(pooled), f.brow = reinterpret_cast<const float4 *>(a.brow);
     f.bcol = reinterpret_cast<const float4 *>(a.bcol), f.bits = pooled_packed;
