@@ -1,6 +1,8 @@
 """The direct 3x3 binary convolution at the sizes where its kernels and the rule that picks one of them can go wrong:
 tiles that are not full in pixels or channels, both sides of every switch, windows that fit no kernel but the last one,
 and operands whose bits are all equal (the largest and the smallest count).  Counts are whole numbers: bit for bit."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -64,3 +66,28 @@ def test_bconv_at_the_edges_of_its_kernels(n, h, w, cin, cout, stride, pad, bits
     if cout % 64 == 0:
         fused, packed = dab.bconv_3x3_affine_add_sign(dev(x), dev(wgt), dev(a), dev(b), dev(shortcut), stride, pad)
         assert torch.equal(fused, sep) and torch.equal(packed, dab.pack_mat(sep))
+
+
+# The last tile of a walking kernel is ragged: its rows past the tensor, and channels past the last, are stored nowhere.
+@pytest.mark.parametrize("n,h,w,cin,cout", [(13, 57, 33, 64, 56), (67, 41, 35, 64, 72), (30, 27, 31, 128, 328), (25, 21, 31, 512, 136),
+                                            (11, 27, 29, 256, 320), (1, 1, 1, 64, 8)])
+def test_bconv_stores_nothing_past_its_output(n, h, w, cin, cout):
+    import dabnn_amd as dab
+    from dabnn_amd import capi
+    r = np.random.default_rng(cin + cout)
+    x = dev(r.integers(0, 2**64, size=(n, h, w, cin // 64), dtype=np.uint64))
+    wgt = dev(r.integers(0, 2**64, size=(cout, 9 * cin // 64), dtype=np.uint64))
+    a, b = dev(r.standard_normal(cout).astype(np.float32)), dev(r.standard_normal(cout).astype(np.float32))
+    size, guard = n * h * w * cout, 64 * cout  # a tile reaches 64 pixels at most
+    ptr = lambda t, at=0: ctypes.c_void_p(t.data_ptr() + at)
+    for fused in (False, True):
+        buf = torch.full((guard + size + guard,), -7.0, device="cuda")
+        if fused:
+            want = dab.bconv_3x3_affine_add(x, wgt, a, b, None, 1, 1)
+            capi.check(capi.lib.dab_bconv3x3_affine_add(ptr(x), n, h, w, cin, ptr(wgt), cout, 1, 1, ptr(a), ptr(b), None, ptr(buf, 4 * guard), None))
+        else:
+            want = dab.bconv_3x3(x, wgt, 1, 1)
+            capi.check(capi.lib.dab_bconv3x3(ptr(x), n, h, w, cin, ptr(wgt), cout, 1, 1, ptr(buf, 4 * guard), None))
+        torch.cuda.synchronize()
+        assert torch.equal(buf[guard:guard + size], want.reshape(-1))
+        assert bool((buf[:guard] == -7).all()) and bool((buf[guard + size:] == -7).all())
