@@ -983,9 +983,14 @@ static int fconv_impl(const char *fn, const float *x, int n, int h, int w, int c
         // a three-channel image too small for 128-pixel tiles (the stem at batch 1): 64-pixel tiles keep the
         // one-load-per-tap loader and still give most CUs a block
         DAB_FCONV_LAUNCH(64, 64, 24, 1, 3);
-    } else if (big_tiles < simd_count() / 4 && vec4 && small_1x1_tiles(kh * kw, M, cout) == 1) {
-        DAB_FCONV_LAUNCH(64, 128, 32, 1, 4);
-    } else if (big_tiles < simd_count() / 4 && vec4 && small_1x1_tiles(kh * kw, M, cout) == 2) {
+    } else if (vec4 && taps == 1 && cout > 64 && ((M + 63) / 64) * ((cout + 63) / 64) >= 3ll * simd_count() / 16 &&
+               (a.K <= 512 || big_tiles < simd_count())) {
+        // 1x1 from three quarters of the CUs on: 64 x 64 tiles in 32-deep slices.  Four blocks of a CU cover each other's
+        // loads, and the last round of blocks is a shorter one than with 128 x 128 tiles in 16-deep slices (16 x 16 x 256 ->
+        // 128, 128 images: 22.1 us against 25.4; x 192 -> 192: 28.4 against 32.9; 14 x 14 x 512 -> 256, 256 images: 116
+        // against 132) or with 64 x 128 tiles (14 x 14 x 256 -> 512, 64 images: 34.5 against 40.0).  Deep and large
+        // problems stay with the larger tile, which reads the operands half as often (16 x 16 x 1024 -> 256, 256 images:
+        // 290 us against 277, 128 images 140 either way).
         DAB_FCONV_LAUNCH(64, 64, 32, 1, 4);
     } else if (big_tiles < simd_count() / 4 && vec4 && small_1x1_tiles(kh * kw, M, cout) == 3) {
         DAB_FCONV_LAUNCH(32, 32, 64, 4, 4);
