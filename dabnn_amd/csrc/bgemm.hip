@@ -111,7 +111,7 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t tile_rsrc(const float *t, cons
 enum Epilogue { kStoreCounts, kAddCounts, kAffine, kAffineSign };
 
 // Few tiles, or a depth that does not fit LDS as filters: a block is one tile of 32 pixels x 32 * NT channels, its four
-// waves take every fourth unit of the depth each and load their operands straight from memory, five units at a time; the
+// waves take every fourth unit of the depth each and load their operands straight from memory, kUnitsAhead units at a time; the
 // partial sums meet in LDS.  Both operands +-1 (fp4_core.h).  m512 k72 n3136, accumulating: 7.8 us against 16.2 for the
 // xor/popcount kernel before.
 constexpr int kUnitsAhead = 3;
