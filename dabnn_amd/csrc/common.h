@@ -88,10 +88,7 @@ struct FastDiv {
 // ---------------------------------------------------------------- blocks and XCDs
 // The blocks of a launch are dealt to the eight XCDs in turn (block b runs on XCD b % 8) and every XCD has an L2 of
 // its own.  This renumbering gives every XCD a contiguous range of numbers, so that blocks whose work is adjacent
-// (neighbouring runs of rows of an image) read the same lines through the same L2.  Not for the xor/popcount kernels:
-// their waves' ranges, renumbered this way, took 4-25 % longer per launch (every XCD then walks all filters for an
-// eighth of the pixels, and the remainder units land on one XCD unless they are spread, which breaks whole staging
-// windows apart).
+// (neighbouring runs of rows of an image) read the same lines through the same L2.
 __device__ __forceinline__ uint32_t xcd_contiguous_block(uint32_t b, uint32_t grid) {
     const uint32_t q = grid >> 3, r = grid & 7u, x = b & 7u;
     return x * q + (x < r ? x : r) + (b >> 3);
@@ -271,8 +268,6 @@ __device__ __forceinline__ void mfma6_16x16x32_two_sums(f32x4w &acc0, f32x4w &ac
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x3 __attribute__((ext_vector_type(3)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x8 __attribute__((ext_vector_type(8)));
-typedef uint32_t u32x16 __attribute__((ext_vector_type(16)));
 
 // Raw buffer descriptor over [p, p + bytes): loads with an offset at or beyond
 // `bytes` return zero, which is how out-of-image taps read a zero word.
