@@ -1,0 +1,91 @@
+"""3x3 convolutions over 32 channels with two work items and more per wave, on f16 parts: pixels and filters of any magnitude (each
+item of 16 x 4 pixels and each filter has a power of two of its own), values too far below the largest for the parts, infinities
+and NaN; with and without the MaxPool; against 64-bit sums."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+import dabnn_amd as dab
+
+pytestmark = pytest.mark.gpu
+N = 22  # 112 x 112: 4312 items on 2048 waves
+
+
+def inputs(cout, seed):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    return torch.randn(N, 112, 112, 32, device="cuda", generator=g).relu_(), torch.randn(cout, 3, 3, 32, device="cuda", generator=g) / 17
+
+
+def reference(x, w, pooled):
+    wt, xt = w.double().cpu().permute(0, 3, 1, 2), x.double().cpu().permute(0, 3, 1, 2)
+    pool = (lambda t: F.max_pool2d(t, 3, 2, 1)) if pooled else (lambda t: t)
+    return tuple(pool(F.conv2d(v, k, padding=1)).permute(0, 2, 3, 1) for v, k in ((xt, wt), (xt.abs(), wt.abs())))
+
+
+def run(x, w, pooled):
+    if pooled:
+        return dab.fconv_maxpool(x, w, None, None, None, False, 3, 3, 1, 1, 1, 1, want_sign=w.shape[0] == 64)[0]
+    return dab.fconv(x, w, None, 3, 3, 1, 1, 1, 1)
+
+
+def check(x, w, pooled):
+    got = run(x, w, pooled)
+    few = torch.cat([got[:2], got[-1:]]).double().cpu()
+    want, size = reference(torch.cat([x[:2], x[-1:]]), w, pooled)
+    # the operands' parts and the term left out: 2^-21 of a product; 288 additions of half an ulp at most; denormal results
+    bound = (2.0**-21 + 288 * 2.0**-24) * size + 2.0**-148
+    assert bool(((few - want).abs() <= bound).all())
+    return float((few - want).norm() / want.norm())
+
+
+@pytest.mark.parametrize("cout", [32, 64])
+@pytest.mark.parametrize("pooled", [False, True])
+def test_no_larger_error_than_the_six_bf16_products(cout, pooled):
+    error = check(*inputs(cout, cout), pooled)
+    print("relative 2-norm error %.3g" % error)
+    assert error < 2.0e-7  # six bf16 products in one sum: 2.4e-7, the fp32 instruction 3.0e-7
+
+
+@pytest.mark.parametrize("cout,pooled", [(32, False), (64, False), (64, True)])
+@pytest.mark.parametrize("case", ["scales", "large", "tiny", "far pixels", "far filters", "denormal"])
+def test_magnitudes(cout, pooled, case):
+    x, w = inputs(cout, 3)
+    if case == "scales":
+        x *= 2.0 ** (torch.arange(N, device="cuda") % 9 * 20.0 - 80).view(-1, 1, 1, 1)
+        x[:, ::16] *= 2.0**-11
+        w *= 2.0 ** (torch.arange(cout, device="cuda") % 16 * 2.0 - 16).view(-1, 1, 1, 1)
+    elif case == "large":
+        x *= 2.0**120
+        w *= 2.0**-10
+    elif case == "tiny":
+        x *= 2.0**-100
+        w *= 2.0**60
+    elif case == "far pixels":
+        x[:, 40:60, 32:80] *= 2.0**-40  # inside items, and items of nothing else
+        x[0, :8, :40] = 0
+    elif case == "far filters":
+        w[5::9, :, :, 3:] *= 2.0**-33
+        x[..., :3] = 0
+    else:
+        x *= 2.0**-126
+        x *= 2.0**-6
+        w *= 2.0**30
+    check(x, w, pooled)
+
+
+@pytest.mark.parametrize("cout", [32, 64])
+@pytest.mark.parametrize("where", ["pixels", "filters"])
+def test_infinities_and_nan(cout, where):
+    x, w = inputs(cout, 4)
+    values = torch.tensor([float("inf"), float("-inf"), float("nan")], device="cuda")
+    if where == "pixels":
+        x.view(-1)[7000:7000 + 40001 * 3:40001] = values
+    else:
+        w.view(-1)[100:100 + 401 * 3:401] = values
+    w.view(-1)[5::7] = 0
+    got = run(x, w, False)[:2].cpu().double()
+    want, _ = reference(x[:2], w, False)
+    assert torch.equal(got.isnan(), want.isnan())
+    assert torch.equal(got[got.isinf()], want[want.isinf()])
+    ok = want.isfinite()
+    assert torch.allclose(got[ok], want[ok], rtol=1e-4, atol=1e-4)
