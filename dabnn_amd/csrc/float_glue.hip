@@ -1240,6 +1240,30 @@ extern "C" int dab_concat_channels(const float *a, int ca, const float *b, int c
     return DAB_OK;
 }
 
+namespace dab {
+// 16 bytes a thread where both sides allow it.  Between device memory and pinned host memory the link bounds it; up to a
+// megabyte that beats the copy engine, which the kernels behind it have to wait for (602 KB to the device and 22 short kernels
+// as one graph: 76 us; by the engine 87, from pageable memory 93).
+__global__ __launch_bounds__(256) void copy_f32_kernel(float *dst, const float *src, long long n, int wide) {
+    const long long first = blockIdx.x * 256ll + threadIdx.x, step = gridDim.x * 256ll;
+    const long long quads = wide ? n / 4 : 0;
+    for (long long i = first; i < quads; i += step) reinterpret_cast<float4 *>(dst)[i] = reinterpret_cast<const float4 *>(src)[i];
+    for (long long i = 4 * quads + first; i < n; i += step) dst[i] = src[i];
+}
+}  // namespace dab
+
+extern "C" int dab_copy_f32(float *dst, const float *src, int64_t n_elem, dab_stream_t stream) {
+    using namespace dab;
+    DAB_REQUIRE(dst && src, "dab_copy_f32: null pointer");
+    DAB_REQUIRE(n_elem > 0, "dab_copy_f32: n_elem %lld", (long long)n_elem);
+    const int wide = (reinterpret_cast<uintptr_t>(dst) | reinterpret_cast<uintptr_t>(src)) % 16 == 0;
+    const long long blocks = ((wide ? n_elem / 4 : n_elem) + 255) / 256;
+    hipLaunchKernelGGL(copy_f32_kernel, dim3((unsigned)(blocks < 1 ? 1 : blocks > 256 ? 256 : blocks)), dim3(256), 0, as_stream(stream), dst, src,
+                       (long long)n_elem, wide);
+    DAB_LAUNCH_CHECK();
+    return DAB_OK;
+}
+
 extern "C" int dab_fill_f32(float *x, int64_t n_elem, float value, dab_stream_t stream) {
     using namespace dab;
     DAB_REQUIRE(x, "dab_fill_f32: null pointer");

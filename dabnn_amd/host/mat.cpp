@@ -7,6 +7,8 @@
 #include <ostream>
 #include <stdexcept>
 
+#include "staging.h"
+
 namespace bnn {
 
 static void hip_check(hipError_t e, const char *what) {
@@ -107,8 +109,12 @@ void Mat::upload(const void *host, size_t nbytes) {
     host_valid_ = false;
 }
 
-void Mat::download(void *host, size_t nbytes) const {
+void Mat::download(void *host, size_t nbytes, Staging *via) const {
     if (nbytes > bytes()) throw std::runtime_error("Mat::download: destination larger than the tensor");
+    if (via && !ld) {
+        via->download(host, dev, nbytes, copy_stream());
+        return;
+    }
     if (ld) {
         // whole pixels, and what is left of nbytes from the pixel behind them
         const size_t row = (size_t)c * elemsize, pitch = (size_t)ld * elemsize, rows = nbytes / row, rest = nbytes - rows * row;
@@ -139,14 +145,14 @@ std::vector<uint64_t> Mat::to_host_bits() const {
     return out;
 }
 
-void Mat::sync_to_host() const {
+void Mat::sync_to_host(Staging *via) const {
     if (host_valid_) return;
     if (host_.size() != bytes()) {
         host_.resize(bytes());
         data = host_.empty() ? nullptr : host_.data();
     }
     // the copy does not wait for work queued on other streams; a Net synchronises its own stream at the end of run()
-    if (!host_.empty()) download(host_.data(), host_.size());
+    if (!host_.empty()) download(host_.data(), host_.size(), via);
     host_valid_ = true;
 }
 

@@ -28,6 +28,8 @@
 
 namespace bnn {
 
+class Staging;
+
 enum class DataType { Float, Bit };
 
 class BNN_API Mat {
@@ -73,12 +75,12 @@ class BNN_API Mat {
     void gather_to(void *dst, void *stream) const;
 
     void upload(const void *host, size_t nbytes);
-    void download(void *host, size_t nbytes) const;
+    void download(void *host, size_t nbytes, Staging *via = nullptr) const;  // via: through pinned memory
     std::vector<float> to_host_float() const;
     std::vector<uint64_t> to_host_bits() const;
 
     // Brings the host mirror up to date with the device copy (allocates it on first use); waits for the device.
-    void sync_to_host() const;
+    void sync_to_host(Staging *via = nullptr) const;
     // The device copy may have changed: the next host access copies it again.
     void mark_device_written() const { host_valid_ = false; }
 

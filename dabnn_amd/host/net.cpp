@@ -1,6 +1,7 @@
 #include "net.h"
 
 #include <algorithm>
+#include <cstring>
 
 #include <hip/hip_runtime_api.h>
 
@@ -13,6 +14,7 @@
 #include "../../include/dabnn_hip_tuning.h"
 #include "layers.h"
 #include "model.h"
+#include "staging.h"
 
 namespace bnn {
 
@@ -63,12 +65,16 @@ Net::Net() {
 
 Net::~Net() {
     std::lock_guard<std::mutex> lock(capture_mutex());
-    if (graph_exec_) (void)hipGraphExecDestroy(static_cast<hipGraphExec_t>(graph_exec_));
+    for (const Graph &g : graphs_)
+        if (g.exec) (void)hipGraphExecDestroy(static_cast<hipGraphExec_t>(g.exec));
     if (input_own_dev_ && mat_map_.count(input_name_)) mat_map_[input_name_]->dev = input_own_dev_;  // freed by its Mat
     layers.clear();
     columns_.clear();
     contiguous_.clear();
+    mirrors_.clear();
     mat_map_.clear();
+    staging_.reset();
+    if (mirror_memory_) (void)hipHostFree(mirror_memory_);
     if (stream_) (void)hipStreamDestroy(static_cast<hipStream_t>(stream_));
 }
 
@@ -114,8 +120,18 @@ void Net::add_mat(const std::string &name, std::shared_ptr<Mat> mat) { mat_map_[
 
 std::shared_ptr<Mat> Net::get_blob(const std::string &name) {
     auto m = blob(name);
-    m->sync_to_host();
+    m->sync_to_host(staging_.get());
     return m;
+}
+
+void Net::download(const std::shared_ptr<Mat> &m, void *host, size_t bytes) {
+    if (mirrors_valid_)
+        for (const Mirror &mirror : mirrors_)
+            if (mirror.mat == m && bytes <= m->bytes()) {
+                std::memcpy(host, mirror.host, bytes);
+                return;
+            }
+    m->download(host, bytes, staging_.get());
 }
 
 std::shared_ptr<Mat> Net::blob(const std::string &name) {
@@ -278,6 +294,8 @@ void Net::prepare(const void *buf, size_t len) {
     allocate_blobs();
     // an in-place layer on the input blob would write into a caller's buffer that is read in place
     copy_input_ = layers_write_input();
+    staging_ = std::make_unique<Staging>(blob(input_name_)->bytes());
+    plan_mirrors();
     hip_check(hipStreamSynchronize(static_cast<hipStream_t>(stream_)), "hipStreamSynchronize");
     prepared_ = true;
 }
@@ -349,6 +367,38 @@ bool Net::layers_write_input() {
             if (m == in) return true;
     }
     return false;
+}
+
+// Float blobs of up to 2 MB in all that layers write and none but in-place ones read: the net's outputs.  A copy of its own
+// takes 20 to 100 us of a call (from the device to pageable memory, and a second synchronisation); behind the layers it
+// takes 2 (4 KB) to 20 us (1 MB: 66 us of a call before).  Above that size the link would hold up callers who ask for another blob.
+void Net::plan_mirrors() {
+    constexpr size_t kMost = 2u << 20;
+    std::vector<const Mat *> rd, wr;
+    std::set<const Mat *> read, written;
+    for (const auto &l : layers) {
+        layer_io(l, rd, wr);
+        for (const Mat *m : wr) written.insert(m);
+        for (const Mat *m : rd)
+            if (std::find(wr.begin(), wr.end(), m) == wr.end()) read.insert(m);
+    }
+    size_t total = 0;
+    for (const auto &kv : mat_map_) {
+        const auto &m = kv.second;
+        const bool known = std::any_of(mirrors_.begin(), mirrors_.end(), [&](const Mirror &x) { return x.mat == m; });
+        if (known || m->data_type != DataType::Float || m->ld || !m->dev || !written.count(m.get()) || read.count(m.get()) ||
+            m->bytes() == 0 || total + m->bytes() > kMost)
+            continue;
+        mirrors_.push_back(Mirror{m, nullptr});
+        total += (m->bytes() + 255) / 256 * 256;
+    }
+    if (mirrors_.empty()) return;
+    hip_check(hipHostMalloc(&mirror_memory_, total, 0), "hipHostMalloc");
+    auto *at = static_cast<unsigned char *>(mirror_memory_);
+    for (Mirror &x : mirrors_) {
+        x.host = reinterpret_cast<float *>(at);
+        at += (x.mat->bytes() + 255) / 256 * 256;
+    }
 }
 
 static bool contains(const std::vector<const Mat *> &v, const Mat *m) {
@@ -674,38 +724,53 @@ void Net::store_concats_in_place() {
     }
 }
 
+// Host inputs of up to a megabyte are put into pinned memory, from where the layers' first kernel takes them; larger ones
+// go through it in blocks, and memory that the caller has pinned is copied from where it lies.
 void Net::run(const void *host_input) {
     BNN_ASSERT(prepared_, "run before read");
     BNN_ASSERT(host_input != nullptr, "run: null input");
-    bind_input(nullptr);
     auto in = blob(input_name_);
-    hip_check(hipMemcpyAsync(in->dev, host_input, in->bytes(), hipMemcpyHostToDevice, static_cast<hipStream_t>(stream_)),
-              "hipMemcpyAsync");
-    launch_layers();
+    hipPointerAttribute_t where;
+    bool pageable = true;
+    if (hipPointerGetAttributes(&where, host_input) == hipSuccess)
+        pageable = where.type == hipMemoryTypeUnregistered;
+    else
+        (void)hipGetLastError();
+    const bool staged = pageable && in->bytes() <= (1u << 20) && in->bytes() <= staging_->bytes();
+    bind_input(nullptr, staged);
+    if (staged)
+        std::memcpy(staging_->memory(), host_input, in->bytes());
+    else if (pageable)
+        staging_->upload(in->dev, host_input, in->bytes(), stream_);
+    else
+        hip_check(hipMemcpyAsync(in->dev, host_input, in->bytes(), hipMemcpyHostToDevice, static_cast<hipStream_t>(stream_)),
+                  "hipMemcpyAsync");
+    launch_layers(staged);
 }
 
 void Net::run_device(const void *device_input) {
     BNN_ASSERT(prepared_, "run before read");
-    bind_input(device_input);
-    launch_layers();
+    bind_input(device_input, false);
+    launch_layers(false);
 }
 
 // Points the input blob at the memory this run reads: the caller's device buffer in place, or the blob's own
 // allocation (host inputs, unaligned buffers, callers whose buffers keep changing), filled here from device_input.
-void Net::bind_input(const void *device_input) {
+void Net::bind_input(const void *device_input, bool staged_input) {
     auto in = blob(input_name_);
     const bool in_place = device_input != nullptr && !copy_input_ && reinterpret_cast<uintptr_t>(device_input) % 256 == 0;
     void *want = in_place ? const_cast<void *>(device_input) : input_own_dev_;
-    if (graph_exec_ && graph_input_ != want) {
+    Graph &graph = graphs_[staged_input];
+    if (graph.exec && graph.input != want) {
         // the graph's kernels hold the address they were captured with
         if (in_place && ++input_rebinds_ >= 3) {
             copy_input_ = true;
             want = input_own_dev_;
         }
-        if (graph_input_ != want) {
+        if (graph.input != want) {
             std::lock_guard<std::mutex> lock(capture_mutex());
-            (void)hipGraphExecDestroy(static_cast<hipGraphExec_t>(graph_exec_));
-            graph_exec_ = nullptr;
+            (void)hipGraphExecDestroy(static_cast<hipGraphExec_t>(graph.exec));
+            graph.exec = nullptr;
         }
     }
     in->dev = want;
@@ -714,34 +779,46 @@ void Net::bind_input(const void *device_input) {
                   "hipMemcpyAsync");
 }
 
-void Net::launch_layers() {
+void Net::enqueue_layers(bool staged_input) {
+    if (staged_input) {
+        const auto in = blob(input_name_);
+        dab_check(dab_copy_f32(static_cast<float *>(in->dev), reinterpret_cast<const float *>(staging_->memory()), (int64_t)in->total(), stream_));
+    }
+    for (const auto &layer : layers) layer->forward();
+    for (const Mirror &m : mirrors_)
+        dab_check(dab_copy_f32(m.host, static_cast<const float *>(m.mat->dev), (int64_t)m.mat->total(), stream_));
+}
+
+void Net::launch_layers(bool staged_input) {
     BNN_ASSERT(!(strict && !run_fconv), "fconv must be run in strict mode");
     hipStream_t s = static_cast<hipStream_t>(stream_);
+    Graph &graph = graphs_[staged_input];
+    mirrors_valid_ = false;
     if (profile || !use_graph) {
-        for (const auto &layer : layers) layer->forward();
-    } else if (graph_exec_) {
-        hip_check(hipGraphLaunch(static_cast<hipGraphExec_t>(graph_exec_), s), "hipGraphLaunch");
+        enqueue_layers(staged_input);
+    } else if (graph.exec) {
+        hip_check(hipGraphLaunch(static_cast<hipGraphExec_t>(graph.exec), s), "hipGraphLaunch");
     } else if (runs_ >= 2) {
         // capture the kernels of one forward pass; nothing in the layers allocates, synchronises or memsets
         std::lock_guard<std::mutex> lock(capture_mutex());
-        hipGraph_t graph = nullptr;
+        hipGraph_t captured = nullptr;
         hip_check(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture");
         try {
-            for (const auto &layer : layers) layer->forward();
+            enqueue_layers(staged_input);
         } catch (...) {
-            (void)hipStreamEndCapture(s, &graph);
-            if (graph) (void)hipGraphDestroy(graph);
+            (void)hipStreamEndCapture(s, &captured);
+            if (captured) (void)hipGraphDestroy(captured);
             throw;
         }
-        hip_check(hipStreamEndCapture(s, &graph), "hipStreamEndCapture");
+        hip_check(hipStreamEndCapture(s, &captured), "hipStreamEndCapture");
         hipGraphExec_t exec = nullptr;
-        hip_check(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0), "hipGraphInstantiate");
-        (void)hipGraphDestroy(graph);
-        graph_exec_ = exec;
-        graph_input_ = blob(input_name_)->dev;
+        hip_check(hipGraphInstantiate(&exec, captured, nullptr, nullptr, 0), "hipGraphInstantiate");
+        (void)hipGraphDestroy(captured);
+        graph.exec = exec;
+        graph.input = blob(input_name_)->dev;
         hip_check(hipGraphLaunch(exec, s), "hipGraphLaunch");
     } else {
-        for (const auto &layer : layers) layer->forward();
+        enqueue_layers(staged_input);
     }
     for (const auto &kv : contiguous_) kv.first->gather_to(kv.second->dev, s);
     for (const auto &bc : columns_) bc->fill_columns();
@@ -749,6 +826,7 @@ void Net::launch_layers() {
     hip_check(hipStreamSynchronize(s), "hipStreamSynchronize");
     for (const auto &kv : contiguous_) kv.second->mark_device_written();
     for (const auto &kv : mat_map_) kv.second->mark_device_written();  // host mirrors show the previous run
+    mirrors_valid_ = true;
 }
 
 std::vector<std::string> Net::layer_descriptions() const {

@@ -21,6 +21,7 @@
 namespace bnn {
 
 class BinConv;
+class Staging;
 
 class BNN_API Net : public std::enable_shared_from_this<Net> {
    public:
@@ -48,6 +49,9 @@ class BNN_API Net : public std::enable_shared_from_this<Net> {
     std::shared_ptr<Mat> blob(const std::string &name);
     // The blob as the layers hold it, slice or not; Mat::download and the host accessors work on both.
     std::shared_ptr<Mat> stored_blob(const std::string &name);
+    // The blob's device memory to the host, contiguous, at most `bytes` of it (what dabnet_get_blob does): outputs of the last run
+    // are in pinned memory already.
+    void download(const std::shared_ptr<Mat> &m, void *host, size_t bytes);
     // If `m` is the column matrix of a layer that convolves without one: makes it, and keeps it up to date from now on.
     void make_columns(const std::shared_ptr<Mat> &m);
     bool has_blob(const std::string &name) const { return mat_map_.count(name) != 0; }
@@ -94,14 +98,29 @@ class BNN_API Net : public std::enable_shared_from_this<Net> {
     std::map<const Mat *, std::shared_ptr<Mat>> contiguous_;  // slice -> the copy that blob() handed out
     std::vector<std::shared_ptr<const BinConv>> columns_;  // layers whose column matrix somebody asked for
     int runs_ = 0;
-    void *graph_exec_ = nullptr;
+    // The captured layers and the input address that their kernels hold: [1] begins with the copy of a small host input
+    // from staging_.
+    struct Graph {
+        void *exec = nullptr;
+        const void *input = nullptr;
+    } graphs_[2];
     void *input_own_dev_ = nullptr;       // the input blob's own allocation
-    const void *graph_input_ = nullptr;   // the input address the graph's kernels hold
     int input_rebinds_ = 0;               // captures thrown away because the caller's buffer changed
     bool copy_input_ = false;             // the caller's buffers keep changing: copy into the own blob
-    void bind_input(const void *device_input);
+    void bind_input(const void *device_input, bool staged_input);
     bool layers_write_input();
-    void launch_layers();
+    void launch_layers(bool staged_input);
+    void enqueue_layers(bool staged_input);
+    std::unique_ptr<Staging> staging_;    // pinned memory for inputs, and for blobs that are asked for
+    // Small blobs that no layer reads are copied to pinned memory behind the layers of every run.
+    struct Mirror {
+        std::shared_ptr<Mat> mat;
+        float *host;
+    };
+    std::vector<Mirror> mirrors_;
+    void *mirror_memory_ = nullptr;
+    bool mirrors_valid_ = false;          // they hold what the last run left
+    void plan_mirrors();
 };
 
 }  // namespace bnn

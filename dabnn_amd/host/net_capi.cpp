@@ -133,7 +133,7 @@ int dabnet_get_blob(dabnet_t *net, const char *name, void *host_out, size_t byte
         auto m = net->net->stored_blob(name ? name : "");
         if (!host_out) throw std::runtime_error("get_blob: null destination");
         net->net->make_columns(m);
-        m->download(host_out, bytes);
+        net->net->download(m, host_out, bytes);
     });
 }
 

@@ -1,0 +1,76 @@
+// Pinned host memory between a Net and its callers' pageable buffers.
+//
+// A copy from or to pageable memory goes through the runtime's own small staging or pins the caller's pages for the call: 24 MB
+// to the device took 650 to 890 us (430 from pinned memory), 256 KB either way 106 us (13), 160 KB from the device 70.
+// A Staging holds up to 32 MB of pinned memory for the life of its Net.  Large inputs run through it in blocks of 256 KB that the
+// calling thread and up to three helpers copy in, and leave it in transfers of 1, 2, 4 and then 8 MB, each started as soon
+// as its blocks are there: one transfer costs 15 us beside its bytes, and the first should not wait long (24 MB in equal
+// transfers of 512 KB, 2 MB and 4 MB: 960, 675 and 720 us; the link alone takes 430).
+#pragma once
+
+#include <atomic>
+#include <condition_variable>
+#include <cstddef>
+#include <mutex>
+#include <thread>
+#include <vector>
+
+namespace bnn {
+
+class Staging {
+   public:
+    static constexpr size_t kBlock = 256u << 10, kMost = 32u << 20, kLargest = 8u << 20;
+    static constexpr size_t kPiece = 512u << 10;  // of a download: its first piece is copied out while the next ones arrive
+
+    // Room for `bytes`, 512 KB at least and 32 MB at most; allocates.
+    explicit Staging(size_t bytes);
+    ~Staging();
+    Staging(const Staging &) = delete;
+    Staging &operator=(const Staging &) = delete;
+
+    unsigned char *memory() const { return memory_; }
+    size_t bytes() const { return bytes_; }
+
+    // Copies host memory to the device on `stream`; `src` may change once the call returns.  The caller synchronises the
+    // stream before the next call (a Net's runs do).
+    void upload(void *dst, const void *src, size_t bytes, void *stream);
+    // Copies device memory to the host on `stream` and waits.
+    void download(void *dst, const void *src, size_t bytes, void *stream);
+
+   private:
+    struct Transfer {
+        size_t first, blocks;
+    };
+    void wait_for_room(size_t block);  // what the block is about to overwrite has been transferred
+    void copy_block(size_t block);
+    void copy_blocks();  // takes blocks until there are none left (a helper's share of an upload)
+    void helper();
+    void start_helpers();
+
+    unsigned char *memory_ = nullptr;
+    size_t bytes_ = 0;
+    int device_ = 0;
+    static constexpr size_t kEvents = 16;
+    std::vector<void *> events_;  // of transfer i: i % kEvents
+
+    // the upload at hand
+    unsigned char *dst_ = nullptr;
+    const unsigned char *src_ = nullptr;
+    size_t size_ = 0, blocks_ = 0, ring_ = 0;  // ring_: blocks in the pinned memory
+    std::vector<Transfer> transfers_;
+    std::vector<size_t> transfer_of_;  // a block's
+    std::atomic<size_t> next_{0}, issued_{0};
+    std::atomic<bool> failed_{false};
+    std::vector<std::atomic<bool>> done_;
+
+    std::vector<std::thread> helpers_;
+    std::mutex mutex_;
+    std::condition_variable wake_, idle_;
+    size_t generation_ = 0;
+    bool open_ = false;  // the upload at hand takes helpers
+    int busy_ = 0;       // and has this many
+    bool stop_ = false;
+    std::mutex use_;  // one upload or download at a time
+};
+
+}  // namespace bnn

@@ -112,9 +112,10 @@ class Net:
             _check(hostlib.dabnet_run_device(self._h, ctypes.c_void_p(x.data_ptr())))
             return self
         a = np.ascontiguousarray(x, dtype=np.float32)
-        _, _, nbytes = self.blob_info(self.input_name)
-        if a.nbytes != nbytes:
-            raise ValueError("input has %d bytes, the model wants %d" % (a.nbytes, nbytes))
+        if self._input_bytes is None:
+            self._input_bytes = self.blob_info(self.input_name)[2]
+        if a.nbytes != self._input_bytes:
+            raise ValueError("input has %d bytes, the model wants %d" % (a.nbytes, self._input_bytes))
         _check(hostlib.dabnet_run(self._h, a.ctypes.data_as(ctypes.c_void_p)))
         return self
 

@@ -329,6 +329,12 @@ DAB_API int dab_concat_channels(const float *a, int ca, const float *b, int cb, 
 /* Mat::fill<float> (dabnn/mat.h:351-443): x[i] = value; the zero-fill before bgemm (dabnn/layers/BinConv.cpp:153). */
 DAB_API int dab_fill_f32(float *x, int64_t n_elem, float value, dab_stream_t stream);
 
+/*
+ * dst[i] = src[i] for n_elem floats, as a kernel on `stream` (so a captured graph can hold it).  Either side may be pinned host
+ * memory; the two must not overlap.  No reference counterpart: a Net brings its input in and its outputs out with it.
+ */
+DAB_API int dab_copy_f32(float *dst, const float *src, int64_t n_elem, dab_stream_t stream);
+
 /* ave_pool_fallback (dabnn/layers/AvePool.cpp:84-123): mean over in-bounds taps. */
 DAB_API int dab_ave_pool(const float *x, int n, int h, int w, int c, int kh, int kw, int pad_h, int pad_w, int stride_h,
                  int stride_w, float *out, dab_stream_t stream);
