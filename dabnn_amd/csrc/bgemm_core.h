@@ -36,4 +36,8 @@ int bit_gemm(const char *fn, const BitGemm &g, FilterLayout layout, hipStream_t 
 // Whether the limits of the window form (32-bit offsets within the packed images) hold.
 bool bit_gemm_takes_images(long long image_words, long long filter_words, long long rows, int cols);
 
+// bconv_float.hip: the convolution of fp32 input in one launch; 1 = done, 0 = not its problem (pack and convolve), negative = error.
+int bconv_float_try(const float *x, int n, int h, int w, int c, const uint64_t *wgt, int words, int kh, int kw, int pad_h, int pad_w, int stride_h, int stride_w,
+                    int cout, float *out, int oh, int ow, hipStream_t s);
+
 }  // namespace dab

@@ -70,8 +70,13 @@ extern "C" int dab_binconv_forward(const float *x, int n, int h, int w, int c, c
         DAB_REQUIRE(wgt, "dab_binconv_forward: direct method needs wgt");
         DAB_REQUIRE(hwc_words == 9 * (c / 64), "dab_binconv_forward: %d words per filter, expected %d", hwc_words,
                     9 * (c / 64));
+        int rc = c <= 512 ? bconv_float_try(x, n, h, w, c, wgt, hwc_words, kh, kw, pad_h, pad_w, stride_h, stride_w, cout, out, oh, ow, as_stream(stream)) : 0;
+        if (rc != 0) {
+            if (rc > 0 && method_out) *method_out = 0;
+            return rc > 0 ? DAB_OK : rc;
+        }
         uint64_t *packed = static_cast<uint64_t *>(workspace);
-        int rc = dab_bitpack_nhwc(x, packed, (int64_t)n * h * w, c, stream);
+        rc = dab_bitpack_nhwc(x, packed, (int64_t)n * h * w, c, stream);
         if (rc != DAB_OK) return rc;
         rc = dab_bconv3x3(packed, n, h, w, c, wgt, cout, stride_h, pad_h, out, stream);
         if (rc == DAB_OK && method_out) *method_out = 0;
@@ -88,8 +93,13 @@ extern "C" int dab_binconv_forward(const float *x, int n, int h, int w, int c, c
         // The column matrix is fused_binarize_im2col of the input, kh * kw times its packed copy: the convolution reads
         // the packed pixels of a window where they are instead (8 x 14 x 14 x 256, 5 x 5: 11 us against 26 with the
         // column matrix and its GEMM).
+        int rc = bconv_float_try(x, n, h, w, c, wgt, hwc_words, kh, kw, pad_h, pad_w, stride_h, stride_w, cout, out, oh, ow, as_stream(stream));
+        if (rc != 0) {
+            if (rc > 0 && method_out) *method_out = 1;
+            return rc > 0 ? DAB_OK : rc;
+        }
         uint64_t *packed = static_cast<uint64_t *>(workspace);
-        int rc = dab_bitpack_nhwc(x, packed, (int64_t)n * h * w, c, stream);
+        rc = dab_bitpack_nhwc(x, packed, (int64_t)n * h * w, c, stream);
         if (rc != DAB_OK) return rc;
         rc = dab_bconv(packed, c / 64, n, h, w, c, wgt, hwc_words, kh, kw, pad_h, pad_w, stride_h, stride_w, cout, nullptr, nullptr,
                        nullptr, out, cout, nullptr, 0, stream);
