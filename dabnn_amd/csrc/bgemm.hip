@@ -427,9 +427,12 @@ static int launch_bit_gemm(const char *fn, BitGemmArgs &p, hipStream_t s) {
     const long long per_channel = (long long)p.units * 2 * (CC == 3 ? 16 : CC * 4);
     // The walking kernel where its filters fit and its waves find tiles for every SIMD; also for one to three units of
     // depth, which are no work for four waves.
-    // 64 channels a wave for plain matrices (m128 k18 n50176: 12.6 us against 16.4), 32 for windows, whose lanes spend
-    // more on addresses than on filters (100 x 25 x 25 x 192 -> 472, 5 x 5, stride 2: 34 us against 43).
-    const bool two = L == kFilterColumns && p.g.cols > 32 && pieces >= 2048;
+    // 64 channels a wave for plain matrices (m128 k18 n50176: 12.6 us against 16.4); for windows, whose lanes spend more on
+    // addresses than on filters, where the filters are no more than that, so that every window is fetched once (3x3 over 64, 128 and
+    // 192 channels -> 64, 131 072 pixels: 20.1, 18.5 and 20.7 -> 15.1, 15.3 and 17.5 us; 23 x 56 x 56 x 384 -> 40, 5x5: 69 -> 48;
+    // below 4096 pieces not for part of a second 32: 582 x 8 x 8 x 128 -> 40 7.8 against 8.9), else 32 (100 x 25 x 25 x 192 -> 472,
+    // 5 x 5, stride 2: 34 us against 43).
+    const bool two = L == kFilterColumns ? p.g.cols > 32 && pieces >= 2048 : p.g.cols > 32 && p.g.cols <= 64 && pieces >= (p.g.cols == 64 ? 2048 : 4096);
     const int ch = two ? 64 : 32;
     if ((pieces >= 2048 || p.units < 4) && per_channel * ch <= kFilterLdsBytes) {
         p.col_tiles = (p.g.cols + ch - 1) / ch;
@@ -452,10 +455,7 @@ static int launch_bit_gemm(const char *fn, BitGemmArgs &p, hipStream_t s) {
             return DAB_OK;
         };
         int rc = DAB_OK;
-        if constexpr (L == kFilterColumns)
-            rc = two ? launch(std::integral_constant<int, 2>{}) : launch(std::integral_constant<int, 1>{});
-        else
-            rc = launch(std::integral_constant<int, 1>{});
+        rc = two ? launch(std::integral_constant<int, 2>{}) : launch(std::integral_constant<int, 1>{});
         if (rc != DAB_OK) return rc;
     } else {
         const int split_ch = p.g.cols > 32 && pieces >= 1024 ? 64 : 32;
