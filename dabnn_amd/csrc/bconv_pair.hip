@@ -1,0 +1,211 @@
+// Two residual layers of a first-stage block in one pass: v1 = a1 * bconv3x3(sign(v0)) + b1 + v0, v2 = a2 * bconv3x3(sign(v1)) + b2 + v1,
+// 64 channels, stride 1, pad 1 (dabnn/layers/BinConv.cpp:144-191, Affine.cpp:10-23, Add.cpp:7-17, twice).
+//
+// One such layer is bound by memory: at batch 256 of 56 x 56 it reads a 205 MB shortcut and writes a 205 MB result in 72 to 80
+// us.  Here v1 never leaves the chip: a block makes R rows of v2 of one image, and with them the rows of v1 that they need --
+// R + 2, two of which its neighbours make too.  v1 stays in the accumulator layout in registers, where it is the second layer's
+// shortcut; its sign bits go through LDS, where they are the second layer's input.
+//
+// Pixels are tiles of 32 that lie one behind the other in memory, full rows, so that a tile's values and sign bits are contiguous.
+// Tile `above` starts with the strip's first pixel; the tiles before it hold the row above the strip.  A wave owns four tiles
+// and all 64 channels (128 registers of v1), and multiplies two of them at a time by the filters, which LDS holds in the matrix
+// instruction's form (fp4_core.h): an expanded pixel serves two channel groups, a fetched filter two tiles.
+#include "fp4_core.h"
+
+namespace dab {
+
+struct BconvPairArgs {
+    const uint64_t *x;        // sign bits of v0
+    const float *shortcut;    // v0
+    const uint64_t *w[2];
+    const float *a[2], *b[2];
+    float *out;
+    uint64_t *bits;           // of v2, or null
+    int H, W;
+    int rows, bands;          // of a strip, strips of an image
+    int above;                // tiles before the strip: ceil(W / 32)
+    FastDiv div_bands, div_w;
+};
+
+constexpr int kPairTiles = 16;  // of a block: four waves with four each
+constexpr int kPairFilterBytes = 9 * 2 * 64 * 16;
+
+template <bool SIGN>
+__global__ __launch_bounds__(256, 2) void bconv3x3_pair_kernel(const BconvPairArgs p) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+    __shared__ uint32_t pop[2][64];  // set bits per filter
+    const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5, l32 = lane & 31;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t item = xcd_contiguous_block(blockIdx.x, gridDim.x);  // neighbouring strips share rows: on one XCD
+    const int img = (int)p.div_bands.div(item), r0 = ((int)item - img * p.bands) * p.rows;
+    const int rows = p.H - r0 < p.rows ? p.H - r0 : p.rows;
+    const int pitch = (p.W + 2) * 8;                           // of a row of packed pixels in LDS, zero words either side
+    unsigned char *const bits0 = lds + 2 * kPairFilterBytes;   // image rows r0 - 2 .. r0 + rows + 1
+    unsigned char *const bits1 = bits0 + (p.rows + 4) * pitch;  // of v1: r0 - 1 .. r0 + rows
+    const size_t strip = ((size_t)img * p.H + r0) * p.W;       // its first pixel
+
+    // v0 of the wave's tiles, asked for before anything else; 0 where there is nothing (above the image, past its end)
+    auto tile_of = [&](int i) { return 2 * wave + (i & 1) + 8 * (i >> 1); };
+    const int lane_off = half * 4 * 256 + l32 * 4;
+    auto row_off = [](int n, int v) { return (8 * (v / 4) + v % 4) * 256 + n * 128; };
+    const int image_left = (p.H - r0) * p.W;  // pixels from the strip's first to the image's end
+    float val[4][2][16];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int first = (tile_of(i) - p.above) * 32;
+        const bool there = (first >= 0 || r0 > 0) && first < image_left;
+        const __amdgpu_buffer_rsrc_t rs = make_rsrc(p.shortcut + (strip + (there ? first : 0)) * 64, there ? (uint32_t)(image_left - first) * 256u : 0u);
+#pragma unroll
+        for (int n = 0; n < 2; ++n)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) val[i][n][v] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, lane_off, row_off(n, v), 0));
+    }
+
+    if (tid < 128) pop[tid >> 6][tid & 63] = 0;
+    const int bit_bytes = (2 * p.rows + 6) * pitch;
+    for (int i = tid * 8; i < bit_bytes; i += 256 * 8) *reinterpret_cast<uint64_t *>(bits0 + i) = 0;
+    __syncthreads();
+    // the packed input, row by row
+    const int in0 = r0 >= 2 ? r0 - 2 : 0, in1 = r0 + rows + 2 < p.H ? r0 + rows + 2 : p.H;
+    const uint64_t *src = p.x + ((size_t)img * p.H + in0) * p.W;
+    for (int j = tid; j < (in1 - in0) * p.W; j += 256) {
+        const int row = (int)p.div_w.div(j), col = j - row * p.W;
+        *reinterpret_cast<uint64_t *>(bits0 + (in0 - (r0 - 2) + row) * pitch + (col + 1) * 8) = src[j];
+    }
+    // the filters, expanded: [layer][tap][32 channels][half][channel] of 16 bytes
+    for (int j = tid; j < 2 * 64 * 9; j += 256) {
+        const int layer = j >= 64 * 9, c = j - layer * (64 * 9), ch = c / 9, tap = c - ch * 9;
+        const uint64_t word = p.w[layer][c];
+        unsigned char *d = lds + layer * kPairFilterBytes + ((tap * 2 + (ch >> 5)) * 64 + (ch & 31)) * 16;
+        *reinterpret_cast<i32x4 *>(d) = lower_half(bitspm((uint32_t)word));
+        *reinterpret_cast<i32x4 *>(d + 32 * 16) = lower_half(bitspm((uint32_t)(word >> 32)));
+        atomicAdd(&pop[layer][ch], (uint32_t)__popcll(word));
+    }
+    __syncthreads();
+
+    auto layer = [&](auto which) __attribute__((always_inline)) {
+        constexpr int L = decltype(which)::value;
+        float init[2], ea[2], eb[2];
+#pragma unroll
+        for (int n = 0; n < 2; ++n) {
+            init[n] = (float)pop[L][n * 32 + l32];
+            ea[n] = p.a[L][n * 32 + l32], eb[n] = p.b[L][n * 32 + l32];
+        }
+        const unsigned char *filter = lds + L * kPairFilterBytes + lane * 16;
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            // two neighbouring tiles; first0: the first one's first pixel, counted from the strip's
+            const int first0 = (tile_of(2 * s) - p.above) * 32;
+            if (L == 0 ? first0 >= (rows + 1) * p.W : (first0 + 64 <= 0 || first0 >= rows * p.W)) continue;
+            int row[2], col[2];  // row: from r0 - 2 on
+            f32x16m acc[2][2];
+            const unsigned char *window[2];
+#pragma unroll
+            for (int m = 0; m < 2; ++m) {
+                const int u = first0 + m * 32 + l32 + 2 * p.W;
+                row[m] = (int)p.div_w.div(u < 0 ? 0 : u), col[m] = u - row[m] * p.W;
+                // v1's rows are 1 .. rows + 2, v2's 2 .. rows + 1; what lies outside is computed from some window and not used
+                const int lowest = 1 + L, highest = rows + 2 - L, r = row[m] < lowest ? lowest : row[m] > highest ? highest : row[m];
+                window[m] = (L == 0 ? bits0 : bits1) + (r - lowest) * pitch + col[m] * 8 + half * 4;
+#pragma unroll
+                for (int n = 0; n < 2; ++n)
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) acc[m][n][v] = init[n];
+            }
+#pragma unroll
+            for (int tap = 0; tap < 9; ++tap) {
+                i32x8 a[2];
+#pragma unroll
+                for (int m = 0; m < 2; ++m) a[m] = bits01(*reinterpret_cast<const uint32_t *>(window[m] + (tap / 3) * pitch + (tap % 3) * 8));
+#pragma unroll
+                for (int n = 0; n < 2; ++n) {
+                    const i32x8 b = upper_zero(*reinterpret_cast<const i32x4 *>(filter + (tap * 2 + n) * 64 * 16));
+#pragma unroll
+                    for (int m = 0; m < 2; ++m) mfma_fp4<32>(acc[m][n], a[m], b);
+                }
+            }
+#pragma unroll
+            for (int m = 0; m < 2; ++m) {
+                const int i = 2 * s + m, first = first0 + m * 32;
+                const bool inside = L == 1 && first >= 0 && first < rows * p.W;  // (a tile of v2)
+                const __amdgpu_buffer_rsrc_t ro = make_rsrc(p.out + (strip + (inside ? first : 0)) * 64, inside ? (uint32_t)(rows * p.W - first) * 256u : 0u);
+                uint32_t word[2] = {0, 0};
+#pragma unroll
+                for (int v = 0; v < 16; ++v)
+#pragma unroll
+                    for (int n = 0; n < 2; ++n) {
+#pragma clang fp contract(off)
+                        float r = ea[n] * acc[m][n][v];
+                        r = r + eb[n];
+                        r = r + val[i][n][v];
+                        if constexpr (L == 0)
+                            val[i][n][v] = r;
+                        else
+                            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, r), ro, lane_off, row_off(n, v), kStoreStream);
+                        if constexpr (L == 0 || SIGN) {
+                            const uint64_t mask = __ballot(r > 0.f);
+                            word[n] = dab_writelane((uint32_t)mask, 8 * (v / 4) + v % 4, word[n]);
+                            word[n] = dab_writelane((uint32_t)(mask >> 32), 8 * (v / 4) + v % 4 + 4, word[n]);
+                        }
+                    }
+                if constexpr (L == 0) {
+                    const int y = r0 - 2 + row[m];
+                    if (half == 0 && row[m] >= 1 && row[m] <= rows + 2 && y >= 0 && y < p.H)
+                        *reinterpret_cast<u32x2 *>(bits1 + (row[m] - 1) * pitch + (col[m] + 1) * 8) = u32x2{word[0], word[1]};
+                } else if constexpr (SIGN) {
+                    if (half == 0 && inside && first + l32 < rows * p.W) p.bits[strip + first + l32] = ((uint64_t)word[1] << 32) | word[0];
+                }
+            }
+        }
+    };
+    layer(std::integral_constant<int, 0>{});
+    __syncthreads();
+    layer(std::integral_constant<int, 1>{});
+}
+
+// Rows of a strip for images of h x w: as many as 16 tiles hold with the row above and the row below, or fewer where a launch
+// would leave CUs without a block; 0 if the kernel does not take them.
+static int pair_rows(int n, int h, int w) {
+    const int above = (w + 31) / 32;
+    if (above * 32 > 2 * w) return 0;  // a tile's first pixel is at most two rows above the strip
+    int most = ((kPairTiles - above) * 32) / w - 1;
+    if (most > h) most = h;
+    if (most < 1) return 0;
+    if (most * w < above * 32 && most < h) return 0;  // the tiles before the second strip would start before the tensor
+    const int cus = simd_count() / 4;
+    // equal strips
+    int bands = (h + most - 1) / most;
+    while ((long long)n * bands < cus && (h + bands) / (bands + 1) * w >= above * 32 && (h + bands) / (bands + 1) >= 2) ++bands;
+    return (h + bands - 1) / bands;
+}
+
+}  // namespace dab
+
+extern "C" int dab_bconv3x3_pair(const uint64_t *x, const float *shortcut, int n, int h, int w, const uint64_t *w1, const float *a1, const float *b1,
+                                 const uint64_t *w2, const float *a2, const float *b2, float *out, uint64_t *out_packed, dab_stream_t stream) {
+    using namespace dab;
+    const char *fn = "dab_bconv3x3_pair";
+    DAB_REQUIRE(x && shortcut && w1 && a1 && b1 && w2 && a2 && b2 && out, "%s: null pointer", fn);
+    DAB_REQUIRE(n > 0 && h > 0 && w > 0, "%s: non-positive dimension", fn);
+    DAB_REQUIRE(out != shortcut && out_packed != x, "%s: the result must not alias the input", fn);
+    DAB_REQUIRE((reinterpret_cast<uintptr_t>(x) & 7) == 0 && (reinterpret_cast<uintptr_t>(w1) & 7) == 0 && (reinterpret_cast<uintptr_t>(w2) & 7) == 0 &&
+                    (reinterpret_cast<uintptr_t>(out_packed) & 7) == 0 && (reinterpret_cast<uintptr_t>(out) & 3) == 0 && (reinterpret_cast<uintptr_t>(shortcut) & 3) == 0,
+                "%s: misaligned pointer", fn);
+    const int rows = pair_rows(n, h, w);
+    const long long pixels = (long long)h * w, bands = rows ? (h + rows - 1) / rows : 0;
+    if (rows == 0 || pixels * 256 >= (1ll << 31) || (long long)n * bands >= kMostBlocks)
+        return fail(DAB_EUNSUPPORTED, "%s: images of %d x %d are not covered", fn, h, w);
+    BconvPairArgs p;
+    p.x = x, p.shortcut = shortcut, p.out = out, p.bits = out_packed;
+    p.w[0] = w1, p.w[1] = w2, p.a[0] = a1, p.a[1] = a2, p.b[0] = b1, p.b[1] = b2;
+    p.H = h, p.W = w, p.rows = rows, p.bands = (int)bands, p.above = (w + 31) / 32;
+    p.div_bands = FastDiv((uint32_t)bands), p.div_w = FastDiv((uint32_t)w);
+    const size_t lds = 2 * kPairFilterBytes + (size_t)(2 * rows + 6) * (w + 2) * 8;
+    const dim3 grid((unsigned)(n * bands));
+    if (out_packed)
+        hipLaunchKernelGGL(bconv3x3_pair_kernel<true>, grid, dim3(256), lds, as_stream(stream), p);
+    else
+        hipLaunchKernelGGL(bconv3x3_pair_kernel<false>, grid, dim3(256), lds, as_stream(stream), p);
+    DAB_LAUNCH_CHECK();
+    return DAB_OK;
+}

@@ -129,6 +129,23 @@ bool BinConv::reads_packed() const {
 bool BinConv::has_slices() const { return output_mat->ld || binarized_mat->ld || (fused_sign_out && fused_sign_out->ld); }
 
 void BinConv::forward_impl() const {
+    if (inside_pass) return;
+    if (!next_in_pass) {
+        forward_alone();
+        return;
+    }
+    const BinConv &second = *next_in_pass;
+    const auto *x = static_cast<const float *>(input_mat->dev);
+    auto *packed = static_cast<uint64_t *>(binarized_mat->dev);
+    if (!input_prepacked) dab_check(dab_bitpack_nhwc(x, packed, (int64_t)input_mat->n * input_mat->h * input_mat->w, input_mat->elem_c, stream()));
+    dab_check(dab_bconv3x3_pair(packed, x, input_mat->n, input_mat->h, input_mat->w, static_cast<const uint64_t *>(weight_mat->dev),
+                                static_cast<const float *>(fused_a->dev), static_cast<const float *>(fused_b->dev),
+                                static_cast<const uint64_t *>(second.weight_mat->dev), static_cast<const float *>(second.fused_a->dev),
+                                static_cast<const float *>(second.fused_b->dev), static_cast<float *>(second.output_mat->dev),
+                                second.fused_sign_out ? static_cast<uint64_t *>(second.fused_sign_out->dev) : nullptr, stream()));
+}
+
+void BinConv::forward_alone() const {
     binarized_mat->allocate();  // there already in a net that was read; a layer of the caller's own takes it here
     void *s = stream();
     const auto *x = static_cast<const float *>(input_mat->dev);
@@ -214,6 +231,8 @@ std::string BinConv::to_str() const {
     if (input_prepacked) ss << ", packed input from its producer";
     if (fused_a) ss << (fused_shortcut ? " + Affine + Add" : " + Affine");
     if (fused_sign_out) ss << " + Sign";
+    if (next_in_pass) ss << ", in one pass with the next layer";
+    if (inside_pass) ss << ", in the pass of the layer before";
     return ss.str();
 }
 

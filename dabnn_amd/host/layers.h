@@ -33,6 +33,13 @@ class BNN_API BinConv : public Layer {
     // takes the distance between pixels, whatever the method.
     bool has_slices() const;
 
+    // Also set by Net::prepare: this layer and the next one, `next_in_pass`, run as one pass (dab_bconv3x3_pair), which writes
+    // neither this layer's output nor its packed copy; the next layer's own forward() has nothing left to do (inside_pass).
+    std::shared_ptr<BinConv> next_in_pass;
+    bool inside_pass = false;
+    // The layer by itself, for who asks for those blobs (which must have memory) after a run.
+    void forward_alone() const;
+
     BinConv(NetCP net, css name, css input, css weight, css output, int pad_h, int pad_w, int stride_h, int stride_w);
     void forward_impl() const override;
     std::string to_str() const override;

@@ -52,7 +52,8 @@ class BNN_API Net : public std::enable_shared_from_this<Net> {
     // The blob's device memory to the host, contiguous, at most `bytes` of it (what dabnet_get_blob does): outputs of the last run
     // are in pinned memory already.
     void download(const std::shared_ptr<Mat> &m, void *host, size_t bytes);
-    // If `m` is the column matrix of a layer that convolves without one: makes it, and keeps it up to date from now on.
+    // If `m` is the column matrix of a layer that convolves without one, or a blob inside two layers' one pass: makes it, and
+    // keeps it up to date from now on.
     void make_columns(const std::shared_ptr<Mat> &m);
     bool has_blob(const std::string &name) const { return mat_map_.count(name) != 0; }
     std::vector<std::string> layer_descriptions() const;
@@ -87,6 +88,7 @@ class BNN_API Net : public std::enable_shared_from_this<Net> {
     void fuse_prelu();
     void allocate_blobs();
     void store_concats_in_place();
+    void pair_residual_layers();
     std::weak_ptr<Net> get_weak() { return shared_from_this(); }
     std::vector<std::shared_ptr<Layer>> layers;
     std::map<std::string, std::vector<uint32_t>> shapes_;  // NHWC with N = 1, as stored in the model
@@ -97,6 +99,7 @@ class BNN_API Net : public std::enable_shared_from_this<Net> {
     bool prepared_ = false;
     std::map<const Mat *, std::shared_ptr<Mat>> contiguous_;  // slice -> the copy that blob() handed out
     std::vector<std::shared_ptr<const BinConv>> columns_;  // layers whose column matrix somebody asked for
+    std::vector<std::shared_ptr<const BinConv>> alone_;    // and the first layers of a pass whose own results somebody did
     int runs_ = 0;
     // The captured layers and the input address that their kernels hold: [1] begins with the copy of a small host input
     // from staging_.
