@@ -369,8 +369,8 @@ __global__ __launch_bounds__(kBandThreads) void fconv_maxpool_kernel(const Fconv
 // 64 filters, each with its own, once for all of the block's bands, in the order the instruction wants them (a lane's eight depths
 // are 16 contiguous bytes).  A band whose rows or filters hold an infinity, or a value 2^28 times smaller than the largest one that
 // it shares its power of two with, is multiplied on the fp32 instruction from memory instead -- flags in LDS say so.
-// Batch 256, 224 x 224 x 3 -> 64 with Affine and sign bits: 408 -> 312 us (six bf16 products, three planes, rows and
-// staged band in one LDS area), batch 40: 80 -> 66; relative distance from 64-bit sums 1.6e-7 -> 9.3e-8.  Per band a wave
+// Batch 256, 224 x 224 x 3 -> 64 with Affine and sign bits: 408 -> 295 us (six bf16 products, three planes, rows and
+// staged band in one LDS area; 312 with a tile row 692 elements long, whose half-wave reads met in banks), batch 40: 80 -> 66; relative distance from 64-bit sums 1.6e-7 -> 9.3e-8.  Per band a wave
 // issues 210 matrix instructions and 1 100 others, which now bound it together: the three phases below still add up.
 //
 // A depth group is four slots of eight depths, slot g = lane / 16; the 147 depths make 19 slots: q = 0..13: kernel row q / 2,
@@ -383,9 +383,9 @@ __global__ __launch_bounds__(kBandThreads) void fconv_maxpool_kernel(const Fconv
 // neighbouring pixels of a row, so the maxima over the columns 2*px-1 .. 2*px+1 of two pooled columns
 // need one value from the lane 16 below; only those maxima -- half of the band -- are staged in LDS for the pass
 // down the rows.
-constexpr int kTileStride = 692;                    // elements per tile row: 115 pixel pairs x 6, + 2
 constexpr int kTileRows = 13, kTilePairs = 115;
-constexpr int kPlaneZero = 9000;                    // eight zeros behind the 13 x 692 tile elements
+constexpr int kTileStride = 736;                    // elements per tile row: 115 pixel pairs x 6, and 16 banks of 32 from row to row
+constexpr int kPlaneZero = kTileRows * kTileStride;  // eight zeros behind the tile's elements
 constexpr int kPlaneT20 = kPlaneZero + 8;           // [112 output columns][16]: tile rows of element 6 * ox + 20
 constexpr int kPlane = kPlaneT20 + 112 * 16;        // f16 elements per plane
 constexpr int kStemDepth = 160;                     // 5 groups x 4 slots x 8
@@ -572,7 +572,8 @@ __global__ __launch_bounds__(kBandThreads) void fconv7x7s2_maxpool_kernel(const 
     };
     // where a filter's place (slot q = place / 8, element t = place % 8) is in its 7 x 21 values: kernel row * 21 + k', or -1
     auto depth_of = [](int q, int t) {
-        if (q < 14) return (q >> 1) * 21 + 8 * (q & 1) + t;
+        if (q < 12) return (2 * (q >> 2) + (q & 1)) * 21 + 8 * ((q >> 1) & 1) + t;
+        if (q < 14) return 6 * 21 + 8 * (q & 1) + t;
         const int ky = 2 * (q - 14) + (t >> 2);
         if (q < 18) return ky < 7 ? ky * 21 + 16 + (t & 3) : -1;
         return q == 18 && t < 7 ? t * 21 + 20 : -1;
@@ -640,9 +641,9 @@ __global__ __launch_bounds__(kBandThreads) void fconv7x7s2_maxpool_kernel(const 
             // eight consecutive k' of kernel row 2 * G + g / 2: group 0's offsets plus a constant.  The other slots of group
             // 3 and group 4 have offsets of their own.  (The filter planes are laid out slot by slot when they are filled.)
             const int base_a = 2 * wm * kTileStride + 6 * f_i;
-            const int a_main = base_a + (f_s >> 1) * kTileStride + 8 * (f_s & 1);
+            const int a_main = base_a + (f_s & 1) * kTileStride + 8 * (f_s >> 1);
             // group 3: slots 12, 13 (kernel row 6), 14, 15 (k' = 16..19 of kernel rows (0, 1) and (2, 3))
-            const int a0_g3 = f_s < 2 ? a_main + 6 * kTileStride : base_a + 2 * (f_s - 2) * kTileStride + 16;
+            const int a0_g3 = f_s < 2 ? base_a + 6 * kTileStride + 8 * f_s : base_a + 2 * (f_s - 2) * kTileStride + 16;
             const int a1_g3 = a0_g3 + (f_s < 2 ? 4 : kTileStride);
             // group 4: slots 16 (kernel rows 4, 5), 17 (row 6, nothing), 18 (k' = 20 of all rows), 19 (nothing)
             const int a0_g4 = f_s < 2 ? base_a + (4 + 2 * f_s) * kTileStride + 16 : f_s == 2 ? kPlaneT20 + f_i * 16 + 2 * wm : kPlaneZero;
