@@ -975,6 +975,10 @@ static int fconv_impl(const char *fn, const float *x, int n, int h, int w, int c
                                      dil_h, dil_w, cout, a.oh, a.ow, out, s);
         if (rc != 0) return rc < 0 ? rc : DAB_OK;
     }
+    if (kh == 1 && kw == 1 && pad_h == 0 && pad_w == 0 && stride_h == 1 && stride_w == 1) {
+        const int rc = fconv_1x1_try(x, M, c, wgt, bias, aff_a, aff_b, relu, a.slope, a.slope_n, cout, out, a.out_ld, a.bits, a.bits_ld, nullptr, nullptr, s);
+        if (rc != 0) return rc < 0 ? rc : DAB_OK;
+    }
     // without padding every tap of every window is inside the image and the bounds test is dropped
     const bool padded = pad_h != 0 || pad_w != 0 || (a.oh - 1) * stride_h + (kh - 1) * dil_h >= h ||
                         (a.ow - 1) * stride_w + (kw - 1) * dil_w >= w;
@@ -1117,6 +1121,11 @@ extern "C" int dab_ave_pool2_fconv1x1(const float *x, int n, int h, int w, int c
     if (span_imgs * h * w * c * 4 >= (1ll << 30) || 128ll * a.K * 4 >= (1ll << 30) || 128ll * cout * 4 >= (1ll << 30))
         return fail(DAB_EUNSUPPORTED, "%s: image, filter or channel count too large for 32-bit tile offsets", fn);
     hipStream_t s = as_stream(stream);
+    {
+        const Pool2Window window = {h, w, a.oh, a.ow};
+        const int rc = fconv_1x1_try(x, M, c, wgt, bias, aff_a, aff_b, relu, nullptr, 0, cout, out, cout, nullptr, 0, pooled, &window, s);
+        if (rc != 0) return rc < 0 ? rc : DAB_OK;
+    }
     const int bn = cout <= 32 ? 32 : cout <= 64 ? 64 : 128;
     const long long big_tiles = ((M + 127) / 128) * ((cout + bn - 1) / bn);
 #define DAB_POOLED_LAUNCH(BM, BN, SK, KSPLIT)                                                                     \
