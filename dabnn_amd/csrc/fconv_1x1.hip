@@ -1,12 +1,13 @@
 // FpConv2D (dabnn/fconv.h:14-76) with 1x1 windows over 64, 128, 192 or 256 channels, large problems, on the f16 matrix cores with
 // split operands and fp32 accuracy (common.h): the shortcut branches of down-sampling blocks, with the AvePool 2x2 stride 2 before
-// them (dabnn/layers/AvePool.cpp) in the loader, and the transitions of dense blocks, with Affine, Relu or PRelu and the sign bits.
+// them (dabnn/layers/AvePool.cpp) in the loader, and the transitions of dense blocks, with the MaxPool 2x2 stride 2
+// (dabnn/layers/MaxPool.cpp) there, Affine, Relu or PRelu and the sign bits.
 //
 // Bound: memory, which the fp32 kernel (float_glue.hip) does not reach: its matrix instruction takes five times as long as
 // three of f16, every column of blocks reads and averages the input again, and each slice of depth ends in a barrier.  Here a
 // block is persistent and has 256 output channels (128 where there are no more), so the input is read once or twice.  A wave
 // holds its 16 or 32 filters, split, in registers; the tiles of 16 or 32 pixels pass through two LDS buffers that all eight waves
-// read.  The loads of the next tile (for the averages: of its four taps) are under way during the products of this one, and the
+// read.  The loads of the next tile (with a pool: of its four taps) are under way during the products of this one, and the
 // pixel's channels are with 16 or 32 neighbouring lanes, which find its power of two, split and store.  Output channels are the
 // rows of the matrix instruction: a lane stores four of a pixel at once.
 //
@@ -16,10 +17,13 @@
 //
 // Measured against the fp32 kernel, us a launch (pixels x channels -> channels):
 //   averages  49152 x 128 -> 256:  37.9 -> 31.2    12288 x 256 -> 512: 43.0 -> 27.6
+//   maxima    32768 x 256 -> 128:  24.1 (the pool by itself) + 22.8 -> 28.8
 //   plain     32768 x 256 -> 128:  22.8 -> 18.6    131072 x 128 -> 128: 51.2 -> 30.2    131072 x 256 -> 256: 143.5 -> 69.5
 // The last reads and writes 268 MB, 3.9 TB/s.  Error against 64-bit sums, relative to the results' root mean square:
 // 2.03e-7 -> 1.11e-7 for 128 channels, 2.87e-7 -> 1.32e-7 for 256.  Filters split into LDS by every block instead, with the waves loading
 // their pixels themselves: the averages 40 to 60 % slower than the fp32 kernel, since a wave waited for each of its loads.
+#include <float.h>
+
 #include "common.h"
 
 namespace dab {
@@ -40,16 +44,16 @@ constexpr int k1x1Threads = 512;
 constexpr int kSpecialPixel = 1 << 20;  // in an exponent's place
 
 // G: groups of 32 input channels.  CT: tiles of 16 output channels a wave.  PX: pixels a tile.
-template <int G, int CT, int PX, bool POOL>
+template <int G, int CT, int PX>
 struct Form1x1 {
     static constexpr int K = 32 * G, channels = 8 * 16 * CT, row = K + 8, plane = PX * row;
     static constexpr int lanes = k1x1Threads / PX, quads = K / 4 / lanes;  // threads of a pixel, and their quadruples of channels
     static constexpr size_t lds = 2 * 2 * plane * 2;
 };
 
-template <int G, int CT, int PX, bool POOL, int WPE>
+template <int G, int CT, int PX, Pool2 POOL, int WPE>
 __global__ __launch_bounds__(k1x1Threads, WPE) void fconv_1x1_kernel(const Fconv1x1Args p) {
-    using F = Form1x1<G, CT, PX, POOL>;
+    using F = Form1x1<G, CT, PX>;
     constexpr int K = F::K, CH = F::channels, ROW = F::row, PLANE = F::plane, LANES = F::lanes, QUADS = F::quads, MT = PX / 16;
     typedef HalfFrag8::u4 u4;
     typedef float f4 __attribute__((ext_vector_type(4)));
@@ -67,7 +71,7 @@ __global__ __launch_bounds__(k1x1Threads, WPE) void fconv_1x1_kernel(const Fconv
     // a pixel's address in x, pooled: of its window
     auto address = [&](int pix) __attribute__((always_inline)) -> const float * {
         const int at = pix < p.M ? pix : p.M - 1;
-        if constexpr (POOL) {
+        if constexpr (POOL != Pool2::none) {
             const uint32_t t = p.div_ow.div((uint32_t)at);
             const int ox = at - (int)t * (int)p.div_ow.d;
             const uint32_t img = p.div_oh.div(t);
@@ -77,7 +81,7 @@ __global__ __launch_bounds__(k1x1Threads, WPE) void fconv_1x1_kernel(const Fconv
             return p.x + (size_t)at * K;
         }
     };
-    constexpr int TAPS = POOL ? 4 : 1;
+    constexpr int TAPS = POOL != Pool2::none ? 4 : 1;
     f4 raw[QUADS][TAPS];
     auto load = [&](int tile) __attribute__((always_inline)) {
         const float *base = address(tile * PX + s_px) + 4 * s_q;
@@ -86,12 +90,20 @@ __global__ __launch_bounds__(k1x1Threads, WPE) void fconv_1x1_kernel(const Fconv
 #pragma unroll
             for (int t = 0; t < TAPS; ++t) raw[k][t] = *reinterpret_cast<const f4 *>(base + (t >> 1) * (size_t)p.wd * K + (t & 1) * K + 4 * LANES * k);
     };
-    // as ave_pool adds and scales
-    auto average = [](const f4 (&v)[TAPS]) __attribute__((always_inline)) -> f4 {
-        if constexpr (POOL)
+    // as pool_vec4_kernel adds and scales, or compares
+    auto of_window = [](const f4 (&v)[TAPS]) __attribute__((always_inline)) -> f4 {
+        if constexpr (POOL == Pool2::average) {
             return ((((f4{0.f, 0.f, 0.f, 0.f} + v[0]) + v[1]) + v[2]) + v[3]) * 0.25f;
-        else
+        } else if constexpr (POOL == Pool2::largest) {
+            f4 m = {-FLT_MAX, -FLT_MAX, -FLT_MAX, -FLT_MAX};
+#pragma unroll
+            for (int t = 0; t < TAPS; ++t)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) m[e] = v[t][e] > m[e] ? v[t][e] : m[e];
+            return m;
+        } else {
             return v[0];
+        }
     };
     auto stage = [&](int tile, int buf) __attribute__((always_inline)) {
         f4 v[QUADS];
@@ -99,11 +111,11 @@ __global__ __launch_bounds__(k1x1Threads, WPE) void fconv_1x1_kernel(const Fconv
         uint32_t smallest = ~0u;
 #pragma unroll
         for (int k = 0; k < QUADS; ++k) {
-            v[k] = average(raw[k]);
+            v[k] = of_window(raw[k]);
             largest = max3_magnitude(v[k].z, v[k].w, max3_magnitude(v[k].x, v[k].y, largest));
             smallest = smallest_magnitude(smallest_magnitude(smallest, v[k].x, v[k].y), v[k].z, v[k].w);
         }
-        if constexpr (POOL) {
+        if constexpr (POOL == Pool2::average) {
             if (p.pooled != nullptr && ch0 == 0 && tile * PX + s_px < p.M) {
 #pragma unroll
                 for (int k = 0; k < QUADS; ++k) *reinterpret_cast<f4 *>(p.pooled + (size_t)(tile * PX + s_px) * K + 4 * (s_q + LANES * k)) = v[k];
@@ -233,7 +245,7 @@ __global__ __launch_bounds__(k1x1Threads, WPE) void fconv_1x1_kernel(const Fconv
                             f4 tap[TAPS];
 #pragma unroll
                             for (int t = 0; t < TAPS; ++t) tap[t] = *reinterpret_cast<const f4 *>(x_at + (t >> 1) * (size_t)p.wd * K + (t & 1) * K + off);
-                            const f4 u = average(tap), w = *reinterpret_cast<const f4 *>(w_at + off);
+                            const f4 u = of_window(tap), w = *reinterpret_cast<const f4 *>(w_at + off);
                             even = __builtin_amdgcn_mfma_f32_16x16x4f32(w.x, u.x, even, 0, 0, 0);
                             odd = __builtin_amdgcn_mfma_f32_16x16x4f32(w.y, u.y, odd, 0, 0, 0);
                             even = __builtin_amdgcn_mfma_f32_16x16x4f32(w.z, u.z, even, 0, 0, 0);
@@ -285,13 +297,13 @@ __global__ __launch_bounds__(k1x1Threads, WPE) void fconv_1x1_kernel(const Fconv
 // launch must have the pixels or the outputs to make up for it.  Times of the fp32 kernel over this one's, over 64 to 512 output channels,
 // averages and plain: 0.83 to 1.31 at pixels * channels = 1.6 M, 0.86 to 1.54 at 3 M, 0.98 to 1.52 at 4 M, 1.03 to 1.8 from 6 M on; below
 // that, the wide outputs: 1.02 to 1.32 at pixels * channels * outputs = 2^30, 0.87 to 1.2 at half of that.
-static bool fconv_1x1_takes(long long M, int K, int cout) {
+bool fconv_1x1_takes(long long M, int K, int cout) {
     if (K % 64 != 0 || K > 256 || cout < 64 || cout % 32 != 0 || M < 1024) return false;
     return M * K >= 4ll << 20 || M * K * cout >= 1ll << 30;
 }
 
 int fconv_1x1_try(const float *x, long long M, int K, const float *wgt, const float *bias, const float *aff_a, const float *aff_b, int relu, const float *slope,
-                  int slope_n, int cout, float *out, int out_ld, uint32_t *bits, int bits_ld, float *pooled, const Pool2Window *pool, hipStream_t s) {
+                  int slope_n, int cout, float *out, int out_ld, uint32_t *bits, int bits_ld, float *pooled, Pool2 kind, const Pool2Window *pool, hipStream_t s) {
     if (!fconv_1x1_takes(M, K, cout)) return 0;
     if ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(wgt) | reinterpret_cast<uintptr_t>(pooled)) % 16 != 0) return 0;
     Fconv1x1Args a;
@@ -303,8 +315,8 @@ int fconv_1x1_try(const float *x, long long M, int K, const float *wgt, const fl
     const int cus = simd_count() / 4;
     auto launch = [&](auto groups, auto channels, auto pixels, auto pooling, auto waves) {
         constexpr int G = decltype(groups)::value, CT = decltype(channels)::value, PX = decltype(pixels)::value, WPE = decltype(waves)::value;
-        constexpr bool POOL = decltype(pooling)::value;
-        using F = Form1x1<G, CT, PX, POOL>;
+        constexpr Pool2 POOL = decltype(pooling)::value;
+        using F = Form1x1<G, CT, PX>;
         constexpr auto kernel = fconv_1x1_kernel<G, CT, PX, POOL, WPE>;
         a.cols = (cout + F::channels - 1) / F::channels, a.tiles = (int)((M + PX - 1) / PX);
         a.div_cols = FastDiv((uint32_t)a.cols);
@@ -321,26 +333,29 @@ int fconv_1x1_try(const float *x, long long M, int K, const float *wgt, const fl
     constexpr integral_constant<int, 4> four;
     constexpr integral_constant<int, 16> px16;
     constexpr integral_constant<int, 32> px32;
-    constexpr std::true_type pooling;
-    constexpr std::false_type plain;
+    constexpr integral_constant<int, 6> six;
+    constexpr integral_constant<int, 8> eight;
+    constexpr integral_constant<Pool2, Pool2::none> plain;
+    constexpr integral_constant<Pool2, Pool2::average> average;
+    constexpr integral_constant<Pool2, Pool2::largest> largest;
     // (64 output channels as 16 a wave leave half of the waves without products; the time is the memory's)
-    switch (K / 64 * 4 + (cout <= 128 ? 2 : 0) + (pool ? 1 : 0)) {
-        case 4: return launch(two, two, px32, plain, four);
-        case 5: return launch(two, two, px32, pooling, two);
-        case 6: return launch(two, one, px32, plain, four);
-        case 7: return launch(two, one, px32, pooling, four);
-        case 8: return launch(four, two, px32, plain, two);
-        case 9: return launch(four, two, px32, pooling, two);
-        case 10: return launch(four, one, px32, plain, four);
-        case 11: return launch(four, one, px32, pooling, two);
-        case 12: return launch(integral_constant<int, 6>{}, two, px32, plain, two);
-        case 13: return launch(integral_constant<int, 6>{}, two, px32, pooling, two);
-        case 14: return launch(integral_constant<int, 6>{}, one, px32, plain, two);
-        case 15: return launch(integral_constant<int, 6>{}, one, px32, pooling, two);
-        case 16: return launch(integral_constant<int, 8>{}, two, px32, plain, two);
-        case 17: return launch(integral_constant<int, 8>{}, two, px16, pooling, two);
-        case 18: return launch(integral_constant<int, 8>{}, one, px32, plain, two);
-        default: return launch(integral_constant<int, 8>{}, one, px16, pooling, two);
+    const bool narrow = cout <= 128;
+    switch (kind) {
+        case Pool2::none:
+            if (K == 64) return narrow ? launch(two, one, px32, plain, four) : launch(two, two, px32, plain, four);
+            if (K == 128) return narrow ? launch(four, one, px32, plain, four) : launch(four, two, px32, plain, two);
+            if (K == 192) return narrow ? launch(six, one, px32, plain, two) : launch(six, two, px32, plain, two);
+            return narrow ? launch(eight, one, px32, plain, two) : launch(eight, two, px32, plain, two);
+        case Pool2::average:
+            if (K == 64) return narrow ? launch(two, one, px32, average, four) : launch(two, two, px32, average, two);
+            if (K == 128) return narrow ? launch(four, one, px32, average, two) : launch(four, two, px32, average, two);
+            if (K == 192) return narrow ? launch(six, one, px32, average, two) : launch(six, two, px32, average, two);
+            return narrow ? launch(eight, one, px16, average, two) : launch(eight, two, px16, average, two);
+        default:
+            if (K == 64) return narrow ? launch(two, one, px32, largest, four) : launch(two, two, px32, largest, two);
+            if (K == 128) return narrow ? launch(four, one, px32, largest, two) : launch(four, two, px32, largest, two);
+            if (K == 192) return narrow ? launch(six, one, px32, largest, two) : launch(six, two, px32, largest, two);
+            return narrow ? launch(eight, one, px16, largest, two) : launch(eight, two, px16, largest, two);
     }
 }
 

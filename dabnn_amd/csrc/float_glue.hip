@@ -976,7 +976,7 @@ static int fconv_impl(const char *fn, const float *x, int n, int h, int w, int c
         if (rc != 0) return rc < 0 ? rc : DAB_OK;
     }
     if (kh == 1 && kw == 1 && pad_h == 0 && pad_w == 0 && stride_h == 1 && stride_w == 1) {
-        const int rc = fconv_1x1_try(x, M, c, wgt, bias, aff_a, aff_b, relu, a.slope, a.slope_n, cout, out, a.out_ld, a.bits, a.bits_ld, nullptr, nullptr, s);
+        const int rc = fconv_1x1_try(x, M, c, wgt, bias, aff_a, aff_b, relu, a.slope, a.slope_n, cout, out, a.out_ld, a.bits, a.bits_ld, nullptr, Pool2::none, nullptr, s);
         if (rc != 0) return rc < 0 ? rc : DAB_OK;
     }
     // without padding every tap of every window is inside the image and the bounds test is dropped
@@ -1083,6 +1083,35 @@ extern "C" int dab_global_ave_pool_fconv1x1(const float *x, int n, int h, int w,
     return DAB_OK;
 }
 
+extern "C" int dab_max_pool2_fconv1x1_takes(int n, int h, int w, int c, int cout) {
+    using namespace dab;
+    if (n < 1 || h < 2 || w < 2 || c < 1 || cout < 1) return 0;
+    const long long M = (long long)n * (h / 2) * (w / 2), span_imgs = 128 / ((long long)(h / 2) * (w / 2)) + 2;
+    return M < (1ll << 31) - 128 && (long long)n * h * w * c < (1ll << 31) && span_imgs * h * w * c * 4 < (1ll << 30) && 128ll * cout * 4 < (1ll << 30) &&
+           fconv_1x1_takes(M, c, cout);
+}
+
+extern "C" int dab_max_pool2_fconv1x1(const float *x, int n, int h, int w, int c, const float *wgt, const float *bias, const float *aff_a, const float *aff_b,
+                                      int relu, const float *slope, int slope_n, int cout, float *out, int64_t out_ld, uint64_t *out_packed, int64_t packed_ld,
+                                      dab_stream_t stream) {
+    using namespace dab;
+    const char *fn = "dab_max_pool2_fconv1x1";
+    DAB_REQUIRE(x && wgt && out, "%s: null pointer", fn);
+    DAB_REQUIRE(n > 0 && h >= 2 && w >= 2 && c > 0 && cout > 0, "%s: bad dimension (the input must hold a 2x2 window)", fn);
+    DAB_REQUIRE((aff_a == nullptr) == (aff_b == nullptr), "%s: affine needs both coefficient vectors", fn);
+    DAB_REQUIRE(!slope || (!relu && (slope_n == 1 || slope_n == cout)), "%s: slopes go without a Relu and number 1 or cout (%d), got %d", fn, cout, slope_n);
+    DAB_REQUIRE(out_ld >= cout && (!out_packed || packed_ld * 64 >= cout), "%s: leading dimension smaller than the row", fn);
+    DAB_REQUIRE((reinterpret_cast<uintptr_t>(out_packed) & 7) == 0, "%s: misaligned packed output", fn);
+    if ((out_packed && cout % 64 != 0) || 128 * out_ld * 4 >= (1ll << 30) || packed_ld >= (1 << 24))
+        return fail(DAB_EUNSUPPORTED, "%s: sign bits need cout %% 64 == 0, leading dimensions 32-bit tile offsets", fn);
+    if (!dab_max_pool2_fconv1x1_takes(n, h, w, c, cout) || (reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(wgt)) % 16 != 0)
+        return fail(DAB_EUNSUPPORTED, "%s: not a problem of the one-launch form, or x or wgt not 16-byte aligned", fn);
+    const Pool2Window window = {h, w, h / 2, w / 2};
+    const int rc = fconv_1x1_try(x, (long long)n * window.oh * window.ow, c, wgt, bias, aff_a, aff_b, relu, slope, slope_n, cout, out, (int)out_ld,
+                                 reinterpret_cast<uint32_t *>(out_packed), (int)(2 * packed_ld), nullptr, Pool2::largest, &window, as_stream(stream));
+    return rc < 0 ? rc : DAB_OK;
+}
+
 extern "C" int dab_ave_pool2_fconv1x1(const float *x, int n, int h, int w, int c, const float *wgt, const float *bias,
                                       const float *aff_a, const float *aff_b, int relu, int cout, float *pooled, float *out,
                                       dab_stream_t stream) {
@@ -1123,7 +1152,7 @@ extern "C" int dab_ave_pool2_fconv1x1(const float *x, int n, int h, int w, int c
     hipStream_t s = as_stream(stream);
     {
         const Pool2Window window = {h, w, a.oh, a.ow};
-        const int rc = fconv_1x1_try(x, M, c, wgt, bias, aff_a, aff_b, relu, nullptr, 0, cout, out, cout, nullptr, 0, pooled, &window, s);
+        const int rc = fconv_1x1_try(x, M, c, wgt, bias, aff_a, aff_b, relu, nullptr, 0, cout, out, cout, nullptr, 0, pooled, Pool2::average, &window, s);
         if (rc != 0) return rc < 0 ? rc : DAB_OK;
     }
     const int bn = cout <= 32 ? 32 : cout <= 64 ? 64 : 128;

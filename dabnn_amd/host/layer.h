@@ -29,6 +29,8 @@ class BNN_API Layer {
     void forward();
     virtual void forward_impl() const = 0;
     virtual std::string to_str() const;
+    // What forward() would do if no other layer did it in its pass: makes the blobs that such a pass does not write.
+    virtual void forward_alone() const { forward_impl(); }
 
     std::string name_;
     std::string type_;

@@ -281,6 +281,17 @@ void FloatConv::check_operands() const {
 }
 
 void FloatConv::forward_impl() const {
+    if (fused_pool_max) {
+        const Mat &in = *fused_pool_input, &o = *output_mat;
+        dab_check(dab_max_pool2_fconv1x1(
+            static_cast<const float *>(in.dev), in.n, in.h, in.w, in.c, static_cast<const float *>(weight_mat->dev),
+            bias_mat ? static_cast<const float *>(bias_mat->dev) : nullptr, fused_a ? static_cast<const float *>(fused_a->dev) : nullptr,
+            fused_b ? static_cast<const float *>(fused_b->dev) : nullptr, fused_relu ? 1 : 0,
+            fused_slope ? static_cast<const float *>(fused_slope->dev) : nullptr, fused_slope ? (int)fused_slope->total() : 0, o.c,
+            static_cast<float *>(o.dev), o.ld ? o.ld : o.c, fused_sign_out ? static_cast<uint64_t *>(fused_sign_out->dev) : nullptr,
+            fused_sign_out ? (fused_sign_out->ld ? fused_sign_out->ld : fused_sign_out->c) : 0, stream()));
+        return;
+    }
     if (fused_pool_input) {
         dab_check((fused_pool_global ? dab_global_ave_pool_fconv1x1 : dab_ave_pool2_fconv1x1)(
             static_cast<const float *>(fused_pool_input->dev), fused_pool_input->n, fused_pool_input->h, fused_pool_input->w,
@@ -332,7 +343,7 @@ std::string FloatConv::to_str() const {
     if (fused_slope) ss << " + PRelu";
     if (fused_sign_out) ss << " + Sign";
     if (fused_pool_input)
-        ss << ", AvePool " << (fused_pool_global ? "over all" : "2x2") << " of " << fused_pool_input->h << "x" << fused_pool_input->w << " inside";
+        ss << (fused_pool_max ? ", MaxPool " : ", AvePool ") << (fused_pool_global ? "over all" : "2x2") << " of " << fused_pool_input->h << "x" << fused_pool_input->w << " inside";
     if (fused_maxpool_out) ss << " + MaxPool 3x3 stride 2" << (fused_maxpool_sign ? " + Sign" : "");
     return ss.str();
 }
@@ -461,7 +472,13 @@ MaxPool::MaxPool(NetCP net, css name, css input, css output, int kernel_h_, int 
     check_window_output("MaxPool", *input_mat, *output_mat, kernel_h, kernel_w, pad_h, pad_w, stride_h, stride_w, 1, 1, input_mat->c);
 }
 
+std::string MaxPool::to_str() const { return Layer::to_str() + (inside_conv ? ", inside the convolution that reads it" : ""); }
+
 void MaxPool::forward_impl() const {
+    if (!inside_conv) forward_alone();
+}
+
+void MaxPool::forward_alone() const {
     if (fused_sign_out) {
         dab_check(dab_max_pool_sign(static_cast<const float *>(input_mat->dev), input_mat->n, input_mat->h, input_mat->w,
                                     input_mat->c, kernel_h, kernel_w, pad_h, pad_w, stride_h, stride_w,

@@ -38,7 +38,7 @@ class BNN_API BinConv : public Layer {
     std::shared_ptr<BinConv> next_in_pass;
     bool inside_pass = false;
     // The layer by itself, for who asks for those blobs (which must have memory) after a run.
-    void forward_alone() const;
+    void forward_alone() const override;
 
     BinConv(NetCP net, css name, css input, css weight, css output, int pad_h, int pad_w, int stride_h, int stride_w);
     void forward_impl() const override;
@@ -70,6 +70,9 @@ class BNN_API FloatConv : public Layer {
     MatP fused_pool_input;
     // The same for a global AvePool (one window over the whole image) at small batch: fused_pool_input is its input.
     bool fused_pool_global = false;
+    // The same for a MaxPool 2x2 stride 2 before large problems, with a Relu or a PRelu and slices: the pooled blob is only
+    // made for who asks for it (MaxPool::inside_conv).
+    bool fused_pool_max = false;
     // Set by Net::prepare when a MaxPool 3x3 stride 2 pad 1 is the only reader of the output: the pool's output blob,
     // the packed copy of it a direct BinConv wants (or null) and the workspace of the one-pass kernel.  output_mat is
     // null then: the convolution's result is never written.
@@ -155,10 +158,13 @@ class BNN_API MaxPool : public Layer {
     MatP input_mat, output_mat;
     // Set by Net::prepare when a direct BinConv reads the pooled blob: its packed input, written in the same pass.
     MatP fused_sign_out;
+    bool inside_conv = false;  // set by Net::prepare: the 1x1 convolution behind it pools for itself
     const int kernel_h, kernel_w, pad_h, pad_w, stride_h, stride_w;
     MaxPool(NetCP net, css name, css input, css output, int kernel_h, int kernel_w, int pad_h, int pad_w, int stride_h,
             int stride_w);
     void forward_impl() const override;
+    void forward_alone() const override;
+    std::string to_str() const override;
 };
 
 }  // namespace bnn

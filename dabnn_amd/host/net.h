@@ -88,6 +88,7 @@ class BNN_API Net : public std::enable_shared_from_this<Net> {
     void fuse_prelu();
     void allocate_blobs();
     void store_concats_in_place();
+    void pool_inside_convs();
     void pair_residual_layers();
     std::weak_ptr<Net> get_weak() { return shared_from_this(); }
     std::vector<std::shared_ptr<Layer>> layers;
@@ -99,7 +100,7 @@ class BNN_API Net : public std::enable_shared_from_this<Net> {
     bool prepared_ = false;
     std::map<const Mat *, std::shared_ptr<Mat>> contiguous_;  // slice -> the copy that blob() handed out
     std::vector<std::shared_ptr<const BinConv>> columns_;  // layers whose column matrix somebody asked for
-    std::vector<std::shared_ptr<const BinConv>> alone_;    // and the first layers of a pass whose own results somebody did
+    std::vector<std::shared_ptr<const Layer>> alone_;      // and those inside another's pass whose own results somebody did
     int runs_ = 0;
     // The captured layers and the input address that their kernels hold: [1] begins with the copy of a small host input
     // from staging_.
