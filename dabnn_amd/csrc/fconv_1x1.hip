@@ -5,7 +5,7 @@
 //
 // Bound: memory, which the fp32 kernel (float_glue.hip) does not reach: its matrix instruction takes five times as long as
 // three of f16, every column of blocks reads and averages the input again, and each slice of depth ends in a barrier.  Here a
-// block is persistent and has 256 output channels (128 where there are no more), so the input is read once or twice.  A wave
+// block is persistent and has 256 output channels (or 128), so the input is read once or twice.  A wave
 // holds its 16 or 32 filters, split, in registers; the tiles of 16 or 32 pixels pass through two LDS buffers that all eight waves
 // read.  The loads of the next tile (with a pool: of its four taps) are under way during the products of this one, and the
 // pixel's channels are with 16 or 32 neighbouring lanes, which find its power of two, split and store.  Output channels are the
@@ -16,7 +16,7 @@
 // convolution of the pooled tensor.
 //
 // Measured against the fp32 kernel, us a launch (pixels x channels -> channels):
-//   averages  49152 x 128 -> 256:  37.9 -> 31.2    12288 x 256 -> 512: 43.0 -> 27.6
+//   averages  49152 x 128 -> 256:  37.9 -> 31.2    24576 x 256 -> 512: 62.7 -> 41.0    in a net, 4900 x 256 -> 512: 28.4 -> 20.7
 //   maxima    32768 x 256 -> 128:  24.1 (the pool by itself) + 22.8 -> 28.8
 //   plain     32768 x 256 -> 128:  22.8 -> 18.6    131072 x 128 -> 128: 51.2 -> 30.2    131072 x 256 -> 256: 143.5 -> 69.5
 // The last reads and writes 268 MB, 3.9 TB/s.  Error against 64-bit sums, relative to the results' root mean square:
@@ -293,13 +293,14 @@ __global__ __launch_bounds__(k1x1Threads, WPE) void fconv_1x1_kernel(const Fconv
     }
 }
 
-// Splitting a block's filters takes 3 (64 channels) to 12 us (256 channels, 32 filters a wave) before its first product, so a
-// launch must have the pixels or the outputs to make up for it.  Times of the fp32 kernel over this one's, over 64 to 512 output channels,
-// averages and plain: 0.83 to 1.31 at pixels * channels = 1.6 M, 0.86 to 1.54 at 3 M, 0.98 to 1.52 at 4 M, 1.03 to 1.8 from 6 M on; below
-// that, the wide outputs: 1.02 to 1.32 at pixels * channels * outputs = 2^30, 0.87 to 1.2 at half of that.
+// Loading and splitting a block's filters takes 2 (64 channels, 16 filters a wave) to 11 us (256 channels, 32 filters) before its first
+// product, so a launch must have work enough to make up for it.  Times of the fp32 kernel over this one's, 64 to 512 output channels,
+// plain and averages: from 192 channels on 1.02 to 1.27 at pixels * channels * outputs = 5 * 2^26, 0.93 to 1.05 at three quarters of
+// that; with 64 and 128 channels 1.0 to 1.3 at 2^29 (outputs of 256 and more), 0.89 to 1.27 at 3/4; narrow outputs, which are bound
+// by the input: 0.98 to 1.19 at pixels * channels = 4 M.
 bool fconv_1x1_takes(long long M, int K, int cout) {
     if (K % 64 != 0 || K > 256 || cout < 64 || cout % 32 != 0 || M < 1024) return false;
-    return M * K >= 4ll << 20 || M * K * cout >= 1ll << 30;
+    return M * K >= 4ll << 20 || M * K * cout >= (K >= 192 ? 5ll << 26 : 1ll << 29);
 }
 
 int fconv_1x1_try(const float *x, long long M, int K, const float *wgt, const float *bias, const float *aff_a, const float *aff_b, int relu, const float *slope,
@@ -338,8 +339,11 @@ int fconv_1x1_try(const float *x, long long M, int K, const float *wgt, const fl
     constexpr integral_constant<Pool2, Pool2::none> plain;
     constexpr integral_constant<Pool2, Pool2::average> average;
     constexpr integral_constant<Pool2, Pool2::largest> largest;
-    // (64 output channels as 16 a wave leave half of the waves without products; the time is the memory's)
-    const bool narrow = cout <= 128;
+    // Sixteen filters a wave where 32 do not fill the outputs, and where blocks of 256 channels would have three tiles of pixels or
+    // fewer each: splitting half of the filters saves more than reading the pixels twice costs (us with 16 / 32 a wave, 256 -> 256
+    // channels: 8192 pixels 12.3 / 15.7, 16384 18.1 / 20.6; 256 -> 512 with averages: 8192 22.1 / 23.0, 16384, four tiles, 35.8 / 32.6).
+    // (64 output channels leave half of the waves without products; the time is the memory's)
+    const bool narrow = cout <= 128 || (M + 31) / 32 * ((cout + 255) / 256) <= 3ll * cus;
     switch (kind) {
         case Pool2::none:
             if (K == 64) return narrow ? launch(two, one, px32, plain, four) : launch(two, two, px32, plain, four);
