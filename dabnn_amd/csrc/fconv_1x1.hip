@@ -339,9 +339,10 @@ int fconv_1x1_try(const float *x, long long M, int K, const float *wgt, const fl
     constexpr integral_constant<Pool2, Pool2::none> plain;
     constexpr integral_constant<Pool2, Pool2::average> average;
     constexpr integral_constant<Pool2, Pool2::largest> largest;
-    // Sixteen filters a wave where 32 do not fill the outputs, and where blocks of 256 channels would have three tiles of pixels or
-    // fewer each: splitting half of the filters saves more than reading the pixels twice costs (us with 16 / 32 a wave, 256 -> 256
-    // channels: 8192 pixels 12.3 / 15.7, 16384 18.1 / 20.6; 256 -> 512 with averages: 8192 22.1 / 23.0, 16384, four tiles, 35.8 / 32.6).
+    // Sixteen filters a wave where 32 do not fill the outputs, and where blocks of 256 channels would have three tiles of
+    // pixels or fewer each: splitting half of the filters saves more than reading the pixels twice costs (us with 16 / 32 a
+    // wave, 256 -> 256 channels: 8192 pixels 12.3 / 15.7, 16384 18.1 / 20.6; 256 -> 512 with averages: 8192 22.1 / 23.0,
+    // 16384, four tiles, 35.8 / 32.6).
     // (64 output channels leave half of the waves without products; the time is the memory's)
     const bool narrow = cout <= 128 || (M + 31) / 32 * ((cout + 255) / 256) <= 3ll * cus;
     switch (kind) {

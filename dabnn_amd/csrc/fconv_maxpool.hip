@@ -369,12 +369,14 @@ __global__ __launch_bounds__(kBandThreads) void fconv_maxpool_kernel(const Fconv
 // 64 filters, each with its own, once for all of the block's bands, in the order the instruction wants them (a lane's eight depths
 // are 16 contiguous bytes).  A band whose rows or filters hold an infinity, or a value 2^28 times smaller than the largest one that
 // it shares its power of two with, is multiplied on the fp32 instruction from memory instead -- flags in LDS say so.
-// Batch 256, 224 x 224 x 3 -> 64 with Affine and sign bits: 408 -> 295 us (six bf16 products, three planes, rows and
-// staged band in one LDS area; 312 with a tile row 692 elements long, whose half-wave reads met in banks), batch 40: 80 -> 66; relative distance from 64-bit sums 1.6e-7 -> 9.3e-8.  Per band a wave
-// issues 210 matrix instructions and 1 100 others, which now bound it together: the three phases below still add up.
+// Batch 256, 224 x 224 x 3 -> 64 with Affine and sign bits: 408 -> 295 us, batch 40: 80 -> 61 (before: six bf16 products, three
+// planes, rows and staged band in one LDS area); 312 with a tile row 692 elements long, whose half-wave reads met in banks.
+// Relative distance from 64-bit sums 1.6e-7 -> 9.3e-8.  Per band a wave issues 210 matrix instructions and 1 100 others, which
+// now bound it together: the three phases below still add up.
 //
-// A depth group is four slots of eight depths, slot g = lane / 16; the 147 depths make 19 slots: q = 0..13: kernel row q / 2,
-// k' = 0..7 or 8..15; q = 14..17: k' = 16..19 of kernel rows (0, 1), (2, 3), (4, 5), (6, none); q = 18: k' = 20 of the seven
+// A depth group is four slots of eight depths, slot g = lane / 16; the 147 depths make 19 slots: q = 0..11: kernel row
+// 2 * (q / 4) + q % 2 (the two slots of a half-wave are rows next to each other), k' = 0..7 or 8..15; q = 12, 13: the same of kernel
+// row 6; q = 14..17: k' = 16..19 of kernel rows (0, 1), (2, 3), (4, 5), (6, none); q = 18: k' = 20 of the seven
 // kernel rows, which a second small array per plane holds transposed (T20[ox][tile row]) so that they are contiguous
 // too; q = 19 is empty.  Empty halves read a zero area of the plane; the eighth element of slot 18 is masked (it is a
 // real tile value, and zero times a NaN would be a NaN).  160 depths for 147, five groups.
@@ -638,8 +640,8 @@ __global__ __launch_bounds__(kBandThreads) void fconv7x7s2_maxpool_kernel(const 
             asm volatile("" : "+v"(f_s), "+v"(f_i));  // what follows is worked out per band: held across the loop it is spilled
             // lane constants of the tile reads: the plane elements of a slot's two halves of four (tile i of the wave's
             // row: + 96 * i; slot 18: + 256 * i; the zero area: + 0).  Groups 0..2 and the first two slots of group 3 are
-            // eight consecutive k' of kernel row 2 * G + g / 2: group 0's offsets plus a constant.  The other slots of group
-            // 3 and group 4 have offsets of their own.  (The filter planes are laid out slot by slot when they are filled.)
+            // eight consecutive k' of kernel row 2 * G + g % 2 (group 3: row 6): group 0's offsets plus a constant.  The other
+            // slots of group 3 and group 4 have offsets of their own.  (The filter planes are laid out slot by slot when they are filled.)
             const int base_a = 2 * wm * kTileStride + 6 * f_i;
             const int a_main = base_a + (f_s & 1) * kTileStride + 8 * (f_s >> 1);
             // group 3: slots 12, 13 (kernel row 6), 14, 15 (k' = 16..19 of kernel rows (0, 1) and (2, 3))

@@ -343,7 +343,8 @@ std::string FloatConv::to_str() const {
     if (fused_slope) ss << " + PRelu";
     if (fused_sign_out) ss << " + Sign";
     if (fused_pool_input)
-        ss << (fused_pool_max ? ", MaxPool " : ", AvePool ") << (fused_pool_global ? "over all" : "2x2") << " of " << fused_pool_input->h << "x" << fused_pool_input->w << " inside";
+        ss << (fused_pool_max ? ", MaxPool " : ", AvePool ") << (fused_pool_global ? "over all" : "2x2") << " of "
+           << fused_pool_input->h << "x" << fused_pool_input->w << " inside";
     if (fused_maxpool_out) ss << " + MaxPool 3x3 stride 2" << (fused_maxpool_sign ? " + Sign" : "");
     return ss.str();
 }
