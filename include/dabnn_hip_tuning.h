@@ -62,12 +62,6 @@ DAB_API int dab_bconv3x3_fused_shares_tiles(int64_t n_out_pixels, int cin, int c
 DAB_API int dab_global_ave_pool_fconv1x1_takes(int n, int h, int w, int c, int cout);
 
 /*
- * 1 for the shapes dab_max_pool2_fconv1x1 covers: those where it takes less time than dab_max_pool and the convolution (c 64, 128,
- * 192 or 256, cout a multiple of 32 from 64 on, and pixels enough).
- */
-DAB_API int dab_max_pool2_fconv1x1_takes(int n, int h, int w, int c, int cout);
-
-/*
  * 1 when dab_fconv_maxpool takes the shape and the problem is large enough on the current device for the one pass to
  * beat dab_fconv_affine_relu + dab_max_pool_sign, 0 otherwise.
  */
