@@ -66,16 +66,6 @@ int fconv_c32_pool_run(const float *x, int n, int h, int w, const float *wgt, co
                        const float *aff_b, int relu, int pad_h, int pad_w, int cout, int oh, int ow, float *pooled,
                        uint64_t *pooled_packed, float *work, hipStream_t s);
 
-// fconv_1x1.hip: 1x1 float convolutions over 64 to 256 channels, large problems, stride 1, the M pixels of x (kind: 2x2 averages or
-// maxima of its windows) one behind the other; 1 = done, 0 = not its problem, negative = error.
-enum class Pool2 { none, average, largest };
-struct Pool2Window {
-    int h, w, oh, ow;
-};
-bool fconv_1x1_takes(long long M, int K, int cout);  // by the sizes alone
-int fconv_1x1_try(const float *x, long long M, int K, const float *wgt, const float *bias, const float *aff_a, const float *aff_b, int relu, const float *slope,
-                  int slope_n, int cout, float *out, int out_ld, uint32_t *bits, int bits_ld, float *pooled, Pool2 kind, const Pool2Window *pool, hipStream_t s);
-
 // A launch has fewer than 2^32 threads (hipLaunchKernel refuses more): grids that grow with the problem are launched in
 // pieces of this many blocks of up to 256 threads.
 constexpr long long kMostBlocks = 1ll << 23;

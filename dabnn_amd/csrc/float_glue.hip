@@ -33,10 +33,12 @@ namespace dab {
 // depths) takes a third of the load instructions and of the address and bounds
 // arithmetic per depth.  CV = 4 does the same with 16-byte loads of four
 // consecutive channels when the channel count is a multiple of 4.  POOL (1x1
-// convolutions with CV = 4) averages 2x2 windows of the input on the way in --
-// an AvePool 2x2 stride 2 followed by the convolution, the shortcut branch of a
-// down-sampling block, in one launch; the pooled tensor is written too unless
-// p.pooled is null.
+// convolutions with CV = 4) takes the averages or the maxima of 2x2 windows of
+// the input on the way in -- a pool 2x2 stride 2 followed by the convolution, in
+// one launch: the shortcut branch of a down-sampling block (averages; the pooled
+// tensor is written too unless p.pooled is null) and the transition of a dense
+// block (maxima).
+enum class Pool2 { none, average, largest };
 struct FconvArgs {
     const float *x;
     const float *w;
@@ -44,7 +46,7 @@ struct FconvArgs {
     const float *aff_a;
     const float *aff_b;
     float *out;
-    float *pooled;  // POOL kernels: the 2x2-averaged input, written as a side product
+    float *pooled;  // averages: the pooled input, written as a side product
     int n, h, wd, c;
     int kw, dil_h, dil_w;
     int pad_h, pad_w, stride_h, stride_w;
@@ -70,7 +72,7 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 constexpr uint32_t kOob = 0x80000000u;     // descriptors here are shorter than 2^30 bytes
 constexpr uint32_t kOobRow = 0x40000000u;  // kOobRow + kOob and kOobRow + (anything < 2^30) stay out of range
 
-template <int BM, int BN, int SK, int KSPLIT, bool PADDED, int CV = 1, bool POOL = false>
+template <int BM, int BN, int SK, int KSPLIT, bool PADDED, int CV = 1, Pool2 POOL = Pool2::none>
 __global__ __launch_bounds__(256) void fconv_kernel(const FconvArgs p) {
     constexpr int WAVES_MN = 4 / KSPLIT;
     constexpr int WAVES_N = (WAVES_MN >= 2 && BN >= 64) ? 2 : 1, WAVES_M = WAVES_MN / WAVES_N;
@@ -85,8 +87,8 @@ __global__ __launch_bounds__(256) void fconv_kernel(const FconvArgs p) {
     static_assert(WK % 8 == 0 && 256 % LK == 0 && APT >= 1 && BPT >= 1, "slice");
     static_assert(CV == 1 || CV == 4 || (CV == 3 && KSPLIT == 1), "channel-vector loader");
     static_assert(KSPLIT == 1 || (KSPLIT == 4 && BM == 32 && BN == 32), "a split depth: the four waves share one 32 x 32 tile");
-    static_assert(!POOL || (CV == 4 && !PADDED), "the pooling loader takes whole 2x2 windows of four channels");
-    constexpr int NW = POOL ? 4 : 1;  // loads per tile element: the window of the pooled input
+    static_assert(POOL == Pool2::none || (CV == 4 && !PADDED), "the pooling loader takes whole 2x2 windows of four channels");
+    constexpr int NW = POOL != Pool2::none ? 4 : 1;  // loads per tile element: the window of the pooled input
     constexpr bool B_PARTIAL = BN < RP;  // fewer weight rows than loader rows: the upper loader rows fetch nothing
     __shared__ __attribute__((aligned(16))) float As[2][BM][RS];
     __shared__ __attribute__((aligned(16))) float Bs[2][BN][RS];
@@ -184,7 +186,7 @@ __global__ __launch_bounds__(256) void fconv_kernel(const FconvArgs p) {
                 off = ((unsigned)y < (unsigned)p.h && (unsigned)xx < (unsigned)p.wd) ? off : kOob;
             }
             a_reg[i][0] = load_cv(x_rsrc, off);
-            if constexpr (POOL) {
+            if constexpr (POOL != Pool2::none) {
                 // the window's other three pixels: right, below, below right (out-of-range elements carry kOob and
                 // stay out of range with these small additions)
                 const uint32_t right = (uint32_t)p.c * 4u, below = (uint32_t)p.wd * right;
@@ -201,7 +203,7 @@ __global__ __launch_bounds__(256) void fconv_kernel(const FconvArgs p) {
 #pragma unroll
         for (int i = 0; i < APT; ++i) {
             f32xcv v = a_reg[i][0];
-            if constexpr (POOL) {
+            if constexpr (POOL == Pool2::average) {
                 // ave_pool_fallback (dabnn/layers/AvePool.cpp:84-123) for a 2x2 window without padding: the taps are
                 // added to zero in row-major order and divided by 4 (a multiplication by 0.25 rounds the same way)
 #pragma clang fp contract(off)
@@ -214,6 +216,17 @@ __global__ __launch_bounds__(256) void fconv_kernel(const FconvArgs p) {
                 const int pix = m0 + l_r + RP * i, k = k0 + CV * l_k;
                 if (p.pooled != nullptr && blockIdx.y == 0 && pix < p.M && k < p.K)
                     *reinterpret_cast<f32xcv *>(p.pooled + (size_t)pix * p.K + k) = v;
+            } else if constexpr (POOL == Pool2::largest) {
+                // max_pool_fallback (dabnn/layers/MaxPool.cpp:209-246): row-major from the lowest value on, passing over NaNs.
+                // (The depth is whole slices here, so that this value never stands where the loader fetched nothing but in
+                // rows past the last pixel, which are not stored.)
+#pragma unroll
+                for (int c = 0; c < CV; ++c) {
+                    float m = -FLT_MAX;
+#pragma unroll
+                    for (int t = 0; t < NW; ++t) m = a_reg[i][t][c] > m ? a_reg[i][t][c] : m;
+                    v[c] = m;
+                }
             }
 #pragma unroll
             for (int c = 0; c < CV; ++c) As[buf][l_r + RP * i][l_k * CV + c] = v[c];
@@ -302,7 +315,7 @@ __global__ __launch_bounds__(256) void fconv_kernel(const FconvArgs p) {
     };
     // accumulator element e of lane l: row 8*(e/4) + 4*(l/32) + e%4, column l % 32
     auto emit_all = [&](auto has_bias, auto has_affine, auto act) {
-        constexpr bool PRELU = std::is_same<decltype(act), Prelu>::value;
+        constexpr bool PRELU = std::is_same<decltype(act), Prelu>::value, SIGNS = PRELU || POOL == Pool2::largest;
         if constexpr (KSPLIT == 1) {
 #pragma unroll
             for (int j = 0; j < TN; ++j) {
@@ -320,9 +333,9 @@ __global__ __launch_bounds__(256) void fconv_kernel(const FconvArgs p) {
                         constexpr int e = decltype(e_)::value;
                         const float v = emit(has_bias, has_affine, act, lane_off + (uint32_t)(i * 32 + 8 * (e / 4) + (e % 4)) * row_bytes,
                                              acc[i][j][e], bias, fa, fb, slope);
-                        if constexpr (PRELU) keep_signs(signs, e_, v);
+                        if constexpr (SIGNS) keep_signs(signs, e_, v);
                     });
-                    if constexpr (PRELU)
+                    if constexpr (SIGNS)
                         if (p.bits) store_signs(signs, wm * WTM + i * 32, n0 + wn * WTN + j * 32, true);
                 }
             }
@@ -343,9 +356,9 @@ __global__ __launch_bounds__(256) void fconv_kernel(const FconvArgs p) {
 #pragma unroll
                 for (int s = 1; s < KSPLIT; ++s) v = __fadd_rn(v, red[(s * 16 + e) * 64 + lane]);
                 v = emit(has_bias, has_affine, act, lane_off + (uint32_t)(8 * (e / 4) + (e % 4)) * row_bytes, v, bias, fa, fb, slope);
-                if constexpr (PRELU) keep_signs(signs, q_, v);  // a wave's four elements are eight consecutive rows
+                if constexpr (SIGNS) keep_signs(signs, q_, v);  // a wave's four elements are eight consecutive rows
             });
-            if constexpr (PRELU)
+            if constexpr (SIGNS)
                 if (p.bits) store_signs(signs, 8 * wave, n0, f_i < 8);
         }
     };
@@ -357,7 +370,7 @@ __global__ __launch_bounds__(256) void fconv_kernel(const FconvArgs p) {
     using T = std::true_type;
     using F = std::false_type;
     const int steps = (p.bias ? 4 : 0) | (p.aff_a ? 2 : 0) | (p.relu ? 1 : 0);
-    if constexpr (!POOL) {
+    if constexpr (POOL != Pool2::average) {
         if (p.slope != nullptr) {
             switch (steps) {
                 case 0: emit_all(F{}, F{}, Prelu{}); break;
@@ -975,10 +988,6 @@ static int fconv_impl(const char *fn, const float *x, int n, int h, int w, int c
                                      dil_h, dil_w, cout, a.oh, a.ow, out, s);
         if (rc != 0) return rc < 0 ? rc : DAB_OK;
     }
-    if (kh == 1 && kw == 1 && pad_h == 0 && pad_w == 0 && stride_h == 1 && stride_w == 1) {
-        const int rc = fconv_1x1_try(x, M, c, wgt, bias, aff_a, aff_b, relu, a.slope, a.slope_n, cout, out, a.out_ld, a.bits, a.bits_ld, nullptr, Pool2::none, nullptr, s);
-        if (rc != 0) return rc < 0 ? rc : DAB_OK;
-    }
     // without padding every tap of every window is inside the image and the bounds test is dropped
     const bool padded = pad_h != 0 || pad_w != 0 || (a.oh - 1) * stride_h + (kh - 1) * dil_h >= h ||
                         (a.ow - 1) * stride_w + (kw - 1) * dil_w >= w;
@@ -1088,7 +1097,8 @@ extern "C" int dab_max_pool2_fconv1x1_takes(int n, int h, int w, int c, int cout
     if (n < 1 || h < 2 || w < 2 || c < 1 || cout < 1) return 0;
     const long long M = (long long)n * (h / 2) * (w / 2), span_imgs = 128 / ((long long)(h / 2) * (w / 2)) + 2;
     return M < (1ll << 31) - 128 && (long long)n * h * w * c < (1ll << 31) && span_imgs * h * w * c * 4 < (1ll << 30) && 128ll * cout * 4 < (1ll << 30) &&
-           fconv_1x1_takes(M, c, cout);
+           c % 64 == 0 && c <= 256 && cout >= 64 && cout % 32 == 0 && M >= 1024 &&
+           (M * c >= 4ll << 20 || M * c * cout >= (c >= 192 ? 5ll << 26 : 1ll << 29));
 }
 
 extern "C" int dab_max_pool2_fconv1x1(const float *x, int n, int h, int w, int c, const float *wgt, const float *bias, const float *aff_a, const float *aff_b,
@@ -1106,10 +1116,29 @@ extern "C" int dab_max_pool2_fconv1x1(const float *x, int n, int h, int w, int c
         return fail(DAB_EUNSUPPORTED, "%s: sign bits need cout %% 64 == 0, leading dimensions 32-bit tile offsets", fn);
     if (!dab_max_pool2_fconv1x1_takes(n, h, w, c, cout) || (reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(wgt)) % 16 != 0)
         return fail(DAB_EUNSUPPORTED, "%s: not a problem of the one-launch form, or x or wgt not 16-byte aligned", fn);
-    const Pool2Window window = {h, w, h / 2, w / 2};
-    const int rc = fconv_1x1_try(x, (long long)n * window.oh * window.ow, c, wgt, bias, aff_a, aff_b, relu, slope, slope_n, cout, out, (int)out_ld,
-                                 reinterpret_cast<uint32_t *>(out_packed), (int)(2 * packed_ld), nullptr, Pool2::largest, &window, as_stream(stream));
-    return rc < 0 ? rc : DAB_OK;
+    FconvArgs a = {};
+    a.x = x, a.w = wgt, a.bias = bias, a.aff_a = aff_a, a.aff_b = aff_b, a.relu = relu, a.out = out;
+    a.slope = slope, a.slope_n = slope_n, a.bits = reinterpret_cast<uint32_t *>(out_packed), a.bits_ld = (int)(2 * packed_ld), a.out_ld = (int)out_ld;
+    a.n = n, a.h = h, a.wd = w, a.c = c, a.K = c, a.cout = cout;
+    a.stride_h = 2, a.stride_w = 2, a.kw = 1, a.dil_h = 1, a.dil_w = 1;
+    a.oh = h / 2, a.ow = w / 2, a.M = n * a.oh * a.ow;
+    a.div_ow = FastDiv((uint32_t)a.ow), a.div_oh = FastDiv((uint32_t)a.oh), a.div_c = FastDiv((uint32_t)c), a.div_kw = FastDiv(1u);
+    hipStream_t s = as_stream(stream);
+#define DAB_POOLED_LAUNCH(BM, BN, SK)                                                                  \
+    hipLaunchKernelGGL((fconv_kernel<BM, BN, SK, 1, false, 4, Pool2::largest>),                        \
+                       dim3((unsigned)((a.M + BM - 1) / BM), (unsigned)((cout + BN - 1) / BN)), dim3(256), 0, s, a)
+    // a tile's sums run over the depth in order, as those of dab_fconv_affine_prelu for problems of this size: the result is bit for bit
+    // that of the two calls.  Whole 128-byte lines of a pixel a slice where one tile holds all output channels; wider ones take the
+    // maxima once for every 256 channels.
+    if (cout <= 64)
+        DAB_POOLED_LAUNCH(128, 64, 32);
+    else if (cout <= 128)
+        DAB_POOLED_LAUNCH(64, 128, 32);
+    else
+        DAB_POOLED_LAUNCH(64, 256, 16);
+#undef DAB_POOLED_LAUNCH
+    DAB_LAUNCH_CHECK();
+    return DAB_OK;
 }
 
 extern "C" int dab_ave_pool2_fconv1x1(const float *x, int n, int h, int w, int c, const float *wgt, const float *bias,
@@ -1150,15 +1179,10 @@ extern "C" int dab_ave_pool2_fconv1x1(const float *x, int n, int h, int w, int c
     if (span_imgs * h * w * c * 4 >= (1ll << 30) || 128ll * a.K * 4 >= (1ll << 30) || 128ll * cout * 4 >= (1ll << 30))
         return fail(DAB_EUNSUPPORTED, "%s: image, filter or channel count too large for 32-bit tile offsets", fn);
     hipStream_t s = as_stream(stream);
-    {
-        const Pool2Window window = {h, w, a.oh, a.ow};
-        const int rc = fconv_1x1_try(x, M, c, wgt, bias, aff_a, aff_b, relu, nullptr, 0, cout, out, cout, nullptr, 0, pooled, Pool2::average, &window, s);
-        if (rc != 0) return rc < 0 ? rc : DAB_OK;
-    }
     const int bn = cout <= 32 ? 32 : cout <= 64 ? 64 : 128;
     const long long big_tiles = ((M + 127) / 128) * ((cout + bn - 1) / bn);
 #define DAB_POOLED_LAUNCH(BM, BN, SK, KSPLIT)                                                                     \
-    hipLaunchKernelGGL((fconv_kernel<BM, BN, SK, KSPLIT, false, 4, true>),                                        \
+    hipLaunchKernelGGL((fconv_kernel<BM, BN, SK, KSPLIT, false, 4, Pool2::average>),                                        \
                        dim3((unsigned)((M + BM - 1) / BM), (unsigned)((cout + BN - 1) / BN)), dim3(256), 0, s, a)
     // Bit for bit the 1x1 convolution of the pooled tensor: a tile's sums run over the depth in order, whatever the tile and
     // its slices, but where the depth is split over the waves -- that is done here for the problems for which

@@ -757,9 +757,11 @@ void Net::store_concats_in_place() {
 }
 
 // MaxPool 2x2 stride 2 whose one reader is a 1x1 FloatConv (the transition of a dense block): the convolution's loader takes the
-// maxima where the library has that in one launch.  Nothing may rewrite what the pool reads, so that the pooled blob can
-// still be made for who asks for it.  256 channels, 32 x 32 -> 16 x 16 x 128 at 128 images:
-// 24.1 + 20.4 -> 28.8 us, bound by the 134 MB that it reads.
+// maxima where the library has that in one launch and one tile holds all output channels, so that the maxima are taken once.  Two
+// launches / one, us: 10 240 pixels x 256 -> 128 23.2 / 19.1, 32 768 x 256 -> 128 47.9 / 30.7 (134 MB read, 4.4 TB/s), 131 072 x 128 ->
+// 64 84 / 54, 65 536 x 64 -> 128 30.5 / 25.1; all of 40 problems of up to 131 072 pixels 1.14 to 1.78 times as fast.  With 160 to 256
+// channels 0.65 to 1.3 (34 816 x 256 -> 160 61 / 76), with more 0.6 to 1.1.  Nothing may rewrite what the pool reads, so that the
+// pooled blob can still be made for who asks for it.
 void Net::pool_inside_convs() {
     std::vector<const Mat *> rd, wr;
     for (size_t i = 0; i + 1 < layers.size(); ++i) {
@@ -781,7 +783,7 @@ void Net::pool_inside_convs() {
         }
         if (!ok || !reader || reader->input_mat != pool->output_mat || reader->fused_pool_input || reader->fused_maxpool_out || reader->weight_mat->h != 1 ||
             reader->weight_mat->w != 1 || reader->pad_h != 0 || reader->pad_w != 0 || reader->stride_h != 1 || reader->stride_w != 1 || reader->dilation != 1 ||
-            !dab_max_pool2_fconv1x1_takes(in.n, in.h, in.w, in.c, reader->output_mat->c))
+            reader->output_mat->c > 128 || !dab_max_pool2_fconv1x1_takes(in.n, in.h, in.w, in.c, reader->output_mat->c))
             continue;
         reader->fused_pool_input = pool->input_mat;
         reader->fused_pool_max = true;

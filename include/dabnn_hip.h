@@ -284,9 +284,9 @@ DAB_API int dab_ave_pool2_fconv1x1(const float *x, int n, int h, int w, int c, c
  * MaxPool 2x2, stride 2, no padding (max_pool_fallback, dabnn/layers/MaxPool.cpp:209-246) followed by a 1x1 FpConv2D
  * (dabnn/fconv.h:14-76), the optional Affine, and a Relu or a PRelu (slope not null; slope_n = 1 or cout) or neither, in one
  * launch: the transition of a dense block.  out and out_packed as for dab_fconv_affine_prelu, with the values of dab_max_pool and
- * that call.  x and wgt must be 16-byte aligned and the shapes those that dab_max_pool2_fconv1x1_takes answers with 1, where the
- * launch takes less time than the two calls, which serve the others (DAB_EUNSUPPORTED): c 64, 128, 192 or 256, cout a multiple of
- * 32 from 64 on, and pixels enough.
+ * that call.  x and wgt must be 16-byte aligned and the shapes those that dab_max_pool2_fconv1x1_takes answers with 1 (the two
+ * calls serve the others: DAB_EUNSUPPORTED): c 64, 128, 192 or 256, cout a multiple of 32 from 64 on, and pixels enough.  Faster
+ * than the two calls with up to 128 output channels; with more it may take up to 1.6 times as long.
  */
 DAB_API int dab_max_pool2_fconv1x1(const float *x, int n, int h, int w, int c, const float *wgt, const float *bias,
                                    const float *a, const float *b, int relu, const float *slope, int slope_n, int cout,

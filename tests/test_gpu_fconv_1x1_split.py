@@ -1,5 +1,5 @@
-"""1x1 float convolutions with 64 to 256 input channels on the f16 matrix cores: errors against 64-bit sums, pixels that fill no
-tile, channels that fill no column, channel slices with sign bits, averages of odd images, infinities and values far apart."""
+"""1x1 float convolutions with 64 to 256 input channels, large problems: errors against 64-bit sums, operands kept whole, pixels that fill
+no tile, channels that fill no column, channel slices with sign bits, averages of odd images, infinities and values far apart."""
 import pytest
 import torch
 
@@ -20,8 +20,7 @@ def sums(x, wgt, bias):
     return rows @ wt.t() + bias, bound
 
 
-# the smallest that are taken (pixels * channels = 4 M; with the outputs 2^29, from 192 channels on 5 * 2^26) and one pixel fewer,
-# pixels that fill no tile, both sides of the switch from 16 to 32 filters a wave
+# pixels * channels = 4 M, with the outputs 2^29, from 192 channels on 5 * 2^26, and one pixel fewer; pixels that fill no tile
 @pytest.mark.parametrize("m,c,cout", [
     (65536, 64, 64), (65535, 64, 64), (70001, 64, 320), (32768, 128, 96), (33001, 128, 416), (131071, 128, 128), (2048, 128, 2048), (2047, 128, 2048),
     (21846, 192, 160), (22001, 192, 128), (16384, 256, 64), (16399, 256, 256), (8192, 256, 512), (16401, 256, 288),
@@ -34,9 +33,9 @@ def test_against_64_bit_sums(m, c, cout):
     want, bound = sums(x, wgt, bias)
     err = (got.reshape(-1, cout).double() - want).abs()
     assert bool((err <= bound).all())
-    # no worse than c products in fp32 one after the other: roundings of 0.41 * 2^-24 of partial sums that grow as the square root
-    if m * c >= 4 << 20 or m * c * cout >= (5 << 26 if c >= 192 else 1 << 29):
-        assert float((err**2).mean().sqrt() / (want**2).mean().sqrt()) < 0.41 * 2.0**-24 * (c / 2)**0.5
+    # no worse than c products and a bias in fp32 one after the other: c + 1 roundings, each spread evenly over half an ulp of at most 2^-23
+    # of its partial sum (2^-24 / sqrt(3) of it in the root mean square), of sums whose variances 1, 2 .. c + 1 make (c + 1) * (c + 2) / 2
+    assert float((err**2).mean().sqrt() / (want**2).mean().sqrt()) < 2.0**-24 / 3**0.5 * ((c + 2) / 2)**0.5
     sep = got.clone()
     dab.affine_inplace(sep, a, b)
     assert torch.equal(dab.fconv_affine_relu(x, wgt, bias, a, b, False, 1, 1, 0, 0, 1, 1), sep)
@@ -98,3 +97,26 @@ def test_special_values(c):
     assert bool((got.isnan() == want.isnan()).all())
     assert bool(((got - want).abs() <= bound)[finite].all())
     assert torch.equal(got[~finite & ~want.isnan()], want[~finite & ~want.isnan()])
+
+
+# every output channel copies one input channel: no operand loses a bit on its way to the products, so the values come back exactly
+@pytest.mark.parametrize("pool", ["none", "average", "maxima"])
+@pytest.mark.parametrize("hw,c,cout", [(128, 256, 512), (128, 192, 256), (182, 128, 416), (256, 64, 128)])
+def test_copied_channels_are_exact(pool, hw, c, cout):
+    import dabnn_amd as dab
+    from dabnn_amd import capi
+    gen = torch.Generator(device="cuda").manual_seed(c)
+    n = 1 if pool == "none" else 4
+    x = torch.randn((n, hw, hw, c), device="cuda", generator=gen)
+    wgt = torch.zeros((cout, 1, 1, c), device="cuda")
+    wgt[torch.arange(cout), 0, 0, torch.arange(cout) % c] = 1
+    if pool == "none":
+        want, got = x, dab.fconv(x, wgt, None, 1, 1, 0, 0, 1, 1)
+    elif pool == "average":
+        want, got = dab.ave_pool(x, 2, 2, 0, 0, 2, 2), dab.ave_pool2_fconv1x1(x, wgt, None, None, None, False, False)[1]
+    else:
+        want, got = dab.max_pool(x, 2, 2, 0, 0, 2, 2), torch.empty((n, hw // 2, hw // 2, cout), device="cuda")
+        capi.check(capi.lib.dab_max_pool2_fconv1x1(x.data_ptr(), n, hw, hw, c, wgt.data_ptr(), None, None, None, 0, None, 0, cout,
+                                                   got.data_ptr(), cout, None, 0, None))
+        torch.cuda.synchronize()
+    assert torch.equal(got, want[..., torch.arange(cout) % c])
