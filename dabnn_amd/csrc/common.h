@@ -149,19 +149,28 @@ __device__ __forceinline__ uint32_t or_from_lane_above(uint32_t v) {
 // ---------------------------------------------------------------- fp32 products on the bf16 matrix cores
 // An fp32 value is the exact sum of three bf16 values (8 + 8 + 8 significand bits, fp32's exponent range):
 // hi = the upper 16 bits of x, mid = the upper 16 bits of x - hi, lo = x - hi - mid.  A product x*w is then
-// hi*hi + (hi*mid + mid*hi) + (hi*lo + mid*mid + lo*hi) + terms below 2^-24 of it: six bf16 matrix instructions (16 cycles for
-// 32 depths; the fp32 instruction takes 32 for 4), the cross terms in a sum of their own: over 160 and 288 products 7.1e-8 and
-// 9.5e-8 away from 64-bit sums, an fp32 loop 2.3e-7 and 3.0e-7.
-// An infinity or a NaN makes a NaN of the sum (an infinity times a zero mid or lo part is one), and for values below 2^-110
-// the mid and lo parts are bf16 denormals and lose bits (activations around 2^-120: 3.5e-5 relative, filters 1.2e-3).
-// The kernels that use it (the small forms of fconv_c32.hip) look for such values and make the sums they are in on the fp32
-// matrix instruction.
+// hi*hi + (hi*mid + mid*hi) + (hi*lo + mid*mid + lo*hi) + terms below 2^-24 of it: six bf16 matrix instructions,
+// accumulated in fp32 from the smallest term up, give a dot product whose error is that of an fp32 loop (measured on
+// a 160-deep product against fp64: 1.6e-7 of the sum of magnitudes, an fp32 loop 2.0e-7; the three leading terms
+// alone: 1.1e-5) at up to 2.6 times the rate of the fp32 matrix instruction (v_mfma_f32_32x32x16_bf16 issues in 33
+// cycles, six of them for 16 depths: 404 TFLOP/s fp32-equivalent against 156; v_mfma_f32_16x16x32_bf16 in 16-19 for
+// 32 depths; the splitting runs on the vector pipe while another wave's matrix instructions are in flight).
+// An infinity or a NaN stays whole in hi and takes part in the hi*hi term only, where it meets the other operand's
+// leading part -- the same sign, and zero where the operand is zero -- so x*w is infinite or NaN where the fp32
+// product is, as long as the other operand's leading part is a normal bf16 or an exact zero; the cross terms use
+// `hif`, hi with non-finite values replaced by zero (an infinity times a zero mid or lo part would be a NaN).  A NaN
+// keeps a quiet bit in its upper half.
+// Limits: the leading part of a nonzero |w| below 2^-126 (an fp32 denormal) is zero or a bf16 denormal, which the
+// matrix core may flush, so inf * w can come out as NaN or 0 where fp32 arithmetic gives an infinity; and for finite
+// operands within 2^16 of the smallest normal the mid and lo parts are bf16 denormals, so the fp32-equivalent error
+// bound above holds only for magnitudes of 2^-110 and more (activations around 2^-120: 3.5e-5 relative, filters 1.2e-3).
+// The kernels for large problems have these limits; the small forms of fconv_c32.hip look for such values and make the
+// sums they are in on the fp32 matrix instruction.
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4w __attribute__((ext_vector_type(4)));
 
 struct SplitParts {
-    uint32_t hi, mid, lo;  // bf16 in the upper halves
-    bool special;          // an infinity or a NaN, whole in hi
+    uint32_t hi, hif, mid, lo;  // bf16 in the upper halves
 };
 __device__ __forceinline__ SplitParts split_bf16x3(float x) {
     const uint32_t xb = __builtin_bit_cast(uint32_t, x);
@@ -171,14 +180,16 @@ __device__ __forceinline__ SplitParts split_bf16x3(float x) {
     r = special ? 0.f : r;
     const uint32_t rb = __builtin_bit_cast(uint32_t, r);
     const float l = r - __builtin_bit_cast(float, rb & 0xffff0000u);
-    return SplitParts{hb, rb, __builtin_bit_cast(uint32_t, l), special};
+    return SplitParts{hb, special ? 0u : hb, rb, __builtin_bit_cast(uint32_t, l)};
 }
 // the upper halves of two dwords as one: a in the lower 16 bits, b in the upper
 __device__ __forceinline__ uint32_t pack_upper_halves(uint32_t a, uint32_t b) { return __builtin_amdgcn_perm(b, a, 0x07060302u); }
 
 // The same split for a pair of finite values with the hardware's round-to-nearest conversions (v_cvt_pk_bf16_f32
 // packs two): hi = bf16(x), mid = bf16(x - hi), lo = bf16(x - hi - mid), both subtractions and the last conversion
-// exact.  5.5 vector instructions per value against about 10 for the truncating form with its tests.
+// exact.  5.5 vector instructions per value against about 10 for the truncating form with its tests.  An infinity or a
+// NaN would come out as NaN in mid and lo: callers check with bf16_pair_max / bf16_pairs_finite and take the
+// truncating form for the rare group that holds one.
 typedef __bf16 bf16x2v __attribute__((ext_vector_type(2)));
 typedef float f32x2v __attribute__((ext_vector_type(2)));
 typedef unsigned short u16x2v __attribute__((ext_vector_type(2)));
@@ -196,6 +207,15 @@ __device__ __forceinline__ SplitPair split_pair_finite(float x0, float x1) {
     s.lo = __builtin_bit_cast(uint32_t, __builtin_convertvector(r2, bf16x2v));
     return s;
 }
+// Running maximum of the magnitudes of bf16 pairs (as 16-bit integers, half by half), and the test of the result.
+__device__ __forceinline__ uint32_t bf16_pair_max(uint32_t running, uint32_t pair) {
+    const u16x2v a = __builtin_bit_cast(u16x2v, running), b = __builtin_bit_cast(u16x2v, pair & 0x7fff7fffu);
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(a, b));
+}
+__device__ __forceinline__ bool bf16_pairs_finite(uint32_t running) {
+    return (running & 0xffffu) < 0x7f80u && (running >> 16) < 0x7f80u;
+}
+
 // Whether one of the values is not zero and below 2^-110, where the parts of the split are bf16 denormals and lose bits:
 // running minimum over pairs of values (from ~0u on), and the test of the result.  Three instructions a pair.
 __device__ __forceinline__ uint32_t smallest_magnitude(uint32_t running, float x0, float x1) {
@@ -206,28 +226,72 @@ __device__ __forceinline__ uint32_t smallest_magnitude(uint32_t running, float x
 }
 __device__ __forceinline__ bool loses_bits_when_split(uint32_t running) { return running < (((127u - 110u) << 24) - 1u); }
 
-// Eight consecutive depths of one row or column as three planes of eight bf16.
+// Two bf16 in a dword, each replaced by zero when it is an infinity or a NaN.
+__device__ __forceinline__ uint32_t finite_bf16_pair(uint32_t w) {
+    const uint32_t lo_ok = (w & 0x00007f80u) != 0x00007f80u ? 0x0000ffffu : 0u;
+    const uint32_t hi_ok = (w & 0x7f800000u) != 0x7f800000u ? 0xffff0000u : 0u;
+    return w & (lo_ok | hi_ok);
+}
+
+// Eight consecutive depths of one row or column as four planes of eight bf16.
 struct SplitFrag8 {
     typedef uint32_t u4 __attribute__((ext_vector_type(4)));
-    u4 hi, mid, lo;
+    u4 hi, hif, mid, lo;
+    // finite values only (see split_pair_finite); hif = hi; returns the running magnitude maximum with these values in
+    __device__ __forceinline__ uint32_t set_finite(const float (&x)[8], uint32_t running) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const SplitPair s = split_pair_finite(x[2 * i], x[2 * i + 1]);
+            hi[i] = s.hi, mid[i] = s.mid, lo[i] = s.lo;
+            running = bf16_pair_max(running, s.hi);
+        }
+        hif = hi;
+        return running;
+    }
+    __device__ __forceinline__ void set(const float (&x)[8]) {
+        SplitParts s[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) s[i] = split_bf16x3(x[i]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            hi[i] = pack_upper_halves(s[2 * i].hi, s[2 * i + 1].hi);
+            hif[i] = pack_upper_halves(s[2 * i].hif, s[2 * i + 1].hif);
+            mid[i] = pack_upper_halves(s[2 * i].mid, s[2 * i + 1].mid);
+            lo[i] = pack_upper_halves(s[2 * i].lo, s[2 * i + 1].lo);
+        }
+    }
 };
 
-// acc += A * B over 32 depths for two 16 x 16 tiles that share A, the five cross terms in sums of their own (the caller adds acc
-// and cross at the end): lane l holds row / column l % 16, depths 8 * (l / 16) .. + 7 (any assignment of depths to lanes and
-// elements works as long as A and B use the same one).  The accumulators alternate so that no instruction waits for the one
-// before it.
+// acc += A * B over 32 depths for two 16 x 16 tiles that share A: lane l holds row / column l % 16, depths
+// 8 * (l / 16) .. + 7 (any assignment of depths to lanes and elements works as long as A and B use the same one).
+// The two accumulators alternate so that no instruction waits for the one before it.
+__device__ __forceinline__ void mfma6_16x16x32(f32x4w &acc0, f32x4w &acc1, const SplitFrag8 &a, const SplitFrag8 &b0,
+                                               const SplitFrag8 &b1) {
+    auto v = [](SplitFrag8::u4 w) { return __builtin_bit_cast(bf16x8, w); };
+#define DAB_MFMA2(A, B)                                                               \
+    acc0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v(a.A), v(b0.B), acc0, 0, 0, 0);  \
+    acc1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v(a.A), v(b1.B), acc1, 0, 0, 0);
+    DAB_MFMA2(lo, hif)
+    DAB_MFMA2(hif, lo)
+    DAB_MFMA2(mid, mid)
+    DAB_MFMA2(mid, hif)
+    DAB_MFMA2(hif, mid)
+    DAB_MFMA2(hi, hi)
+#undef DAB_MFMA2
+}
+// The same with the five cross terms in sums of their own: the caller adds acc and cross at the end.
 __device__ __forceinline__ void mfma6_16x16x32_two_sums(f32x4w &acc0, f32x4w &acc1, f32x4w &cross0, f32x4w &cross1, const SplitFrag8 &a,
                                                         const SplitFrag8 &b0, const SplitFrag8 &b1) {
     auto v = [](SplitFrag8::u4 w) { return __builtin_bit_cast(bf16x8, w); };
 #define DAB_MFMA2(S, A, B)                                                           \
     S##0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v(a.A), v(b0.B), S##0, 0, 0, 0);  \
     S##1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v(a.A), v(b1.B), S##1, 0, 0, 0);
-    DAB_MFMA2(cross, lo, hi)
-    DAB_MFMA2(cross, hi, lo)
+    DAB_MFMA2(cross, lo, hif)
+    DAB_MFMA2(cross, hif, lo)
     DAB_MFMA2(cross, mid, mid)
     DAB_MFMA2(acc, hi, hi)
-    DAB_MFMA2(cross, mid, hi)
-    DAB_MFMA2(cross, hi, mid)
+    DAB_MFMA2(cross, mid, hif)
+    DAB_MFMA2(cross, hif, mid)
 #undef DAB_MFMA2
 }
 

@@ -1,7 +1,6 @@
 // FpConv2D (dabnn/fconv.h:14-76) for 3x3, stride 1 convolutions over 32 input channels -- the second and third
-// convolution of a three-convolution stem -- on the 16-bit matrix cores with split operands and fp32 accuracy (common.h: two f16
-// parts and three products per depth group; small problems three bf16 parts and six products), with the optional Affine and Relu of
-// dab_fconv_affine_relu in the same pass.
+// convolution of a three-convolution stem -- on the bf16 matrix cores with split operands (common.h: six products
+// per depth group, fp32 accuracy), with the optional Affine and Relu of dab_fconv_affine_relu in the same pass.
 //
 // A depth group of the matrix instruction (32 depths) is one tap's 32 channels, so there is no im2col stage and no
 // pixel tile in LDS: a wave owns a column of four 16-pixel tiles (four consecutive output rows at one x tile) and all
@@ -10,7 +9,7 @@
 // splits them in registers, once: a split row serves the three output rows it is a vertical tap of, and the three
 // horizontal taps are the same values one lane over (lane-shifting moves, with the two pixels beside the tile fetched
 // and split as a seventh row).  Out-of-image taps read zero through the buffer descriptor.  The next item's rows are
-// in flight while this one's last products are made.  The filters are split once per block into planes of 16-bit parts
+// in flight while this one's last products are made.  The filters are split once per block into three planes of bf16
 // in LDS ([plane][output channel][tap][32] with eight elements of padding per channel: a quarter wave's 16-byte reads
 // hit all banks); a filter fragment (16 channels x 32 depths of one tap) is read once per tap and used for the wave's
 // four tiles.  The output channels are the rows of the matrix instruction and the pixels its columns, so a lane ends
@@ -49,26 +48,18 @@ constexpr uint32_t kC32Oob = 0x80000000u;  // beyond the descriptor (images here
 // and c32_pool_complete_kernel takes the maxima with those afterwards.  oh must be a multiple of 4.
 //
 // NT: 16-channel tiles of the output that a block makes; NY blocks (blockIdx.y) make the cout = 16 * NT * NY channels.
-// TWO_SUMS: three bf16 parts; the five cross terms are summed by themselves, 2^-8 of the result and less, and added to the sum of
-// the hi * hi products at the end, so that a result takes 9 roundings at its own size instead of 54.  That form has the
+// TWO_SUMS: the five cross terms are summed by themselves, 2^-8 of the result and less, and added to the sum of the
+// hi * hi products at the end, so that a result takes 9 roundings at its own size instead of 54.  That form has the
 // registers for it because its blocks make 32 channels at most, which small problems want anyway (more work items).
-// Otherwise two f16 parts with a power of two per item and per filter: half the matrix instructions, two thirds of the
-// registers and lane moves.  Bound by vector instructions (32 output channels: 810 an item beside 216 matrix
-// instructions, the two hardly overlap) and for 64 channels by both.  112 x 112, 100 images: 32 channels 117 -> 101 us, 64 channels
-// with the MaxPool 211 -> 142 against six bf16 products in one sum; distance from 64-bit sums 2.4e-7 -> 1.4e-7 and 1.3e-7.
-// Both are as exact as fp32 arithmetic over fp32's whole range: items with an infinity, (bf16) a NaN or a value so small that
-// its split loses bits (below 2^-110, f16: 2^-28 of the item's or filter's largest) are made again on the fp32 matrix instruction.
+// It is as exact as fp32 arithmetic over fp32's whole range: items with an infinity, a NaN or a value so small that its
+// split loses bits (below 2^-110) are made again on the fp32 matrix instruction.
 template <int NT, int NY, int KH, int KW, bool POOL, bool TWO_SUMS>
 __global__ __launch_bounds__(kC32Threads) void fconv_c32_kernel(const FconvC32Args p) {
     constexpr int TAPS = KH * KW, PT = kC32PixelTiles, CH = 16 * NT, COUT = CH * NY;
     constexpr int ROW = TAPS * 32 + 8;     // bf16 elements per output channel in a plane
-    constexpr int PLANE = CH * ROW;        // elements per plane
-    constexpr int PLANES = TWO_SUMS ? 3 : 2;  // hi, mid, lo in bf16 / hi, lo in f16
-    // NT > 2 has no registers for a second set of sums: the cross terms of all taps first, scaled, then the hi * hi products
-    constexpr bool TWO_PASSES = !TWO_SUMS && NT > 2, TWO_SETS = !TWO_PASSES;
-    __shared__ __attribute__((aligned(16))) uint16_t planes[PLANES * PLANE];
-    __shared__ __attribute__((aligned(16))) int filter_exp[TWO_SUMS ? 4 : CH];  // f16: a filter was scaled by two to this
-    __shared__ int filter_special;  // a filter value is an infinity, (bf16) a NaN, or too small for the split
+    constexpr int PLANE = CH * ROW;        // elements per plane (hi, mid, lo)
+    __shared__ __attribute__((aligned(16))) uint16_t planes[3 * PLANE];
+    __shared__ int filter_special;  // a filter value is an infinity or a NaN (TWO_SUMS: or too small for the split)
     __shared__ int next_item;       // the first item of the block's range that no wave has taken
     // bias, Affine a and b per output channel (zeros where the layer has none): read from here when an item is written,
     // so that no load is outstanding among the stores -- loads and stores share one counter and complete in no fixed
@@ -155,7 +146,7 @@ __global__ __launch_bounds__(kC32Threads) void fconv_c32_kernel(const FconvC32Ar
         per_channel[2][tid] = p.aff_a ? p.aff_b[ch0 + tid] : 0.f;
     }
     __syncthreads();
-    if constexpr (TWO_SUMS) {
+    {
         bool special = false;
         uint32_t lost = 0;  // lower halves: what the third part could not hold
         // pairs of consecutive depths: one dword per plane
@@ -163,44 +154,19 @@ __global__ __launch_bounds__(kC32Threads) void fconv_c32_kernel(const FconvC32Ar
             const int co = idx / (TAPS * 16), r = idx - co * (TAPS * 16);  // r: pair index in the channel's 288 depths
             const float2 v = *reinterpret_cast<const float2 *>(p.w + (size_t)(ch0 + co) * (TAPS * 32) + 2 * r);
             const SplitParts s0 = split_bf16x3(v.x), s1 = split_bf16x3(v.y);
-            special |= s0.special || s1.special;
-            lost |= s0.lo | s1.lo;
+            special |= s0.hif != s0.hi || s1.hif != s1.hi;
+            if constexpr (TWO_SUMS) lost |= s0.lo | s1.lo;
             uint32_t *d = reinterpret_cast<uint32_t *>(planes + co * ROW + 2 * r);
             d[0] = pack_upper_halves(s0.hi, s1.hi);
             d[PLANE / 2] = pack_upper_halves(s0.mid, s1.mid);
             d[2 * (PLANE / 2)] = pack_upper_halves(s0.lo, s1.lo);
         }
         if (special || (lost & 0xffffu) != 0) filter_special = 1;
-    } else if (tid < CH * 8) {
-        // eight threads for a filter, which has a power of two of its own
-        const int co = tid >> 3, part = tid & 7;
-        const float2 *w = reinterpret_cast<const float2 *>(p.w + (size_t)(ch0 + co) * (TAPS * 32)) + part;
-        float2 v[TAPS * 2];
-        float largest = 0.f;
-        uint32_t smallest = ~0u;
-#pragma unroll
-        for (int k = 0; k < TAPS * 2; ++k) {
-            v[k] = w[8 * k];
-            largest = max3_magnitude(v[k].x, v[k].y, largest);
-            smallest = smallest_magnitude(smallest, v[k].x, v[k].y);
-        }
-#pragma unroll
-        for (int step = 1; step < 8; step *= 2) largest = max3_magnitude(__shfl_xor(largest, step, 8), 0.f, largest);
-        const int e = f16_scale_exponent(largest);
-        const float up = exp2_int(e), up11 = exp2_int(e + 11);
-#pragma unroll
-        for (int k = 0; k < TAPS * 2; ++k) {
-            const HalfPair sp = split_pair_f16(v[k].x, v[k].y, up, up11);
-            uint32_t *d = reinterpret_cast<uint32_t *>(planes + co * ROW + 2 * (part + 8 * k));
-            d[0] = sp.hi, d[PLANE / 2] = sp.lo;
-        }
-        if (part == 0) filter_exp[co] = e;
-        if (!(largest < __builtin_inff()) || too_small_for_f16(smallest, e)) filter_special = 1;
     }
     __syncthreads();
     const bool w_special = __builtin_amdgcn_readfirstlane(filter_special) != 0;
 
-    f32x4w acc[PT][NT], cross[TWO_SETS ? PT : 1][TWO_SETS ? NT : 1];
+    f32x4w acc[PT][NT], cross[TWO_SUMS ? PT : 1][TWO_SUMS ? NT : 1];
     // max_pool's step, `v > m ? v : m` from -FLT_MAX on, as the hardware's maximum: a NaN is passed over either way (the
     // running maximum never is one); where +0 and -0 tie the hardware gives +0 and max_pool the earlier tap, which no
     // comparison and no sign bit of the result can tell apart
@@ -241,9 +207,9 @@ __global__ __launch_bounds__(kC32Threads) void fconv_c32_kernel(const FconvC32Ar
         const size_t cell = ((size_t)at.img * (p.oh >> 1) + (at.oy0 >> 1) + (f_i & 1)) * (p.ow >> 1) + at.xt * 8 + (f_i >> 1);
         *reinterpret_cast<float4 *>(p.out + cell * COUT + ch0 + nt * 16 + 4 * g_now) = make_float4(out[0], out[1], out[2], out[3]);
     };
-    // Writes the item at `at`, whose sums are in acc, in f16 times two to `scaled` and the filters' exponents (special: an
-    // infinity among its pixels or in the filters, with TWO_SUMS a NaN, or a value too small for the split).
-    auto write_item = [&](const Place &at, bool special, int scaled) __attribute__((always_inline)) {
+    // Writes the item at `at`, whose sums are in acc (special: an infinity or a NaN among its pixels or in the filters, or
+    // with TWO_SUMS a value too small for the split).
+    auto write_item = [&](const Place &at, bool special) __attribute__((always_inline)) {
         int g_now = g;
         asm volatile("" : "+v"(g_now));  // what follows is read per item: hoisted out of the item loop it would be spilled
         if constexpr (TWO_SUMS) {
@@ -263,20 +229,6 @@ __global__ __launch_bounds__(kC32Threads) void fconv_c32_kernel(const FconvC32Ar
                         top = bits > top ? bits : top;
                     }
             special |= __builtin_amdgcn_ballot_w64(top >= 0xff000000u) != 0;
-        } else {
-#pragma unroll
-            for (int nt = 0; nt < NT; ++nt) {
-                const int4 f = *reinterpret_cast<const int4 *>(filter_exp + nt * 16 + 4 * g_now);
-                const int down[4] = {-(scaled + f.x), -(scaled + f.y), -(scaled + f.z), -(scaled + f.w)};
-#pragma unroll
-                for (int t = 0; t < PT; ++t)
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        float v = acc[t][nt][e];
-                        if constexpr (TWO_SETS) v = __builtin_fmaf(cross[t][nt][e], 1.f / 2048.f, v);
-                        acc[t][nt][e] = __builtin_ldexpf(v, down[e]);
-                    }
-            }
         }
         if (!special) {
             float bs[NT][4], as[NT][4], bb[NT][4];
@@ -363,7 +315,9 @@ __global__ __launch_bounds__(kC32Threads) void fconv_c32_kernel(const FconvC32Ar
             }
             }
         } else {
-            // The item is made again in fp32, one tile and one tap at a time.
+            // The item is made again, one tile and one tap at a time: with TWO_SUMS in fp32, otherwise with the split that
+            // keeps an infinity or a NaN whole in hi and takes copies with the non-finite values zeroed for the cross terms
+            // (Inf * 0 would make a NaN of a sum that is an infinity).
 #pragma unroll 1
             for (int nt = 0; nt < NT; ++nt) {
                 const int co = nt * 16 + 4 * g_now;
@@ -381,17 +335,28 @@ __global__ __launch_bounds__(kC32Threads) void fconv_c32_kernel(const FconvC32Ar
                         f32x4r r[2];
                         fetch(at, true, t + ty, tx, r);
                         const float v[8] = {r[0][0], r[0][1], r[0][2], r[0][3], r[1][0], r[1][1], r[1][2], r[1][3]};
-                        const float *w = p.w + (size_t)(ch0 + nt * 16 + f_i) * (TAPS * 32) + tap * 32 + 8 * g_now;
-                        const f32x4r w0 = *reinterpret_cast<const f32x4r *>(w), w1 = *reinterpret_cast<const f32x4r *>(w + 4);
+                        if constexpr (TWO_SUMS) {
+                            const float *w = p.w + (size_t)(ch0 + nt * 16 + f_i) * (TAPS * 32) + tap * 32 + 8 * g_now;
+                            const f32x4r w0 = *reinterpret_cast<const f32x4r *>(w), w1 = *reinterpret_cast<const f32x4r *>(w + 4);
 #pragma unroll
-                        for (int e = 0; e < 2; ++e) {  // four sums, a quarter of the depth each
-                            one = __builtin_amdgcn_mfma_f32_16x16x4f32(w0[e], v[e], one, 0, 0, 0);
-                            none = __builtin_amdgcn_mfma_f32_16x16x4f32(w0[e + 2], v[e + 2], none, 0, 0, 0);
-                            two = __builtin_amdgcn_mfma_f32_16x16x4f32(w1[e], v[e + 4], two, 0, 0, 0);
-                            three = __builtin_amdgcn_mfma_f32_16x16x4f32(w1[e + 2], v[e + 6], three, 0, 0, 0);
+                            for (int e = 0; e < 2; ++e) {  // four sums, a quarter of the depth each
+                                one = __builtin_amdgcn_mfma_f32_16x16x4f32(w0[e], v[e], one, 0, 0, 0);
+                                none = __builtin_amdgcn_mfma_f32_16x16x4f32(w0[e + 2], v[e + 2], none, 0, 0, 0);
+                                two = __builtin_amdgcn_mfma_f32_16x16x4f32(w1[e], v[e + 4], two, 0, 0, 0);
+                                three = __builtin_amdgcn_mfma_f32_16x16x4f32(w1[e + 2], v[e + 6], three, 0, 0, 0);
+                            }
+                            continue;
                         }
+                        SplitFrag8 px, f;
+                        px.set(v);
+                        const uint16_t *src = filter_at(nt, ty, tx);
+                        f.hi = *reinterpret_cast<const u4 *>(src), f.mid = *reinterpret_cast<const u4 *>(src + PLANE);
+                        f.lo = *reinterpret_cast<const u4 *>(src + 2 * PLANE);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) f.hif[e] = finite_bf16_pair(f.hi[e]);
+                        mfma6_16x16x32(one, none, f, px, px);
                     }
-                    one = (one + none) + (two + three);
+                    if constexpr (TWO_SUMS) one = (one + none) + (two + three);
                     const float4 fin = make_float4(finish(one[0], bias.x, fa.x, fb.x), finish(one[1], bias.y, fa.y, fb.y),
                                                    finish(one[2], bias.z, fa.z, fb.z), finish(one[3], bias.w, fa.w, fb.w));
                     if constexpr (POOL) {
@@ -419,27 +384,23 @@ __global__ __launch_bounds__(kC32Threads) void fconv_c32_kernel(const FconvC32Ar
     // loads and stores complete in no fixed order), which by then has long happened.
     Place done = here;
     bool have_done = false, done_special = false;
-    int done_scaled = 0;
     struct Row {
-        u4 hi, mid, lo;  // (f16: no mid)
+        u4 hi, mid, lo;
     };
-    auto split_row = [&](const f32x4r (&r)[2], uint32_t &running, float up, float up11) __attribute__((always_inline)) {
+    auto split_row = [&](const f32x4r (&r)[2], uint32_t &running) __attribute__((always_inline)) {
         float v[8] = {r[0][0], r[0][1], r[0][2], r[0][3], r[1][0], r[1][1], r[1][2], r[1][3]};
+        if constexpr (TWO_SUMS) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) running = smallest_magnitude(running, v[2 * e], v[2 * e + 1]);
-        // the minimum first, the split then: the compiler would keep all rows' values for a minimum taken last
-        if constexpr (TWO_SUMS)
+            for (int e = 0; e < 4; ++e) running = smallest_magnitude(running, v[2 * e], v[2 * e + 1]);
+            // the minimum first, the split then: the compiler would keep all rows' values for a minimum taken last
             asm("" : "+v"(running), "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]), "+v"(v[6]), "+v"(v[7]));
+        }
         Row out;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            if constexpr (TWO_SUMS) {
-                const SplitPair sp = split_pair_finite(v[2 * e], v[2 * e + 1]);
-                out.hi[e] = sp.hi, out.mid[e] = sp.mid, out.lo[e] = sp.lo;
-            } else {
-                const HalfPair sp = split_pair_f16(v[2 * e], v[2 * e + 1], up, up11);
-                out.hi[e] = sp.hi, out.lo[e] = sp.lo;
-            }
+            const SplitPair sp = split_pair_finite(v[2 * e], v[2 * e + 1]);
+            out.hi[e] = sp.hi, out.mid[e] = sp.mid, out.lo[e] = sp.lo;
+            if constexpr (!TWO_SUMS) running = bf16_pair_max(running, sp.hi);
         }
         return out;
     };
@@ -449,40 +410,26 @@ __global__ __launch_bounds__(kC32Threads) void fconv_c32_kernel(const FconvC32Ar
         const int next_index = __builtin_amdgcn_readfirstlane(taken);
         const Place next = locate(next_index);
         const bool next_ok = next_index < last;
-        uint32_t running = ~0u;
-        float largest = 0.f, up = 1.f, up11 = 1.f;
-        int scaled = 0;
-        if constexpr (!TWO_SUMS) {  // the power of two of the item's pixels
-            auto enlarge = [&](const f32x4r (&r)[2]) __attribute__((always_inline)) {
-#pragma unroll
-                for (int k = 0; k < 2; ++k) largest = max3_magnitude(r[k][2], r[k][3], max3_magnitude(r[k][0], r[k][1], largest));
-            };
-#pragma unroll
-            for (int j = 0; j < ROWS; ++j) enlarge(raw[j]);
-            enlarge(raw_halo);
-            largest = wave_max(largest);
-            scaled = f16_scale_exponent(largest);
-            up = exp2_int(scaled), up11 = exp2_int(scaled + 11);
-        }
+        uint32_t running = TWO_SUMS ? ~0u : 0u;
         // Every pixel is fetched and split once: the pixels of horizontal tap 1, and the halo.  Taps 0 and 2 are the
         // same values one lane over (a lane's neighbours in its group of 16 hold the neighbouring pixels' same eight
         // channels), moved with the lane-shifting form of v_mov; the end lane takes its value from the halo row.
         Row centre[ROWS];
 #pragma unroll
-        for (int j = 0; j < ROWS; ++j) centre[j] = split_row(raw[j], running, up, up11);
-        const Row halo = split_row(raw_halo, running, up, up11);
+        for (int j = 0; j < ROWS; ++j) centre[j] = split_row(raw[j], running);
+        const Row halo = split_row(raw_halo, running);
 
-        if (have_done) write_item(done, done_special, done_scaled);
+        if (have_done) write_item(done, done_special);
 #pragma unroll
         for (int t = 0; t < PT; ++t)
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt) {
                 acc[t][nt] = f32x4w{0.f, 0.f, 0.f, 0.f};
-                if constexpr (TWO_SETS) cross[t][nt] = acc[t][nt];
+                if constexpr (TWO_SUMS) cross[t][nt] = acc[t][nt];
             }
 
         // input row j as horizontal tap TX sees it
-        auto shifted = [&](auto tx_c, auto j_c, auto with_lo) __attribute__((always_inline)) {
+        auto shifted = [&](auto tx_c, auto j_c) __attribute__((always_inline)) {
             constexpr int TX = decltype(tx_c)::value, J = decltype(j_c)::value;
             if constexpr (TX == 1) {
                 return centre[J];
@@ -502,102 +449,60 @@ __global__ __launch_bounds__(kC32Threads) void fconv_c32_kernel(const FconvC32Ar
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     out.hi[e] = move(centre[J].hi[e], halo.hi[e]);
-                    if constexpr (TWO_SUMS) out.mid[e] = move(centre[J].mid[e], halo.mid[e]);
-                    if constexpr (decltype(with_lo)::value) out.lo[e] = move(centre[J].lo[e], halo.lo[e]);
+                    out.mid[e] = move(centre[J].mid[e], halo.mid[e]);
+                    out.lo[e] = move(centre[J].lo[e], halo.lo[e]);
                 }
                 return out;
             }
         };
         auto frag = [](const u4 &h, const u4 &m, const u4 &l) {
             SplitFrag8 f;
-            f.hi = h, f.mid = m, f.lo = l;
+            f.hi = h, f.hif = h, f.mid = m, f.lo = l;
             return f;
         };
         auto of_row = [&](const Row &r) { return frag(r.hi, r.mid, r.lo); };
         // rows of the product = output channels (the filter fragment), columns = pixels; output row t takes input row
         // t + ty.  The rows of a tap are made as the vertical taps first need them: four, then one, then one.
-        // CROSS / MAIN: the cross terms, the hi * hi products or both.
-        auto phase = [&](auto tx_c, auto cross_c, auto main_c, auto &&after_first) __attribute__((always_inline)) {
+        auto phase = [&](auto tx_c, auto &&after_first) __attribute__((always_inline)) {
             constexpr int TX = decltype(tx_c)::value;
-            constexpr bool CROSS = decltype(cross_c)::value, MAIN = decltype(main_c)::value;
-            auto row = [&](auto j_c) __attribute__((always_inline)) { return shifted(tx_c, j_c, cross_c); };
-            const Row r0 = row(std::integral_constant<int, 0>{}), r1 = row(std::integral_constant<int, 1>{});
-            const Row r2 = row(std::integral_constant<int, 2>{}), r3 = row(std::integral_constant<int, 3>{});
+            Row r0 = shifted(tx_c, std::integral_constant<int, 0>{}), r1 = shifted(tx_c, std::integral_constant<int, 1>{});
+            Row r2 = shifted(tx_c, std::integral_constant<int, 2>{}), r3 = shifted(tx_c, std::integral_constant<int, 3>{});
             auto products = [&](int ty, const Row &a, const Row &b, const Row &c, const Row &d) __attribute__((always_inline)) {
 #pragma unroll
                 for (int nt = 0; nt < NT; ++nt) {
                     const uint16_t *src = filter_at(nt, ty, TX);
+                    const SplitFrag8 f = frag(*reinterpret_cast<const u4 *>(src), *reinterpret_cast<const u4 *>(src + PLANE),
+                                              *reinterpret_cast<const u4 *>(src + 2 * PLANE));
                     if constexpr (TWO_SUMS) {
-                        const SplitFrag8 f = frag(*reinterpret_cast<const u4 *>(src), *reinterpret_cast<const u4 *>(src + PLANE),
-                                                  *reinterpret_cast<const u4 *>(src + 2 * PLANE));
                         mfma6_16x16x32_two_sums(acc[0][nt], acc[1][nt], cross[0][nt], cross[1][nt], f, of_row(a), of_row(b));
                         mfma6_16x16x32_two_sums(acc[2][nt], acc[3][nt], cross[2][nt], cross[3][nt], f, of_row(c), of_row(d));
                     } else {
-                        const u4 hi = *reinterpret_cast<const u4 *>(src);
-                        const Row *px[PT] = {&a, &b, &c, &d};
-                        auto add = [&](f32x4w (&sum)[PT][NT], u4 f, auto part) __attribute__((always_inline)) {
-#pragma unroll
-                            for (int t = 0; t < PT; ++t)
-                                sum[t][nt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, f), __builtin_bit_cast(f16x8, part(*px[t])), sum[t][nt], 0, 0, 0);
-                        };
-                        auto hi_of = [](const Row &r) { return r.hi; };
-                        auto lo_of = [](const Row &r) { return r.lo; };
-                        if constexpr (CROSS) {
-                            const u4 lo = *reinterpret_cast<const u4 *>(src + PLANE);
-                            if constexpr (TWO_SETS) {
-                                add(cross, lo, hi_of);
-                                if constexpr (MAIN) add(acc, hi, hi_of);
-                                add(cross, hi, lo_of);
-                            } else {
-                                add(acc, lo, hi_of);
-                                add(acc, hi, lo_of);
-                            }
-                        } else {
-                            add(acc, hi, hi_of);
-                        }
+                        mfma6_16x16x32(acc[0][nt], acc[1][nt], f, of_row(a), of_row(b));
+                        mfma6_16x16x32(acc[2][nt], acc[3][nt], f, of_row(c), of_row(d));
                     }
                 }
                 __builtin_amdgcn_sched_barrier(0);  // rows and filter fragments are made as they are needed, not up front
             };
             products(0, r0, r1, r2, r3);
             after_first();
-            const Row r4 = row(std::integral_constant<int, 4>{});
+            const Row r4 = shifted(tx_c, std::integral_constant<int, 4>{});
             products(1, r1, r2, r3, r4);
-            const Row r5 = row(std::integral_constant<int, 5>{});
+            const Row r5 = shifted(tx_c, std::integral_constant<int, 5>{});
             products(2, r2, r3, r4, r5);
         };
-        using std::integral_constant;
-        auto fetch_next = [&]() __attribute__((always_inline)) {
+        phase(std::integral_constant<int, 1>{}, [] {});
+        phase(std::integral_constant<int, 0>{}, [] {});
+        phase(std::integral_constant<int, 2>{}, [&]() __attribute__((always_inline)) {
 #pragma unroll
             for (int j = 0; j < ROWS; ++j) fetch(next, next_ok, j, 1, raw[j]);
             fetch_halo(next, next_ok, raw_halo);
-        };
-        constexpr std::true_type yes{};
-        constexpr std::false_type no{};
-        if constexpr (TWO_PASSES) {
-            phase(integral_constant<int, 1>{}, yes, no, [] {});
-            phase(integral_constant<int, 0>{}, yes, no, [] {});
-            phase(integral_constant<int, 2>{}, yes, no, [] {});
-#pragma unroll
-            for (int t = 0; t < PT; ++t)
-#pragma unroll
-                for (int nt = 0; nt < NT; ++nt) acc[t][nt] = acc[t][nt] * (1.f / 2048.f);
-            phase(integral_constant<int, 2>{}, no, yes, [] {});
-            phase(integral_constant<int, 0>{}, no, yes, fetch_next);
-            phase(integral_constant<int, 1>{}, no, yes, [] {});
-        } else {
-            phase(integral_constant<int, 1>{}, yes, yes, [] {});
-            phase(integral_constant<int, 0>{}, yes, yes, [] {});
-            phase(integral_constant<int, 2>{}, yes, yes, fetch_next);
-        }
+        });
 
         done = here, have_done = true;
-        done_scaled = scaled;
-        done_special = w_special || !(largest < __builtin_inff()) ||
-                       __builtin_amdgcn_ballot_w64(TWO_SUMS ? loses_bits_when_split(running) : too_small_for_f16(running, scaled)) != 0;
+        done_special = w_special || __builtin_amdgcn_ballot_w64(TWO_SUMS ? loses_bits_when_split(running) : !bf16_pairs_finite(running)) != 0;
         here = next, item = next_index;
     }
-    if (have_done) write_item(done, done_special, done_scaled);
+    if (have_done) write_item(done, done_special);
 }
 
 // The pass behind fconv_c32_kernel<..., POOL>: a pooled cell of an even pooled row (the first of its tile column) takes
@@ -690,8 +595,8 @@ bool fconv_c32_many_items(int n, int oh, int ow) {
 // (14.8 / 12.2), 6 images 22.7 / 15.5 (28.7 / 20.6), 20 images 52 / 32 (60 / 39); 64 channels, 1 image 11.2 / 9.4
 // (15.7 / 12.9), 6 images 36.0 / 22.5 (44.0 / 29.4), 20 images 85 / 49 (102 / 58).  Blocks of 16 against 32 of the 64
 // channels: 25.4 / 24.8 at 4 images, 35.8 / 38.1 at 8, 44.4 / 42.4 at 12, 62 / 59 at 20: the line is at one item per wave.
-// Distance from 64-bit sums, relative: 8.3e-8, the f16 form 1.4e-7 (so it does not take these sizes over), the fp32 kernels
-// 2.2e-7; with pixels or filters around 2^-120 1.6e-7, as the fp32 kernels (from the split 3.5e-5 and 1.2e-3).  Looking for such values costs 0.2 us of a lone
+// Distance from 64-bit sums, relative: 8.3e-8, the fp32 kernels 2.2e-7 and one sum 2.4e-7; with pixels or filters around
+// 2^-120 1.6e-7, as the fp32 kernels (from the split 3.5e-5 and 1.2e-3).  Looking for such values costs 0.2 us of a lone
 // item's 7.4 and nothing that shows from 196 items on.
 template <bool POOL>
 static int launch_c32(const FconvC32Args &a, hipStream_t s, const char *what) {
