@@ -295,84 +295,6 @@ __device__ __forceinline__ void mfma6_16x16x32_two_sums(f32x4w &acc0, f32x4w &ac
 #undef DAB_MFMA2
 }
 
-// ---------------------------------------------------------------- fp32 products on the f16 matrix cores
-// The same with two parts of 11 significand bits: X = x * 2^s, hi = f16(X), lo = f16((X - hi) * 2^11), so that
-// x = (hi + lo * 2^-11) * 2^-s to 2^-23 of its size, and x*w is hi*hi + 2^-11 * (lo*hi + hi*lo) but for terms below 2^-22: three
-// matrix instructions where bf16 needs six, the scaled cross terms in a sum of their own.  Distance from 64-bit sums over 160 and
-// 288 normally distributed products: 1.16e-7 and 1.36e-7 of the result (2-norm), the six bf16 products in one sum 1.76e-7 and
-// 2.45e-7, the fp32 instruction 2.27e-7 and 3.05e-7; the six bf16 products in two sums 7.1e-8 and 9.5e-8, so forms that have the
-// registers for those and are not bound by the matrix cores keep them.
-// f16 has five exponent bits, so the values that share a scale must not be too far apart: s puts the largest magnitude into
-// [2^14, 2^15), and a value that is then not zero and below 2^-14 has no full hi part.  Callers look for such values (and for
-// infinities) and make their sums on the fp32 instruction.  A NaN makes a NaN of all sums that it is in, as it should.
-typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-
-// The power of two for a group of values whose largest magnitude is `largest` (not an infinity; zero: any).  At most 100, so that 2^(s + 11) is
-// a float; groups below 2^-86 then keep less than their 28 octaves.
-__device__ __forceinline__ int f16_scale_exponent(float largest) {
-    const int e = (int)(__builtin_bit_cast(uint32_t, largest) >> 23) - 127;
-    const int s = 14 - e;
-    return s < 100 ? s : 100;
-}
-__device__ __forceinline__ float exp2_int(int e) { return __builtin_bit_cast(float, (uint32_t)(127 + e) << 23); }  // -126 .. 127
-// Whether the running minimum of smallest_magnitude() lies below 2^-14 once scaled by 2^s.
-__device__ __forceinline__ bool too_small_for_f16(uint32_t running, int s) { return running < ((uint32_t)(127 - 14 - s) << 24) - 1u; }
-struct HalfPair {
-    uint32_t hi, lo;  // two f16 each, the first value in the lower half
-};
-// up = 2^s, up11 = 2^(s + 11)
-__device__ __forceinline__ HalfPair split_pair_f16(float x0, float x1, float up, float up11) {
-    // three instructions a value: conversions fused with the products (v_fma_mixlo_f16, v_fma_mixhi_f16)
-    const f16x2 h = {(_Float16)__builtin_fmaf(x0, up, 0.f), (_Float16)__builtin_fmaf(x1, up, 0.f)};
-    HalfPair r;
-    r.hi = __builtin_bit_cast(uint32_t, h);
-    asm("" : "+v"(r.hi));  // seeing through this, the compiler makes both halves a second time for what follows
-    const f16x2 k = __builtin_bit_cast(f16x2, r.hi);
-    const f16x2 l = {(_Float16)__builtin_fmaf((float)k.x, -2048.f, x0 * up11), (_Float16)__builtin_fmaf((float)k.y, -2048.f, x1 * up11)};
-    r.lo = __builtin_bit_cast(uint32_t, l);
-    return r;
-}
-// max(|a|, |b|, m), passing over NaNs
-__device__ __forceinline__ float max3_magnitude(float a, float b, float m) {
-    float r;
-    asm("v_max3_f32 %0, |%1|, |%2|, %3" : "=v"(r) : "v"(a), "v"(b), "v"(m));
-    return r;
-}
-// The largest of the wave's values (none below zero), the same in every lane.
-__device__ __forceinline__ float wave_max(float v) {
-    int m = __builtin_bit_cast(int, v);  // bits of floats >= 0 are ordered as integers
-    auto step = [&](auto ctrl, auto rows) {
-        const int o = __builtin_amdgcn_update_dpp(0, m, decltype(ctrl)::value, decltype(rows)::value, 0xf, false);
-        m = o > m ? o : m;
-    };
-    using std::integral_constant;
-    step(integral_constant<int, 0x111>{}, integral_constant<int, 0xf>{});  // row_shr:1, 2, 4, 8: lane 15 of a row has the row's
-    step(integral_constant<int, 0x112>{}, integral_constant<int, 0xf>{});
-    step(integral_constant<int, 0x114>{}, integral_constant<int, 0xf>{});
-    step(integral_constant<int, 0x118>{}, integral_constant<int, 0xf>{});
-    step(integral_constant<int, 0x142>{}, integral_constant<int, 0xa>{});  // row_bcast:15 into rows 1 and 3
-    step(integral_constant<int, 0x143>{}, integral_constant<int, 0xc>{});  // row_bcast:31 into rows 2 and 3
-    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(m, 63));
-}
-
-// Eight consecutive depths of one row or column as two planes of eight f16, and
-// acc += A * B, cross += 2^11 * (its cross terms), as mfma6_16x16x32_two_sums.
-struct HalfFrag8 {
-    typedef uint32_t u4 __attribute__((ext_vector_type(4)));
-    u4 hi, lo;
-};
-__device__ __forceinline__ void mfma3_16x16x32(f32x4w &acc0, f32x4w &acc1, f32x4w &cross0, f32x4w &cross1, const HalfFrag8 &a, const HalfFrag8 &b0,
-                                               const HalfFrag8 &b1) {
-    auto v = [](HalfFrag8::u4 w) { return __builtin_bit_cast(f16x8, w); };
-    cross0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(v(a.lo), v(b0.hi), cross0, 0, 0, 0);
-    cross1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(v(a.lo), v(b1.hi), cross1, 0, 0, 0);
-    acc0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(v(a.hi), v(b0.hi), acc0, 0, 0, 0);
-    acc1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(v(a.hi), v(b1.hi), acc1, 0, 0, 0);
-    cross0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(v(a.hi), v(b0.lo), cross0, 0, 0, 0);
-    cross1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(v(a.hi), v(b1.lo), cross1, 0, 0, 0);
-}
-
 // ---------------------------------------------------------------- buffer resources
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x3 __attribute__((ext_vector_type(3)));

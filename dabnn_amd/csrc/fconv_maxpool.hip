@@ -363,50 +363,47 @@ __global__ __launch_bounds__(kBandThreads) void fconv_maxpool_kernel(const Fconv
 // channels; an output pixel's 21 values of one kernel row are contiguous (tile elements 6*ox + k', k' = 3*tx + ch),
 // so a lane's operand addresses are a base plus constants.
 //
-// The products run on the f16 matrix cores with fp32 accuracy (split operands, three v_mfma_f32_16x16x32_f16 per 32 depths;
-// common.h): 48 cycles where the eight fp32 instructions for the same depth take 256 and six bf16 ones 96.  A band's rows are
-// split once, on their way into LDS, into two planes of f16 (hi, lo) with the band's own power of two, and so are the block's
-// 64 filters, each with its own, once for all of the block's bands, in the order the instruction wants them (a lane's eight depths
-// are 16 contiguous bytes).  A band whose rows or filters hold an infinity, or a value 2^28 times smaller than the largest one that
-// it shares its power of two with, is multiplied on the fp32 instruction from memory instead -- flags in LDS say so.
-// Batch 256, 224 x 224 x 3 -> 64 with Affine and sign bits: 408 -> 295 us, batch 40: 80 -> 61 (before: six bf16 products, three
-// planes, rows and staged band in one LDS area); 312 with a tile row 692 elements long, whose half-wave reads met in banks.
-// Relative distance from 64-bit sums 1.6e-7 -> 9.3e-8.  Per band a wave issues 210 matrix instructions and 1 100 others, which
-// now bound it together: the three phases below still add up.
-//
-// A depth group is four slots of eight depths, slot g = lane / 16; the 147 depths make 19 slots: q = 0..11: kernel row
-// 2 * (q / 4) + q % 2 (the two slots of a half-wave are rows next to each other), k' = 0..7 or 8..15; q = 12, 13: the same of kernel
-// row 6; q = 14..17: k' = 16..19 of kernel rows (0, 1), (2, 3), (4, 5), (6, none); q = 18: k' = 20 of the seven
+// The products run on the bf16 matrix cores with fp32 accuracy (split operands, six v_mfma_f32_16x16x32_bf16 per 32
+// depths; common.h): the instruction takes 19 cycles where the eight fp32 ones for the same depth take 256.  The tile
+// is split once, on its way into LDS, into three planes of bf16 (hi, mid, lo), and so are the block's 64 filters, once
+// for all of its bands, in the order the instruction wants them (a lane's eight depths are 16 contiguous bytes).  The
+// cross terms need hi with non-finite values taken out (common.h); a band with an infinity or a NaN in its rows or in
+// the filters -- flags in LDS say so -- takes a second copy of the loop that derives it from hi in registers, all
+// other bands use hi as it is.  A depth group is
+// four slots of eight depths, slot g = lane / 16; the 147 depths make 19 slots: q = 0..13: kernel row q / 2, k' = 0..7
+// or 8..15; q = 14..17: k' = 16..19 of kernel rows (0, 1), (2, 3), (4, 5), (6, none); q = 18: k' = 20 of the seven
 // kernel rows, which a second small array per plane holds transposed (T20[ox][tile row]) so that they are contiguous
 // too; q = 19 is empty.  Empty halves read a zero area of the plane; the eighth element of slot 18 is masked (it is a
-// real tile value, and zero times a NaN would be a NaN).  160 depths for 147, five groups.
-// The next band's rows are fetched into registers while the current one is multiplied and split while it is pooled: planes and
-// staged maxima have LDS of their own, so a band takes two barriers.  Pooling starts in registers: a lane holds four
-// neighbouring pixels of a row, so the maxima over the columns 2*px-1 .. 2*px+1 of two pooled columns
+// real tile value, and zero times an infinity would be a NaN).  160 depths for 147, five groups.
+// The next band's rows are fetched into registers while the current one is pooled.  Pooling starts in registers: a
+// lane holds four neighbouring pixels of a row, so the maxima over the columns 2*px-1 .. 2*px+1 of two pooled columns
 // need one value from the lane 16 below; only those maxima -- half of the band -- are staged in LDS for the pass
 // down the rows.
+constexpr int kTileStride = 692;                    // elements per tile row: 115 pixel pairs x 6, + 2
 constexpr int kTileRows = 13, kTilePairs = 115;
-constexpr int kTileStride = 736;                    // elements per tile row: 115 pixel pairs x 6, and 16 banks of 32 from row to row
-constexpr int kPlaneZero = kTileRows * kTileStride;  // eight zeros behind the tile's elements
+constexpr int kPlaneZero = 9000;                    // eight zeros behind the 13 x 692 tile elements
 constexpr int kPlaneT20 = kPlaneZero + 8;           // [112 output columns][16]: tile rows of element 6 * ox + 20
-constexpr int kPlane = kPlaneT20 + 112 * 16;        // f16 elements per plane
+constexpr int kPlane = kPlaneT20 + 112 * 16;        // bf16 elements per plane
 constexpr int kStemDepth = 160;                     // 5 groups x 4 slots x 8
-constexpr int kFilterRow = kStemDepth + 8;          // f16 elements per filter in a plane
+constexpr int kFilterRow = kStemDepth + 8;          // bf16 elements per filter in a plane
 constexpr int kFilterPlane = kBandChannels * kFilterRow;
 constexpr int kStemStageStride = 72;                // floats per pooled column of the staged maxima: two columns on are 16 banks on
 constexpr int kStemStageFloats = 4 * 56 * kStemStageStride;
+constexpr int kStemWorkBytes = 3 * kPlane * 2 > kStemStageFloats * 4 ? 3 * kPlane * 2 : kStemStageFloats * 4;  // the planes share the staged maxima's space
 constexpr int kPairLoads = (kTileRows * kTilePairs + kBandThreads - 1) / kBandThreads;
 constexpr int kStemKeepSlots = 2;  // 56 pooled columns x 16 channel groups on 512 threads
 static_assert(56 * 16 <= kStemKeepSlots * kBandThreads, "pooled columns of the stem");
 static_assert(kTileStride * kTileRows <= kPlaneZero && (kPlaneT20 * 2) % 16 == 0 && (kPlane * 2) % 16 == 0, "plane layout");
-static_assert((kFilterRow * 2) % 16 == 0, "filter rows are 16-byte aligned");
+static_assert((kFilterRow * 2) % 16 == 0 && kStemWorkBytes % 16 == 0, "filter rows and the work area are 16-byte aligned");
 
 // The stem's finished band (accumulator element e of lane l: pixel 16*i + 4*(l/16) + e of row wm, channel l % 16 of
 // tile j): + bias, Affine (a*v + b, two roundings), Relu, in the reference's order; then the maxima over the columns
-// of the two pooled columns 8*i + 2*(l/16) and the next one go to LDS; stem_pool, behind a barrier, walks down the four rows.
+// of the two pooled columns 8*i + 2*(l/16) and the next one go to LDS, and pool_band_rows walks down the four rows.
 // All threads of the block call it after a barrier that ended every other use of `stage`.
-__device__ __forceinline__ void stem_stage(const FconvPoolArgs &p, float *stage, const f32x4v (&acc)[7][2], const BandOut o, int tid, int wm,
-                                           int wn, int f_s, int f_i) {
+template <bool SIGN>
+__device__ __forceinline__ void stem_epilogue(const FconvPoolArgs &p, float *stage, const f32x4v (&acc)[7][2], const BandOut o,
+                                              int tid, int wm, int wn, int f_s, int f_i, float4 (&keep)[kStemKeepSlots],
+                                              bool fold, bool write_carry) {
     constexpr int TM = 7, TN = 2;
     const int below = (((tid & 63) - 16) & 63) * 4;  // ds_bpermute address of the lane 16 below (lanes 0..15: 48 above)
     auto stage_all = [&](auto has_bias, auto has_affine, auto has_relu) {
@@ -453,10 +450,7 @@ __device__ __forceinline__ void stem_stage(const FconvPoolArgs &p, float *stage,
         case 6: stage_all(T{}, T{}, F{}); break;
         default: stage_all(T{}, T{}, T{}); break;
     }
-}
-template <bool SIGN>
-__device__ __forceinline__ void stem_pool(const FconvPoolArgs &p, const float *stage, const BandOut o, int tid, float4 (&keep)[kStemKeepSlots],
-                                          bool fold, bool write_carry) {
+    __syncthreads();
     pool_band_rows<SIGN, kStemKeepSlots, 4>(p, o, tid, keep, fold, write_carry, [&](int px, int c4) {
         const float *col = &stage[px * kStemStageStride + c4 * 4];
         return [=](int r) { return *reinterpret_cast<const float4 *>(col + r * (56 * kStemStageStride)); };
@@ -466,14 +460,12 @@ __device__ __forceinline__ void stem_pool(const FconvPoolArgs &p, const float *s
 template <bool SIGN>
 __global__ __launch_bounds__(kBandThreads) void fconv7x7s2_maxpool_kernel(const FconvPoolArgs p) {
     constexpr int BN = kBandChannels, TM = 7, TN = 2;
-    __shared__ __attribute__((aligned(16))) uint16_t fplanes[2 * kFilterPlane];  // the filters: hi, lo
-    __shared__ __attribute__((aligned(16))) uint16_t planes[2 * kPlane];         // the band's rows: hi, lo
-    __shared__ __attribute__((aligned(16))) float stage[kStemStageFloats];
-    __shared__ int filter_exp[BN];      // a filter was scaled by two to this
-    __shared__ int special_filters;     // 1 + the first channel of a channel tile with a filter that f16 parts cannot hold, or 0
-    // of the band at hand and the next one, in turn: the bits of the largest magnitude of its rows, and whether they hold a
-    // value that f16 parts cannot
-    __shared__ int rows_max[2], rows_special[2];
+    typedef uint32_t u32x2a __attribute__((ext_vector_type(2), aligned(4)));
+    __shared__ __attribute__((aligned(16))) uint16_t fplanes[3 * kFilterPlane];  // the filters: hi, mid, lo
+    __shared__ __attribute__((aligned(16))) float stage[kStemWorkBytes / 4];
+    uint16_t *const planes = reinterpret_cast<uint16_t *>(stage);  // the band's rows: hi, mid, lo, kPlane elements each
+    __shared__ int special_flag;    // the band's rows hold an infinity or a NaN
+    __shared__ int special_filters;  // 1 + the first channel of a channel tile whose filters hold one, or 0
 
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = wave >> 1, wn = wave & 1;
@@ -508,22 +500,20 @@ __global__ __launch_bounds__(kBandThreads) void fconv7x7s2_maxpool_kernel(const 
     };
     typedef float f32x3v __attribute__((ext_vector_type(3)));
     f32x3v pf0[kPairLoads], pf1[kPairLoads];
-    BandOut at;
+    int img, band, row0, n0;
     auto enter = [&](int it) {
         const int bi = (int)p.div_ytiles.div((uint32_t)it);
-        at.ytile = it - bi * p.ytiles;
-        at.n0 = at.ytile * BN;
-        at.img = (int)p.div_bands.div((uint32_t)bi);
-        at.band = bi - at.img * p.bands;
-        at.row0 = at.band * 4;
+        n0 = (it - bi * p.ytiles) * BN;
+        img = (int)p.div_bands.div((uint32_t)bi);
+        band = bi - img * p.bands;
+        row0 = band * 4;
     };
-    // One descriptor per image: rows above and below it have offsets that are negative modulo 2^32 or at least
-    // the image's size, and read as zero; columns outside carry kPoolOob, which stays out of range after the
-    // addition of a row offset of magnitude below 2^30.
-    auto image_rsrc = [&](int img) { return make_rsrc(p.x + (size_t)img * p.h * p.wd * 3, img_bytes); };
     auto fetch_tile = [&]() {
-        const auto x_rsrc = image_rsrc(at.img);
-        const uint32_t base = (uint32_t)((2 * at.row0 - 3) * p.wd * 12);
+        // One descriptor per image: rows above and below it have offsets that are negative modulo 2^32 or at least
+        // the image's size, and read as zero; columns outside carry kPoolOob, which stays out of range after the
+        // addition of a row offset of magnitude below 2^30.
+        const auto x_rsrc = make_rsrc(p.x + (size_t)img * p.h * p.wd * 3, img_bytes);
+        const uint32_t base = (uint32_t)((2 * row0 - 3) * p.wd * 12);
 #pragma unroll
         for (int j = 0; j < kPairLoads; ++j) {
             const PairPlace q = pair_place(j);
@@ -531,246 +521,194 @@ __global__ __launch_bounds__(kBandThreads) void fconv7x7s2_maxpool_kernel(const 
             pf1[j] = __builtin_bit_cast(f32x3v, __builtin_amdgcn_raw_buffer_load_b96(x_rsrc, (int)(base + q.off1), 0, 0));
         }
     };
-    // the fetched rows' largest magnitude goes into rows_max[slot] (a block's threads all call it, a barrier follows)
-    auto publish_max = [&](int slot) {
-        float m = 0.f;
+
+    // lane constants of the tile reads: the plane elements of a slot's two halves of four (tile i of the wave's
+    // row: + 96 * i; slot 18: + 256 * i; the zero area: + 0).  Groups 0..2 and the first two slots of group 3 are
+    // eight consecutive k' of kernel row 2 * G + g / 2: group 0's offsets plus a constant.  The other slots of group
+    // 3 and group 4 have offsets of their own.  (The filter planes are laid out slot by slot when they are filled.)
+    const int base_a = 2 * wm * kTileStride + 6 * f_i;
+    const int a_main = base_a + (f_s >> 1) * kTileStride + 8 * (f_s & 1);
+    // group 3: slots 12, 13 (kernel row 6), 14, 15 (k' = 16..19 of kernel rows (0, 1) and (2, 3))
+    const int a0_g3 = f_s < 2 ? a_main + 6 * kTileStride : base_a + 2 * (f_s - 2) * kTileStride + 16;
+    const int a1_g3 = a0_g3 + (f_s < 2 ? 4 : kTileStride);
+    // group 4: slots 16 (kernel rows 4, 5), 17 (row 6, nothing), 18 (k' = 20 of all rows), 19 (nothing)
+    const int a0_g4 = f_s < 2 ? base_a + (4 + 2 * f_s) * kTileStride + 16 : f_s == 2 ? kPlaneT20 + f_i * 16 + 2 * wm : kPlaneZero;
+    const int a1_g4 = f_s == 0 ? a0_g4 + kTileStride : f_s == 2 ? a0_g4 + 4 : kPlaneZero;
+    const int s0_g4 = f_s < 2 ? 96 : f_s == 2 ? 256 : 0, s1_g4 = f_s == 0 ? 96 : f_s == 2 ? 256 : 0;
+    const uint32_t keep_g4 = f_s == 2 ? 0x0000ffffu : 0xffffffffu;  // slot 18: seven kernel rows, the eighth element out
+
+    enter(item);
+    fetch_tile();
+    if (tid == 0) special_flag = 0, special_filters = 0;
+    __syncthreads();
+    int filters_of = -1;  // the channel tile whose filters are in LDS
+    for (;;) {
+        // here: the band's rows are in registers (or on their way), every thread is past its last read of the LDS
+        if (n0 != filters_of) {
+            filters_of = n0;
+            const int rows_n = p.cout - n0 < BN ? p.cout - n0 : BN;
+            bool special = false;
+            // two consecutive places of a filter's 160: slot q = place / 8, element t = place % 8
+            for (int idx = tid; idx < BN * (kStemDepth / 2); idx += kBandThreads) {
+                const int co = idx / (kStemDepth / 2), pr = idx - co * (kStemDepth / 2);
+                SplitParts sp[2];
 #pragma unroll
-        for (int j = 0; j < kPairLoads; ++j) {
-            m = max3_magnitude(pf0[j][0], pf0[j][1], m);
-            m = max3_magnitude(pf0[j][2], pf1[j][0], m);
-            m = max3_magnitude(pf1[j][1], pf1[j][2], m);
+                for (int e = 0; e < 2; ++e) {
+                    const int q = (2 * pr + e) >> 3, t = (2 * pr + e) & 7;
+                    int k = -1;  // the place's depth in the filter's (kernel row, k') order
+                    if (q < 14) {
+                        k = (q >> 1) * 21 + 8 * (q & 1) + t;
+                    } else if (q < 18) {
+                        const int ky = 2 * (q - 14) + (t >> 2);
+                        if (ky < 7) k = ky * 21 + 16 + (t & 3);
+                    } else if (q == 18 && t < 7) {
+                        k = t * 21 + 20;
+                    }
+                    sp[e] = split_bf16x3((co < rows_n && k >= 0) ? p.w[(size_t)(n0 + co) * 147 + k] : 0.f);
+                    special |= sp[e].hif != sp[e].hi;
+                }
+                uint32_t *d = reinterpret_cast<uint32_t *>(fplanes + co * kFilterRow + 2 * pr);
+                d[0] = pack_upper_halves(sp[0].hi, sp[1].hi);
+                d[kFilterPlane / 2] = pack_upper_halves(sp[0].mid, sp[1].mid);
+                d[2 * (kFilterPlane / 2)] = pack_upper_halves(sp[0].lo, sp[1].lo);
+            }
+            if (special) special_filters = n0 + 1;
         }
-        m = wave_max(m);
-        if (lane == 0) atomicMax(&rows_max[slot], __builtin_bit_cast(int, m));
-    };
-    // the fetched rows as f16 parts
-    auto split_rows = [&](int slot) {
-        const float largest = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(rows_max[slot]));
-        const int s = f16_scale_exponent(largest);
-        const float up = exp2_int(s), up11 = exp2_int(s + 11);
-        uint32_t smallest = ~0u;
-        if (tid < 8) reinterpret_cast<uint32_t *>(planes + (tid >> 2) * kPlane + kPlaneZero)[tid & 3] = 0u;
+        if (tid < 12) reinterpret_cast<uint32_t *>(planes + (tid >> 2) * kPlane + kPlaneZero)[tid & 3] = 0u;
+        bool any_special = false;
 #pragma unroll
         for (int j = 0; j < kPairLoads; ++j) {
             const PairPlace q = pair_place(j);
             if (q.lds >= 0) {
+                // the six values as three pairs through the packed conversions; a triple with an infinity, a NaN or a
+                // value that rounds up to an infinity is split again the slow way (and sends the band through the
+                // loop that derives the finite parts, which is right for finite values too)
                 const float v[6] = {pf0[j][0], pf0[j][1], pf0[j][2], pf1[j][0], pf1[j][1], pf1[j][2]};
-                HalfPair sp[3];
+                SplitPair sp[3];
+                uint32_t magnitudes = 0;
+#pragma unroll
+                for (int e = 0; e < 3; ++e) {
+                    sp[e] = split_pair_finite(v[2 * e], v[2 * e + 1]);
+                    magnitudes = bf16_pair_max(magnitudes, sp[e].hi);
+                }
+                if (!bf16_pairs_finite(magnitudes)) {
+                    any_special = true;
+#pragma unroll
+                    for (int e = 0; e < 3; ++e) {
+                        const SplitParts s0 = split_bf16x3(v[2 * e]), s1 = split_bf16x3(v[2 * e + 1]);
+                        sp[e].hi = pack_upper_halves(s0.hi, s1.hi);
+                        sp[e].mid = pack_upper_halves(s0.mid, s1.mid);
+                        sp[e].lo = pack_upper_halves(s0.lo, s1.lo);
+                    }
+                }
                 uint32_t *d = reinterpret_cast<uint32_t *>(planes + q.lds);
 #pragma unroll
                 for (int e = 0; e < 3; ++e) {
-                    smallest = smallest_magnitude(smallest, v[2 * e], v[2 * e + 1]);
-                    sp[e] = split_pair_f16(v[2 * e], v[2 * e + 1], up, up11);
                     d[e] = sp[e].hi;
-                    d[kPlane / 2 + e] = sp[e].lo;
+                    d[kPlane / 2 + e] = sp[e].mid;
+                    d[2 * (kPlane / 2) + e] = sp[e].lo;
                 }
                 if (q.t20 >= 0) {  // the pair's third value: the first of the second pair
                     planes[q.t20] = (uint16_t)sp[1].hi;
-                    planes[kPlane + q.t20] = (uint16_t)sp[1].lo;
+                    planes[kPlane + q.t20] = (uint16_t)sp[1].mid;
+                    planes[2 * kPlane + q.t20] = (uint16_t)sp[1].lo;
                 }
             }
         }
-        if (!(largest < __builtin_inff()) || too_small_for_f16(smallest, s)) rows_special[slot] = 1;
-    };
-    // where a filter's place (slot q = place / 8, element t = place % 8) is in its 7 x 21 values: kernel row * 21 + k', or -1
-    auto depth_of = [](int q, int t) {
-        if (q < 12) return (2 * (q >> 2) + (q & 1)) * 21 + 8 * ((q >> 1) & 1) + t;
-        if (q < 14) return 6 * 21 + 8 * (q & 1) + t;
-        const int ky = 2 * (q - 14) + (t >> 2);
-        if (q < 18) return ky < 7 ? ky * 21 + 16 + (t & 3) : -1;
-        return q == 18 && t < 7 ? t * 21 + 20 : -1;
-    };
-    // the filters of the channel tile at n0 as f16 parts, eight threads for a filter
-    auto fill_filters = [&](int n0) {
-        const int co = tid >> 3, part = tid & 7;
-        const bool there = n0 + co < p.cout;
-        const float *w = p.w + (size_t)(n0 + co) * 147;
-        float m = 0.f;
-        for (int k = part; k < 147; k += 8) m = max3_magnitude(there ? w[k] : 0.f, 0.f, m);
-#pragma unroll
-        for (int step = 1; step < 8; step *= 2) m = max3_magnitude(__shfl_xor(m, step, 8), 0.f, m);
-        const int s = f16_scale_exponent(m);
-        const float up = exp2_int(s), up11 = exp2_int(s + 11);
-        uint32_t smallest = ~0u;
-        for (int pr = part; pr < kStemDepth / 2; pr += 8) {
-            float v[2];
-#pragma unroll
-            for (int e = 0; e < 2; ++e) {
-                const int k = depth_of((2 * pr + e) >> 3, (2 * pr + e) & 7);
-                v[e] = there && k >= 0 ? w[k] : 0.f;
-            }
-            smallest = smallest_magnitude(smallest, v[0], v[1]);
-            const HalfPair sp = split_pair_f16(v[0], v[1], up, up11);
-            uint32_t *d = reinterpret_cast<uint32_t *>(fplanes + co * kFilterRow + 2 * pr);
-            d[0] = sp.hi;
-            d[kFilterPlane / 2] = sp.lo;
-        }
-        if (part == 0) filter_exp[co] = s;
-        if (!(m < __builtin_inff()) || too_small_for_f16(smallest, s)) special_filters = n0 + 1;
-    };
+        if (any_special) special_flag = 1;
+        __syncthreads();
 
-    enter(item);
-    fetch_tile();
-    if (tid == 0) special_filters = 0;
-    if (tid < 2) rows_max[tid] = 0, rows_special[tid] = 0;
-    __syncthreads();
-    fill_filters(at.n0);
-    publish_max(0);
-    __syncthreads();
-    split_rows(0);
-    __syncthreads();
-    int slot = 0;
-    for (;;) {
-        // here: the band's rows and filters are in LDS, every thread is past its last read of the staged band before
-        const BandOut o = at;
+        const BandOut o{img, band, row0, n0, n0 / BN};
         const int next = item + range.step;
         const bool has_next = next < range.end;
-        if (has_next) {  // the next band's rows come while this one is multiplied
-            enter(next);
-            fetch_tile();
-        }
-        f32x4v acc[TM][TN], cross[TM][TN];
+
+        f32x4v acc[TM][TN];
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
-            for (int j = 0; j < TN; ++j) acc[i][j] = cross[i][j] = f32x4v{0.f, 0.f, 0.f, 0.f};
-        const bool special = __builtin_amdgcn_readfirstlane(rows_special[slot]) != 0 || __builtin_amdgcn_readfirstlane(special_filters) == o.n0 + 1;
-        if (!special) {
-            int f_s = lane >> 4, f_i = lane & 15;
-            asm volatile("" : "+v"(f_s), "+v"(f_i));  // what follows is worked out per band: held across the loop it is spilled
-            // lane constants of the tile reads: the plane elements of a slot's two halves of four (tile i of the wave's
-            // row: + 96 * i; slot 18: + 256 * i; the zero area: + 0).  Groups 0..2 and the first two slots of group 3 are
-            // eight consecutive k' of kernel row 2 * G + g % 2 (group 3: row 6): group 0's offsets plus a constant.  The other
-            // slots of group 3 and group 4 have offsets of their own.  (The filter planes are laid out slot by slot when they are filled.)
-            const int base_a = 2 * wm * kTileStride + 6 * f_i;
-            const int a_main = base_a + (f_s & 1) * kTileStride + 8 * (f_s >> 1);
-            // group 3: slots 12, 13 (kernel row 6), 14, 15 (k' = 16..19 of kernel rows (0, 1) and (2, 3))
-            const int a0_g3 = f_s < 2 ? base_a + 6 * kTileStride + 8 * f_s : base_a + 2 * (f_s - 2) * kTileStride + 16;
-            const int a1_g3 = a0_g3 + (f_s < 2 ? 4 : kTileStride);
-            // group 4: slots 16 (kernel rows 4, 5), 17 (row 6, nothing), 18 (k' = 20 of all rows), 19 (nothing)
-            const int a0_g4 = f_s < 2 ? base_a + (4 + 2 * f_s) * kTileStride + 16 : f_s == 2 ? kPlaneT20 + f_i * 16 + 2 * wm : kPlaneZero;
-            const int a1_g4 = f_s == 0 ? a0_g4 + kTileStride : f_s == 2 ? a0_g4 + 4 : kPlaneZero;
-            const int s0_g4 = f_s < 2 ? 96 : f_s == 2 ? 256 : 0, s1_g4 = f_s == 0 ? 96 : f_s == 2 ? 256 : 0;
-            const uint32_t keep_g4 = f_s == 2 ? 0x0000ffffu : 0xffffffffu;  // slot 18: seven kernel rows, the eighth element out
-            // A slot's eight f16 of both planes are two halves of four, each 4-byte aligned and read as a pair of dwords
-            // behind a base that the compiler does not see through: with long constant offsets it makes an 8-byte read of the
-            // pair, which takes 50 cycles where it is off by four (the kernel then took 555 us at batch 256).
-            typedef const uint32_t __attribute__((address_space(3))) *LdsWords;
-            LdsWords h0, l0, h1, l1;  // first half, hi and lo, and second half
-            auto base = [&](int e) {
-                LdsWords q = (LdsWords)(planes + e);
-                asm("" : "+v"(q));
-                return q;
-            };
-            auto frag_at = [&](int d0, int d1, uint32_t keep_mask) {
-                return HalfFrag8{HalfFrag8::u4{h0[d0], h0[d0 + 1], h1[d1], h1[d1 + 1] & keep_mask}, HalfFrag8::u4{l0[d0], l0[d0 + 1], l1[d1], l1[d1 + 1] & keep_mask}};
-            };
-            // called for the tiles in order: the bases serve tiles 0..3 and 4..6 of a group (offsets of such a read end at 255)
-            auto tile_frag = [&](int G, int i) {
-                const int i0 = i & 4;
-                if (G < 4) {
-                    const int e0 = (G < 3 ? a_main + 2 * G * kTileStride : a0_g3) + 96 * i0;
-                    if (i == i0) h0 = base(e0), l0 = base(kPlane + e0);
-                    if (G == 3 && i == i0) h1 = base(a1_g3 + 96 * i0), l1 = base(kPlane + a1_g3 + 96 * i0);
-                    if (G < 3) h1 = h0, l1 = l0;
-                    return frag_at(48 * (i - i0), 48 * (i - i0) + (G < 3 ? 2 : 0), 0xffffffffu);
-                }
-                h0 = base(a0_g4 + s0_g4 * i), l0 = base(kPlane + a0_g4 + s0_g4 * i);
-                h1 = base(a1_g4 + s1_g4 * i), l1 = base(kPlane + a1_g4 + s1_g4 * i);
-                return frag_at(0, 0, keep_g4);
-            };
-            auto b_frag = [&](int G, int j) {
-                const uint16_t *row = fplanes + (wn * 32 + j * 16 + f_i) * kFilterRow + G * 32 + f_s * 8;
-                return HalfFrag8{*reinterpret_cast<const HalfFrag8::u4 *>(row), *reinterpret_cast<const HalfFrag8::u4 *>(row + kFilterPlane)};
-            };
-            // 35 steps of six matrix instructions (depth group G = step / 7, pixel tile i = step % 7); a step's reads are
-            // the next step's tile fragment (four reads) and, in the middle of a group, the next group's filter fragments
-            // (four more), dealt out between its matrix instructions
-            HalfFrag8 a[2], b[2][TN];
+            for (int j = 0; j < TN; ++j) acc[i][j] = f32x4v{0.f, 0.f, 0.f, 0.f};
+        // a slot's eight bf16 of every plane: two halves of four (each 4-byte aligned)
+        auto a_frag = [&](auto derive_finite, int e0, int e1, uint32_t keep_mask) {
+            SplitFrag8 f;
+            const u32x2a h0 = *reinterpret_cast<const u32x2a *>(planes + e0), h1 = *reinterpret_cast<const u32x2a *>(planes + e1);
+            const u32x2a m0 = *reinterpret_cast<const u32x2a *>(planes + kPlane + e0), m1 = *reinterpret_cast<const u32x2a *>(planes + kPlane + e1);
+            const u32x2a l0 = *reinterpret_cast<const u32x2a *>(planes + 2 * kPlane + e0), l1 = *reinterpret_cast<const u32x2a *>(planes + 2 * kPlane + e1);
+            f.hi = SplitFrag8::u4{h0.x, h0.y, h1.x, h1.y & keep_mask};
+            f.mid = SplitFrag8::u4{m0.x, m0.y, m1.x, m1.y & keep_mask};
+            f.lo = SplitFrag8::u4{l0.x, l0.y, l1.x, l1.y & keep_mask};
+            if constexpr (decltype(derive_finite)::value) {
 #pragma unroll
-            for (int j = 0; j < TN; ++j) b[0][j] = b_frag(0, j);
-            a[0] = tile_frag(0, 0);
+                for (int e = 0; e < 4; ++e) f.hif[e] = finite_bf16_pair(f.hi[e]);
+            } else {
+                f.hif = f.hi;
+            }
+            return f;
+        };
+        auto b_frag = [&](auto derive_finite, int G, int j) {
+            const uint16_t *row = fplanes + (wn * 32 + j * 16 + f_i) * kFilterRow + G * 32 + f_s * 8;
+            SplitFrag8 f;
+            f.hi = *reinterpret_cast<const SplitFrag8::u4 *>(row);
+            f.mid = *reinterpret_cast<const SplitFrag8::u4 *>(row + kFilterPlane);
+            f.lo = *reinterpret_cast<const SplitFrag8::u4 *>(row + 2 * kFilterPlane);
+            if constexpr (decltype(derive_finite)::value) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) f.hif[e] = finite_bf16_pair(f.hi[e]);
+            } else {
+                f.hif = f.hi;
+            }
+            return f;
+        };
+        auto tile_frag = [&](auto derive_finite, int G, int i) {
+            return G < 3    ? a_frag(derive_finite, a_main + 2 * G * kTileStride + 96 * i, a_main + 2 * G * kTileStride + 96 * i + 4, 0xffffffffu)
+                   : G == 3 ? a_frag(derive_finite, a0_g3 + 96 * i, a1_g3 + 96 * i, 0xffffffffu)
+                            : a_frag(derive_finite, a0_g4 + s0_g4 * i, a1_g4 + s1_g4 * i, keep_g4);
+        };
+        // 35 steps of twelve matrix instructions (depth group G = step / 7, pixel tile i = step % 7); a step's reads are
+        // the next step's tile fragment (six reads) and, in the middle of a group, the next group's filter fragments
+        // (six more), dealt out between its matrix instructions
+        auto multiply = [&](auto derive_finite) {
+            SplitFrag8 a[2], b[2][TN];
+#pragma unroll
+            for (int j = 0; j < TN; ++j) b[0][j] = b_frag(derive_finite, 0, j);
+            a[0] = tile_frag(derive_finite, 0, 0);
 #pragma unroll
             for (int step = 0; step < 5 * TM; ++step) {
                 const int G = step / TM, i = step - G * TM;
                 const bool more_tiles = step + 1 < 5 * TM, more_filters = i == 3 && G + 1 < 5;
-                if (more_tiles) a[(step + 1) & 1] = tile_frag((step + 1) / TM, (step + 1) % TM);
+                if (more_tiles) a[(step + 1) & 1] = tile_frag(derive_finite, (step + 1) / TM, (step + 1) % TM);
                 if (more_filters) {
 #pragma unroll
-                    for (int j = 0; j < TN; ++j) b[(G + 1) & 1][j] = b_frag(G + 1, j);
+                    for (int j = 0; j < TN; ++j) b[(G + 1) & 1][j] = b_frag(derive_finite, G + 1, j);
                 }
-                mfma3_16x16x32(acc[i][0], acc[i][1], cross[i][0], cross[i][1], a[step & 1], b[G & 1][0], b[G & 1][1]);
+                mfma6_16x16x32(acc[i][0], acc[i][1], a[step & 1], b[G & 1][0], b[G & 1][1]);
+                if constexpr (!decltype(derive_finite)::value) {
 #pragma unroll
-                for (int k = 0; k < 6; ++k) {
-                    if (more_tiles && k < 4) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);    // one LDS read
-                    if (more_filters && k < 4) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // and one of the filters'
-                    __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);                               // a matrix instruction
-                }
-            }
-            const int s_rows = f16_scale_exponent(__builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(rows_max[slot])));
-#pragma unroll
-            for (int j = 0; j < TN; ++j) {
-                const int down = -(s_rows + filter_exp[wn * 32 + j * 16 + f_i]);
-#pragma unroll
-                for (int i = 0; i < TM; ++i)
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) acc[i][j][e] = __builtin_ldexpf(__builtin_fmaf(cross[i][j][e], 1.f / 2048.f, acc[i][j][e]), down);
-            }
-        } else {
-            // the same slots in fp32 from memory, in two sums
-            const auto x_rsrc = image_rsrc(o.img);
-            int f_s = lane >> 4, f_i = lane & 15;
-            asm volatile("" : "+v"(f_s), "+v"(f_i));  // nothing of this path is held across the band loop
-#pragma unroll 1
-            for (int G = 0; G < 5; ++G) {
-                const int q = 4 * G + f_s;
-                float wv[TN][8];
-#pragma unroll
-                for (int j = 0; j < TN; ++j)
-#pragma unroll
-                    for (int t = 0; t < 8; ++t) {
-                        const int co = o.n0 + wn * 32 + j * 16 + f_i, k = depth_of(q, t);
-                        wv[j][t] = co < p.cout && k >= 0 ? p.w[(size_t)co * 147 + k] : 0.f;
+                    for (int k = 0; k < 6; ++k) {
+                        if (more_tiles) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);    // one LDS read
+                        if (more_filters) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // and one of the filters'
+                        __builtin_amdgcn_sched_group_barrier(0x8, 2, 0);                      // two matrix instructions
                     }
-#pragma unroll
-                for (int i = 0; i < TM; ++i) {
-                    float xv[8];
-#pragma unroll
-                    for (int t = 0; t < 8; ++t) {
-                        const int k = depth_of(q, t), ky = k / 21;
-                        const int e = 6 * (16 * i + f_i) + k - 21 * ky - 9;  // float of the image's row
-                        const bool in = k >= 0 && (unsigned)e < (unsigned)(3 * p.wd);
-                        const uint32_t off = (uint32_t)(((2 * (o.row0 + wm) - 3 + ky) * p.wd * 3 + e) * 4);
-                        xv[t] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(x_rsrc, (int)(in ? off : kPoolOob), 0, 0));
-                    }
-#pragma unroll
-                    for (int t = 0; t < 8; ++t)
-#pragma unroll
-                        for (int j = 0; j < TN; ++j) {
-                            f32x4v &sum = t & 1 ? cross[i][j] : acc[i][j];
-                            sum = __builtin_amdgcn_mfma_f32_16x16x4f32(xv[t], wv[j][t], sum, 0, 0, 0);
-                        }
                 }
             }
-#pragma unroll
-            for (int i = 0; i < TM; ++i)
-#pragma unroll
-                for (int j = 0; j < TN; ++j) acc[i][j] = acc[i][j] + cross[i][j];
-        }
+        };
+        if (__builtin_amdgcn_readfirstlane(special_flag) != 0 || __builtin_amdgcn_readfirstlane(special_filters) == n0 + 1)
+            multiply(std::true_type{});
+        else
+            multiply(std::false_type{});
         int tid_band = tid;
         asm volatile("" : "+v"(tid_band));  // the epilogue's addresses are worked out per band, not held (spilled) across the loop
-        stem_stage(p, stage, acc, o, tid_band, wm, wn, f_s, f_i);
-        if (has_next) publish_max(slot ^ 1);
-        __syncthreads();
-        stem_pool<SIGN>(p, stage, o, tid_band, keep, fold && o.band > 0, !p.chained || !has_next);
+        // the next band's rows come while this band is pooled (their registers are free of the multiplication)
+        if (has_next) {
+            enter(next);
+            fetch_tile();
+        }
+        __syncthreads();  // the planes are dead: the staged band takes their place
+        if (tid == 0) special_flag = 0;  // the next band's rows set it again, after the barrier that ends this pass
+        stem_epilogue<SIGN>(p, stage, acc, o, tid_band, wm, wn, f_s, f_i, keep, fold && o.band > 0, !p.chained || !has_next);
         if (!has_next) break;
-        if (at.n0 != o.n0) fill_filters(at.n0);
-        split_rows(slot ^ 1);
-        if (tid == 0) rows_max[slot] = 0, rows_special[slot] = 0;
-        slot ^= 1;
         fold = p.chained != 0;
         item = next;
-        __syncthreads();
+        __syncthreads();  // the staged band is dead
     }
 }
 

@@ -1,5 +1,5 @@
-"""The one-pass 7x7 stem on f16 parts: rows and filters of any magnitude (each band and each filter has a scale of its own), values too
-far below their band's or filter's largest for the parts, infinities, NaN, several channel tiles; against 64-bit sums."""
+"""The one-pass 7x7 stem on three bf16 parts: operands kept whole, rows and filters of magnitudes far apart, infinities, NaN, several
+channel tiles; against 64-bit sums."""
 import pytest
 import torch
 import torch.nn.functional as F
@@ -20,8 +20,8 @@ def operands(n, h, w, cout, seed):
     return torch.randn((n, h, w, 3), device="cuda", generator=gen), torch.randn((cout, 7, 7, 3), device="cuda", generator=gen) * 0.1
 
 
-# A product is off by 2^-23 of it for each operand's parts and 2^-22 for the term left out, a sum of 10 to 160 partial sums by half an ulp
-# each: 2^-21 + 160 * 2^-24 of the sum of magnitudes is above all of it.
+# The terms left out are below 2^-24 of a product; 30 matrix instructions round the sum five times each at most, half an ulp a time:
+# 2^-21 + 160 * 2^-24 of the sum of magnitudes is above all of it.
 BOUND = 2.0**-21 + 160 * 2.0**-24
 
 
@@ -81,11 +81,29 @@ def test_infinities_and_nan(value, where):
     assert torch.allclose(pooled[ok], want[ok], rtol=1e-5, atol=1e-5)
 
 
-def test_no_larger_error_than_the_six_bf16_products():
+# every output channel copies one input channel at one tap: no operand loses a bit on its way to the products
+@pytest.mark.parametrize("n,h,w,cout", [(2, 16, 224, 64), (3, 40, 223, 128)])
+def test_copied_channels_are_exact(n, h, w, cout):
+    import dabnn_amd as dab
+    x, wgt = operands(n, h, w, cout, 8)
+    wgt = torch.zeros_like(wgt)
+    padded, oh, ow = F.pad(x, (0, 0, 3, 3, 3, 3)), (h - 1) // 2 + 1, (w - 1) // 2 + 1
+    copies = []
+    for co in range(cout):
+        ky, kx, c = co % 7, co // 7 % 7, co % 3
+        wgt[co, ky, kx, c] = 1
+        copies.append(padded[:, ky:ky + 2 * oh - 1:2, kx:kx + 2 * ow - 1:2, c])
+    got, _ = dab.fconv_maxpool(x, wgt, None, None, None, False, 7, 7, 3, 3, 2, 2)
+    assert torch.equal(got, dab.max_pool(torch.stack(copies, -1).contiguous(), 3, 3, 1, 1, 2, 2))
+
+
+def test_no_larger_error_than_an_fp32_sum():
     import dabnn_amd as dab
     x, wgt = operands(8, 112, 224, 64, 7)
     got, _ = dab.fconv_maxpool(x, wgt, None, None, None, False, 7, 7, 3, 3, 2, 2)
     want, _ = reference(x, wgt)
     error = float((got.double().cpu() - want).norm() / want.norm())
     print("relative 2-norm error %.3g" % error)
-    assert error < 1.5e-7  # six bf16 products in one sum: 1.76e-7 of a sum, the fp32 instruction 2.27e-7
+    # 147 products in fp32 one after the other: roundings spread evenly over half an ulp (2^-24 / sqrt(3) in the root mean square) of
+    # partial sums whose variances 1, 2 .. 147 add up to 147 * 148 / 2
+    assert error < 2.0**-24 / 3**0.5 * (148 / 2)**0.5
