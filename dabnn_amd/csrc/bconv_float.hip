@@ -9,6 +9,8 @@
 // Bound by latency: one launch from the host (4.3 us with the call), one round trip for the input and filters, one pass over
 // the depth, the store.  So all of a wave's input is asked for at once (48 words: with 32 at a time 16 x 56 x 56 x 64 took 8.1
 // us instead of 6.6), in groups of 16 so that small strips do not pack what is not there (1 to 1.5 us of them).
+#include <functional>
+
 #include "bgemm_core.h"
 #include "fp4_core.h"
 
@@ -271,6 +273,9 @@ static bool plan_float_conv(FloatConvPlan &plan, const float *x, int n, int h, i
 int bconv_float_try(const float *x, int n, int h, int w, int c, const uint64_t *wgt, int words, int kh, int kw, int pad_h, int pad_w, int stride_h, int stride_w,
                     int cout, float *out, int oh, int ow, hipStream_t s) {
     FloatConvPlan p;
+    // A layer run in place, or into a buffer that its input reaches into: here blocks store while others still read their rows.
+    const float *x_end = x + (size_t)n * h * w * c, *out_end = out + (size_t)n * oh * ow * cout;
+    if (std::less<const float *>()(x, out_end) && std::less<const float *>()(out, x_end)) return 0;
     if ((reinterpret_cast<uintptr_t>(wgt) & 7) != 0 || (reinterpret_cast<uintptr_t>(out) & 3) != 0 || (reinterpret_cast<uintptr_t>(x) & 3) != 0) return 0;
     if (!plan_float_conv(p, x, n, h, w, c, wgt, words, kh, kw, pad_h, pad_w, stride_h, stride_w, cout, out, oh, ow)) return 0;
     const int rc = p.ds == 1   ? launch_float_conv<1>(p.a, p.grid, p.lds, s)

@@ -201,8 +201,9 @@ DAB_API int dab_bconv3x3_pair(const uint64_t *x, const float *shortcut, int n, i
  * bgemm on `wgt_t` (the transposed weights; may be NULL when the direct kernel
  * applies).  The counts are the same.
  * hwc_words = words per filter (weight.total()/weight.n).
- * workspace must hold dab_binconv_workspace_bytes(...) bytes.
+ * workspace must hold dab_binconv_workspace_bytes(...) bytes
  * (room for the column matrix, whether or not the call makes one).
+ * out may be x, or overlap it: x is packed before out is written then.
  * method_out (optional) receives 0 = DIRECT_CONV, 1 = BGEMM.
  */
 DAB_API size_t dab_binconv_workspace_bytes(int n, int h, int w, int c, int kh, int kw, int pad_h, int pad_w, int stride_h,

@@ -67,3 +67,24 @@ def test_nothing_is_stored_past_the_output(cin, cout, k):
                                             out.data_ptr() + 4 * guard, ws.data_ptr(), need, None, torch.cuda.current_stream().cuda_stream))
     assert bool((out[:guard] == -7).all()) and bool((out[-guard:] == -7).all())
     assert torch.equal(out[guard:-guard].view(n, h, w, cout).cpu(), reference(x.cpu(), wf, (1, 1), (k // 2, k // 2)))
+
+
+# a layer run in place, and into buffers that begin before its input's end or end behind its start (counted in output elements from x)
+@pytest.mark.parametrize("n,h,w,c,k", [(2, 12, 12, 64, 3), (16, 56, 56, 64, 3), (3, 20, 21, 128, 1), (2, 14, 14, 192, 3), (1, 9, 9, 256, 5)])
+@pytest.mark.parametrize("where", [0.0, 0.5, -0.75])
+def test_output_over_input(n, h, w, c, k, where):
+    from dabnn_amd import capi
+    r = np.random.default_rng(c + k)
+    weight = torch.from_numpy(models.pack_weight(r.standard_normal((c, k, k, c)).astype(np.float32)).view(np.int64)).cuda()
+    x = torch.randn((n, h, w, c), device="cuda", generator=torch.Generator(device="cuda").manual_seed(n + c))
+    want = dab.BinConv(weight, k, k, k // 2, k // 2, 1, 1)(x)
+    size = x.numel()
+    buf = torch.empty(3 * size, device="cuda")
+    buf[size:2 * size] = x.view(-1)
+    at = size + int(where * size) // 4 * 4
+    need = capi.lib.dab_binconv_workspace_bytes(n, h, w, c, k, k, k // 2, k // 2, 1, 1)
+    ws = torch.empty(need, dtype=torch.uint8, device="cuda")
+    wt = dab.weight_transpose(weight)
+    capi.check(capi.lib.dab_binconv_forward(buf.data_ptr() + 4 * size, n, h, w, c, weight.data_ptr(), wt.data_ptr(), weight.shape[1], k, k, k // 2, k // 2, 1, 1, c,
+                                            buf.data_ptr() + 4 * at, ws.data_ptr(), need, None, torch.cuda.current_stream().cuda_stream))
+    assert torch.equal(buf[at:at + size].view_as(want), want)
