@@ -60,6 +60,7 @@ extern "C" int dab_binconv_forward(const float *x, int n, int h, int w, int c, c
     using namespace dab;
     DAB_REQUIRE(x && out && workspace, "dab_binconv_forward: null pointer");
     DAB_REQUIRE(n > 0 && h > 0 && w > 0 && c > 0 && cout > 0 && kh > 0 && kw > 0, "dab_binconv_forward: non-positive dimension");
+    DAB_REQUIRE(pad_h >= 0 && pad_w >= 0 && stride_h > 0 && stride_w > 0, "dab_binconv_forward: bad pad/stride");
     DAB_REQUIRE(c % 64 == 0, "dab_binconv_forward: c %d is not a multiple of 64", c);
     DAB_REQUIRE(workspace_bytes >= dab_binconv_workspace_bytes(n, h, w, c, kh, kw, pad_h, pad_w, stride_h, stride_w),
                 "dab_binconv_forward: workspace too small");
@@ -70,6 +71,8 @@ extern "C" int dab_binconv_forward(const float *x, int n, int h, int w, int c, c
         DAB_REQUIRE(wgt, "dab_binconv_forward: direct method needs wgt");
         DAB_REQUIRE(hwc_words == 9 * (c / 64), "dab_binconv_forward: %d words per filter, expected %d", hwc_words,
                     9 * (c / 64));
+        DAB_REQUIRE((reinterpret_cast<uintptr_t>(workspace) & 15) == 0 && (reinterpret_cast<uintptr_t>(wgt) & 7) == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0,
+                    "dab_binconv_forward: buffers must be 16-byte aligned");
         int rc = c <= 512 ? bconv_float_try(x, n, h, w, c, wgt, hwc_words, kh, kw, pad_h, pad_w, stride_h, stride_w, cout, out, oh, ow, as_stream(stream)) : 0;
         if (rc != 0) {
             if (rc > 0 && method_out) *method_out = 0;
@@ -93,6 +96,7 @@ extern "C" int dab_binconv_forward(const float *x, int n, int h, int w, int c, c
         // The column matrix is fused_binarize_im2col of the input, kh * kw times its packed copy: the convolution reads
         // the packed pixels of a window where they are instead (8 x 14 x 14 x 256, 5 x 5: 11 us against 26 with the
         // column matrix and its GEMM).
+        DAB_REQUIRE((reinterpret_cast<uintptr_t>(workspace) & 7) == 0 && (reinterpret_cast<uintptr_t>(out) & 3) == 0, "dab_binconv_forward: misaligned pointer");
         int rc = bconv_float_try(x, n, h, w, c, wgt, hwc_words, kh, kw, pad_h, pad_w, stride_h, stride_w, cout, out, oh, ow, as_stream(stream));
         if (rc != 0) {
             if (rc > 0 && method_out) *method_out = 1;

@@ -106,3 +106,16 @@ def test_workspace_and_row_words():
     # direct method needs the packed input, bgemm method the column matrix
     assert lib.dab_binconv_workspace_bytes(1, 56, 56, 64, 3, 3, 1, 1, 1, 1) == 56 * 56 * 10 * 8
     assert lib.dab_binconv_workspace_bytes(2, 7, 7, 512, 3, 3, 1, 1, 1, 1) == 2 * 49 * 72 * 8
+
+
+# the 3x3 route and the general one: sizes of which every call behind dab_binconv_forward refuses the arguments, however small the problem
+@pytest.mark.parametrize("cout", [64, 60])
+@pytest.mark.parametrize("change", [dict(pad_h=-1, pad_w=-1), dict(pad_w=-1), dict(stride_h=0), dict(stride_w=-1), dict(workspace=20), dict(out=18)])
+def test_binconv_forward_refuses_what_its_parts_refuse(cout, change):
+    from dabnn_amd import capi
+    a = dict(pad_h=1, pad_w=1, stride_h=1, stride_w=1, workspace=32, out=32)
+    a.update(change)
+    vp = ctypes.c_void_p
+    rc = capi.lib.dab_binconv_forward(vp(16), 2, 8, 9, 64, vp(16), vp(16), 9, 3, 3, a["pad_h"], a["pad_w"], a["stride_h"], a["stride_w"], cout, vp(a["out"]),
+                                      vp(a["workspace"]), 1 << 30, None, vp(None))
+    assert rc == capi.DAB_EINVAL, capi.last_error()
