@@ -273,6 +273,8 @@ static bool plan_float_conv(FloatConvPlan &plan, const float *x, int n, int h, i
 int bconv_float_try(const float *x, int n, int h, int w, int c, const uint64_t *wgt, int words, int kh, int kw, int pad_h, int pad_w, int stride_h, int stride_w,
                     int cout, float *out, int oh, int ow, hipStream_t s) {
     FloatConvPlan p;
+    // (with a stride of two and more the output of a window larger than the padded image is rounded up to one pixel)
+    if (h + 2ll * pad_h < kh || w + 2ll * pad_w < kw) return 0;
     // A layer run in place, or into a buffer that its input reaches into: here blocks store while others still read their rows.
     const float *x_end = x + (size_t)n * h * w * c, *out_end = out + (size_t)n * oh * ow * cout;
     if (std::less<const float *>()(x, out_end) && std::less<const float *>()(out, x_end)) return 0;

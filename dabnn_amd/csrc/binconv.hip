@@ -71,6 +71,7 @@ extern "C" int dab_binconv_forward(const float *x, int n, int h, int w, int c, c
         DAB_REQUIRE(wgt, "dab_binconv_forward: direct method needs wgt");
         DAB_REQUIRE(hwc_words == 9 * (c / 64), "dab_binconv_forward: %d words per filter, expected %d", hwc_words,
                     9 * (c / 64));
+        DAB_REQUIRE(h + 2 * pad_h >= 3 && w + 2 * pad_w >= 3, "dab_binconv_forward: input smaller than the kernel");
         DAB_REQUIRE((reinterpret_cast<uintptr_t>(workspace) & 15) == 0 && (reinterpret_cast<uintptr_t>(wgt) & 7) == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0,
                     "dab_binconv_forward: buffers must be 16-byte aligned");
         int rc = c <= 512 ? bconv_float_try(x, n, h, w, c, wgt, hwc_words, kh, kw, pad_h, pad_w, stride_h, stride_w, cout, out, oh, ow, as_stream(stream)) : 0;

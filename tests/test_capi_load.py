@@ -119,3 +119,12 @@ def test_binconv_forward_refuses_what_its_parts_refuse(cout, change):
     rc = capi.lib.dab_binconv_forward(vp(16), 2, 8, 9, 64, vp(16), vp(16), 9, 3, 3, a["pad_h"], a["pad_w"], a["stride_h"], a["stride_w"], cout, vp(a["out"]),
                                       vp(a["workspace"]), 1 << 30, None, vp(None))
     assert rc == capi.DAB_EINVAL, capi.last_error()
+
+
+def test_binconv_forward_refuses_images_smaller_than_the_direct_kernel():
+    """Stride 2 over two padded rows or columns: (2 - 3) / 2 + 1 is one output pixel in C, but no 3x3 window fits."""
+    from dabnn_amd import capi
+    vp = ctypes.c_void_p
+    for h, w, pad in [(2, 9, 0), (9, 2, 0), (2, 2, 0)]:
+        rc = capi.lib.dab_binconv_forward(vp(16), 2, h, w, 64, vp(16), vp(16), 9, 3, 3, pad, pad, 2, 2, 64, vp(32), vp(32), 1 << 30, None, vp(None))
+        assert rc == capi.DAB_EINVAL and "smaller than the kernel" in capi.last_error(), capi.last_error()

@@ -88,3 +88,22 @@ def test_output_over_input(n, h, w, c, k, where):
     capi.check(capi.lib.dab_binconv_forward(buf.data_ptr() + 4 * size, n, h, w, c, weight.data_ptr(), wt.data_ptr(), weight.shape[1], k, k, k // 2, k // 2, 1, 1, c,
                                             buf.data_ptr() + 4 * at, ws.data_ptr(), need, None, torch.cuda.current_stream().cuda_stream))
     assert torch.equal(buf[at:at + size].view_as(want), want)
+
+
+# windows larger than the padded image, whose output is rounded up to one pixel: those rows and columns are padding
+@pytest.mark.parametrize("h,w,c,k,stride", [(9, 3, 64, (3, 5), (1, 3)), (3, 9, 128, (5, 3), (4, 1)), (6, 2, 192, (1, 4), (2, 4)), (2, 2, 64, (3, 3), (3, 2))])
+def test_windows_larger_than_the_image(h, w, c, k, stride):
+    from dabnn_amd import capi
+    r = np.random.default_rng(h)
+    cout, n = 40, 3
+    wf = r.standard_normal((cout, *k, c)).astype(np.float32)
+    weight = torch.from_numpy(models.pack_weight(wf).view(np.int64)).cuda()
+    x = torch.from_numpy(r.standard_normal((n, h, w, c)).astype(np.float32)).cuda()
+    oh, ow = (int((s - f) / t) + 1 for s, f, t in zip((h, w), k, stride))
+    want = reference(F.pad(x, (0, 0, 0, k[1], 0, k[0]), value=-1.0).cpu(), wf, stride, (0, 0))[:, :oh, :ow]
+    need = capi.lib.dab_binconv_workspace_bytes(n, h, w, c, *k, 0, 0, *stride)
+    ws, wt, out = torch.empty(need, dtype=torch.uint8, device="cuda"), dab.weight_transpose(weight), torch.empty((n, oh, ow, cout), device="cuda")
+    # (strides that differ make the 3x3 case the general route's)
+    capi.check(capi.lib.dab_binconv_forward(x.data_ptr(), n, h, w, c, weight.data_ptr(), wt.data_ptr(), weight.shape[1], *k, 0, 0, *stride, cout,
+                                            out.data_ptr(), ws.data_ptr(), need, None, torch.cuda.current_stream().cuda_stream))
+    assert torch.equal(out.cpu(), want)
