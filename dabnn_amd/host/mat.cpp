@@ -112,7 +112,7 @@ void Mat::upload(const void *host, size_t nbytes) {
 void Mat::download(void *host, size_t nbytes, Staging *via) const {
     if (nbytes > bytes()) throw std::runtime_error("Mat::download: destination larger than the tensor");
     if (via && !ld) {
-        via->download(host, dev, nbytes, copy_stream());
+        via->download(host, dev, nbytes);
         return;
     }
     if (ld) {

@@ -38,6 +38,7 @@ Staging::~Staging() {
     wake_.notify_all();
     for (auto &t : helpers_) t.join();
     for (void *e : events_) (void)hipEventDestroy(static_cast<hipEvent_t>(e));
+    if (download_stream_) (void)hipStreamDestroy(static_cast<hipStream_t>(download_stream_));
     (void)hipHostFree(memory_);
 }
 
@@ -166,9 +167,22 @@ void Staging::upload(void *dst, const void *src, size_t bytes, void *stream) {
     wait_for_helpers();
 }
 
-void Staging::download(void *dst, const void *src, size_t bytes, void *stream) {
+// (one that does not synchronise with the null stream, as Mat's copies)
+void Staging::make_download_stream() {
+    int current = 0;
+    hip_check(hipGetDevice(&current), "hipGetDevice");
+    if (current != device_) hip_check(hipSetDevice(device_), "hipSetDevice");
+    hipStream_t s = nullptr;
+    const hipError_t e = hipStreamCreateWithFlags(&s, hipStreamNonBlocking);
+    if (current != device_) hip_check(hipSetDevice(current), "hipSetDevice");
+    hip_check(e, "hipStreamCreate");
+    download_stream_ = s;
+}
+
+void Staging::download(void *dst, const void *src, size_t bytes) {
     std::lock_guard<std::mutex> one(use_);
-    hipStream_t s = static_cast<hipStream_t>(stream);
+    if (!download_stream_) make_download_stream();
+    hipStream_t s = static_cast<hipStream_t>(download_stream_);
     const size_t pieces = (bytes + kPiece - 1) / kPiece, window = std::min(kEvents, bytes_ / kPiece);  // (an event each)
     try {
         for (size_t i = 0; i < pieces + window; ++i) {

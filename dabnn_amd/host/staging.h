@@ -34,8 +34,9 @@ class Staging {
     // Copies host memory to the device on `stream`; `src` may change once the call returns.  The caller synchronises the
     // stream before the next call (a Net's runs do).
     void upload(void *dst, const void *src, size_t bytes, void *stream);
-    // Copies device memory to the host on `stream` and waits.
-    void download(void *dst, const void *src, size_t bytes, void *stream);
+    // Copies device memory to the host and waits.  The stream is the Staging's own, of the device that its events are of: the runtime
+    // records no event of one device on a stream of another.
+    void download(void *dst, const void *src, size_t bytes);
 
    private:
     struct Transfer {
@@ -46,12 +47,14 @@ class Staging {
     void copy_blocks();  // takes blocks until there are none left (a helper's share of an upload)
     void helper();
     void start_helpers();
+    void make_download_stream();
 
     unsigned char *memory_ = nullptr;
     size_t bytes_ = 0;
     int device_ = 0;
     static constexpr size_t kEvents = 16;
     std::vector<void *> events_;  // of transfer i: i % kEvents
+    void *download_stream_ = nullptr;  // made by the first download
 
     // the upload at hand
     unsigned char *dst_ = nullptr;

@@ -1,0 +1,95 @@
+// Staging and Mat's copies through it over a runtime of two devices that lives in host memory: what the real one refuses -- an event
+// of one device on a stream of another -- is refused here too.  Run by tests/test_staging.py, without a GPU.
+#include <hip/hip_runtime_api.h>
+
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <vector>
+
+#include "../../dabnn_amd/host/mat.h"
+#include "../../dabnn_amd/host/staging.h"
+
+static thread_local int current = 0;
+static int pinned = 0, streams = 0, events = 0;  // alive
+struct Owned {
+    int device;
+};
+static int device_of(const void *p) { return static_cast<const Owned *>(p)->device; }
+
+extern "C" {
+const char *hipGetErrorString(hipError_t e) { return e == hipSuccess ? "success" : "refused"; }
+hipError_t hipGetDevice(int *d) { return *d = current, hipSuccess; }
+hipError_t hipSetDevice(int d) { return current = d, hipSuccess; }
+hipError_t hipMalloc(void **p, size_t n) { return *p = malloc(n), hipSuccess; }
+hipError_t hipFree(void *p) { return free(p), hipSuccess; }
+hipError_t hipHostMalloc(void **p, size_t n, unsigned) { return ++pinned, *p = malloc(n), hipSuccess; }
+hipError_t hipHostFree(void *p) { return --pinned, free(p), hipSuccess; }
+hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) { return ++streams, *s = reinterpret_cast<hipStream_t>(new Owned{current}), hipSuccess; }
+hipError_t hipStreamDestroy(hipStream_t s) { return --streams, delete reinterpret_cast<Owned *>(s), hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) { return ++events, *e = reinterpret_cast<hipEvent_t>(new Owned{current}), hipSuccess; }
+hipError_t hipEventDestroy(hipEvent_t e) { return --events, delete reinterpret_cast<Owned *>(e), hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) { return device_of(e) == device_of(s) ? hipSuccess : hipErrorInvalidHandle; }
+hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipStream_t) { return memcpy(d, s, n), hipSuccess; }
+hipError_t hipMemcpy2DAsync(void *d, size_t dp, const void *s, size_t sp, size_t w, size_t h, hipMemcpyKind, hipStream_t) {
+    for (size_t y = 0; y < h; ++y) memcpy(static_cast<char *>(d) + y * dp, static_cast<const char *>(s) + y * sp, w);
+    return hipSuccess;
+}
+}
+
+#define CHECK(x)                                               \
+    do {                                                       \
+        if (!(x)) {                                            \
+            printf("%s:%d: %s\n", __FILE__, __LINE__, #x);     \
+            return 1;                                          \
+        }                                                      \
+    } while (0)
+
+static int round_trip(bnn::Staging &staging, int device, size_t floats) {
+    current = device;
+    std::vector<float> in(floats), out(floats, -1.f);
+    for (size_t i = 0; i < floats; ++i) in[i] = (float)(i % 1000003);
+    auto m = bnn::Mat::planned(1, 1, 1, (int)floats, bnn::DataType::Float, "m");
+    m->allocate();
+    hipStream_t s;
+    (void)hipStreamCreateWithFlags(&s, 0);
+    staging.upload(m->dev, in.data(), floats * 4, s);
+    (void)hipStreamDestroy(s);
+    m->download(out.data(), floats * 4, &staging);
+    CHECK(out == in);
+    return 0;
+}
+
+int main() {
+    try {
+        {
+            // a copy without a Staging first: Mat's own stream is of device 0
+            std::vector<float> some(64, 3.f);
+            auto plain = bnn::Mat::planned(1, 1, 1, 64, bnn::DataType::Float, "plain");
+            plain->allocate();
+            plain->upload(some.data(), 256);
+            plain->download(some.data(), 256);
+        }
+        const int streams_before = streams;
+        for (int device : {0, 1}) {
+            current = device;
+            bnn::Staging staging(10 << 20);
+            for (size_t floats : {1000, 400000, 2000001, 21000000}) {  // one piece, pieces, a round of the events, longer than the pinned memory
+                CHECK(round_trip(staging, device, floats) == 0);
+            }
+            // asked for from a thread whose current device is another one, which stays what it was
+            current = 1 - device;
+            std::vector<float> in(200000, 2.f), out(200000);
+            staging.download(out.data(), in.data(), in.size() * 4);
+            CHECK(out == in && current == 1 - device);
+        }
+        CHECK(pinned == 0 && events == 0 && streams == streams_before);
+    } catch (const std::exception &e) {
+        printf("exception: %s\n", e.what());
+        return 1;
+    }
+    puts("ok");
+    return 0;
+}
