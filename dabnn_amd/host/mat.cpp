@@ -53,16 +53,11 @@ Mat::~Mat() {
     if (dev && !external_memory) (void)hipFree(dev);
 }
 
-// Copies between host and device go over one stream of their own that does not synchronise with the null stream, and
-// wait for it.  A plain hipMemcpy works on the null stream, and a null-stream operation issued by one thread while
-// another thread's Net captures its HIP graph fails and invalidates that capture.
+// Copies between host and device go over the current device's copy stream and wait for it.
 static hipStream_t copy_stream() {
-    static hipStream_t s = [] {
-        hipStream_t created = nullptr;
-        hip_check(hipStreamCreateWithFlags(&created, hipStreamNonBlocking), "hipStreamCreate");
-        return created;
-    }();
-    return s;
+    int device = 0;
+    hip_check(hipGetDevice(&device), "hipGetDevice");
+    return static_cast<hipStream_t>(copy_stream(device));
 }
 
 std::shared_ptr<Mat> Mat::planned(int n, int h, int w, int c, DataType type, const std::string &name) {

@@ -4,6 +4,7 @@
 
 #include <algorithm>
 #include <cstring>
+#include <map>
 #include <stdexcept>
 #include <string>
 
@@ -11,6 +12,22 @@ namespace bnn {
 
 static void hip_check(hipError_t e, const char *what) {
     if (e != hipSuccess) throw std::runtime_error(std::string(what) + ": " + hipGetErrorString(e));
+}
+
+void *copy_stream(int device) {
+    static std::mutex mutex;
+    static std::map<int, hipStream_t> streams;
+    std::lock_guard<std::mutex> lock(mutex);
+    hipStream_t &s = streams[device];
+    if (!s) {
+        int current = 0;
+        hip_check(hipGetDevice(&current), "hipGetDevice");
+        if (current != device) hip_check(hipSetDevice(device), "hipSetDevice");
+        const hipError_t e = hipStreamCreateWithFlags(&s, hipStreamNonBlocking);
+        if (current != device) hip_check(hipSetDevice(current), "hipSetDevice");
+        hip_check(e, "hipStreamCreate");
+    }
+    return s;
 }
 
 Staging::Staging(size_t bytes) {
@@ -38,7 +55,6 @@ Staging::~Staging() {
     wake_.notify_all();
     for (auto &t : helpers_) t.join();
     for (void *e : events_) (void)hipEventDestroy(static_cast<hipEvent_t>(e));
-    if (download_stream_) (void)hipStreamDestroy(static_cast<hipStream_t>(download_stream_));
     (void)hipHostFree(memory_);
 }
 
@@ -167,22 +183,9 @@ void Staging::upload(void *dst, const void *src, size_t bytes, void *stream) {
     wait_for_helpers();
 }
 
-// (one that does not synchronise with the null stream, as Mat's copies)
-void Staging::make_download_stream() {
-    int current = 0;
-    hip_check(hipGetDevice(&current), "hipGetDevice");
-    if (current != device_) hip_check(hipSetDevice(device_), "hipSetDevice");
-    hipStream_t s = nullptr;
-    const hipError_t e = hipStreamCreateWithFlags(&s, hipStreamNonBlocking);
-    if (current != device_) hip_check(hipSetDevice(current), "hipSetDevice");
-    hip_check(e, "hipStreamCreate");
-    download_stream_ = s;
-}
-
 void Staging::download(void *dst, const void *src, size_t bytes) {
     std::lock_guard<std::mutex> one(use_);
-    if (!download_stream_) make_download_stream();
-    hipStream_t s = static_cast<hipStream_t>(download_stream_);
+    hipStream_t s = static_cast<hipStream_t>(copy_stream(device_));
     const size_t pieces = (bytes + kPiece - 1) / kPiece, window = std::min(kEvents, bytes_ / kPiece);  // (an event each)
     try {
         for (size_t i = 0; i < pieces + window; ++i) {

@@ -17,6 +17,12 @@
 
 namespace bnn {
 
+// The stream (a hipStream_t) for copies between host and device memory that belong to no net's own stream: one per device, for the
+// life of the process (making one takes 150 to 200 us), and one that does not synchronise with the null stream.  A plain hipMemcpy works
+// on the null stream, and a null-stream operation issued by one thread while another thread's Net captures its HIP graph fails and
+// invalidates that capture.
+void *copy_stream(int device);
+
 class Staging {
    public:
     static constexpr size_t kBlock = 256u << 10, kMost = 32u << 20, kLargest = 8u << 20;
@@ -34,7 +40,7 @@ class Staging {
     // Copies host memory to the device on `stream`; `src` may change once the call returns.  The caller synchronises the
     // stream before the next call (a Net's runs do).
     void upload(void *dst, const void *src, size_t bytes, void *stream);
-    // Copies device memory to the host and waits.  The stream is the Staging's own, of the device that its events are of: the runtime
+    // Copies device memory to the host and waits, over the copy stream of the device that the Staging's events are of: the runtime
     // records no event of one device on a stream of another.
     void download(void *dst, const void *src, size_t bytes);
 
@@ -47,14 +53,12 @@ class Staging {
     void copy_blocks();  // takes blocks until there are none left (a helper's share of an upload)
     void helper();
     void start_helpers();
-    void make_download_stream();
 
     unsigned char *memory_ = nullptr;
     size_t bytes_ = 0;
     int device_ = 0;
     static constexpr size_t kEvents = 16;
     std::vector<void *> events_;  // of transfer i: i % kEvents
-    void *download_stream_ = nullptr;  // made by the first download
 
     // the upload at hand
     unsigned char *dst_ = nullptr;
