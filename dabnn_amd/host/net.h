@@ -49,8 +49,8 @@ class BNN_API Net : public std::enable_shared_from_this<Net> {
     std::shared_ptr<Mat> blob(const std::string &name);
     // The blob as the layers hold it, slice or not; Mat::download and the host accessors work on both.
     std::shared_ptr<Mat> stored_blob(const std::string &name);
-    // The blob's device memory to the host, contiguous, at most `bytes` of it (what dabnet_get_blob does): outputs of the last run
-    // are in pinned memory already.
+    // The blob's device memory to the host, contiguous, at most `bytes` of it (what dabnet_get_blob does): outputs of the last
+    // run that are asked for run after run are in pinned memory already.
     void download(const std::shared_ptr<Mat> &m, void *host, size_t bytes);
     // If `m` is the column matrix of a layer that convolves without one, or a blob inside two layers' one pass: makes it, and
     // keeps it up to date from now on.
@@ -107,6 +107,7 @@ class BNN_API Net : public std::enable_shared_from_this<Net> {
     struct Graph {
         void *exec = nullptr;
         const void *input = nullptr;
+        int copies = 0;  // of mirrors
     } graphs_[2];
     void *input_own_dev_ = nullptr;       // the input blob's own allocation
     int input_rebinds_ = 0;               // captures thrown away because the caller's buffer changed
@@ -116,14 +117,17 @@ class BNN_API Net : public std::enable_shared_from_this<Net> {
     void launch_layers(bool staged_input);
     void enqueue_layers(bool staged_input);
     std::unique_ptr<Staging> staging_;    // pinned memory for inputs, and for blobs that are asked for
-    // Small blobs that no layer reads are copied to pinned memory behind the layers of every run.
+    // Small blobs that no layer reads are copied to pinned memory behind the layers of the first two runs, and of every run once they
+    // have been asked for.
     struct Mirror {
         std::shared_ptr<Mat> mat;
         float *host;
+        bool asked = false;
+        bool copied = false;  // by the run at hand
+        bool valid = false;   // holds what the last run left
     };
     std::vector<Mirror> mirrors_;
     void *mirror_memory_ = nullptr;
-    bool mirrors_valid_ = false;          // they hold what the last run left
     void plan_mirrors();
 };
 

@@ -71,3 +71,42 @@ def test_several_nets_and_threads():
         t.join()
     for a, b in zip(got, want):
         assert np.array_equal(a, b)
+
+
+def copies_in_a_run(n, x):
+    """Launches of the copy kernel in one run of a net without a graph."""
+    from torch.profiler import ProfilerActivity, profile
+    with profile(activities=[ProfilerActivity.CUDA]) as p:
+        n.run(x)
+        torch.cuda.synchronize()
+    names = [e.name for e in p.events()]
+    assert any("fconv" in s for s in names), names  # the trace shows the layers
+    return sum("copy_f32" in s for s in names)
+
+
+def test_outputs_are_copied_for_who_asks():
+    n = make(2, 32)
+    n.set_use_graph(False)
+    x = torch.randn(2, 32, 32, 3, device="cuda")
+    for _ in range(3):
+        n.run(x)
+    assert copies_in_a_run(n, x) == 0
+    want = n.get_blob("logits")
+    assert np.array_equal(n.get_blob("logits"), want)
+    assert copies_in_a_run(n, x) == 1
+    assert np.array_equal(n.get_blob("logits"), want)
+
+
+# the copies begin before the graph is captured, in the graph's place, and behind either kind of input
+@pytest.mark.parametrize("first_look", [1, 2, 3, 5])
+def test_blobs_asked_for_late(first_look):
+    n = make(2, 32)
+    r = np.random.default_rng(first_look)
+    for i in range(1, 12):
+        x = r.standard_normal((2, 32, 32, 3)).astype(np.float32)
+        n.run(x if i % 3 else torch.from_numpy(x).cuda())
+        if i >= first_look:
+            got = n.get_blob("logits")
+            other = make(2, 32).run(x)
+            assert np.array_equal(got, other.get_blob("logits")), i
+            other.close()
