@@ -179,7 +179,17 @@ static int pair_rows(int n, int h, int w) {
     return (h + bands - 1) / bands;
 }
 
+// Strips of an image, or 0 where the kernel does not take the problem.
+static int pair_bands(int n, int h, int w) {
+    const int rows = pair_rows(n, h, w);
+    if (rows == 0) return 0;
+    const int bands = (h + rows - 1) / rows;
+    return (long long)h * w * 256 < (1ll << 31) && (long long)n * bands < kMostBlocks ? bands : 0;
+}
+
 }  // namespace dab
+
+extern "C" int dab_bconv3x3_pair_takes(int n, int h, int w) { return n > 0 && h > 0 && w > 0 && dab::pair_bands(n, h, w) > 0; }
 
 extern "C" int dab_bconv3x3_pair(const uint64_t *x, const float *shortcut, int n, int h, int w, const uint64_t *w1, const float *a1, const float *b1,
                                  const uint64_t *w2, const float *a2, const float *b2, float *out, uint64_t *out_packed, dab_stream_t stream) {
@@ -191,14 +201,13 @@ extern "C" int dab_bconv3x3_pair(const uint64_t *x, const float *shortcut, int n
     DAB_REQUIRE((reinterpret_cast<uintptr_t>(x) & 7) == 0 && (reinterpret_cast<uintptr_t>(w1) & 7) == 0 && (reinterpret_cast<uintptr_t>(w2) & 7) == 0 &&
                     (reinterpret_cast<uintptr_t>(out_packed) & 7) == 0 && (reinterpret_cast<uintptr_t>(out) & 3) == 0 && (reinterpret_cast<uintptr_t>(shortcut) & 3) == 0,
                 "%s: misaligned pointer", fn);
+    const int bands = pair_bands(n, h, w);
+    if (bands == 0) return fail(DAB_EUNSUPPORTED, "%s: %d images of %d x %d are not covered", fn, n, h, w);
     const int rows = pair_rows(n, h, w);
-    const long long pixels = (long long)h * w, bands = rows ? (h + rows - 1) / rows : 0;
-    if (rows == 0 || pixels * 256 >= (1ll << 31) || (long long)n * bands >= kMostBlocks)
-        return fail(DAB_EUNSUPPORTED, "%s: images of %d x %d are not covered", fn, h, w);
     BconvPairArgs p;
     p.x = x, p.shortcut = shortcut, p.out = out, p.bits = out_packed;
     p.w[0] = w1, p.w[1] = w2, p.a[0] = a1, p.a[1] = a2, p.b[0] = b1, p.b[1] = b2;
-    p.H = h, p.W = w, p.rows = rows, p.bands = (int)bands, p.above = (w + 31) / 32;
+    p.H = h, p.W = w, p.rows = rows, p.bands = bands, p.above = (w + 31) / 32;
     p.div_bands = FastDiv((uint32_t)bands), p.div_w = FastDiv((uint32_t)w);
     const size_t lds = 2 * kPairFilterBytes + (size_t)(2 * rows + 6) * (w + 2) * 8;
     const dim3 grid((unsigned)(n * bands));

@@ -805,8 +805,8 @@ void Net::pair_residual_layers() {
     auto residual = [&](const std::shared_ptr<BinConv> &bc) {
         const Mat &in = *bc->input_mat;
         return bc->method() == BinConv::DIRECT_CONV && in.elem_c == 64 && bc->weight_mat->n == 64 && bc->stride_h == 1 && bc->pad_h == 1 && bc->fused_a &&
-               bc->fused_shortcut == bc->input_mat && !bc->has_slices() && !in.ld && bc->output_mat != bc->input_mat && in.w >= 16 && in.w <= 64 &&
-               (long long)in.h * in.w < (1 << 22) && (long long)in.n * in.h * in.w >= 48000;
+               bc->fused_shortcut == bc->input_mat && !bc->has_slices() && !in.ld && bc->output_mat != bc->input_mat && in.w <= 64 &&
+               (long long)in.n * in.h * in.w >= 48000 && dab_bconv3x3_pair_takes(in.n, in.h, in.w);
     };
     for (size_t i = 0; i + 1 < layers.size(); ++i) {
         auto first = std::dynamic_pointer_cast<BinConv>(layers[i]), second = std::dynamic_pointer_cast<BinConv>(layers[i + 1]);

@@ -185,11 +185,12 @@ DAB_API int dab_bconv3x3_affine_add_sign(const uint64_t *x, int n, int h, int w,
  * Two residual layers in one pass (no reference counterpart; BinConv, Affine, Add twice): v1 = a1 * bconv_3x3(x, w1) + b1 + shortcut,
  * out = a2 * bconv_3x3(sign bits of v1, w2) + b2 + v1, each operation rounded by itself, for 64 channels everywhere, stride 1, pad 1;
  * x: [n][h][w] words, the sign bits of `shortcut`.  v1 is not written.  out_packed (may be NULL): the sign bits of out.
- * Bit for bit two calls of dab_bconv3x3_affine_add_sign.  DAB_EUNSUPPORTED for widths whose strips do not fit the kernel (above 240
- * or so, and below 16).
+ * Bit for bit two calls of dab_bconv3x3_affine_add_sign.  DAB_EUNSUPPORTED for shapes that dab_bconv3x3_pair_takes answers with 0: it
+ * takes images of 16 to 128 columns and of 160, those of a single row up to 160, and fewer than 2^23 strips in all.
  */
 DAB_API int dab_bconv3x3_pair(const uint64_t *x, const float *shortcut, int n, int h, int w, const uint64_t *w1, const float *a1, const float *b1,
                               const uint64_t *w2, const float *a2, const float *b2, float *out, uint64_t *out_packed, dab_stream_t stream);
+DAB_API int dab_bconv3x3_pair_takes(int n, int h, int w);
 
 /*
  * BinConv::forward_impl (dabnn/layers/BinConv.cpp:144-191) for a batch of

@@ -128,3 +128,18 @@ def test_binconv_forward_refuses_images_smaller_than_the_direct_kernel():
     for h, w, pad in [(2, 9, 0), (9, 2, 0), (2, 2, 0)]:
         rc = capi.lib.dab_binconv_forward(vp(16), 2, h, w, 64, vp(16), vp(16), 9, 3, 3, pad, pad, 2, 2, 64, vp(32), vp(32), 1 << 30, None, vp(None))
         assert rc == capi.DAB_EINVAL and "smaller than the kernel" in capi.last_error(), capi.last_error()
+
+
+def test_shapes_that_two_layers_take_in_one_pass():
+    """dab_bconv3x3_pair_takes says what the call refuses, at the edges that the header states."""
+    from dabnn_amd import capi
+    vp = ctypes.c_void_p
+    takes = capi.lib.dab_bconv3x3_pair_takes
+    for h in (2, 7, 56, 300):
+        assert [w for w in range(1, 600) if takes(4, h, w)] == list(range(16, 129)) + [160]
+    assert [w for w in range(1, 600) if takes(4, 1, w)] == list(range(16, 161))
+    assert takes(2**22, 1, 16) and not takes(2**23, 1, 16) and not takes(2**20, 300, 64) and not takes(1, 2**23, 16)
+    assert not takes(0, 8, 16) and not takes(1, 0, 16) and not takes(1, 8, -1)
+    for n, h, w in [(4, 7, 15), (4, 7, 129), (4, 7, 159), (4, 7, 161), (2**23, 1, 16), (2**20, 300, 64)]:
+        rc = capi.lib.dab_bconv3x3_pair(vp(16), vp(16), n, h, w, vp(16), vp(16), vp(16), vp(16), vp(16), vp(16), vp(32), vp(64), vp(None))
+        assert rc == capi.DAB_EUNSUPPORTED and not takes(n, h, w), (n, h, w)
