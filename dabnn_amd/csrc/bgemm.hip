@@ -427,24 +427,46 @@ static int launch_bit_gemm(const char *fn, BitGemmArgs &p, hipStream_t s) {
     const long long per_channel = (long long)p.units * 2 * (CC == 3 ? 16 : CC * 4);
     // The walking kernel where its filters fit and its waves find tiles for every SIMD; also for one to three units of
     // depth, which are no work for four waves.
-    // 64 channels a wave for plain matrices (m128 k18 n50176: 12.6 us against 16.4); for windows, whose lanes spend more on
-    // addresses than on filters, where the filters are no more than that, so that every window is fetched once (3x3 over 64, 128 and
-    // 192 channels -> 64, 131 072 pixels: 20.1, 18.5 and 20.7 -> 15.1, 15.3 and 17.5 us; 23 x 56 x 56 x 384 -> 40, 5x5: 69 -> 48;
-    // below 4096 pieces not for part of a second 32: 582 x 8 x 8 x 128 -> 40 7.8 against 8.9), else 32 (100 x 25 x 25 x 192 -> 472,
-    // 5 x 5, stride 2: 34 us against 43).
-    const bool two = L == kFilterColumns ? p.g.cols > 32 && pieces >= 2048 : p.g.cols > 32 && p.g.cols <= 64 && pieces >= (p.g.cols == 64 ? 2048 : 4096);
-    const int ch = two ? 64 : 32;
-    if ((pieces >= 2048 || p.units < 4) && per_channel * ch <= kFilterLdsBytes) {
-        p.col_tiles = (p.g.cols + ch - 1) / ch;
+    struct Walk {
+        int col_tiles, lds;
+        bool fits;
+        long long groups;
+        long long rounds;  // tiles that the waves of the fullest CU walk
+    };
+    auto walk = [&](int ch) {
+        Walk w;
+        w.col_tiles = (p.g.cols + ch - 1) / ch;
+        w.fits = per_channel * ch <= kFilterLdsBytes;
+        w.lds = w.fits ? (int)(per_channel * ch) : 0;
+        const int cus = simd_count() / 4, by_registers = ch == 64 ? 3 : 4, by_lds = 160 * 1024 / (w.lds + 1024);
+        const long long most = (long long)cus * (by_lds < by_registers ? by_lds : by_registers) / w.col_tiles, want = (p.row_tiles + 3) / 4;
+        w.groups = want < most ? want : most < 1 ? 1 : most;
+        const long long per_wave = (p.row_tiles + w.groups * 4 - 1) / (w.groups * 4);
+        w.groups = (p.row_tiles + 4 * per_wave - 1) / (4 * per_wave);
+        w.rounds = (w.groups * w.col_tiles + cus - 1) / cus * per_wave;
+        return w;
+    };
+    // 64 channels a wave for plain matrices (m128 k18 n50176: 12.6 us against 16.4).  For windows, whose lanes spend more on addresses
+    // than on filters, with 33 to 64 channels, so that every window is fetched once, from 4096 pieces on (2048 with all 64: 582 x 8 x 8 x
+    // 128 -> 40 7.8 us with 32 against 8.9).  A tile of 64 takes 1.5 to 1.9 times as long as one of 32, so not where the fullest CU walks
+    // two thirds as many of them (45 such layers: 0.95).  570 random layers: into slices of their output 1.17 times as fast (0.93 to 1.8),
+    // into an output of their own 1.06 (30 words a filter and more 0.94 to 1.3; fewer, bound by the stores, 0.89 to 1.6).  3x3 over 128
+    // channels -> 64, into slices of 256, 131 072 pixels: 18.5 -> 15.3 us.  With more channels 32 (100 x 25 x 25 x 192 -> 472, 5 x 5, stride 2:
+    // 34 us against 43).
+    const bool wide = L == kFilterColumns ? p.g.cols > 32 && pieces >= 2048 : p.g.cols > 32 && p.g.cols <= 64 && pieces >= (p.g.cols == 64 ? 2048 : 4096);
+    const Walk by32 = walk(32), by64 = walk(64);
+    // Where 64 filters do not fit (above 144 words, or 108 in chunks of three), windows leave the walking kernel for the one that splits the
+    // depth, 64 channels a block: 23 x 56 x 56 x 384 -> 40, 5x5, 50 us with 32 channels a wave, 32 split; 41 x 56 x 56 x 384 -> 64, 6x6, 113 and
+    // 85.  Not in chunks of one word or two from 8000 pieces on, but for few channels and pieces (82 x 56 x 56 x 320 -> 64, 6x6, 269 and 375;
+    // -> 40 270 and 256, 459 x 33 x 33 458 and 500).
+    const bool split = wide && !by64.fits && (L == kFilterColumns || CC >= 3 || pieces < 8000 || (p.g.cols <= 40 && pieces < 20000));
+    const bool two = wide && by64.fits && (L == kFilterColumns || 2 * by32.rounds > 3 * by64.rounds);
+    const Walk &w = two ? by64 : by32;
+    if ((pieces >= 2048 || p.units < 4) && w.fits && !split) {
+        p.col_tiles = w.col_tiles;
         p.div_col_tiles = FastDiv((uint32_t)p.col_tiles);
-        const size_t lds = (size_t)(per_channel * ch);
-        int per_cu = (int)(160 * 1024 / (lds + 1024));
-        const int by_registers = two ? 3 : 4;
-        per_cu = per_cu > by_registers ? by_registers : per_cu;
-        const long long most = (long long)(simd_count() / 4) * per_cu / p.col_tiles, want = (p.row_tiles + 3) / 4;
-        long long groups = want < most ? want : most < 1 ? 1 : most;
-        const long long per_wave = (p.row_tiles + groups * 4 - 1) / (groups * 4);
-        groups = (p.row_tiles + 4 * per_wave - 1) / (4 * per_wave);
+        const size_t lds = (size_t)w.lds;
+        const long long groups = w.groups;
         auto launch = [&](auto nt) {
             constexpr auto kernel = bit_gemm_stream_kernel<CC, L, E, decltype(nt)::value, LONG>;
             if (lds > 64 * 1024) {

@@ -14,6 +14,11 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("n,h,w,cin,cout,k,stride,pad", [
     (1, 256, 128, 192, 64, 3, 1, 1), (1, 255, 128, 192, 64, 3, 1, 1), (2, 255, 128, 64, 40, 5, 1, 2), (1, 255, 256, 64, 33, 1, 1, 0),
     (3, 157, 139, 320, 56, 3, 1, 1), (1, 256, 256, 128, 64, 5, 2, 2), (33, 45, 47, 128, 64, 1, 1, 0), (1, 256, 256, 192, 65, 3, 1, 1),
+    # 150 to 250 words a filter, of which 64 do not fit: the depth split from 4096 pieces on, but 32 channels a wave in chunks of one word or
+    # two from 8000 on (with up to 40 channels from 20 000); 108 and 144 words, which fit
+    (5, 128, 128, 320, 64, 6, 1, 3), (8, 128, 128, 320, 64, 6, 1, 3), (8, 128, 128, 320, 40, 6, 1, 3), (20, 128, 128, 640, 40, 4, 1, 2),
+    (5, 128, 128, 384, 56, 5, 1, 2), (9, 128, 128, 512, 33, 5, 1, 2), (6, 128, 128, 640, 64, 5, 1, 2), (8, 128, 128, 576, 64, 4, 1, 2),
+    (4, 128, 128, 768, 48, 3, 1, 1),
 ])
 @pytest.mark.parametrize("epilogue", ["counts", "affine", "sign"])
 def test_windows(n, h, w, cin, cout, k, stride, pad, epilogue):
