@@ -25,10 +25,10 @@ struct FloatBconvArgs {
     int kw, taps;
     int words;         // of a filter, the converter's padding word included
     int rows, bands;   // output rows of a block, blocks one below the other
-    int in_rows, in_w;  // input rows and padded columns in LDS
+    int in_rows;        // input rows in LDS
     int px_bytes, row_bytes, filter_bytes;  // LDS strides
     int groups;        // of 64 channels
-    int zero_at, filters_at, part_at;       // LDS offsets
+    int filters_at, part_at;                // LDS offsets
     uint32_t w_words;  // in the filter tensor
     uint32_t row_words;  // packed words of an input row
     FastDiv div_groups, div_bands, div_words, div_row_words, div_cw, div_ow, div_kw;
@@ -255,14 +255,14 @@ static bool plan_float_conv(FloatConvPlan &plan, const float *x, int n, int h, i
         best = cycles;
         plan.ds = ds, plan.lds = (size_t)lds, plan.grid = (unsigned)blocks;
         plan.a.rows = rows, plan.a.bands = bands, plan.a.in_rows = in_rows;
-        plan.a.zero_at = (int)(in_rows * row_bytes), plan.a.filters_at = (int)packed, plan.a.part_at = (int)(packed + filters);
+        plan.a.filters_at = (int)packed, plan.a.part_at = (int)(packed + filters);
     }
     if (best > kFloatConvCycles || best >= 1e30) return false;
     FloatBconvArgs &a = plan.a;
     a.x = x, a.w = wgt, a.out = out;
     a.H = h, a.W = w, a.CW = cw, a.OH = oh, a.OW = ow, a.cout = cout;
     a.stride_h = stride_h, a.stride_w = stride_w, a.pad_h = pad_h, a.pad_w = pad_w;
-    a.kw = kw, a.taps = taps, a.words = words, a.in_w = (int)in_w;
+    a.kw = kw, a.taps = taps, a.words = words;
     a.px_bytes = (int)px_bytes, a.row_bytes = (int)row_bytes, a.filter_bytes = (int)filter_bytes;
     a.groups = groups, a.w_words = (uint32_t)((long long)cout * words), a.row_words = (uint32_t)(w * cw);
     a.div_groups = FastDiv((uint32_t)groups), a.div_bands = FastDiv((uint32_t)a.bands), a.div_words = FastDiv((uint32_t)words);

@@ -843,7 +843,7 @@ void Net::run(const void *host_input) {
         pageable = where.type == hipMemoryTypeUnregistered;
     else
         (void)hipGetLastError();
-    const bool staged = pageable && in->bytes() <= (1u << 20) && in->bytes() <= staging_->bytes();
+    const bool staged = pageable && in->bytes() <= (1u << 20);  // (staging_ holds that much)
     bind_input(nullptr, staged);
     if (staged)
         std::memcpy(staging_->memory(), host_input, in->bytes());

@@ -119,11 +119,6 @@ void Staging::upload(void *dst, const void *src, size_t bytes, void *stream) {
     if (bytes == 0) return;
     std::lock_guard<std::mutex> one(use_);
     hipStream_t s = static_cast<hipStream_t>(stream);
-    if (bytes <= std::min<size_t>(bytes_, 1u << 20)) {
-        std::memcpy(memory_, src, bytes);
-        hip_check(hipMemcpyAsync(dst, memory_, bytes, hipMemcpyHostToDevice, s), "hipMemcpyAsync");
-        return;
-    }
     start_helpers();
     dst_ = static_cast<unsigned char *>(dst), src_ = static_cast<const unsigned char *>(src);
     size_ = bytes, blocks_ = (bytes + kBlock - 1) / kBlock;

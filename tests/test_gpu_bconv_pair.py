@@ -28,6 +28,12 @@ def pair(v0, ws, ab, want_bits=True, guard=0):
     return rc, out, bits
 
 
+def same(a, b):
+    """Bit for bit, but for the bits of a NaN."""
+    nan = b.isnan()
+    return torch.equal(a.isnan(), nan) and torch.equal(a[~nan].view(torch.int32), b[~nan].view(torch.int32))
+
+
 @pytest.mark.parametrize("n,h,w", [
     (1, 56, 56), (2, 56, 56), (37, 56, 56), (300, 56, 56), (1, 1, 16), (1, 2, 31), (3, 3, 32), (2, 5, 33), (3, 17, 17), (40, 28, 28), (5, 14, 18),
     (2, 57, 55), (1, 61, 64), (3, 23, 65), (2, 9, 100), (2, 7, 160), (70, 15, 57), (1, 200, 40), (260, 16, 16),
@@ -41,12 +47,12 @@ def test_equals_two_layers(n, h, w):
     guard = 1024
     rc, out, bits = pair(v0, ws, ab, guard=guard)
     assert rc == capi.DAB_OK
-    assert torch.equal(out[guard:-guard].view(torch.int32), v2.view(-1).view(torch.int32)) or torch.equal(torch.nan_to_num(out[guard:-guard], nan=-9.0), torch.nan_to_num(v2.view(-1), nan=-9.0))
+    assert same(out[guard:-guard], v2.view(-1))
     assert torch.equal(bits[guard:-guard], x2.view(-1))
     assert bool((out[:guard] == -5).all()) and bool((out[-guard:] == -5).all()) and bool((bits[:guard] == -5).all()) and bool((bits[-guard:] == -5).all())
     rc, alone, untouched = pair(v0, ws, ab, want_bits=False)
     assert rc == capi.DAB_OK and bool((untouched == -5).all())
-    assert torch.equal(torch.nan_to_num(alone, nan=-9.0), torch.nan_to_num(v2.view(-1), nan=-9.0))
+    assert same(alone, v2.view(-1))
 
 
 @pytest.mark.parametrize("h,w", [(8, 15), (8, 300), (8, 129)])
