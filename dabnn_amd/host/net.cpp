@@ -832,7 +832,7 @@ void Net::pair_residual_layers() {
 }
 
 // Host inputs of up to a megabyte are put into pinned memory, from where the layers' first kernel takes them; larger ones
-// go through it in blocks, and memory that the caller has pinned is copied from where it lies.
+// go through it in blocks from the second on, and memory that the caller has pinned is copied from where it lies.
 void Net::run(const void *host_input) {
     BNN_ASSERT(prepared_, "run before read");
     BNN_ASSERT(host_input != nullptr, "run: null input");
@@ -847,11 +847,16 @@ void Net::run(const void *host_input) {
     bind_input(nullptr, staged);
     if (staged)
         std::memcpy(staging_->memory(), host_input, in->bytes());
-    else if (pageable)
+    else if (pageable && uploaded_) {
+        {
+            std::lock_guard<std::mutex> lock(capture_mutex());
+            staging_->grow(in->bytes());
+        }
         staging_->upload(in->dev, host_input, in->bytes(), stream_);
-    else
+    } else
         hip_check(hipMemcpyAsync(in->dev, host_input, in->bytes(), hipMemcpyHostToDevice, static_cast<hipStream_t>(stream_)),
                   "hipMemcpyAsync");
+    uploaded_ = uploaded_ || (pageable && !staged);
     launch_layers(staged);
 }
 

@@ -117,6 +117,7 @@ class BNN_API Net : public std::enable_shared_from_this<Net> {
     void launch_layers(bool staged_input);
     void enqueue_layers(bool staged_input);
     std::unique_ptr<Staging> staging_;    // pinned memory for inputs, and for blobs that are asked for
+    bool uploaded_ = false;               // a large input from pageable memory
     // Small blobs that no layer reads are copied to pinned memory behind the layers of the first two runs, and of every run once they
     // have been asked for.
     struct Mirror {

@@ -31,7 +31,7 @@ void *copy_stream(int device) {
 }
 
 Staging::Staging(size_t bytes) {
-    bytes_ = std::min(std::max(bytes, kPiece), kMost);
+    bytes_ = std::min(std::max(bytes, kPiece), kSmall);
     hip_check(hipGetDevice(&device_), "hipGetDevice");
     void *p = nullptr;
     hip_check(hipHostMalloc(&p, bytes_, 0), "hipHostMalloc");
@@ -56,6 +56,16 @@ Staging::~Staging() {
     for (auto &t : helpers_) t.join();
     for (void *e : events_) (void)hipEventDestroy(static_cast<hipEvent_t>(e));
     (void)hipHostFree(memory_);
+}
+
+void Staging::grow(size_t bytes) {
+    std::lock_guard<std::mutex> one(use_);
+    const size_t want = std::min(bytes, kMost);
+    if (want <= bytes_) return;
+    void *p = nullptr;
+    hip_check(hipHostMalloc(&p, want, 0), "hipHostMalloc");
+    (void)hipHostFree(memory_);
+    memory_ = static_cast<unsigned char *>(p), bytes_ = want;
 }
 
 void Staging::wait_for_room(size_t block) {

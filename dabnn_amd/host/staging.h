@@ -2,7 +2,10 @@
 //
 // A copy from or to pageable memory goes through the runtime's own small staging or pins the caller's pages for the call: 24 MB
 // to the device took 650 to 890 us (430 from pinned memory), 256 KB either way 106 us (13), 160 KB from the device 70.
-// A Staging holds up to 32 MB of pinned memory for the life of its Net.  Large inputs run through it in blocks of 256 KB that the
+// A Staging holds 512 KB to 1 MB of pinned memory for the life of its Net, and up to 32 MB from the second large input on: memory
+// that is pinned for the first time is mapped page by page as it is first written, 0.4 ms for 2 MB and 2.5 for 24, which pays after ten
+// to twenty runs (batch 40 of 224 x 224 images: 1.01 ms a run without, 0.87 with it, 3.8 the run that writes it first; 0.92 with 8 MB,
+// 1.06 with 4).  Large inputs run through it in blocks of 256 KB that the
 // calling thread and up to three helpers copy in, and leave it in transfers of 1, 2, 4 and then 8 MB, each started as soon
 // as its blocks are there: one transfer costs 15 us beside its bytes, and the first should not wait long (24 MB in equal
 // transfers of 512 KB, 2 MB and 4 MB: 960, 675 and 720 us; the link alone takes 430).
@@ -25,12 +28,13 @@ void *copy_stream(int device);
 
 class Staging {
    public:
-    static constexpr size_t kBlock = 256u << 10, kMost = 32u << 20, kLargest = 8u << 20;
+    static constexpr size_t kBlock = 256u << 10, kSmall = 1u << 20, kMost = 32u << 20, kLargest = 8u << 20;
     static constexpr size_t kPiece = 512u << 10;  // of a download: its first piece is copied out while the next ones arrive
 
-    // Room for `bytes`, 512 KB at least and 32 MB at most; allocates.
+    // Room for `bytes`, 512 KB at least and 1 MB at most; allocates, and so does grow: up to 32 MB (memory() is another then).
     explicit Staging(size_t bytes);
     ~Staging();
+    void grow(size_t bytes);
     Staging(const Staging &) = delete;
     Staging &operator=(const Staging &) = delete;
 

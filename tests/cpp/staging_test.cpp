@@ -75,9 +75,16 @@ int main() {
         for (int device : {0, 1}) {
             current = device;
             bnn::Staging staging(10 << 20);
-            for (size_t floats : {1000, 400000, 2000001, 21000000}) {  // one piece, pieces, a round of the events, longer than the pinned memory
+            CHECK(staging.bytes() == 1 << 20);
+            for (size_t floats : {1000, 400000}) CHECK(round_trip(staging, device, floats) == 0);  // one piece, longer than the pinned memory
+            staging.grow(10 << 20);
+            staging.grow(5 << 20);
+            CHECK(staging.bytes() == 10 << 20 && pinned == 1);
+            for (size_t floats : {1000, 400000, 2000001, 21000000}) {  // pieces, a round of the events, longer than the pinned memory
                 CHECK(round_trip(staging, device, floats) == 0);
             }
+            staging.grow(100 << 20);
+            CHECK(staging.bytes() == 32 << 20 && round_trip(staging, device, 21000000) == 0);
             // asked for from a thread whose current device is another one, which stays what it was
             current = 1 - device;
             std::vector<float> in(200000, 2.f), out(200000);
