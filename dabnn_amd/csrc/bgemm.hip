@@ -428,17 +428,17 @@ static int launch_bit_gemm(const char *fn, BitGemmArgs &p, hipStream_t s) {
     // The walking kernel where its filters fit and its waves find tiles for every SIMD; also for one to three units of
     // depth, which are no work for four waves.
     struct Walk {
-        int col_tiles, lds;
-        bool fits;
+        int channels, col_tiles;
+        size_t lds;
         long long groups;
         long long rounds;  // tiles that the waves of the fullest CU walk
     };
+    auto fits = [&](int ch) { return per_channel * ch <= kFilterLdsBytes; };
     auto walk = [&](int ch) {
         Walk w;
-        w.col_tiles = (p.g.cols + ch - 1) / ch;
-        w.fits = per_channel * ch <= kFilterLdsBytes;
-        w.lds = w.fits ? (int)(per_channel * ch) : 0;
-        const int cus = simd_count() / 4, by_registers = ch == 64 ? 3 : 4, by_lds = 160 * 1024 / (w.lds + 1024);
+        w.channels = ch, w.col_tiles = (p.g.cols + ch - 1) / ch;
+        w.lds = (size_t)(per_channel * ch);
+        const int cus = simd_count() / 4, by_registers = ch == 64 ? 3 : 4, by_lds = (int)(160 * 1024 / (w.lds + 1024));
         const long long most = (long long)cus * (by_lds < by_registers ? by_lds : by_registers) / w.col_tiles, want = (p.row_tiles + 3) / 4;
         w.groups = want < most ? want : most < 1 ? 1 : most;
         const long long per_wave = (p.row_tiles + w.groups * 4 - 1) / (w.groups * 4);
@@ -454,18 +454,20 @@ static int launch_bit_gemm(const char *fn, BitGemmArgs &p, hipStream_t s) {
     // channels -> 64, into slices of 256, 131 072 pixels: 18.5 -> 15.3 us.  With more channels 32 (100 x 25 x 25 x 192 -> 472, 5 x 5, stride 2:
     // 34 us against 43).
     const bool wide = L == kFilterColumns ? p.g.cols > 32 && pieces >= 2048 : p.g.cols > 32 && p.g.cols <= 64 && pieces >= (p.g.cols == 64 ? 2048 : 4096);
-    const Walk by32 = walk(32), by64 = walk(64);
     // Where 64 filters do not fit (above 144 words, or 108 in chunks of three), windows leave the walking kernel for the one that splits the
     // depth, 64 channels a block: 23 x 56 x 56 x 384 -> 40, 5x5, 50 us with 32 channels a wave, 32 split; 41 x 56 x 56 x 384 -> 64, 6x6, 113 and
     // 85.  Not in chunks of one word or two from 8000 pieces on, but for few channels and pieces (82 x 56 x 56 x 320 -> 64, 6x6, 269 and 375;
     // -> 40 270 and 256, 459 x 33 x 33 458 and 500).
-    const bool split = wide && !by64.fits && (L == kFilterColumns || CC >= 3 || pieces < 8000 || (p.g.cols <= 40 && pieces < 20000));
-    const bool two = wide && by64.fits && (L == kFilterColumns || 2 * by32.rounds > 3 * by64.rounds);
-    const Walk &w = two ? by64 : by32;
-    if ((pieces >= 2048 || p.units < 4) && w.fits && !split) {
+    const bool split = wide && !fits(64) && (L == kFilterColumns || CC >= 3 || pieces < 8000 || (p.g.cols <= 40 && pieces < 20000));
+    if ((pieces >= 2048 || p.units < 4) && fits(32) && !split) {
+        Walk w = walk(32);
+        if (wide && fits(64)) {
+            const Walk by64 = walk(64);
+            if (L == kFilterColumns || 2 * w.rounds > 3 * by64.rounds) w = by64;
+        }
         p.col_tiles = w.col_tiles;
         p.div_col_tiles = FastDiv((uint32_t)p.col_tiles);
-        const size_t lds = (size_t)w.lds;
+        const size_t lds = w.lds;
         const long long groups = w.groups;
         auto launch = [&](auto nt) {
             constexpr auto kernel = bit_gemm_stream_kernel<CC, L, E, decltype(nt)::value, LONG>;
@@ -477,7 +479,7 @@ static int launch_bit_gemm(const char *fn, BitGemmArgs &p, hipStream_t s) {
             return DAB_OK;
         };
         int rc = DAB_OK;
-        rc = two ? launch(std::integral_constant<int, 2>{}) : launch(std::integral_constant<int, 1>{});
+        rc = w.channels == 64 ? launch(std::integral_constant<int, 2>{}) : launch(std::integral_constant<int, 1>{});
         if (rc != DAB_OK) return rc;
     } else {
         const int split_ch = p.g.cols > 32 && pieces >= 1024 ? 64 : 32;
