@@ -280,7 +280,7 @@ __global__ __launch_bounds__(kC32Threads) void fconv_c32_kernel(const FconvC32Ar
                     f32x4w v0, v1;
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
-                        // (from the lowest value on, as max_pool: a cell of nothing but NaNs holds that)
+                        // (from the lowest value on, as max_pool: a cell of nothing but negative infinities and NaNs holds that)
                         v0[e] = max_of_three(acc[0][nt][e], acc[1][nt][e], -FLT_MAX);
                         v1[e] = later_max(max_of_three(acc[1][nt][e], acc[2][nt][e], acc[3][nt][e]), -FLT_MAX);
                     }

@@ -83,6 +83,21 @@ def test_magnitudes(cout, pooled, case):
     check(x, w, pooled)
 
 
+# finite operands whose sums are below every float: max_pool starts at the lowest float, which a cell of nothing but such sums holds
+@pytest.mark.parametrize("cout", [32, 64])
+def test_pool_of_sums_that_overflow(cout):
+    x = torch.full((N, 112, 112, 32), 3e38, device="cuda")
+    x[0] = 1.0
+    w = torch.zeros(cout, 3, 3, 32, device="cuda")
+    w[::2, 1, 1] = -1.0
+    w[1::2, 1, 1, 0] = 0.5
+    full = run(x, w, False)
+    assert bool(full[1:, :, :, ::2].isneginf().all()) and bool(full[:, :, :, 1::2].isfinite().all())
+    got = run(x, w, True)
+    assert torch.equal(got, dab.max_pool(full, 3, 3, 1, 1, 2, 2))
+    assert bool((got[1:, :, :, ::2] == torch.finfo(torch.float32).min).all())
+
+
 @pytest.mark.parametrize("cout", [32, 64])
 @pytest.mark.parametrize("where", ["pixels", "filters"])
 def test_infinities_and_nan(cout, where):
