@@ -16,7 +16,7 @@ static void hip_check(hipError_t e, const char *what) {
 
 void *copy_stream(int device) {
     static std::mutex mutex;
-    static std::map<int, hipStream_t> streams;
+    static auto &streams = *new std::map<int, hipStream_t>;  // never destroyed: a blob may be read while the process ends
     std::lock_guard<std::mutex> lock(mutex);
     hipStream_t &s = streams[device];
     if (!s) {
