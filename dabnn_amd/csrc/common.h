@@ -237,17 +237,6 @@ __device__ __forceinline__ uint32_t finite_bf16_pair(uint32_t w) {
 struct SplitFrag8 {
     typedef uint32_t u4 __attribute__((ext_vector_type(4)));
     u4 hi, hif, mid, lo;
-    // finite values only (see split_pair_finite); hif = hi; returns the running magnitude maximum with these values in
-    __device__ __forceinline__ uint32_t set_finite(const float (&x)[8], uint32_t running) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const SplitPair s = split_pair_finite(x[2 * i], x[2 * i + 1]);
-            hi[i] = s.hi, mid[i] = s.mid, lo[i] = s.lo;
-            running = bf16_pair_max(running, s.hi);
-        }
-        hif = hi;
-        return running;
-    }
     __device__ __forceinline__ void set(const float (&x)[8]) {
         SplitParts s[8];
 #pragma unroll
