@@ -1,0 +1,626 @@
+// The first layer of a down-sampling block with its shortcut branch, in one launch:
+//   out = a * bconv3x3(sign(x), stride 2, pad 1) + b + (sa * (conv1x1(avepool2x2(x)) + bias) + sb)
+// (dabnn/layers/BinConv.cpp:144-191, Affine.cpp:10-23, AvePool.cpp:84-123, FloatConv.cpp, Add.cpp:7-17), with the sign bits of
+// the result.  64, 128 or 256 input channels, even height and width.
+//
+// As two launches the branch's blob is written by one and read by the other; here it stays in the accumulators of the fp32 matrix
+// instruction, which lie like those of the fp4 one that counts (fp4_core.h): lane = channel, register = pixel.  Its values are only
+// written for who asks for them (`sc_out`).
+//
+// Three kernels, chosen by the number of 32-pixel x 32-channel pieces of the output (pick_down has both sides of its lines):
+//   staged  few pieces: a block is one tile, all its operands are asked for at once, eight waves share the branch's depth
+//   tile    a block is 32 pixels x 128 channels, a wave 32 channels
+//   walk    many pieces, 64 and 128 input channels: a wave keeps the filters of 32 channels, blocks walk over pixel tiles
+// One Bi-Real-18 pass, the three layers as two launches each / in one (us, in a graph): batch 1 5.9 + 6.9 + 8.1 / 3.8 + 3.7 + 4.0, batch
+// 6 9.4 + 9.0 + 9.0 / 5.7 + 5.7 + 5.8, batch 40 22 + 18 + 20 / 13.6 + 12.0 + 11.3, batch 256 100 + 68 / 61 + 43 (the third stays two).
+#include "fp4_core.h"
+
+namespace dab {
+
+struct BconvDownArgs {
+    const uint64_t *x;   // sign bits of xf
+    const float *xf;
+    const uint64_t *w;   // of the binary convolution
+    const float *ea, *eb;
+    const float *sw;     // [cout][cin] of the branch
+    const float *bias, *sa, *sb;  // may be null: bias, and sa with sb
+    float *sc_out;       // the branch's result, or null
+    float *out;
+    uint32_t *bits;      // or null
+    int total;           // output pixels
+    int H, W, OH, OW, cout, cols;
+    uint32_t x_bytes, w_bytes;
+    FastDiv div_ow, div_oh, div_cols;
+};
+
+constexpr int kDownOutside = (int)0x80000000;  // beyond any descriptor
+
+struct DownPixel {
+    int n, oy, ox;
+    __device__ __forceinline__ DownPixel(const BconvDownArgs &p, int pix) {
+        const uint32_t t = p.div_ow.div((uint32_t)pix);
+        ox = pix - (int)t * p.OW;
+        n = (int)p.div_oh.div(t);
+        oy = (int)t - n * p.OH;
+    }
+};
+
+// ave_pool_fallback (dabnn/layers/AvePool.cpp:84-123) for a 2x2 window: the taps added to zero in row-major order, divided by 4
+__device__ __forceinline__ f32x4m pool_taps(const f32x4m (&t)[4]) {
+#pragma clang fp contract(off)
+    f32x4m s = {0.f, 0.f, 0.f, 0.f};
+    s = s + t[0];
+    s = s + t[1];
+    s = s + t[2];
+    s = s + t[3];
+    return s * 0.25f;
+}
+// bias, Affine of the branch; Affine of the counts; Add: every operation rounded by itself like the separate layers'
+__device__ __forceinline__ float branch_value(float v, bool with_bias, float bias, bool with_affine, float sa, float sb) {
+#pragma clang fp contract(off)
+    if (with_bias) v = v + bias;
+    if (with_affine) {
+        v = sa * v;
+        v = v + sb;
+    }
+    return v;
+}
+__device__ __forceinline__ float down_value(float cnt, float ea, float eb, float sc) {
+#pragma clang fp contract(off)
+    float r = ea * cnt;
+    r = r + eb;
+    return r + sc;
+}
+
+// ---------------------------------------------------------------- few pieces
+// Bound by latency: a block is T pixels x 16 * NT channels.  Three waves ask for a kernel row's bits each, all eight for the
+// block's floats and filters in whole lines, which meet in LDS; then the waves take 16 pixels and a part of the branch's depth each, and
+// the partial sums meet in LDS too.  (Floats fetched by each lane for its own pixel and depths, without the staging: a load then
+// touches 16 or 32 lines, and 256 input channels took 5.3 to 9 us instead of 4.0 to 5.8.)
+template <int CW, int T, int NT>
+__global__ __launch_bounds__(512) void bconv3x3_down_staged_kernel(const BconvDownArgs p) {
+    constexpr int C = CW * 64, CH = 16 * NT, LD = CH + 4, AS = C + 4, THREADS = 512;
+    constexpr int KB = 64 / T, ND = 2 * CW < KB ? 1 : 2 * CW / KB, NC = CH / T < 1 ? 1 : CH / T;  // counting: T pixels x T channels, NC of them
+    constexpr bool kPair = 2 * CW < KB;
+    constexpr int STEPS = kPair ? 2 : 3;
+    constexpr int XP = T * (C / 4) / THREADS < 1 ? 1 : T * (C / 4) / THREADS, FP = CH * (C / 4) / THREADS < 1 ? 1 : CH * (C / 4) / THREADS;
+    constexpr int PXG = T / 16, DG = 8 / PXG, DEPTH = C / DG;  // the branch: PXG groups of 16 pixels, DG parts of the depth
+    __shared__ __attribute__((aligned(16))) float pooled[T][AS];
+    __shared__ __attribute__((aligned(16))) float filt[CH][AS];
+    __shared__ __attribute__((aligned(16))) float part[3 + DG][T * LD];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int r = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t tile = p.div_cols.div(blockIdx.x);
+    const int ch0 = (int)(blockIdx.x - tile * p.cols) * CH;
+    uint32_t act[STEPS][ND], wt[NC][STEPS][ND];
+    const int lr = lane % T, kb = lane / T;
+    if (r < 3) {
+        const __amdgpu_buffer_rsrc_t rx = make_rsrc(p.x, p.x_bytes), rw = make_rsrc(p.w, p.w_bytes);
+        int pix = (int)tile * T + lr;
+        pix = pix < p.total ? pix : p.total - 1;
+        const DownPixel at(p, pix);
+        const int y0 = 2 * at.oy - 1, x0 = 2 * at.ox - 1;
+        const int base = ((at.n * p.H + y0 + r) * p.W + x0) * (CW * 8);
+        const bool row_ok = (unsigned)(y0 + r) < (unsigned)p.H;
+        const int wbase = (ch0 + lr) * (CW * 72) + r * (CW * 24);
+#pragma unroll
+        for (int s = 0; s < STEPS; ++s) {
+            const int kw = kPair ? s * 2 + (kb >> 1) : s;
+            const int inner = kPair ? (kb & 1) * 4 : kb * (ND * 4);
+            const bool ok = row_ok && (unsigned)(x0 + kw) < (unsigned)p.W && (!kPair || kw < 3);
+            load_dwords<ND>(act[s], rx, ok ? base + kw * (CW * 8) + inner : kDownOutside);
+#pragma unroll
+            for (int n = 0; n < NC; ++n)
+                load_dwords<ND>(wt[n][s], rw, (!kPair || kw < 3) ? wbase + n * T * (CW * 72) + kw * (CW * 8) + inner : kDownOutside);
+        }
+    }
+    f32x4m tap[XP][4], f[FP];
+#pragma unroll
+    for (int i = 0; i < XP; ++i) {
+        const int piece = tid + THREADS * i, pix = (int)tile * T + piece / (C / 4);
+        const DownPixel at(p, pix < p.total ? pix : p.total - 1);
+        const float *src = p.xf + ((size_t)(at.n * p.H + 2 * at.oy) * p.W + 2 * at.ox) * C + (piece % (C / 4)) * 4;
+        const size_t below = (size_t)p.W * C;
+        tap[i][0] = *reinterpret_cast<const f32x4m *>(src), tap[i][1] = *reinterpret_cast<const f32x4m *>(src + C);
+        tap[i][2] = *reinterpret_cast<const f32x4m *>(src + below), tap[i][3] = *reinterpret_cast<const f32x4m *>(src + below + C);
+    }
+#pragma unroll
+    for (int i = 0; i < FP; ++i) {
+        const int piece = tid + THREADS * i;
+        if (piece < CH * (C / 4)) f[i] = *reinterpret_cast<const f32x4m *>(p.sw + (size_t)ch0 * C + piece * 4);
+    }
+    // the store pass's operands: thread t has four channels of a pixel
+    constexpr int Q = T * CH / 4;
+    const int opix = (int)tile * T + tid / (CH / 4), och = ch0 + (tid % (CH / 4)) * 4;
+    const bool ok = tid < Q && opix < p.total;
+    const f32x4m zero = {0.f, 0.f, 0.f, 0.f};
+    f32x4m ea = zero, eb = zero, bias = zero, sa = zero, sb = zero;
+    if (ok) {
+        ea = *reinterpret_cast<const f32x4m *>(p.ea + och), eb = *reinterpret_cast<const f32x4m *>(p.eb + och);
+        if (p.bias) bias = *reinterpret_cast<const f32x4m *>(p.bias + och);
+        if (p.sa) sa = *reinterpret_cast<const f32x4m *>(p.sa + och), sb = *reinterpret_cast<const f32x4m *>(p.sb + och);
+    }
+    __builtin_amdgcn_sched_barrier(0);  // everything is asked for before anything is waited for
+    if (r < 3) {
+        typename Fp4Acc<T>::type acc[NC];
+#pragma unroll
+        for (int n = 0; n < NC; ++n)
+#pragma unroll
+            for (int v = 0; v < Fp4Acc<T>::regs; ++v) acc[n][v] = 0.f;
+#pragma unroll
+        for (int s = 0; s < STEPS; ++s)
+#pragma unroll
+            for (int d = 0; d < ND; ++d) {
+                const i32x8 a = bitspm1(act[s][d]);
+#pragma unroll
+                for (int n = 0; n < NC; ++n) mfma_fp4<T>(acc[n], a, bitspm1(wt[n][s][d]));
+            }
+#pragma unroll
+        for (int n = 0; n < NC; ++n)
+#pragma unroll
+            for (int v = 0; v < Fp4Acc<T>::regs; ++v) part[r][fp4_row<T>(kb, v) * LD + n * T + lr] = acc[n][v];
+    }
+#pragma unroll
+    for (int i = 0; i < XP; ++i) {
+        const int piece = tid + THREADS * i;
+        if (piece < T * (C / 4)) *reinterpret_cast<f32x4m *>(&pooled[piece / (C / 4)][(piece % (C / 4)) * 4]) = pool_taps(tap[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < FP; ++i) {
+        const int piece = tid + THREADS * i;
+        if (piece < CH * (C / 4)) *reinterpret_cast<f32x4m *>(&filt[piece / (C / 4)][(piece % (C / 4)) * 4]) = f[i];
+    }
+    __syncthreads();
+    {
+        const int l16 = lane & 15, k4 = lane >> 4, px = r % PXG, dg = r / PXG;
+        f32x4m acc[NT];
+#pragma unroll
+        for (int n = 0; n < NT; ++n) acc[n] = zero;
+        if constexpr (DEPTH >= 16) {
+#pragma unroll
+            for (int d = 0; d < DEPTH; d += 16) {
+                const int k = dg * DEPTH + d + 4 * k4;
+                const f32x4m a = *reinterpret_cast<const f32x4m *>(&pooled[px * 16 + l16][k]);
+                f32x4m b[NT];
+#pragma unroll
+                for (int n = 0; n < NT; ++n) b[n] = *reinterpret_cast<const f32x4m *>(&filt[n * 16 + l16][k]);
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+#pragma unroll
+                    for (int n = 0; n < NT; ++n) acc[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], b[n][e], acc[n], 0, 0, 0);
+            }
+        } else {
+#pragma unroll
+            for (int d = 0; d < DEPTH; d += 4) {
+                const int k = dg * DEPTH + d + k4;
+                const float a = pooled[px * 16 + l16][k];
+#pragma unroll
+                for (int n = 0; n < NT; ++n) acc[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, filt[n * 16 + l16][k], acc[n], 0, 0, 0);
+            }
+        }
+#pragma unroll
+        for (int n = 0; n < NT; ++n)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) part[3 + dg][(px * 16 + 4 * k4 + v) * LD + n * 16 + l16] = acc[n][v];
+    }
+    __syncthreads();
+    if (tid >= Q) return;  // whole waves
+
+    constexpr float kHalfDepth = 0.5f * (kPair ? 3 * 4 * 64 : 9 * C);
+    const int o = (tid / (CH / 4)) * LD + (tid % (CH / 4)) * 4;
+    f32x4m s[3 + DG], v, sc;
+#pragma unroll
+    for (int i = 0; i < 3 + DG; ++i) s[i] = *reinterpret_cast<f32x4m *>(&part[i][o]);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        float t = (s[3][e] + s[4][e]) + (s[5][e] + s[6][e]);
+        if constexpr (DG == 8) t = t + ((s[7][e] + s[8][e]) + (s[9][e] + s[10][e]));
+        sc[e] = branch_value(t, p.bias != nullptr, bias[e], p.sa != nullptr, sa[e], sb[e]);
+        v[e] = down_value(kHalfDepth - 0.5f * (s[0][e] + s[1][e] + s[2][e]), ea[e], eb[e], sc[e]);
+    }
+    const size_t first = (size_t)opix * p.cout + och;
+    if (ok) {
+        *reinterpret_cast<f32x4m *>(p.out + first) = v;
+        if (p.sc_out) *reinterpret_cast<f32x4m *>(p.sc_out + first) = sc;
+    }
+    if (p.bits) {
+        constexpr int G = CH / 4 < 8 ? CH / 4 : 8;
+        const int g = tid % G;
+        uint32_t word = sign_nibble(make_float4(v[0], v[1], v[2], v[3])) << (4 * g);
+        word = or_from_lane_above<1>(word);
+        word = or_from_lane_above<2>(word);
+        if constexpr (G == 8) word = or_from_lane_above<4>(word);
+        if (ok && g == 0) {
+            if constexpr (G == 8)
+                p.bits[first >> 5] = word;
+            else
+                reinterpret_cast<uint16_t *>(p.bits)[first >> 4] = (uint16_t)word;
+        }
+    }
+}
+
+// ---------------------------------------------------------------- between
+// A wave counts, the block pools its pixels into LDS, the wave multiplies on the fp32 matrix instruction -- 32 of 64 cycles per 64
+// channels of depth, which is what bounds the kernel: 40 images of 28 x 28 x 128 to 256 take 12.0 us.
+template <int CW, int WAVES>
+__global__ __launch_bounds__(WAVES * 64) void bconv3x3_down_tile_kernel(const BconvDownArgs p) {
+    constexpr int C = CW * 64, AS = C + 4, CH = 32 * WAVES, THREADS = 64 * WAVES;  // AS: rows 4 floats off a multiple of 64 banks
+    constexpr int PIECES = 32 * (C / 4) / THREADS;  // 16-byte pieces of the pooled tile per thread
+    constexpr int CHUNK = 8, CHUNKS = C / 8 / CHUNK;  // a wave's filters in steps of 8 depths, asked for CHUNK steps at a time
+    __shared__ __attribute__((aligned(16))) float pooled[32][AS];
+    const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5, l32 = lane & 31;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t item = xcd_contiguous_block(blockIdx.x, gridDim.x);  // a pixel tile's channel blocks share an XCD's L2
+    const uint32_t tile = p.div_cols.div(item);
+    const int ch0 = (int)(item - tile * p.cols) * CH + wave * 32, ch = ch0 + l32;
+    const int m0 = (int)tile * 32;
+    const bool ch_ok = ch0 < p.cout;  // (32 channels are all there or none)
+    const __amdgpu_buffer_rsrc_t rx = make_rsrc(p.x, p.x_bytes), rw = make_rsrc(p.w, p.w_bytes);
+
+    // the bits first: loads come back in order, and counting covers the wait for the floats
+    uint32_t act[9][CW], wt[9][CW];
+    {
+        const int pix = m0 + l32 < p.total ? m0 + l32 : p.total - 1;
+        const DownPixel at(p, pix);
+        const int y0 = 2 * at.oy - 1, x0 = 2 * at.ox - 1, base = ((at.n * p.H + y0) * p.W + x0) * (CW * 8) + half * (CW * 4);
+#pragma unroll
+        for (int t = 0; t < 9; ++t) {
+            const bool ok = (unsigned)(y0 + t / 3) < (unsigned)p.H && (unsigned)(x0 + t % 3) < (unsigned)p.W;
+            load_dwords<CW>(act[t], rx, ok ? base + ((t / 3) * p.W + t % 3) * (CW * 8) : kDownOutside);
+        }
+#pragma unroll
+        for (int t = 0; t < 9; ++t) load_dwords<CW>(wt[t], rw, ch_ok ? ch * (CW * 72) + t * (CW * 8) + half * (CW * 4) : kDownOutside);
+    }
+    f32x4m tap[PIECES][4];
+#pragma unroll
+    for (int i = 0; i < PIECES; ++i) {
+        const int piece = tid + THREADS * i, row = piece / (C / 4), c4 = piece % (C / 4);
+        const DownPixel at(p, m0 + row < p.total ? m0 + row : p.total - 1);
+        const float *src = p.xf + ((size_t)(at.n * p.H + 2 * at.oy) * p.W + 2 * at.ox) * C + c4 * 4;
+        const size_t below = (size_t)p.W * C;
+        tap[i][0] = *reinterpret_cast<const f32x4m *>(src), tap[i][1] = *reinterpret_cast<const f32x4m *>(src + C);
+        tap[i][2] = *reinterpret_cast<const f32x4m *>(src + below), tap[i][3] = *reinterpret_cast<const f32x4m *>(src + below + C);
+    }
+    const float *filter = p.sw + (size_t)(ch_ok ? ch : 0) * C + half * 4;
+    f32x4m f[CHUNKS > 1 ? 2 : 1][CHUNK];
+    auto fetch_filters = [&](int chunk) {
+#pragma unroll
+        for (int s = 0; s < CHUNK; ++s) f[chunk & 1][s] = *reinterpret_cast<const f32x4m *>(filter + (chunk * CHUNK + s) * 8);
+    };
+    fetch_filters(0);
+    float ea = 0.f, eb = 0.f, bias = 0.f, sa = 0.f, sb = 0.f;
+    if (ch_ok) {
+        ea = p.ea[ch], eb = p.eb[ch];
+        if (p.bias) bias = p.bias[ch];
+        if (p.sa) sa = p.sa[ch], sb = p.sb[ch];
+    }
+
+    f32x16m cnt, sum;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) cnt[v] = 0.f, sum[v] = 0.f;
+#pragma unroll
+    for (int t = 0; t < 9; ++t)
+#pragma unroll
+        for (int c = 0; c < CW; ++c) mfma_fp4<32>(cnt, bitspm1(act[t][c]), bitspm1(wt[t][c]));
+#pragma unroll
+    for (int i = 0; i < PIECES; ++i) {
+        const int piece = tid + THREADS * i;
+        *reinterpret_cast<f32x4m *>(&pooled[piece / (C / 4)][(piece % (C / 4)) * 4]) = pool_taps(tap[i]);
+    }
+    __syncthreads();
+    // eight depths at a time, the pairs d and d + 4 in one instruction
+#pragma unroll
+    for (int chunk = 0; chunk < CHUNKS; ++chunk) {
+        if (chunk + 1 < CHUNKS) fetch_filters(chunk + 1);
+#pragma unroll
+        for (int s = 0; s < CHUNK; ++s) {
+            const f32x4m a = *reinterpret_cast<const f32x4m *>(&pooled[l32][(chunk * CHUNK + s) * 8 + half * 4]);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) sum = __builtin_amdgcn_mfma_f32_32x32x2f32(a[e], f[chunk & 1][s][e], sum, 0, 0, 0);
+        }
+    }
+
+    constexpr float kHalfDepth = 0.5f * 9 * C;
+    const size_t base = (size_t)m0 * p.cout;
+    const int rows = p.total - m0 < 32 ? p.total - m0 : 32;
+    const __amdgpu_buffer_rsrc_t ro = make_rsrc(p.out + base, (uint32_t)rows * p.cout * 4u);
+    const __amdgpu_buffer_rsrc_t rs = make_rsrc(p.sc_out + (p.sc_out ? base : 0), p.sc_out ? (uint32_t)rows * p.cout * 4u : 0u);
+    const int lane_off = ch_ok ? (half * 4 * p.cout + ch) * 4 : kDownOutside;
+    uint32_t word = 0;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+        const int row = 8 * (v / 4) + v % 4;
+        const float sc = branch_value(sum[v], p.bias != nullptr, bias, p.sa != nullptr, sa, sb);
+        const float r = down_value(kHalfDepth - 0.5f * cnt[v], ea, eb, sc);
+        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, r), ro, lane_off + row * p.cout * 4, 0, kStoreStream);
+        if (p.sc_out) __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, sc), rs, lane_off + row * p.cout * 4, 0, 0);
+        const uint64_t mask = __ballot(r > 0.f);
+        word = dab_writelane((uint32_t)mask, row, word);
+        word = dab_writelane((uint32_t)(mask >> 32), row + 4, word);
+    }
+    if (p.bits && half == 0 && m0 + l32 < p.total && ch_ok) p.bits[(size_t)(m0 + l32) * (p.cout / 32) + ch0 / 32] = word;
+}
+
+// ---------------------------------------------------------------- many pieces: blocks that walk over pixel tiles
+// A wave keeps the filters of 32 channels for its lifetime, the branch's as three planes of bf16 (common.h: six products per 16
+// depths, fp32 accuracy, the cross terms in a sum of their own), and a block walks over tiles of 32 pixels: it pools and splits a
+// tile into LDS while the next one's floats and bits are on their way.  A tile (or a wave's filters) with an infinity, a NaN or a
+// value too small for the split is made on the fp32 matrix instruction.  With 64 input channels bound by memory: 256 images of
+// 56 x 56 x 64 to 128 move 315 MB in 61 us, 5.2 TB/s, the rate of a copy (tile kernel 75, two launches 100).  With 128 a block has eight
+// waves, so that the floats are read once: 28 x 28 at 256 images 43 us (tile 63, two launches 68; four waves 63).  256 input
+// channels, whose filters take 192 registers, were no faster (64 us, two launches 59).
+template <int CW, int WAVES>
+__global__ __launch_bounds__(WAVES * 64, 2) void bconv3x3_down_walk_kernel(const BconvDownArgs p) {
+    constexpr int C = CW * 64, CH = 32 * WAVES, THREADS = 64 * WAVES;
+    constexpr int PIECES = 32 * (C / 4) / THREADS, GROUPS = C / 16;
+    constexpr int ROW = C + 8, PLANE = 32 * ROW;  // bf16 elements; rows 4 dwords off a multiple of 32: a quarter wave's reads hit all banks
+    extern __shared__ __attribute__((aligned(16))) uint16_t planes[];  // [buffer][plane][pixel][depth]
+    __shared__ int special_tile[2];
+    const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5, l32 = lane & 31;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int group = (int)p.div_cols.div(blockIdx.x), groups = (int)p.div_cols.div(gridDim.x);
+    const int ch0 = ((int)blockIdx.x - group * p.cols) * CH + wave * 32, ch = ch0 + l32;
+    const bool ch_ok = ch0 < p.cout;  // (32 channels are all there or none)
+    const int tiles = (p.total + 31) / 32;
+    const __amdgpu_buffer_rsrc_t rx = make_rsrc(p.x, p.x_bytes), rw = make_rsrc(p.w, p.w_bytes);
+    typedef SplitFrag8::u4 u4;
+
+    f32x4m tap[PIECES][4];
+    uint32_t act[9][CW];
+    auto fetch_floats = [&](int tile) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < PIECES; ++i) {
+            const int piece = tid + THREADS * i, pix = tile * 32 + piece / (C / 4);
+            const DownPixel at(p, pix < p.total ? pix : p.total - 1);
+            const float *src = p.xf + ((size_t)(at.n * p.H + 2 * at.oy) * p.W + 2 * at.ox) * C + (piece % (C / 4)) * 4;
+            const size_t below = (size_t)p.W * C;
+            tap[i][0] = *reinterpret_cast<const f32x4m *>(src), tap[i][1] = *reinterpret_cast<const f32x4m *>(src + C);
+            tap[i][2] = *reinterpret_cast<const f32x4m *>(src + below), tap[i][3] = *reinterpret_cast<const f32x4m *>(src + below + C);
+        }
+    };
+    auto fetch_bits = [&](int tile) __attribute__((always_inline)) {
+        const int pix = tile * 32 + l32 < p.total ? tile * 32 + l32 : p.total - 1;
+        const DownPixel at(p, pix);
+        const int y0 = 2 * at.oy - 1, x0 = 2 * at.ox - 1, base = ((at.n * p.H + y0) * p.W + x0) * (CW * 8) + half * (CW * 4);
+#pragma unroll
+        for (int t = 0; t < 9; ++t) {
+            const bool ok = (unsigned)(y0 + t / 3) < (unsigned)p.H && (unsigned)(x0 + t % 3) < (unsigned)p.W;
+            load_dwords<CW>(act[t], rx, ok ? base + ((t / 3) * p.W + t % 3) * (CW * 8) : kDownOutside);
+        }
+    };
+    int tile = group;
+    if (tile < tiles) fetch_bits(tile), fetch_floats(tile);
+
+    uint32_t wt[9][CW];
+#pragma unroll
+    for (int t = 0; t < 9; ++t) load_dwords<CW>(wt[t], rw, ch_ok ? ch * (CW * 72) + t * (CW * 8) + half * (CW * 4) : kDownOutside);
+    const float *filter = p.sw + (size_t)(ch_ok ? ch : 0) * C;
+    u4 fhi[GROUPS], fmid[GROUPS], flo[GROUPS];
+    uint32_t fsmall = ~0u, ftop = 0;
+#pragma unroll
+    for (int g = 0; g < GROUPS; ++g) {
+        const f32x4m v0 = *reinterpret_cast<const f32x4m *>(filter + g * 16 + half * 8), v1 = *reinterpret_cast<const f32x4m *>(filter + g * 16 + half * 8 + 4);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float a = e < 2 ? v0[2 * e] : v1[2 * e - 4], b = e < 2 ? v0[2 * e + 1] : v1[2 * e - 3];
+            fsmall = smallest_magnitude(fsmall, a, b);
+            const SplitPair sp = split_pair_finite(a, b);
+            ftop = bf16_pair_max(ftop, sp.hi);
+            fhi[g][e] = sp.hi, fmid[g][e] = sp.mid, flo[g][e] = sp.lo;
+        }
+    }
+    const bool filter_special = __builtin_amdgcn_ballot_w64(loses_bits_when_split(fsmall) || !bf16_pairs_finite(ftop)) != 0;
+    uint32_t set = 0;
+#pragma unroll
+    for (int t = 0; t < 9; ++t)
+#pragma unroll
+        for (int c = 0; c < CW; ++c) set += __popc(wt[t][c]);
+    set += __shfl_xor(set, 32);
+    const float init = (float)set;
+    float ea = 0.f, eb = 0.f, bias = 0.f, sa = 0.f, sb = 0.f;
+    if (ch_ok) {
+        ea = p.ea[ch], eb = p.eb[ch];
+        if (p.bias) bias = p.bias[ch];
+        if (p.sa) sa = p.sa[ch], sb = p.sb[ch];
+    }
+    if (tid < 2) special_tile[tid] = -1;
+    __syncthreads();
+
+    for (int buf = 0; tile < tiles; tile += groups, buf ^= 1) {
+        uint16_t *const out_planes = planes + buf * 3 * PLANE;
+        uint32_t small = ~0u, top = 0;
+#pragma unroll
+        for (int i = 0; i < PIECES; ++i) {
+            const int piece = tid + THREADS * i;
+            const f32x4m v = pool_taps(tap[i]);
+            small = smallest_magnitude(smallest_magnitude(small, v[0], v[1]), v[2], v[3]);
+            const SplitPair s0 = split_pair_finite(v[0], v[1]), s1 = split_pair_finite(v[2], v[3]);
+            top = bf16_pair_max(bf16_pair_max(top, s0.hi), s1.hi);
+            uint16_t *d = out_planes + (piece / (C / 4)) * ROW + (piece % (C / 4)) * 4;
+            *reinterpret_cast<u32x2 *>(d) = u32x2{s0.hi, s1.hi};
+            *reinterpret_cast<u32x2 *>(d + PLANE) = u32x2{s0.mid, s1.mid};
+            *reinterpret_cast<u32x2 *>(d + 2 * PLANE) = u32x2{s0.lo, s1.lo};
+        }
+        if (loses_bits_when_split(small) || !bf16_pairs_finite(top)) special_tile[buf] = tile;
+        const bool more = tile + groups < tiles;
+        if (more) fetch_floats(tile + groups);
+        __syncthreads();
+        f32x16m sum;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) sum[v] = 0.f;
+        if (!filter_special && special_tile[buf] != tile) {
+            f32x16m cross = sum;
+            const uint16_t *src = out_planes + l32 * ROW + half * 8;
+            auto v = [](u4 w) { return __builtin_bit_cast(bf16x8, w); };
+#pragma unroll
+            for (int g = 0; g < GROUPS; ++g) {
+                const u4 hi = *reinterpret_cast<const u4 *>(src + g * 16), mid = *reinterpret_cast<const u4 *>(src + g * 16 + PLANE),
+                         lo = *reinterpret_cast<const u4 *>(src + g * 16 + 2 * PLANE);
+                cross = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v(lo), v(fhi[g]), cross, 0, 0, 0);
+                sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v(hi), v(fhi[g]), sum, 0, 0, 0);
+                cross = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v(hi), v(flo[g]), cross, 0, 0, 0);
+                cross = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v(mid), v(fmid[g]), cross, 0, 0, 0);
+                cross = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v(mid), v(fhi[g]), cross, 0, 0, 0);
+                cross = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v(hi), v(fmid[g]), cross, 0, 0, 0);
+            }
+#pragma unroll
+            for (int e = 0; e < 16; ++e) sum[e] = sum[e] + cross[e];
+        } else {
+            const DownPixel at(p, tile * 32 + l32 < p.total ? tile * 32 + l32 : p.total - 1);
+            const float *src = p.xf + ((size_t)(at.n * p.H + 2 * at.oy) * p.W + 2 * at.ox) * C + half * 4;
+            const size_t below = (size_t)p.W * C;
+#pragma unroll 1
+            for (int d = 0; d < C; d += 8) {
+                const f32x4m t[4] = {*reinterpret_cast<const f32x4m *>(src + d), *reinterpret_cast<const f32x4m *>(src + d + C),
+                                     *reinterpret_cast<const f32x4m *>(src + d + below), *reinterpret_cast<const f32x4m *>(src + d + below + C)};
+                const f32x4m a = pool_taps(t), b = *reinterpret_cast<const f32x4m *>(filter + d + half * 4);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) sum = __builtin_amdgcn_mfma_f32_32x32x2f32(a[e], b[e], sum, 0, 0, 0);
+            }
+        }
+#pragma unroll
+        for (int v = 0; v < 16; ++v) sum[v] = branch_value(sum[v], p.bias != nullptr, bias, p.sa != nullptr, sa, sb);
+        f32x16m cnt;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) cnt[v] = init;
+#pragma unroll
+        for (int t = 0; t < 9; ++t)
+#pragma unroll
+            for (int c = 0; c < CW; ++c) {
+                asm volatile("" : "+v"(wt[t][c]));  // expanded here: hoisted out of the loop the expanded filters would not fit
+                mfma_fp4<32>(cnt, bits01(act[t][c]), bitspm(wt[t][c]));
+            }
+        if (more) fetch_bits(tile + groups);
+
+        const size_t base = (size_t)tile * 32 * p.cout;
+        const int rows = p.total - tile * 32 < 32 ? p.total - tile * 32 : 32;
+        const __amdgpu_buffer_rsrc_t ro = make_rsrc(p.out + base, (uint32_t)rows * p.cout * 4u);
+        const __amdgpu_buffer_rsrc_t rs = make_rsrc(p.sc_out + (p.sc_out ? base : 0), p.sc_out ? (uint32_t)rows * p.cout * 4u : 0u);
+        int lane_off = ch_ok ? (half * 4 * p.cout + ch) * 4 : kDownOutside;
+        asm volatile("" : "+v"(lane_off));  // sixteen offsets kept from tile to tile would not fit
+        uint32_t word = 0;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+            const int row = 8 * (v / 4) + v % 4;
+            const float sc = sum[v], r = down_value(cnt[v], ea, eb, sc);
+            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, r), ro, lane_off + row * p.cout * 4, 0, kStoreStream);
+            if (p.sc_out) __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, sc), rs, lane_off + row * p.cout * 4, 0, 0);
+            const uint64_t mask = __ballot(r > 0.f);
+            word = dab_writelane((uint32_t)mask, row, word);
+            word = dab_writelane((uint32_t)(mask >> 32), row + 4, word);
+        }
+        if (p.bits && half == 0 && l32 < rows && ch_ok) p.bits[((size_t)tile * 32 + l32) * (p.cout / 32) + ch0 / 32] = word;
+    }
+}
+
+static bool down_geometry(BconvDownArgs &a, int n, int h, int w, int cin, int cout) {
+    if (!(cin == 64 || cin == 128 || cin == 256) || cout % 64 != 0 || h % 2 != 0 || w % 2 != 0) return false;
+    const long long in_pixels = (long long)n * h * w, total = in_pixels / 4;
+    if (in_pixels >= (1ll << 31) - 64 || in_pixels * (cin / 8) >= (1ll << 31) || (long long)cout * cin * 9 / 8 >= (1ll << 31) || cout >= (1 << 20) ||
+        total * cout >= (1ll << 40))
+        return false;
+    a.H = h, a.W = w, a.OH = h / 2, a.OW = w / 2, a.cout = cout, a.total = (int)total;
+    a.x_bytes = (uint32_t)(in_pixels * (cin / 8)), a.w_bytes = (uint32_t)((long long)cout * 9 * cin / 8);
+    a.div_ow = FastDiv((uint32_t)a.OW), a.div_oh = FastDiv((uint32_t)a.OH);
+    return true;
+}
+
+enum class Down { staged16, staged32, tile, walk };
+// By 32-pixel x 32-channel pieces, us:
+//   16 x 16 tiles up to 128 pieces of 128 and 256 input channels: 28 x 28 x 128 at batch 1 (56 pieces) 3.7 against 4.2, at batch 4
+//   (200) 6.1 against 4.5; 14 x 14 x 256 at batch 2 (64) 4.1 against 5.6, at batch 6 (160) 6.8 against 5.8
+//   32 x 32 tiles up to 700 pieces (64 input channels) and 512: 56 x 56 x 64 at batch 6 (588) 5.7 against the tile kernel's 6.4, at
+//   batch 9 (884) 7.5 against 6.5; 28 x 28 x 128 at batch 9 (448) 6.0 against 7.5, at batch 16 (784) 12.4 against 7.7; 14 x 14 x 256 at
+//   batch 16 (400) 9.7 against 10.8
+//   walking from 2600 pieces: 56 x 56 x 64 at batch 16 (1568) 9.3 against the tile kernel's 9.1, at batch 40 (3920) 13.6 against 15.5;
+//   28 x 28 x 128 at batch 40 (1960) 13.8 against 12.0, at batch 100 (4904) 23 against 27
+static Down pick_down(long long total, int cin, int cout) {
+    const long long pieces = (total + 31) / 32 * (cout / 32);
+    if (cin >= 128 && pieces <= 128) return Down::staged16;
+    if (pieces <= (cin == 64 ? 700 : 512)) return Down::staged32;
+    return cin <= 128 && pieces >= 2600 ? Down::walk : Down::tile;
+}
+
+template <class Kernel>
+static int launch_down(Kernel kernel, BconvDownArgs &a, int px, int ch, int threads, hipStream_t s) {
+    a.cols = (a.cout + ch - 1) / ch;
+    a.div_cols = FastDiv((uint32_t)a.cols);
+    const long long blocks = ((long long)a.total + px - 1) / px * a.cols;
+    if (blocks >= kMostBlocks) return fail(DAB_EUNSUPPORTED, "dab_bconv3x3_down: too many work units");
+    hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(threads), 0, s, a);
+    DAB_LAUNCH_CHECK();
+    return DAB_OK;
+}
+
+template <int CW, int WAVES>
+static int launch_down_walk(BconvDownArgs &a, hipStream_t s) {
+    constexpr int CH = 32 * WAVES;
+    constexpr size_t lds = 2 * 3 * 32 * (CW * 64 + 8) * 2;
+    auto kernel = bconv3x3_down_walk_kernel<CW, WAVES>;
+    a.cols = (a.cout + CH - 1) / CH;
+    a.div_cols = FastDiv((uint32_t)a.cols);
+    if (lds > 64 * 1024) {
+        const int rc = allow_dynamic_lds<bconv3x3_down_walk_kernel<CW, WAVES>>("dab_bconv3x3_down", lds);
+        if (rc != DAB_OK) return rc;
+    }
+    static const int per_cu = [&] {
+        int blocks = 0;
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, kernel, WAVES * 64, lds) != hipSuccess || blocks < 1) blocks = 1;
+        return blocks;
+    }();
+    const int tiles = (int)(((long long)a.total + 31) / 32), most = simd_count() / 4 * per_cu / a.cols;
+    int groups = tiles < most ? tiles : most < 1 ? 1 : most;
+    const int per_block = (tiles + groups - 1) / groups;
+    groups = (tiles + per_block - 1) / per_block;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(groups * a.cols)), dim3(WAVES * 64), lds, s, a);
+    DAB_LAUNCH_CHECK();
+    return DAB_OK;
+}
+
+template <int CW>
+static int launch_bconv_down(BconvDownArgs &a, hipStream_t s) {
+    switch (pick_down(a.total, CW * 64, a.cout)) {
+        case Down::staged16:
+            if constexpr (CW >= 2) return launch_down(bconv3x3_down_staged_kernel<CW, 16, 1>, a, 16, 16, 512, s);
+            [[fallthrough]];
+        case Down::staged32: return launch_down(bconv3x3_down_staged_kernel<CW, 32, 2>, a, 32, 32, 512, s);
+        case Down::walk:
+            if constexpr (CW <= 2) return launch_down_walk<CW, 4 * CW>(a, s);
+            [[fallthrough]];
+        default: return launch_down(bconv3x3_down_tile_kernel<CW, 4>, a, 32, 128, 256, s);
+    }
+}
+
+}  // namespace dab
+
+extern "C" int dab_bconv3x3_down_takes(int n, int h, int w, int cin, int cout) {
+    dab::BconvDownArgs a;
+    return n > 0 && h > 0 && w > 0 && cout > 0 && dab::down_geometry(a, n, h, w, cin, cout) &&
+           ((long long)a.total + 31) / 32 * ((cout + 127) / 128) < dab::kMostBlocks;
+}
+
+extern "C" int dab_bconv3x3_down(const uint64_t *x_packed, const float *x, int n, int h, int w, int cin, const uint64_t *wgt, const float *a,
+                                 const float *b, int cout, const float *sc_wgt, const float *sc_bias, const float *sc_a, const float *sc_b,
+                                 float *shortcut, float *out, uint64_t *out_packed, dab_stream_t stream) {
+    using namespace dab;
+    const char *fn = "dab_bconv3x3_down";
+    DAB_REQUIRE(x_packed && x && wgt && a && b && sc_wgt && out, "%s: null pointer", fn);
+    DAB_REQUIRE(n > 0 && h > 0 && w > 0 && cin > 0 && cout > 0, "%s: non-positive dimension", fn);
+    DAB_REQUIRE((sc_a == nullptr) == (sc_b == nullptr), "%s: affine needs both coefficient vectors", fn);
+    DAB_REQUIRE(out != x && shortcut != x && out != shortcut && out_packed != x_packed, "%s: the results must not alias the input or each other", fn);
+    auto at = [](const void *q) { return reinterpret_cast<uintptr_t>(q); };
+    DAB_REQUIRE(((at(x_packed) | at(x) | at(a) | at(b) | at(sc_wgt) | at(sc_bias) | at(sc_a) | at(sc_b) | at(shortcut) | at(out)) & 15) == 0 &&
+                    ((at(wgt) | at(out_packed)) & 7) == 0,
+                "%s: buffers must be 16-byte aligned", fn);
+    BconvDownArgs p;
+    if (!dab_bconv3x3_down_takes(n, h, w, cin, cout) || !down_geometry(p, n, h, w, cin, cout))
+        return fail(DAB_EUNSUPPORTED, "%s: %d images of %d x %d x %d to %d channels are not covered", fn, n, h, w, cin, cout);
+    p.x = x_packed, p.xf = x, p.w = wgt, p.ea = a, p.eb = b, p.sw = sc_wgt, p.bias = sc_bias, p.sa = sc_a, p.sb = sc_b;
+    p.sc_out = shortcut, p.out = out, p.bits = reinterpret_cast<uint32_t *>(out_packed);
+    hipStream_t s = as_stream(stream);
+    switch (cin) {
+        case 64: return launch_bconv_down<1>(p, s);
+        case 128: return launch_bconv_down<2>(p, s);
+        default: return launch_bconv_down<4>(p, s);
+    }
+}

@@ -130,6 +130,10 @@ bool BinConv::has_slices() const { return output_mat->ld || binarized_mat->ld ||
 
 void BinConv::forward_impl() const {
     if (inside_pass) return;
+    if (branch) {
+        forward_with_branch(nullptr);
+        return;
+    }
     if (!next_in_pass) {
         forward_alone();
         return;
@@ -143,6 +147,17 @@ void BinConv::forward_impl() const {
                                 static_cast<const uint64_t *>(second.weight_mat->dev), static_cast<const float *>(second.fused_a->dev),
                                 static_cast<const float *>(second.fused_b->dev), static_cast<float *>(second.output_mat->dev),
                                 second.fused_sign_out ? static_cast<uint64_t *>(second.fused_sign_out->dev) : nullptr, stream()));
+}
+
+void BinConv::forward_with_branch(float *branch_out) const {
+    auto floats = [](const MatP &m) { return m ? static_cast<const float *>(m->dev) : nullptr; };
+    const auto *x = floats(input_mat);
+    auto *packed = static_cast<uint64_t *>(binarized_mat->dev);
+    const int n = input_mat->n, h = input_mat->h, w = input_mat->w, c = input_mat->elem_c;
+    if (!input_prepacked) dab_check(dab_bitpack_nhwc(x, packed, (int64_t)n * h * w, c, stream()));
+    dab_check(dab_bconv3x3_down(packed, x, n, h, w, c, static_cast<const uint64_t *>(weight_mat->dev), floats(fused_a), floats(fused_b), weight_mat->n,
+                                floats(branch->weight_mat), floats(branch->bias_mat), floats(branch->fused_a), floats(branch->fused_b), branch_out,
+                                static_cast<float *>(output_mat->dev), fused_sign_out ? static_cast<uint64_t *>(fused_sign_out->dev) : nullptr, stream()));
 }
 
 void BinConv::forward_alone() const {
@@ -233,6 +248,7 @@ std::string BinConv::to_str() const {
     if (fused_sign_out) ss << " + Sign";
     if (next_in_pass) ss << ", in one pass with the next layer";
     if (inside_pass) ss << ", in the pass of the layer before";
+    if (branch) ss << ", its shortcut convolution in the same pass";
     return ss.str();
 }
 
@@ -280,7 +296,10 @@ void FloatConv::check_operands() const {
                         dilation, dilation, weight_mat->n);
 }
 
+void FloatConv::forward_alone() const { inside_block->forward_with_branch(static_cast<float *>(output_mat->dev)); }
+
 void FloatConv::forward_impl() const {
+    if (inside_block) return;
     if (fused_pool_max) {
         const Mat &in = *fused_pool_input, &o = *output_mat;
         dab_check(dab_max_pool2_fconv1x1(
@@ -345,6 +364,7 @@ std::string FloatConv::to_str() const {
     if (fused_pool_input)
         ss << (fused_pool_max ? ", MaxPool " : ", AvePool ") << (fused_pool_global ? "over all" : "2x2") << " of "
            << fused_pool_input->h << "x" << fused_pool_input->w << " inside";
+    if (inside_block) ss << ", in the pass of the binary convolution that adds it";
     if (fused_maxpool_out) ss << " + MaxPool 3x3 stride 2" << (fused_maxpool_sign ? " + Sign" : "");
     return ss.str();
 }

@@ -9,6 +9,8 @@ namespace bnn {
 
 using css = const std::string &;
 
+class FloatConv;
+
 class BNN_API BinConv : public Layer {
    public:
     MatP input_mat;
@@ -39,6 +41,11 @@ class BNN_API BinConv : public Layer {
     bool inside_pass = false;
     // The layer by itself, for who asks for those blobs (which must have memory) after a run.
     void forward_alone() const override;
+
+    // Also set by Net::prepare: the 1x1 convolution of this layer's shortcut branch runs in this layer's pass
+    // (dab_bconv3x3_down), which does not write the branch's blob.
+    std::shared_ptr<FloatConv> branch;
+    void forward_with_branch(float *branch_out) const;  // branch_out: where the branch's blob is wanted, or null
 
     BinConv(NetCP net, css name, css input, css weight, css output, int pad_h, int pad_w, int stride_h, int stride_w);
     void forward_impl() const override;
@@ -77,6 +84,10 @@ class BNN_API FloatConv : public Layer {
     // the packed copy of it a direct BinConv wants (or null) and the workspace of the one-pass kernel.  output_mat is
     // null then: the convolution's result is never written.
     MatP fused_maxpool_out, fused_maxpool_sign, fused_maxpool_carry;
+    // Set by Net::prepare: the binary convolution that adds this layer's result runs both (BinConv::branch); the layer by itself
+    // makes output_mat, which must have memory, for who asks for it after a run.
+    const BinConv *inside_block = nullptr;
+    void forward_alone() const override;
     const int pad_h, pad_w, stride_h, stride_w, dilation;
     FloatConv(NetCP net, css name, css input, css weight, css bias, css output, int pad_h, int pad_w, int stride_h,
               int stride_w, int dilation);

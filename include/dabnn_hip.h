@@ -193,6 +193,21 @@ DAB_API int dab_bconv3x3_pair(const uint64_t *x, const float *shortcut, int n, i
 DAB_API int dab_bconv3x3_pair_takes(int n, int h, int w);
 
 /*
+ * The first layer of a down-sampling block and its shortcut branch in one pass (BinConv, Affine, AvePool 2x2, FloatConv 1x1, Affine, Add):
+ *   out = a * bconv3x3(x_packed, stride 2, pad 1) + b + (sc_a * (conv1x1(avepool2x2(x)) + sc_bias) + sc_b)
+ * x [n][h][w][cin] floats with x_packed = pack_mat(x); wgt as dab_bconv3x3, sc_wgt [cout][cin]; sc_bias, and sc_a with sc_b, may be NULL.
+ * out [n][h/2][w/2][cout]; out_packed = pack_mat(out) and shortcut (what the branch adds) are written unless NULL.  No
+ * result may overlap an input.  Every operation behind the sums is rounded by itself, as in the separate layers; the branch's fp32
+ * sums may be added in another order than dab_ave_pool2_fconv1x1's.  Buffers 16-byte aligned (wgt and out_packed 8).
+ * DAB_EUNSUPPORTED for shapes that dab_bconv3x3_down_takes answers with 0: it takes 64, 128 and 256 input channels, multiples of 64
+ * output channels and even h and w, within 32-bit pixel numbers.
+ */
+DAB_API int dab_bconv3x3_down(const uint64_t *x_packed, const float *x, int n, int h, int w, int cin, const uint64_t *wgt, const float *a,
+                              const float *b, int cout, const float *sc_wgt, const float *sc_bias, const float *sc_a, const float *sc_b,
+                              float *shortcut, float *out, uint64_t *out_packed, dab_stream_t stream);
+DAB_API int dab_bconv3x3_down_takes(int n, int h, int w, int cin, int cout);
+
+/*
  * BinConv::forward_impl (dabnn/layers/BinConv.cpp:144-191) for a batch of
  * fp32 NHWC images: binarise + binary convolution, fp32 mismatch counts out.
  * Method selection mirrors BinConv::method() (:80-98): 3x3 with cin in
