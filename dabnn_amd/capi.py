@@ -86,7 +86,9 @@ SIGNATURES = {
     "dab_fill_f32": (_i, [_vp, _i64, ctypes.c_float, _vp]),
     "dab_bconv3x3_pair": (_i, [_vp, _vp, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
     "dab_bconv3x3_pair_takes": (_i, [_i] * 3),
-    "dab_bconv3x3_down": (_i, [_vp, _vp, _i, _i, _i, _i, _vp, _vp, _vp, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
+    "dab_bconv3x3_pair_pool": (_i, [_vp, _vp, _i, _i, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
+    "dab_bconv3x3_pair_pool_takes": (_i, [_i] * 3),
+    "dab_bconv3x3_down": (_i, [_vp, _vp, _i, _i, _i, _i, _i, _vp, _vp, _vp, _i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
     "dab_bconv3x3_down_takes": (_i, [_i] * 5),
     "dab_copy_f32": (_i, [_vp, _vp, _i64, _vp]),
     "dab_ave_pool": (_i, [_vp] + [_i] * 10 + [_vp, _vp]),

@@ -19,7 +19,7 @@ namespace dab {
 
 struct BconvDownArgs {
     const uint64_t *x;   // sign bits of xf
-    const float *xf;
+    const float *xf;     // or the pooled tensor, for the kernels built for that
     const uint64_t *w;   // of the binary convolution
     const float *ea, *eb;
     const float *sw;     // [cout][cin] of the branch
@@ -55,6 +55,28 @@ __device__ __forceinline__ f32x4m pool_taps(const f32x4m (&t)[4]) {
     s = s + t[3];
     return s * 0.25f;
 }
+// Four channels of a pooled pixel as they are asked for: the four taps, or the pooled value where x is pooled already.
+template <bool POOLED>
+struct DownPiece {
+    f32x4m t[POOLED ? 1 : 4];
+    __device__ __forceinline__ void fetch(const BconvDownArgs &p, int pix, int c, int channels) {
+        if constexpr (POOLED) {
+            t[0] = *reinterpret_cast<const f32x4m *>(p.xf + (size_t)pix * channels + c);
+        } else {
+            const DownPixel at(p, pix);
+            const float *src = p.xf + ((size_t)(at.n * p.H + 2 * at.oy) * p.W + 2 * at.ox) * channels + c;
+            const size_t below = (size_t)p.W * channels;
+            t[0] = *reinterpret_cast<const f32x4m *>(src), t[1] = *reinterpret_cast<const f32x4m *>(src + channels);
+            t[2] = *reinterpret_cast<const f32x4m *>(src + below), t[3] = *reinterpret_cast<const f32x4m *>(src + below + channels);
+        }
+    }
+    __device__ __forceinline__ f32x4m value() const {
+        if constexpr (POOLED)
+            return t[0];
+        else
+            return pool_taps(t);
+    }
+};
 // bias, Affine of the branch; Affine of the counts; Add: every operation rounded by itself like the separate layers'
 __device__ __forceinline__ float branch_value(float v, bool with_bias, float bias, bool with_affine, float sa, float sb) {
 #pragma clang fp contract(off)
@@ -114,15 +136,12 @@ __global__ __launch_bounds__(512) void bconv3x3_down_staged_kernel(const BconvDo
                 load_dwords<ND>(wt[n][s], rw, (!kPair || kw < 3) ? wbase + n * T * (CW * 72) + kw * (CW * 8) + inner : kDownOutside);
         }
     }
-    f32x4m tap[XP][4], f[FP];
+    DownPiece<false> x[XP];
+    f32x4m f[FP];
 #pragma unroll
     for (int i = 0; i < XP; ++i) {
         const int piece = tid + THREADS * i, pix = (int)tile * T + piece / (C / 4);
-        const DownPixel at(p, pix < p.total ? pix : p.total - 1);
-        const float *src = p.xf + ((size_t)(at.n * p.H + 2 * at.oy) * p.W + 2 * at.ox) * C + (piece % (C / 4)) * 4;
-        const size_t below = (size_t)p.W * C;
-        tap[i][0] = *reinterpret_cast<const f32x4m *>(src), tap[i][1] = *reinterpret_cast<const f32x4m *>(src + C);
-        tap[i][2] = *reinterpret_cast<const f32x4m *>(src + below), tap[i][3] = *reinterpret_cast<const f32x4m *>(src + below + C);
+        x[i].fetch(p, pix < p.total ? pix : p.total - 1, (piece % (C / 4)) * 4, C);
     }
 #pragma unroll
     for (int i = 0; i < FP; ++i) {
@@ -163,7 +182,7 @@ __global__ __launch_bounds__(512) void bconv3x3_down_staged_kernel(const BconvDo
 #pragma unroll
     for (int i = 0; i < XP; ++i) {
         const int piece = tid + THREADS * i;
-        if (piece < T * (C / 4)) *reinterpret_cast<f32x4m *>(&pooled[piece / (C / 4)][(piece % (C / 4)) * 4]) = pool_taps(tap[i]);
+        if (piece < T * (C / 4)) *reinterpret_cast<f32x4m *>(&pooled[piece / (C / 4)][(piece % (C / 4)) * 4]) = x[i].value();
     }
 #pragma unroll
     for (int i = 0; i < FP; ++i) {
@@ -242,7 +261,7 @@ __global__ __launch_bounds__(512) void bconv3x3_down_staged_kernel(const BconvDo
 // ---------------------------------------------------------------- between
 // A wave counts, the block pools its pixels into LDS, the wave multiplies on the fp32 matrix instruction -- 32 of 64 cycles per 64
 // channels of depth, which is what bounds the kernel: 40 images of 28 x 28 x 128 to 256 take 12.0 us.
-template <int CW, int WAVES>
+template <int CW, int WAVES, bool POOLED>
 __global__ __launch_bounds__(WAVES * 64) void bconv3x3_down_tile_kernel(const BconvDownArgs p) {
     constexpr int C = CW * 64, AS = C + 4, CH = 32 * WAVES, THREADS = 64 * WAVES;  // AS: rows 4 floats off a multiple of 64 banks
     constexpr int PIECES = 32 * (C / 4) / THREADS;  // 16-byte pieces of the pooled tile per thread
@@ -271,15 +290,11 @@ __global__ __launch_bounds__(WAVES * 64) void bconv3x3_down_tile_kernel(const Bc
 #pragma unroll
         for (int t = 0; t < 9; ++t) load_dwords<CW>(wt[t], rw, ch_ok ? ch * (CW * 72) + t * (CW * 8) + half * (CW * 4) : kDownOutside);
     }
-    f32x4m tap[PIECES][4];
+    DownPiece<POOLED> x[PIECES];
 #pragma unroll
     for (int i = 0; i < PIECES; ++i) {
-        const int piece = tid + THREADS * i, row = piece / (C / 4), c4 = piece % (C / 4);
-        const DownPixel at(p, m0 + row < p.total ? m0 + row : p.total - 1);
-        const float *src = p.xf + ((size_t)(at.n * p.H + 2 * at.oy) * p.W + 2 * at.ox) * C + c4 * 4;
-        const size_t below = (size_t)p.W * C;
-        tap[i][0] = *reinterpret_cast<const f32x4m *>(src), tap[i][1] = *reinterpret_cast<const f32x4m *>(src + C);
-        tap[i][2] = *reinterpret_cast<const f32x4m *>(src + below), tap[i][3] = *reinterpret_cast<const f32x4m *>(src + below + C);
+        const int piece = tid + THREADS * i, pix = m0 + piece / (C / 4);
+        x[i].fetch(p, pix < p.total ? pix : p.total - 1, (piece % (C / 4)) * 4, C);
     }
     const float *filter = p.sw + (size_t)(ch_ok ? ch : 0) * C + half * 4;
     f32x4m f[CHUNKS > 1 ? 2 : 1][CHUNK];
@@ -305,7 +320,7 @@ __global__ __launch_bounds__(WAVES * 64) void bconv3x3_down_tile_kernel(const Bc
 #pragma unroll
     for (int i = 0; i < PIECES; ++i) {
         const int piece = tid + THREADS * i;
-        *reinterpret_cast<f32x4m *>(&pooled[piece / (C / 4)][(piece % (C / 4)) * 4]) = pool_taps(tap[i]);
+        *reinterpret_cast<f32x4m *>(&pooled[piece / (C / 4)][(piece % (C / 4)) * 4]) = x[i].value();
     }
     __syncthreads();
     // eight depths at a time, the pairs d and d + 4 in one instruction
@@ -349,7 +364,7 @@ __global__ __launch_bounds__(WAVES * 64) void bconv3x3_down_tile_kernel(const Bc
 // 56 x 56 x 64 to 128 move 315 MB in 61 us, 5.2 TB/s, the rate of a copy (tile kernel 75, two launches 100).  With 128 a block has eight
 // waves, so that the floats are read once: 28 x 28 at 256 images 43 us (tile 63, two launches 68; four waves 63).  256 input
 // channels, whose filters take 192 registers, were no faster (64 us, two launches 59).
-template <int CW, int WAVES>
+template <int CW, int WAVES, bool POOLED>
 __global__ __launch_bounds__(WAVES * 64, 2) void bconv3x3_down_walk_kernel(const BconvDownArgs p) {
     constexpr int C = CW * 64, CH = 32 * WAVES, THREADS = 64 * WAVES;
     constexpr int PIECES = 32 * (C / 4) / THREADS, GROUPS = C / 16;
@@ -365,17 +380,13 @@ __global__ __launch_bounds__(WAVES * 64, 2) void bconv3x3_down_walk_kernel(const
     const __amdgpu_buffer_rsrc_t rx = make_rsrc(p.x, p.x_bytes), rw = make_rsrc(p.w, p.w_bytes);
     typedef SplitFrag8::u4 u4;
 
-    f32x4m tap[PIECES][4];
+    DownPiece<POOLED> x[PIECES];
     uint32_t act[9][CW];
     auto fetch_floats = [&](int tile) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < PIECES; ++i) {
             const int piece = tid + THREADS * i, pix = tile * 32 + piece / (C / 4);
-            const DownPixel at(p, pix < p.total ? pix : p.total - 1);
-            const float *src = p.xf + ((size_t)(at.n * p.H + 2 * at.oy) * p.W + 2 * at.ox) * C + (piece % (C / 4)) * 4;
-            const size_t below = (size_t)p.W * C;
-            tap[i][0] = *reinterpret_cast<const f32x4m *>(src), tap[i][1] = *reinterpret_cast<const f32x4m *>(src + C);
-            tap[i][2] = *reinterpret_cast<const f32x4m *>(src + below), tap[i][3] = *reinterpret_cast<const f32x4m *>(src + below + C);
+            x[i].fetch(p, pix < p.total ? pix : p.total - 1, (piece % (C / 4)) * 4, C);
         }
     };
     auto fetch_bits = [&](int tile) __attribute__((always_inline)) {
@@ -432,7 +443,7 @@ __global__ __launch_bounds__(WAVES * 64, 2) void bconv3x3_down_walk_kernel(const
 #pragma unroll
         for (int i = 0; i < PIECES; ++i) {
             const int piece = tid + THREADS * i;
-            const f32x4m v = pool_taps(tap[i]);
+            const f32x4m v = x[i].value();
             small = smallest_magnitude(smallest_magnitude(small, v[0], v[1]), v[2], v[3]);
             const SplitPair s0 = split_pair_finite(v[0], v[1]), s1 = split_pair_finite(v[2], v[3]);
             top = bf16_pair_max(bf16_pair_max(top, s0.hi), s1.hi);
@@ -466,14 +477,12 @@ __global__ __launch_bounds__(WAVES * 64, 2) void bconv3x3_down_walk_kernel(const
 #pragma unroll
             for (int e = 0; e < 16; ++e) sum[e] = sum[e] + cross[e];
         } else {
-            const DownPixel at(p, tile * 32 + l32 < p.total ? tile * 32 + l32 : p.total - 1);
-            const float *src = p.xf + ((size_t)(at.n * p.H + 2 * at.oy) * p.W + 2 * at.ox) * C + half * 4;
-            const size_t below = (size_t)p.W * C;
+            const int pix = tile * 32 + l32 < p.total ? tile * 32 + l32 : p.total - 1;
 #pragma unroll 1
-            for (int d = 0; d < C; d += 8) {
-                const f32x4m t[4] = {*reinterpret_cast<const f32x4m *>(src + d), *reinterpret_cast<const f32x4m *>(src + d + C),
-                                     *reinterpret_cast<const f32x4m *>(src + d + below), *reinterpret_cast<const f32x4m *>(src + d + below + C)};
-                const f32x4m a = pool_taps(t), b = *reinterpret_cast<const f32x4m *>(filter + d + half * 4);
+            for (int d = half * 4; d < C; d += 8) {
+                DownPiece<POOLED> again;
+                again.fetch(p, pix, d, C);
+                const f32x4m a = again.value(), b = *reinterpret_cast<const f32x4m *>(filter + d);
 #pragma unroll
                 for (int e = 0; e < 4; ++e) sum = __builtin_amdgcn_mfma_f32_32x32x2f32(a[e], b[e], sum, 0, 0, 0);
             }
@@ -552,15 +561,15 @@ static int launch_down(Kernel kernel, BconvDownArgs &a, int px, int ch, int thre
     return DAB_OK;
 }
 
-template <int CW, int WAVES>
+template <int CW, int WAVES, bool POOLED>
 static int launch_down_walk(BconvDownArgs &a, hipStream_t s) {
     constexpr int CH = 32 * WAVES;
     constexpr size_t lds = 2 * 3 * 32 * (CW * 64 + 8) * 2;
-    auto kernel = bconv3x3_down_walk_kernel<CW, WAVES>;
+    auto kernel = bconv3x3_down_walk_kernel<CW, WAVES, POOLED>;
     a.cols = (a.cout + CH - 1) / CH;
     a.div_cols = FastDiv((uint32_t)a.cols);
     if (lds > 64 * 1024) {
-        const int rc = allow_dynamic_lds<bconv3x3_down_walk_kernel<CW, WAVES>>("dab_bconv3x3_down", lds);
+        const int rc = allow_dynamic_lds<bconv3x3_down_walk_kernel<CW, WAVES, POOLED>>("dab_bconv3x3_down", lds);
         if (rc != DAB_OK) return rc;
     }
     static const int per_cu = [&] {
@@ -577,18 +586,16 @@ static int launch_down_walk(BconvDownArgs &a, hipStream_t s) {
     return DAB_OK;
 }
 
-template <int CW>
+template <int CW, bool POOLED>
 static int launch_bconv_down(BconvDownArgs &a, hipStream_t s) {
-    switch (pick_down(a.total, CW * 64, a.cout)) {
-        case Down::staged16:
-            if constexpr (CW >= 2) return launch_down(bconv3x3_down_staged_kernel<CW, 16, 1>, a, 16, 16, 512, s);
-            [[fallthrough]];
-        case Down::staged32: return launch_down(bconv3x3_down_staged_kernel<CW, 32, 2>, a, 32, 32, 512, s);
-        case Down::walk:
-            if constexpr (CW <= 2) return launch_down_walk<CW, 4 * CW>(a, s);
-            [[fallthrough]];
-        default: return launch_down(bconv3x3_down_tile_kernel<CW, 4>, a, 32, 128, 256, s);
-    }
+    const Down kernel = pick_down(a.total, CW * 64, a.cout);
+    if constexpr (CW >= 2 && !POOLED)
+        if (kernel == Down::staged16) return launch_down(bconv3x3_down_staged_kernel<CW, 16, 1>, a, 16, 16, 512, s);
+    if constexpr (!POOLED)
+        if (kernel == Down::staged32) return launch_down(bconv3x3_down_staged_kernel<CW, 32, 2>, a, 32, 32, 512, s);
+    if constexpr (CW <= 2)
+        if (kernel == Down::walk) return launch_down_walk<CW, 4 * CW, POOLED>(a, s);
+    return launch_down(bconv3x3_down_tile_kernel<CW, 4, POOLED>, a, 32, 128, 256, s);
 }
 
 }  // namespace dab
@@ -599,8 +606,8 @@ extern "C" int dab_bconv3x3_down_takes(int n, int h, int w, int cin, int cout) {
            ((long long)a.total + 31) / 32 * ((cout + 127) / 128) < dab::kMostBlocks;
 }
 
-extern "C" int dab_bconv3x3_down(const uint64_t *x_packed, const float *x, int n, int h, int w, int cin, const uint64_t *wgt, const float *a,
-                                 const float *b, int cout, const float *sc_wgt, const float *sc_bias, const float *sc_a, const float *sc_b,
+extern "C" int dab_bconv3x3_down(const uint64_t *x_packed, const float *x, int x_pooled, int n, int h, int w, int cin, const uint64_t *wgt,
+                                 const float *a, const float *b, int cout, const float *sc_wgt, const float *sc_bias, const float *sc_a, const float *sc_b,
                                  float *shortcut, float *out, uint64_t *out_packed, dab_stream_t stream) {
     using namespace dab;
     const char *fn = "dab_bconv3x3_down";
@@ -619,8 +626,8 @@ extern "C" int dab_bconv3x3_down(const uint64_t *x_packed, const float *x, int n
     p.sc_out = shortcut, p.out = out, p.bits = reinterpret_cast<uint32_t *>(out_packed);
     hipStream_t s = as_stream(stream);
     switch (cin) {
-        case 64: return launch_bconv_down<1>(p, s);
-        case 128: return launch_bconv_down<2>(p, s);
-        default: return launch_bconv_down<4>(p, s);
+        case 64: return x_pooled ? launch_bconv_down<1, true>(p, s) : launch_bconv_down<1, false>(p, s);
+        case 128: return x_pooled ? launch_bconv_down<2, true>(p, s) : launch_bconv_down<2, false>(p, s);
+        default: return x_pooled ? launch_bconv_down<4, true>(p, s) : launch_bconv_down<4, false>(p, s);
     }
 }

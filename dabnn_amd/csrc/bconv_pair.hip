@@ -187,6 +187,213 @@ static int pair_bands(int n, int h, int w) {
     return (long long)h * w * 256 < (1ll << 31) && (long long)n * bands < kMostBlocks ? bands : 0;
 }
 
+// ---------------------------------------------------------------- the same for a pass whose result is only pooled
+// Before a down-sampling block the second layer's result is read by an AvePool 2x2 and, as sign bits, by a binary convolution:
+// the pass writes the pooled tensor and the bits, a quarter of the bytes, and its reader fetches a quarter.  A tile's 32 pixels are
+// eight 2x2 windows, in the order of the pooled tensor, one window the four registers of an accumulator quad, so that pooling
+// takes no exchange.  A strip has an even number of rows; the rows above and below it, of which only the sign bits are wanted, are a
+// fifth tile of each wave that no register outlives, so that a strip has eight rows of 56 where the kernel above has seven.
+// 56 x 56 at batch 256, with the block's first layer behind it (bconv_down.hip): 89 + 61 us (one behind the other 164) before, 77 + 47 (131) now.
+struct BconvPairPoolArgs {
+    const uint64_t *x;
+    const float *shortcut;
+    const uint64_t *w[2];
+    const float *a[2], *b[2];
+    float *pooled;
+    uint64_t *bits;
+    int H, W;
+    int rows, bands;
+    uint32_t image_bytes;  // of the shortcut
+    FastDiv div_bands, div_w, div_half_w;
+};
+
+__global__ __launch_bounds__(256, 2) void bconv3x3_pair_pool_kernel(const BconvPairPoolArgs p) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+    __shared__ uint32_t pop[2][64];
+    const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5, l32 = lane & 31;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t item = xcd_contiguous_block(blockIdx.x, gridDim.x);
+    const int img = (int)p.div_bands.div(item), r0 = ((int)item - img * p.bands) * p.rows;
+    const int rows = p.H - r0 < p.rows ? p.H - r0 : p.rows, half_w = p.W >> 1, windows = (rows >> 1) * half_w;
+    const int pitch = (p.W + 2) * 8;
+    unsigned char *const bits0 = lds + 2 * kPairFilterBytes;   // image rows r0 - 2 .. r0 + rows + 1
+    unsigned char *const bits1 = bits0 + (p.rows + 4) * pitch;  // of v1: r0 - 1 .. r0 + rows
+    const size_t image = (size_t)img * p.H * p.W;               // its first pixel
+    auto tile_of = [&](int i) { return 2 * wave + (i & 1) + 8 * (i >> 1); };
+    const __amdgpu_buffer_rsrc_t rs = make_rsrc(p.shortcut + image * 64, p.image_bytes);
+    constexpr int kNowhere = (int)0x80000000;  // beyond the image: loads return zero
+
+    // v0, asked for before anything else: the row above the strip and the one below it (pixel j of the two, one behind the other) ...
+    float edge[2][16];
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+        const int j = wave * 32 + 8 * (v / 4) + 4 * half + v % 4;
+        const int pix = (r0 - 1) * p.W + j + (j >= p.W ? rows * p.W : 0);
+        const int off = j < 2 * p.W && pix >= 0 ? pix * 256 + l32 * 4 : kNowhere;
+#pragma unroll
+        for (int n = 0; n < 2; ++n) edge[n][v] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, off + n * 128, 0, 0));
+    }
+    // ... and of the wave's four tiles
+    float val[4][2][16];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int win = tile_of(i) * 8 + 2 * q + half, rp = (int)p.div_half_w.div((uint32_t)win);
+            const int off = win < windows ? ((r0 + 2 * rp) * p.W + 2 * (win - rp * half_w)) * 256 + l32 * 4 : kNowhere;
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int n = 0; n < 2; ++n)
+                    val[i][n][4 * q + e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, off + (e & 1) * 256 + n * 128, (e >> 1) * p.W * 256, 0));
+        }
+
+    if (tid < 128) pop[tid >> 6][tid & 63] = 0;
+    const int bit_bytes = (2 * p.rows + 6) * pitch;
+    for (int i = tid * 8; i < bit_bytes; i += 256 * 8) *reinterpret_cast<uint64_t *>(bits0 + i) = 0;
+    __syncthreads();
+    const int in0 = r0 >= 2 ? r0 - 2 : 0, in1 = r0 + rows + 2 < p.H ? r0 + rows + 2 : p.H;
+    const uint64_t *src = p.x + image + (size_t)in0 * p.W;
+    for (int j = tid; j < (in1 - in0) * p.W; j += 256) {
+        const int row = (int)p.div_w.div(j), col = j - row * p.W;
+        *reinterpret_cast<uint64_t *>(bits0 + (in0 - (r0 - 2) + row) * pitch + (col + 1) * 8) = src[j];
+    }
+    for (int j = tid; j < 2 * 64 * 9; j += 256) {
+        const int layer = j >= 64 * 9, c = j - layer * (64 * 9), ch = c / 9, tap = c - ch * 9;
+        const uint64_t word = p.w[layer][c];
+        unsigned char *d = lds + layer * kPairFilterBytes + ((tap * 2 + (ch >> 5)) * 64 + (ch & 31)) * 16;
+        *reinterpret_cast<i32x4 *>(d) = lower_half(bitspm((uint32_t)word));
+        *reinterpret_cast<i32x4 *>(d + 32 * 16) = lower_half(bitspm((uint32_t)(word >> 32)));
+        atomicAdd(&pop[layer][ch], (uint32_t)__popcll(word));
+    }
+    __syncthreads();
+
+    auto value = [](float cnt, float a, float b, float add) {
+#pragma clang fp contract(off)
+        float r = a * cnt;
+        r = r + b;
+        return r + add;
+    };
+    auto layer = [&](auto which) __attribute__((always_inline)) {
+        constexpr int L = decltype(which)::value;
+        float init[2], ea[2], eb[2];
+#pragma unroll
+        for (int n = 0; n < 2; ++n) {
+            init[n] = (float)pop[L][n * 32 + l32];
+            ea[n] = p.a[L][n * 32 + l32], eb[n] = p.b[L][n * 32 + l32];
+        }
+        const unsigned char *filter = lds + L * kPairFilterBytes + lane * 16;
+        // counts of M tiles whose lanes' windows are at `window`
+        auto count = [&](auto tiles, const unsigned char *const *window, f32x16m (*acc)[2]) __attribute__((always_inline)) {
+            constexpr int M = decltype(tiles)::value;
+#pragma unroll
+            for (int m = 0; m < M; ++m)
+#pragma unroll
+                for (int n = 0; n < 2; ++n)
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) acc[m][n][v] = init[n];
+#pragma unroll
+            for (int tap = 0; tap < 9; ++tap) {
+                i32x8 a[M];
+#pragma unroll
+                for (int m = 0; m < M; ++m) a[m] = bits01(*reinterpret_cast<const uint32_t *>(window[m] + (tap / 3) * pitch + (tap % 3) * 8));
+#pragma unroll
+                for (int n = 0; n < 2; ++n) {
+                    const i32x8 b = upper_zero(*reinterpret_cast<const i32x4 *>(filter + (tap * 2 + n) * 64 * 16));
+#pragma unroll
+                    for (int m = 0; m < M; ++m) mfma_fp4<32>(acc[m][n], a[m], b);
+                }
+            }
+        };
+        auto put_sign = [](uint32_t (&word)[2], int n, int v, float r) __attribute__((always_inline)) {
+            const uint64_t mask = __ballot(r > 0.f);
+            word[n] = dab_writelane((uint32_t)mask, 8 * (v / 4) + v % 4, word[n]);
+            word[n] = dab_writelane((uint32_t)(mask >> 32), 8 * (v / 4) + v % 4 + 4, word[n]);
+        };
+        if constexpr (L == 0) {
+            const int j = wave * 32 + l32, below = j >= p.W, col = j - (below ? p.W : 0);
+            const bool there = j < 2 * p.W && (below ? r0 + rows < p.H : r0 > 0);
+            if (wave * 32 < 2 * p.W) {
+                const unsigned char *window[1] = {bits0 + (there && below ? rows + 1 : 0) * pitch + (there ? col : 0) * 8 + half * 4};
+                f32x16m acc[1][2];
+                count(std::integral_constant<int, 1>{}, window, acc);
+                uint32_t word[2] = {0, 0};
+#pragma unroll
+                for (int v = 0; v < 16; ++v)
+#pragma unroll
+                    for (int n = 0; n < 2; ++n) put_sign(word, n, v, value(acc[0][n][v], ea[n], eb[n], edge[n][v]));
+                if (half == 0 && there) *reinterpret_cast<u32x2 *>(bits1 + (below ? rows + 1 : 0) * pitch + (col + 1) * 8) = u32x2{word[0], word[1]};
+            }
+        }
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            if (tile_of(2 * s) * 8 >= windows) continue;
+            int row[2], col[2];  // of the lane's pixel, from r0 on
+            bool there[2];
+            const unsigned char *window[2];
+            f32x16m acc[2][2];
+#pragma unroll
+            for (int m = 0; m < 2; ++m) {
+                const int win = tile_of(2 * s + m) * 8 + l32 / 4;
+                there[m] = win < windows;
+                const int rp = (int)p.div_half_w.div((uint32_t)(there[m] ? win : 0));
+                row[m] = 2 * rp + ((l32 >> 1) & 1), col[m] = 2 * ((there[m] ? win : 0) - rp * half_w) + (l32 & 1);
+                window[m] = (L == 0 ? bits0 + pitch : bits1) + row[m] * pitch + col[m] * 8 + half * 4;
+            }
+            count(std::integral_constant<int, 2>{}, window, acc);
+#pragma unroll
+            for (int m = 0; m < 2; ++m) {
+                const int i = 2 * s + m;
+                const size_t first = (size_t)img * (p.H >> 1) * half_w + (size_t)(r0 >> 1) * half_w;  // the strip's first pooled pixel
+                const __amdgpu_buffer_rsrc_t ro = make_rsrc(p.pooled + first * 64, (uint32_t)windows * 256u);
+                uint32_t word[2] = {0, 0};
+#pragma unroll
+                for (int n = 0; n < 2; ++n)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+#pragma clang fp contract(off)
+                        float sum = 0.f;  // ave_pool_fallback's order (dabnn/layers/AvePool.cpp:84-123)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            const int v = 4 * q + e;
+                            const float r = value(acc[m][n][v], ea[n], eb[n], val[i][n][v]);
+                            if constexpr (L == 0)
+                                val[i][n][v] = r;
+                            else
+                                sum = sum + r;
+                            put_sign(word, n, v, r);
+                        }
+                        if constexpr (L == 1)
+                            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, sum * 0.25f), ro,
+                                                                  (tile_of(i) * 8 + 2 * q + half) * 256 + l32 * 4 + n * 128, 0, kStoreStream);
+                    }
+                if (half == 0 && there[m]) {
+                    if constexpr (L == 0)
+                        *reinterpret_cast<u32x2 *>(bits1 + (row[m] + 1) * pitch + (col[m] + 1) * 8) = u32x2{word[0], word[1]};
+                    else
+                        p.bits[image + (size_t)(r0 + row[m]) * p.W + col[m]] = ((uint64_t)word[1] << 32) | word[0];
+                }
+            }
+        }
+    };
+    layer(std::integral_constant<int, 0>{});
+    __syncthreads();
+    layer(std::integral_constant<int, 1>{});
+}
+
+// Rows of a strip, even, or 0 where the kernel does not take the problem.
+static int pair_pool_rows(int n, int h, int w) {
+    if (h % 2 != 0 || w % 2 != 0 || w > 64 || (long long)h * w * 256 >= (1ll << 31)) return 0;
+    int most = (kPairTiles * 32 / w) & ~1;
+    if (most > h) most = h;
+    const int cus = simd_count() / 4;
+    auto even_rows = [&](int bands) { return ((h + bands - 1) / bands + 1) & ~1; };
+    int bands = (h + most - 1) / most;
+    while ((long long)n * bands < cus && even_rows(bands) > 2) ++bands;
+    const int rows = even_rows(bands) < most ? even_rows(bands) : most;
+    return (long long)n * ((h + rows - 1) / rows) < kMostBlocks ? rows : 0;
+}
+
 }  // namespace dab
 
 extern "C" int dab_bconv3x3_pair_takes(int n, int h, int w) { return n > 0 && h > 0 && w > 0 && dab::pair_bands(n, h, w) > 0; }
@@ -215,6 +422,30 @@ extern "C" int dab_bconv3x3_pair(const uint64_t *x, const float *shortcut, int n
         hipLaunchKernelGGL(bconv3x3_pair_kernel<true>, grid, dim3(256), lds, as_stream(stream), p);
     else
         hipLaunchKernelGGL(bconv3x3_pair_kernel<false>, grid, dim3(256), lds, as_stream(stream), p);
+    DAB_LAUNCH_CHECK();
+    return DAB_OK;
+}
+
+extern "C" int dab_bconv3x3_pair_pool_takes(int n, int h, int w) { return n > 0 && h > 0 && w > 0 && dab::pair_pool_rows(n, h, w) > 0; }
+
+extern "C" int dab_bconv3x3_pair_pool(const uint64_t *x, const float *shortcut, int n, int h, int w, const uint64_t *w1, const float *a1, const float *b1,
+                                      const uint64_t *w2, const float *a2, const float *b2, float *pooled, uint64_t *out_packed, dab_stream_t stream) {
+    using namespace dab;
+    const char *fn = "dab_bconv3x3_pair_pool";
+    DAB_REQUIRE(x && shortcut && w1 && a1 && b1 && w2 && a2 && b2 && pooled && out_packed, "%s: null pointer", fn);
+    DAB_REQUIRE(n > 0 && h > 0 && w > 0, "%s: non-positive dimension", fn);
+    DAB_REQUIRE(pooled != shortcut && out_packed != x, "%s: the result must not alias the input", fn);
+    auto at = [](const void *q) { return reinterpret_cast<uintptr_t>(q); };
+    DAB_REQUIRE(((at(x) | at(w1) | at(w2) | at(out_packed)) & 7) == 0 && ((at(pooled) | at(shortcut)) & 3) == 0, "%s: misaligned pointer", fn);
+    const int rows = pair_pool_rows(n, h, w);
+    if (rows == 0) return fail(DAB_EUNSUPPORTED, "%s: %d images of %d x %d are not covered", fn, n, h, w);
+    BconvPairPoolArgs p;
+    p.x = x, p.shortcut = shortcut, p.pooled = pooled, p.bits = out_packed;
+    p.w[0] = w1, p.w[1] = w2, p.a[0] = a1, p.a[1] = a2, p.b[0] = b1, p.b[1] = b2;
+    p.H = h, p.W = w, p.rows = rows, p.bands = (h + rows - 1) / rows, p.image_bytes = (uint32_t)(h * w) * 256u;
+    p.div_bands = FastDiv((uint32_t)p.bands), p.div_w = FastDiv((uint32_t)w), p.div_half_w = FastDiv((uint32_t)w / 2);
+    const size_t lds = 2 * kPairFilterBytes + (size_t)(2 * rows + 6) * (w + 2) * 8;
+    hipLaunchKernelGGL(bconv3x3_pair_pool_kernel, dim3((unsigned)(n * p.bands)), dim3(256), lds, as_stream(stream), p);
     DAB_LAUNCH_CHECK();
     return DAB_OK;
 }

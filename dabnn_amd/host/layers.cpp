@@ -138,15 +138,20 @@ void BinConv::forward_impl() const {
         forward_alone();
         return;
     }
+    forward_pass(next_in_pass->pooled_in_pass != nullptr);
+}
+
+void BinConv::forward_pass(bool pooled) const {
     const BinConv &second = *next_in_pass;
-    const auto *x = static_cast<const float *>(input_mat->dev);
+    auto floats = [](const MatP &m) { return static_cast<const float *>(m->dev); };
+    auto words = [](const MatP &m) { return static_cast<const uint64_t *>(m->dev); };
+    const Mat &in = *input_mat;
     auto *packed = static_cast<uint64_t *>(binarized_mat->dev);
-    if (!input_prepacked) dab_check(dab_bitpack_nhwc(x, packed, (int64_t)input_mat->n * input_mat->h * input_mat->w, input_mat->elem_c, stream()));
-    dab_check(dab_bconv3x3_pair(packed, x, input_mat->n, input_mat->h, input_mat->w, static_cast<const uint64_t *>(weight_mat->dev),
-                                static_cast<const float *>(fused_a->dev), static_cast<const float *>(fused_b->dev),
-                                static_cast<const uint64_t *>(second.weight_mat->dev), static_cast<const float *>(second.fused_a->dev),
-                                static_cast<const float *>(second.fused_b->dev), static_cast<float *>(second.output_mat->dev),
-                                second.fused_sign_out ? static_cast<uint64_t *>(second.fused_sign_out->dev) : nullptr, stream()));
+    if (!input_prepacked) dab_check(dab_bitpack_nhwc(floats(input_mat), packed, (int64_t)in.n * in.h * in.w, in.elem_c, stream()));
+    auto *sign = second.fused_sign_out ? static_cast<uint64_t *>(second.fused_sign_out->dev) : nullptr;
+    dab_check((pooled ? dab_bconv3x3_pair_pool : dab_bconv3x3_pair)(
+        packed, floats(input_mat), in.n, in.h, in.w, words(weight_mat), floats(fused_a), floats(fused_b), words(second.weight_mat), floats(second.fused_a),
+        floats(second.fused_b), static_cast<float *>((pooled ? second.pooled_in_pass : second.output_mat)->dev), sign, stream()));
 }
 
 void BinConv::forward_with_branch(float *branch_out) const {
@@ -155,12 +160,16 @@ void BinConv::forward_with_branch(float *branch_out) const {
     auto *packed = static_cast<uint64_t *>(binarized_mat->dev);
     const int n = input_mat->n, h = input_mat->h, w = input_mat->w, c = input_mat->elem_c;
     if (!input_prepacked) dab_check(dab_bitpack_nhwc(x, packed, (int64_t)n * h * w, c, stream()));
-    dab_check(dab_bconv3x3_down(packed, x, n, h, w, c, static_cast<const uint64_t *>(weight_mat->dev), floats(fused_a), floats(fused_b), weight_mat->n,
+    dab_check(dab_bconv3x3_down(packed, branch_pooled ? floats(branch_pooled) : x, branch_pooled ? 1 : 0, n, h, w, c, static_cast<const uint64_t *>(weight_mat->dev), floats(fused_a), floats(fused_b), weight_mat->n,
                                 floats(branch->weight_mat), floats(branch->bias_mat), floats(branch->fused_a), floats(branch->fused_b), branch_out,
                                 static_cast<float *>(output_mat->dev), fused_sign_out ? static_cast<uint64_t *>(fused_sign_out->dev) : nullptr, stream()));
 }
 
 void BinConv::forward_alone() const {
+    if (pooled_in_pass) {
+        first_in_pass->forward_pass(false);
+        return;
+    }
     binarized_mat->allocate();  // there already in a net that was read; a layer of the caller's own takes it here
     void *s = stream();
     const auto *x = static_cast<const float *>(input_mat->dev);
@@ -248,6 +257,7 @@ std::string BinConv::to_str() const {
     if (fused_sign_out) ss << " + Sign";
     if (next_in_pass) ss << ", in one pass with the next layer";
     if (inside_pass) ss << ", in the pass of the layer before";
+    if (pooled_in_pass) ss << ", written pooled 2x2";
     if (branch) ss << ", its shortcut convolution in the same pass";
     return ss.str();
 }

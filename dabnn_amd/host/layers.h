@@ -39,12 +39,18 @@ class BNN_API BinConv : public Layer {
     // neither this layer's output nor its packed copy; the next layer's own forward() has nothing left to do (inside_pass).
     std::shared_ptr<BinConv> next_in_pass;
     bool inside_pass = false;
+    // Of the second layer of such a pass, where its result is only wanted pooled 2x2 (by `branch` of its reader) and as sign bits
+    // (dab_bconv3x3_pair_pool): the pooled blob.  output_mat is then only made for who asks for it.
+    MatP pooled_in_pass;
+    const BinConv *first_in_pass = nullptr;
+    void forward_pass(bool pooled) const;  // of the first layer: both layers
     // The layer by itself, for who asks for those blobs (which must have memory) after a run.
     void forward_alone() const override;
 
     // Also set by Net::prepare: the 1x1 convolution of this layer's shortcut branch runs in this layer's pass
     // (dab_bconv3x3_down), which does not write the branch's blob.
     std::shared_ptr<FloatConv> branch;
+    MatP branch_pooled;  // the branch's pooled input, where input_mat is not written
     void forward_with_branch(float *branch_out) const;  // branch_out: where the branch's blob is wanted, or null
 
     BinConv(NetCP net, css name, css input, css weight, css output, int pad_h, int pad_w, int stride_h, int stride_w);

@@ -171,6 +171,14 @@ void Net::make_columns(const std::shared_ptr<Mat> &m) {
             alone_.push_back(bc->branch);
             return;
         }
+        if (bc && bc->pooled_in_pass && bc->output_mat == m) {
+            std::lock_guard<std::mutex> lock(capture_mutex());
+            m->allocate();
+            bc->forward_alone();
+            hip_check(hipStreamSynchronize(static_cast<hipStream_t>(stream_)), "hipStreamSynchronize");
+            alone_.push_back(bc);
+            return;
+        }
         if (bc && bc->next_in_pass && (bc->output_mat == m || bc->fused_sign_out == m)) {
             std::lock_guard<std::mutex> lock(capture_mutex());
             bc->output_mat->allocate();
@@ -322,6 +330,7 @@ void Net::prepare(const void *buf, size_t len) {
         pool_inside_convs();
         pair_residual_layers();
         branches_inside_binconvs();
+        pool_inside_pairs();
     }
     allocate_blobs();
     // an in-place layer on the input blob would write into a caller's buffer that is read in place
@@ -337,9 +346,10 @@ static void layer_io(const std::shared_ptr<Layer> &l, std::vector<const Mat *> &
     reads.clear(), writes.clear();
     if (auto bc = std::dynamic_pointer_cast<BinConv>(l)) {
         if (bc->inside_pass) return;
-        reads = {bc->input_mat.get()};
+        reads = {(bc->branch_pooled ? bc->branch_pooled : bc->input_mat).get()};
         if (bc->next_in_pass) {
-            writes = {bc->next_in_pass->output_mat.get(), bc->binarized_mat.get()};
+            const auto &pooled = bc->next_in_pass->pooled_in_pass;
+            writes = {(pooled ? pooled : bc->next_in_pass->output_mat).get(), bc->binarized_mat.get()};
             if (bc->next_in_pass->fused_sign_out) writes.push_back(bc->next_in_pass->fused_sign_out.get());
             return;
         }
@@ -390,6 +400,7 @@ void Net::allocate_blobs() {
         if (bc && bc->reads_packed()) on_demand.insert(bc->col_mat.get());
         if (bc && bc->next_in_pass) on_demand.insert({bc->output_mat.get(), bc->fused_sign_out.get()});
         if (bc && bc->branch) on_demand.insert(bc->branch->output_mat.get());
+        if (bc && bc->pooled_in_pass) on_demand.insert(bc->output_mat.get());
         auto mp = std::dynamic_pointer_cast<MaxPool>(l);
         if (mp && mp->inside_conv) on_demand.insert(mp->output_mat.get());
     }
@@ -837,6 +848,7 @@ void Net::pair_residual_layers() {
         // (the net's input may be a buffer of the caller's, gone after the run)
         if (!ok || first->input_mat == stored_blob(input_name_)) continue;
         first->next_in_pass = second;
+        second->first_in_pass = first.get();
         second->inside_pass = true;
         ++i;
     }
@@ -884,6 +896,32 @@ void Net::branches_inside_binconvs() {
         if (!ok) continue;
         bc->branch = branch;
         branch->inside_block = bc.get();
+    }
+}
+
+// Two residual layers in one pass, in front of a down-sampling block whose branch runs in its BinConv's pass: where nobody else reads
+// the second layer's result, the pass writes it pooled (and its sign bits), a quarter of the bytes, and the block's pass reads that; who
+// asks for the result has the unpooled pass run.  56 x 56, the two passes together, us: 17 images 21.5 -> 18.8, 40 34 -> 33, 100 70 ->
+// 60, 256 164 -> 131.
+void Net::pool_inside_pairs() {
+    std::vector<const Mat *> rd, wr;
+    for (const auto &l : layers) {
+        auto reader = std::dynamic_pointer_cast<BinConv>(l);
+        if (!reader || !reader->branch) continue;
+        const auto &m = reader->input_mat;
+        std::shared_ptr<BinConv> second;
+        bool ok = dab_bconv3x3_pair_pool_takes(m->n, m->h, m->w);
+        for (const auto &other : layers) {
+            layer_io(other, rd, wr);
+            if (other != l && contains(rd, m.get())) ok = false;
+            if (!contains(wr, m.get())) continue;
+            auto first = std::dynamic_pointer_cast<BinConv>(other);
+            ok = ok && first && first->next_in_pass && !second;
+            second = ok ? first->next_in_pass : nullptr;
+        }
+        if (!ok || !second || second->output_mat != m || second->fused_sign_out != reader->binarized_mat || !reader->input_prepacked) continue;
+        second->pooled_in_pass = Mat::planned(m->n, m->h / 2, m->w / 2, m->c, DataType::Float, "pooled_" + m->name);
+        reader->branch_pooled = second->pooled_in_pass;
     }
 }
 

@@ -91,6 +91,7 @@ class BNN_API Net : public std::enable_shared_from_this<Net> {
     void pool_inside_convs();
     void pair_residual_layers();
     void branches_inside_binconvs();
+    void pool_inside_pairs();
     std::weak_ptr<Net> get_weak() { return shared_from_this(); }
     std::vector<std::shared_ptr<Layer>> layers;
     std::map<std::string, std::vector<uint32_t>> shapes_;  // NHWC with N = 1, as stored in the model

@@ -193,18 +193,29 @@ DAB_API int dab_bconv3x3_pair(const uint64_t *x, const float *shortcut, int n, i
 DAB_API int dab_bconv3x3_pair_takes(int n, int h, int w);
 
 /*
+ * dab_bconv3x3_pair and the AvePool 2x2 stride 2 of its result, for who reads that and out_packed and not the result itself:
+ * pooled [n][h/2][w/2][64] = avepool2x2(v2), out_packed = pack_mat(v2).  Bit for bit the separate calls.  Alignment as there; neither
+ * result may overlap an input.  DAB_EUNSUPPORTED for shapes that dab_bconv3x3_pair_pool_takes answers with 0: it takes even h and w,
+ * w up to 64.
+ */
+DAB_API int dab_bconv3x3_pair_pool(const uint64_t *x, const float *shortcut, int n, int h, int w, const uint64_t *w1, const float *a1,
+                                   const float *b1, const uint64_t *w2, const float *a2, const float *b2, float *pooled,
+                                   uint64_t *out_packed, dab_stream_t stream);
+DAB_API int dab_bconv3x3_pair_pool_takes(int n, int h, int w);
+
+/*
  * The first layer of a down-sampling block and its shortcut branch in one pass (BinConv, Affine, AvePool 2x2, FloatConv 1x1, Affine, Add):
  *   out = a * bconv3x3(x_packed, stride 2, pad 1) + b + (sc_a * (conv1x1(avepool2x2(x)) + sc_bias) + sc_b)
- * x [n][h][w][cin] floats with x_packed = pack_mat(x); wgt as dab_bconv3x3, sc_wgt [cout][cin]; sc_bias, and sc_a with sc_b, may be NULL.
+ * x [n][h][w][cin] floats with x_packed = pack_mat(x), or, with x_pooled, avepool2x2(x) [n][h/2][w/2][cin] in its place; wgt as dab_bconv3x3, sc_wgt [cout][cin]; sc_bias, and sc_a with sc_b, may be NULL.
  * out [n][h/2][w/2][cout]; out_packed = pack_mat(out) and shortcut (what the branch adds) are written unless NULL.  No
  * result may overlap an input.  Every operation behind the sums is rounded by itself, as in the separate layers; the branch's fp32
  * sums may be added in another order than dab_ave_pool2_fconv1x1's.  Buffers 16-byte aligned (wgt and out_packed 8).
  * DAB_EUNSUPPORTED for shapes that dab_bconv3x3_down_takes answers with 0: it takes 64, 128 and 256 input channels, multiples of 64
  * output channels and even h and w, within 32-bit pixel numbers.
  */
-DAB_API int dab_bconv3x3_down(const uint64_t *x_packed, const float *x, int n, int h, int w, int cin, const uint64_t *wgt, const float *a,
-                              const float *b, int cout, const float *sc_wgt, const float *sc_bias, const float *sc_a, const float *sc_b,
-                              float *shortcut, float *out, uint64_t *out_packed, dab_stream_t stream);
+DAB_API int dab_bconv3x3_down(const uint64_t *x_packed, const float *x, int x_pooled, int n, int h, int w, int cin, const uint64_t *wgt,
+                              const float *a, const float *b, int cout, const float *sc_wgt, const float *sc_bias, const float *sc_a,
+                              const float *sc_b, float *shortcut, float *out, uint64_t *out_packed, dab_stream_t stream);
 DAB_API int dab_bconv3x3_down_takes(int n, int h, int w, int cin, int cout);
 
 /*

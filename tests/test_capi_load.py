@@ -143,3 +143,22 @@ def test_shapes_that_two_layers_take_in_one_pass():
     for n, h, w in [(4, 7, 15), (4, 7, 129), (4, 7, 159), (4, 7, 161), (2**23, 1, 16), (2**20, 300, 64)]:
         rc = capi.lib.dab_bconv3x3_pair(vp(16), vp(16), n, h, w, vp(16), vp(16), vp(16), vp(16), vp(16), vp(16), vp(32), vp(64), vp(None))
         assert rc == capi.DAB_EUNSUPPORTED and not takes(n, h, w), (n, h, w)
+
+
+def test_shapes_of_the_down_sampling_passes():
+    """dab_bconv3x3_down_takes and dab_bconv3x3_pair_pool_takes say what the calls refuse, at the edges that the header states."""
+    from dabnn_amd import capi
+    vp = ctypes.c_void_p
+    takes = capi.lib.dab_bconv3x3_down_takes
+    assert [c for c in range(1, 1100) if takes(2, 8, 8, c, 64)] == [64, 128, 256] and [c for c in range(1, 300) if takes(2, 8, 8, 64, c)] == [64, 128, 192, 256]
+    assert not takes(2, 7, 8, 64, 64) and not takes(2, 8, 7, 64, 64) and not takes(0, 8, 8, 64, 64) and not takes(2**20, 64, 64, 64, 64)
+    for n, h, w, cin, cout in [(2, 7, 8, 64, 64), (2, 8, 8, 512, 64), (2, 8, 8, 64, 72), (2**20, 64, 64, 64, 64)]:
+        rc = capi.lib.dab_bconv3x3_down(vp(16), vp(32), 0, n, h, w, cin, vp(16), vp(16), vp(16), cout, vp(16), None, None, None, None, vp(64), vp(128), vp(None))
+        assert rc == capi.DAB_EUNSUPPORTED, (n, h, w, cin, cout)
+    rc = capi.lib.dab_bconv3x3_down(vp(16), vp(32), 0, 2, 8, 8, 64, vp(16), vp(16), vp(16), 64, vp(16), None, vp(16), None, None, vp(64), vp(128), vp(None))
+    assert rc == capi.DAB_EINVAL and "both coefficient vectors" in capi.last_error()
+    pool = capi.lib.dab_bconv3x3_pair_pool_takes
+    assert [w for w in range(1, 200) if pool(4, 8, w)] == list(range(2, 65, 2)) and not pool(4, 7, 16) and not pool(0, 8, 16) and not pool(2**23, 2, 2)
+    for n, h, w in [(4, 7, 16), (4, 8, 15), (4, 8, 66), (2**23, 2, 2)]:
+        rc = capi.lib.dab_bconv3x3_pair_pool(vp(16), vp(16), n, h, w, vp(16), vp(16), vp(16), vp(16), vp(16), vp(16), vp(32), vp(64), vp(None))
+        assert rc == capi.DAB_EUNSUPPORTED, (n, h, w)

@@ -20,13 +20,13 @@ def ptr(t):
     return ctypes.c_void_p(0 if t is None else t.data_ptr())
 
 
-def down(gpu, x, packed, w, coef, sw, bias, branch, cout, sign=True, want_branch=True):
+def down(gpu, x, packed, w, coef, sw, bias, branch, cout, sign=True, want_branch=True, pooled=None):
     torch, dab, capi = gpu
     n, h, wd, cin = x.shape
     out = torch.full((n, h // 2, wd // 2, cout), 7.0, device="cuda")
     sc = torch.full_like(out, 7.0) if want_branch else None
     bits = torch.zeros((n, h // 2, wd // 2, cout // 64), dtype=torch.int64, device="cuda") if sign else None
-    rc = capi.lib.dab_bconv3x3_down(ptr(packed), ptr(x), n, h, wd, cin, ptr(w), ptr(coef[0]), ptr(coef[1]), cout, ptr(sw), ptr(bias), ptr(branch[0]),
+    rc = capi.lib.dab_bconv3x3_down(ptr(packed), ptr(x if pooled is None else pooled), pooled is not None, n, h, wd, cin, ptr(w), ptr(coef[0]), ptr(coef[1]), cout, ptr(sw), ptr(bias), ptr(branch[0]),
                                     ptr(branch[1]), ptr(sc), ptr(out), ptr(bits), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
     assert rc == 0, capi.lib.dab_last_error()
     return out, sc, bits
@@ -72,6 +72,12 @@ def check(gpu, x, wt, v, sw, cout, with_bias, with_affine, special=False):
     # without the outputs that may be left out: the same result
     again, _, _ = down(gpu, x, packed, wt, v, sw, bias, branch, cout, sign=False, want_branch=False)
     assert torch.equal(again.nan_to_num(nan=5e37), out.nan_to_num(nan=5e37))
+    # from the pooled tensor: its values, and the same bounds (the kernel for few pieces does not take it)
+    out, sc, bits = down(gpu, x, packed, wt, v, sw, bias, branch, cout, pooled=s)
+    pgot = sc.reshape(-1, cout).double()
+    pgot = pgot[finite] if special else pgot
+    assert bool(((pgot - exact).abs() <= (x.shape[3] + 8) * 2.0 ** -24 * size + 1e-42).all())
+    assert torch.equal(out.nan_to_num(nan=5e37), ((v[0] * cnt + v[1]) + sc).nan_to_num(nan=5e37)) and torch.equal(bits, dab.pack_mat(out))
     rel = ((got - exact).norm() / exact.norm()).item()
     return rel
 
