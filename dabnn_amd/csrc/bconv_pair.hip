@@ -30,10 +30,51 @@ struct BconvPairArgs {
 constexpr int kPairTiles = 16;  // of a block: four waves with four each
 constexpr int kPairFilterBytes = 9 * 2 * 64 * 16;
 
+// The packed rows of a strip and the filters of both layers, which LDS holds before anything is counted.  They are asked for
+// before the floats: loads come back in the order they were asked for, and the floats are only wanted behind the first tile's counts.
+// (The floats first: 56 x 56 at 256 images 89 us instead of 75, the pooled form 77 instead of 65.  The results are written through
+// the L2: the pass behind this one reads them, and both together take 2 to 4 % less than with streaming stores.)
+struct PairStage {
+    // (at most 800 words: five rows of 160)
+    uint64_t rows[4], filters[5];
+    float coefficient;  // a1, b1, a2, b2: one per thread
+    // src: `words` words of the packed rows; bits, w: LDS
+    __device__ __forceinline__ void fetch(const uint64_t *src, int words, const uint64_t *const (&w)[2], const float *const (&a)[2], const float *const (&b)[2], int tid) {
+        coefficient = (tid < 64 ? a[0] : tid < 128 ? b[0] : tid < 192 ? a[1] : b[1])[tid & 63];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) rows[i] = tid + 256 * i < words ? src[tid + 256 * i] : 0;
+#pragma unroll
+        for (int i = 0; i < 5; ++i) {
+            const int j = tid + 256 * i;
+            filters[i] = j < 64 * 9 ? w[0][j] : j < 2 * 64 * 9 ? w[1][j - 64 * 9] : 0;
+        }
+    }
+    // first: of the row that the first word belongs to; the filters expanded, [layer][tap][32 channels][half][channel] of 16 bytes
+    __device__ __forceinline__ void put(unsigned char *first, int words, int pitch, int width, const FastDiv &div_w, unsigned char *lds, uint32_t (*pop)[64], float *coef, int tid) const {
+        coef[tid] = coefficient;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int j = tid + 256 * i, row = (int)div_w.div(j), col = j - row * width;
+            if (j < words) *reinterpret_cast<uint64_t *>(first + row * pitch + (col + 1) * 8) = rows[i];
+        }
+#pragma unroll
+        for (int i = 0; i < 5; ++i) {
+            const int j = tid + 256 * i;
+            if (j >= 2 * 64 * 9) break;
+            const int layer = j >= 64 * 9, c = j - layer * (64 * 9), ch = c / 9, tap = c - ch * 9;
+            unsigned char *d = lds + layer * kPairFilterBytes + ((tap * 2 + (ch >> 5)) * 64 + (ch & 31)) * 16;
+            *reinterpret_cast<i32x4 *>(d) = lower_half(bitspm((uint32_t)filters[i]));
+            *reinterpret_cast<i32x4 *>(d + 32 * 16) = lower_half(bitspm((uint32_t)(filters[i] >> 32)));
+            atomicAdd(&pop[layer][ch], (uint32_t)__popcll(filters[i]));
+        }
+    }
+};
+
 template <bool SIGN>
 __global__ __launch_bounds__(256, 2) void bconv3x3_pair_kernel(const BconvPairArgs p) {
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     __shared__ uint32_t pop[2][64];  // set bits per filter
+    __shared__ float coef[2][2][64];  // a and b of the layers
     const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5, l32 = lane & 31;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t item = xcd_contiguous_block(blockIdx.x, gridDim.x);  // neighbouring strips share rows: on one XCD
@@ -44,7 +85,11 @@ __global__ __launch_bounds__(256, 2) void bconv3x3_pair_kernel(const BconvPairAr
     unsigned char *const bits1 = bits0 + (p.rows + 4) * pitch;  // of v1: r0 - 1 .. r0 + rows
     const size_t strip = ((size_t)img * p.H + r0) * p.W;       // its first pixel
 
-    // v0 of the wave's tiles, asked for before anything else; 0 where there is nothing (above the image, past its end)
+    const int in0 = r0 >= 2 ? r0 - 2 : 0, in1 = r0 + rows + 2 < p.H ? r0 + rows + 2 : p.H, words = (in1 - in0) * p.W;
+    PairStage stage;
+    stage.fetch(p.x + ((size_t)img * p.H + in0) * p.W, words, p.w, p.a, p.b, tid);
+    __builtin_amdgcn_sched_barrier(0);
+    // v0 of the wave's tiles; 0 where there is nothing (above the image, past its end)
     auto tile_of = [&](int i) { return 2 * wave + (i & 1) + 8 * (i >> 1); };
     const int lane_off = half * 4 * 256 + l32 * 4;
     auto row_off = [](int n, int v) { return (8 * (v / 4) + v % 4) * 256 + n * 128; };
@@ -65,22 +110,7 @@ __global__ __launch_bounds__(256, 2) void bconv3x3_pair_kernel(const BconvPairAr
     const int bit_bytes = (2 * p.rows + 6) * pitch;
     for (int i = tid * 8; i < bit_bytes; i += 256 * 8) *reinterpret_cast<uint64_t *>(bits0 + i) = 0;
     __syncthreads();
-    // the packed input, row by row
-    const int in0 = r0 >= 2 ? r0 - 2 : 0, in1 = r0 + rows + 2 < p.H ? r0 + rows + 2 : p.H;
-    const uint64_t *src = p.x + ((size_t)img * p.H + in0) * p.W;
-    for (int j = tid; j < (in1 - in0) * p.W; j += 256) {
-        const int row = (int)p.div_w.div(j), col = j - row * p.W;
-        *reinterpret_cast<uint64_t *>(bits0 + (in0 - (r0 - 2) + row) * pitch + (col + 1) * 8) = src[j];
-    }
-    // the filters, expanded: [layer][tap][32 channels][half][channel] of 16 bytes
-    for (int j = tid; j < 2 * 64 * 9; j += 256) {
-        const int layer = j >= 64 * 9, c = j - layer * (64 * 9), ch = c / 9, tap = c - ch * 9;
-        const uint64_t word = p.w[layer][c];
-        unsigned char *d = lds + layer * kPairFilterBytes + ((tap * 2 + (ch >> 5)) * 64 + (ch & 31)) * 16;
-        *reinterpret_cast<i32x4 *>(d) = lower_half(bitspm((uint32_t)word));
-        *reinterpret_cast<i32x4 *>(d + 32 * 16) = lower_half(bitspm((uint32_t)(word >> 32)));
-        atomicAdd(&pop[layer][ch], (uint32_t)__popcll(word));
-    }
+    stage.put(bits0 + (in0 - (r0 - 2)) * pitch, words, pitch, p.W, p.div_w, lds, pop, &coef[0][0][0], tid);
     __syncthreads();
 
     auto layer = [&](auto which) __attribute__((always_inline)) {
@@ -89,7 +119,7 @@ __global__ __launch_bounds__(256, 2) void bconv3x3_pair_kernel(const BconvPairAr
 #pragma unroll
         for (int n = 0; n < 2; ++n) {
             init[n] = (float)pop[L][n * 32 + l32];
-            ea[n] = p.a[L][n * 32 + l32], eb[n] = p.b[L][n * 32 + l32];
+            ea[n] = coef[L][0][n * 32 + l32], eb[n] = coef[L][1][n * 32 + l32];
         }
         const unsigned char *filter = lds + L * kPairFilterBytes + lane * 16;
 #pragma unroll
@@ -141,7 +171,7 @@ __global__ __launch_bounds__(256, 2) void bconv3x3_pair_kernel(const BconvPairAr
                         if constexpr (L == 0)
                             val[i][n][v] = r;
                         else
-                            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, r), ro, lane_off, row_off(n, v), kStoreStream);
+                            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, r), ro, lane_off, row_off(n, v), kStoreThrough);
                         if constexpr (L == 0 || SIGN) {
                             const uint64_t mask = __ballot(r > 0.f);
                             word[n] = dab_writelane((uint32_t)mask, 8 * (v / 4) + v % 4, word[n]);
@@ -193,7 +223,7 @@ static int pair_bands(int n, int h, int w) {
 // eight 2x2 windows, in the order of the pooled tensor, one window the four registers of an accumulator quad, so that pooling
 // takes no exchange.  A strip has an even number of rows; the rows above and below it, of which only the sign bits are wanted, are a
 // fifth tile of each wave that no register outlives, so that a strip has eight rows of 56 where the kernel above has seven.
-// 56 x 56 at batch 256, with the block's first layer behind it (bconv_down.hip): 89 + 61 us (one behind the other 164) before, 77 + 47 (131) now.
+// 56 x 56 at batch 256, with the block's first layer behind it (bconv_down.hip): 89 + 61 us (one behind the other 164) as it was, 65 + 46 (118) now.
 struct BconvPairPoolArgs {
     const uint64_t *x;
     const float *shortcut;
@@ -210,6 +240,7 @@ struct BconvPairPoolArgs {
 __global__ __launch_bounds__(256, 2) void bconv3x3_pair_pool_kernel(const BconvPairPoolArgs p) {
     extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
     __shared__ uint32_t pop[2][64];
+    __shared__ float coef[2][2][64];
     const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5, l32 = lane & 31;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t item = xcd_contiguous_block(blockIdx.x, gridDim.x);
@@ -223,7 +254,11 @@ __global__ __launch_bounds__(256, 2) void bconv3x3_pair_pool_kernel(const BconvP
     const __amdgpu_buffer_rsrc_t rs = make_rsrc(p.shortcut + image * 64, p.image_bytes);
     constexpr int kNowhere = (int)0x80000000;  // beyond the image: loads return zero
 
-    // v0, asked for before anything else: the row above the strip and the one below it (pixel j of the two, one behind the other) ...
+    const int in0 = r0 >= 2 ? r0 - 2 : 0, in1 = r0 + rows + 2 < p.H ? r0 + rows + 2 : p.H, words = (in1 - in0) * p.W;
+    PairStage stage;
+    stage.fetch(p.x + image + (size_t)in0 * p.W, words, p.w, p.a, p.b, tid);
+    __builtin_amdgcn_sched_barrier(0);
+    // v0: the row above the strip and the one below it (pixel j of the two, one behind the other) ...
     float edge[2][16];
 #pragma unroll
     for (int v = 0; v < 16; ++v) {
@@ -252,20 +287,7 @@ __global__ __launch_bounds__(256, 2) void bconv3x3_pair_pool_kernel(const BconvP
     const int bit_bytes = (2 * p.rows + 6) * pitch;
     for (int i = tid * 8; i < bit_bytes; i += 256 * 8) *reinterpret_cast<uint64_t *>(bits0 + i) = 0;
     __syncthreads();
-    const int in0 = r0 >= 2 ? r0 - 2 : 0, in1 = r0 + rows + 2 < p.H ? r0 + rows + 2 : p.H;
-    const uint64_t *src = p.x + image + (size_t)in0 * p.W;
-    for (int j = tid; j < (in1 - in0) * p.W; j += 256) {
-        const int row = (int)p.div_w.div(j), col = j - row * p.W;
-        *reinterpret_cast<uint64_t *>(bits0 + (in0 - (r0 - 2) + row) * pitch + (col + 1) * 8) = src[j];
-    }
-    for (int j = tid; j < 2 * 64 * 9; j += 256) {
-        const int layer = j >= 64 * 9, c = j - layer * (64 * 9), ch = c / 9, tap = c - ch * 9;
-        const uint64_t word = p.w[layer][c];
-        unsigned char *d = lds + layer * kPairFilterBytes + ((tap * 2 + (ch >> 5)) * 64 + (ch & 31)) * 16;
-        *reinterpret_cast<i32x4 *>(d) = lower_half(bitspm((uint32_t)word));
-        *reinterpret_cast<i32x4 *>(d + 32 * 16) = lower_half(bitspm((uint32_t)(word >> 32)));
-        atomicAdd(&pop[layer][ch], (uint32_t)__popcll(word));
-    }
+    stage.put(bits0 + (in0 - (r0 - 2)) * pitch, words, pitch, p.W, p.div_w, lds, pop, &coef[0][0][0], tid);
     __syncthreads();
 
     auto value = [](float cnt, float a, float b, float add) {
@@ -280,7 +302,7 @@ __global__ __launch_bounds__(256, 2) void bconv3x3_pair_pool_kernel(const BconvP
 #pragma unroll
         for (int n = 0; n < 2; ++n) {
             init[n] = (float)pop[L][n * 32 + l32];
-            ea[n] = p.a[L][n * 32 + l32], eb[n] = p.b[L][n * 32 + l32];
+            ea[n] = coef[L][0][n * 32 + l32], eb[n] = coef[L][1][n * 32 + l32];
         }
         const unsigned char *filter = lds + L * kPairFilterBytes + lane * 16;
         // counts of M tiles whose lanes' windows are at `window`
@@ -365,7 +387,7 @@ __global__ __launch_bounds__(256, 2) void bconv3x3_pair_pool_kernel(const BconvP
                         }
                         if constexpr (L == 1)
                             __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, sum * 0.25f), ro,
-                                                                  (tile_of(i) * 8 + 2 * q + half) * 256 + l32 * 4 + n * 128, 0, kStoreStream);
+                                                                  (tile_of(i) * 8 + 2 * q + half) * 256 + l32 * 4 + n * 128, 0, kStoreThrough);
                     }
                 if (half == 0 && there[m]) {
                     if constexpr (L == 0)
