@@ -27,17 +27,22 @@ typedef uint32_t u32x4u __attribute__((ext_vector_type(4), aligned(8)));
 
 constexpr int kBeyond = (int)0x80000000;  // an offset outside every descriptor: loads return zero
 
-// kFilterColumns goes with a plain matrix (rows of x in memory order), kFilterRows with windows of images.
-template <FilterLayout L>
+// kFilterColumns goes with a plain matrix (rows of x in memory order), kFilterRows with windows of images.  A plain matrix is read
+// through descriptors too, whose scalar offset walks the depth, so that a unit costs no vector address arithmetic, but for LONG
+// ones: rows of 2^26 bytes, or filters of 2^31, and more.
+template <FilterLayout L, bool LONG>
 struct PixelRows {
     __amdgpu_buffer_rsrc_t rsrc;  // windows: the packed images
     int base, y0, x0;
     const uint64_t *row;          // plain matrix
-    __device__ __forceinline__ void start(const BitGemmArgs &p, long long tile_row, int l32) {
+    __device__ __forceinline__ void start(const BitGemmArgs &p, long long tile_row, int l32, int half) {
         long long r = tile_row + l32;
         r = r < p.g.rows ? r : p.g.rows - 1;
-        if constexpr (L == kFilterColumns) {
+        if constexpr (L == kFilterColumns && LONG) {
             row = p.g.x + r * p.g.x_ld;
+        } else if constexpr (L == kFilterColumns) {
+            rsrc = make_rsrc(p.g.x + tile_row * p.g.x_ld, 0x7fffffffu);
+            base = (int)(r - tile_row) * (int)(p.g.x_ld * 8) + half * 16;
         } else {
             rsrc = make_rsrc(p.g.x, p.x_bytes);
             const uint32_t t = p.div_ow.div((uint32_t)r);
@@ -54,6 +59,16 @@ struct PixelRows {
         if constexpr (L == kFilterColumns) {
             static_assert(CC == 4, "a plain matrix is walked four words at a time");
             const int word = u * 4 + half * 2;
+            if constexpr (!LONG) {
+                if (u * 4 + 4 <= p.g.words) {
+                    load_dwords<4>(d, rsrc, base, u * 32);
+                } else {
+                    const u32x2 v0 = __builtin_amdgcn_raw_buffer_load_b64(rsrc, word < p.g.words ? base : kBeyond, u * 32, 0);
+                    const u32x2 v1 = __builtin_amdgcn_raw_buffer_load_b64(rsrc, word + 1 < p.g.words ? base + 8 : kBeyond, u * 32, 0);
+                    d[0] = v0.x, d[1] = v0.y, d[2] = v1.x, d[3] = v1.y;
+                }
+                return;
+            }
             d[0] = d[1] = d[2] = d[3] = 0u;
             if (word + 1 < p.g.words) {
                 const u32x4u v = *reinterpret_cast<const u32x4u *>(row + word);
@@ -78,9 +93,15 @@ struct PixelRows {
 };
 
 // CC dwords of unit u of filter `col` for one half of the lanes
-template <int CC, FilterLayout L>
+template <int CC, FilterLayout L, bool LONG>
 __device__ __forceinline__ void load_filter(uint32_t (&d)[CC], const BitGemmArgs &p, __amdgpu_buffer_rsrc_t rw, int col, int u, int half) {
-    if constexpr (L == kFilterColumns) {
+    if constexpr (L == kFilterColumns && !LONG) {
+        const int word = u * 4 + half * 2, ld = (int)p.g.w_ld * 8, off = col < p.g.cols ? col * 8 + half * 2 * ld : kBeyond;
+        const bool whole = u * 4 + 4 <= p.g.words;
+        const u32x2 v0 = __builtin_amdgcn_raw_buffer_load_b64(rw, whole || word < p.g.words ? off : kBeyond, u * 4 * ld, 0);
+        const u32x2 v1 = __builtin_amdgcn_raw_buffer_load_b64(rw, whole || word + 1 < p.g.words ? off : kBeyond, u * 4 * ld + ld, 0);
+        d[0] = v0.x, d[1] = v0.y, d[2] = v1.x, d[3] = v1.y;
+    } else if constexpr (L == kFilterColumns) {
         const int word = u * 4 + half * 2;
         const uint64_t *src = p.g.w + (long long)word * p.g.w_ld + col;
         const bool ok = col < p.g.cols;
@@ -117,7 +138,7 @@ enum Epilogue { kStoreCounts, kAddCounts, kAffine, kAffineSign };
 // waves take every fourth unit of the depth each and load their operands straight from memory, kUnitsAhead units at a time; the
 // partial sums meet in LDS.  Both operands +-1 (fp4_core.h).  m512 k72 n3136, accumulating: 7.8 us against 16.2 for the
 // xor/popcount kernel before.
-constexpr int kUnitsAhead = 3;
+constexpr int kUnitsAhead = 2;
 template <int CC, FilterLayout L, int E, int NT, bool LONG>
 __global__ __launch_bounds__(256, 4) void bit_gemm_split_kernel(const BitGemmArgs p) {
     constexpr int CH = 32 * NT, LD = CH + 1;
@@ -127,9 +148,9 @@ __global__ __launch_bounds__(256, 4) void bit_gemm_split_kernel(const BitGemmArg
     const uint32_t block_tile = p.div_col_tiles.div(blockIdx.x);
     const int ch0 = (int)(blockIdx.x - block_tile * p.col_tiles) * CH;
     const long long row0 = (block_tile + p.first_tile) * 32;
-    const __amdgpu_buffer_rsrc_t rw = make_rsrc(p.g.w, L == kFilterRows ? p.w_bytes : 0u);
-    PixelRows<L> px;
-    px.start(p, row0, l32);
+    const __amdgpu_buffer_rsrc_t rw = make_rsrc(p.g.w, L == kFilterRows ? p.w_bytes : 0x7fffffffu);
+    PixelRows<L, LONG> px;
+    px.start(p, row0, l32, half);
 
     // this thread's outputs: channel tid % CH of pixels tid / CH + i * (256 / CH)
     constexpr int RPI = 256 / CH, ROWS = 32 / RPI;
@@ -142,6 +163,17 @@ __global__ __launch_bounds__(256, 4) void bit_gemm_split_kernel(const BitGemmArg
         if (ch_ok) ea = p.g.a[ch], eb = p.g.b[ch];
     const int out_off = ch_ok ? (r0 * (int)p.g.out_ld + ch) * 4 : kBeyond, out_step = RPI * (int)p.g.out_ld * 4;
     auto element = [&](int i) { return p.g.out + (row0 + r0 + i * RPI) * p.g.out_ld + ch; };  // LONG: output i
+    uint32_t a[2][kUnitsAhead][CC], w[2][kUnitsAhead][NT][CC];
+    auto fetch = [&](int slot, int u0) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < kUnitsAhead; ++i)
+            if (u0 + 4 * i < p.units) {
+                px.load(a[slot][i], p, u0 + 4 * i, half);
+#pragma unroll
+                for (int n = 0; n < NT; ++n) load_filter<CC, L, LONG>(w[slot][i][n], p, rw, ch0 + n * 32 + l32, u0 + 4 * i, half);
+            }
+    };
+    fetch(0, wib);
     const float *second = E == kAddCounts ? p.g.out : p.g.shortcut;
     if constexpr (LONG) {
         static_assert(L == kFilterColumns, "a plain matrix");
@@ -154,31 +186,28 @@ __global__ __launch_bounds__(256, 4) void bit_gemm_split_kernel(const BitGemmArg
 #pragma unroll
         for (int i = 0; i < ROWS; ++i) old[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, out_off, i * out_step, 0));
     }
-
     f32x16m acc[NT];
 #pragma unroll
     for (int n = 0; n < NT; ++n)
 #pragma unroll
         for (int v = 0; v < 16; ++v) acc[n][v] = 0.f;
-    for (int u0 = wib; u0 < p.units; u0 += 4 * kUnitsAhead) {
-        uint32_t a[kUnitsAhead][CC], w[kUnitsAhead][NT][CC];
-#pragma unroll
-        for (int i = 0; i < kUnitsAhead; ++i)
-            if (u0 + 4 * i < p.units) {
-                px.load(a[i], p, u0 + 4 * i, half);
-#pragma unroll
-                for (int n = 0; n < NT; ++n) load_filter<CC, L>(w[i][n], p, rw, ch0 + n * 32 + l32, u0 + 4 * i, half);
-            }
+    auto multiply = [&](int slot, int u0) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < kUnitsAhead; ++i)
             if (u0 + 4 * i < p.units) {
 #pragma unroll
                 for (int c = 0; c < CC; ++c) {
-                    const i32x8 av = bitspm1(a[i][c]);
+                    const i32x8 av = bitspm1(a[slot][i][c]);
 #pragma unroll
-                    for (int n = 0; n < NT; ++n) mfma_fp4<32>(acc[n], av, bitspm1(w[i][n][c]));
+                    for (int n = 0; n < NT; ++n) mfma_fp4<32>(acc[n], av, bitspm1(w[slot][i][n][c]));
                 }
             }
+    };
+    for (int u0 = wib; u0 < p.units; u0 += 8 * kUnitsAhead) {
+        fetch(1, u0 + 4 * kUnitsAhead);
+        multiply(0, u0);
+        fetch(0, u0 + 8 * kUnitsAhead);
+        multiply(1, u0 + 4 * kUnitsAhead);
     }
 #pragma unroll
     for (int n = 0; n < NT; ++n)
@@ -226,7 +255,7 @@ __global__ __launch_bounds__(256, NT == 2 ? 3 : 4) void bit_gemm_stream_kernel(c
     const int wib = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int group = (int)p.div_col_tiles.div(blockIdx.x), groups = (int)p.div_col_tiles.div(gridDim.x);
     const int ch0 = ((int)blockIdx.x - group * p.col_tiles) * CH;
-    const __amdgpu_buffer_rsrc_t rw = make_rsrc(p.g.w, L == kFilterRows ? p.w_bytes : 0u);
+    const __amdgpu_buffer_rsrc_t rw = make_rsrc(p.g.w, L == kFilterRows ? p.w_bytes : 0x7fffffffu);
     if (tid < CH) pop[tid] = L == kFilterRows && p.g.extra_word ? extra_bits(p, rw, ch0 + tid) : 0u;
     __syncthreads();
     constexpr int kBatch = 3;  // pieces a thread asks for before it puts the first of them away
@@ -247,7 +276,7 @@ __global__ __launch_bounds__(256, NT == 2 ? 3 : 4) void bit_gemm_stream_kernel(c
                 u = r >> 1, h = r & 1;
             }
             chan[j] = c, slot[j] = (u * CH + c) * 2 + h;
-            if (s < n_pieces) load_filter<CC, L>(d[j], p, rw, ch0 + c, u, h);
+            if (s < n_pieces) load_filter<CC, L, LONG>(d[j], p, rw, ch0 + c, u, h);
         }
 #pragma unroll
         for (int j = 0; j < kBatch; ++j) {
@@ -277,8 +306,8 @@ __global__ __launch_bounds__(256, NT == 2 ? 3 : 4) void bit_gemm_stream_kernel(c
 
     for (long long tile = (long long)group * 4 + wib; tile < p.row_tiles; tile += (long long)groups * 4) {
         const long long row0 = tile * 32;
-        PixelRows<L> px;
-        px.start(p, row0, l32);
+        PixelRows<L, LONG> px;
+        px.start(p, row0, l32, half);
         uint32_t a[4][CC];
 #pragma unroll
         for (int i = 0; i < 4; ++i)
@@ -545,7 +574,7 @@ int bit_gemm(const char *fn, const BitGemm &g, FilterLayout layout, hipStream_t 
     if (layout == kFilterColumns && takes_direct(g)) return g.accumulate ? launch_direct<kAddCounts>(p, stream) : launch_direct<kStoreCounts>(p, stream);
     if (layout == kFilterColumns) {
         p.units = (g.words + 3) / 4, p.chunks = p.units;
-        if (g.out_ld >= kLongRow)
+        if (g.out_ld >= kLongRow || g.x_ld * 8 >= (1ll << 26) || g.words * g.w_ld * 8 >= (1ll << 31))
             return g.accumulate ? launch_bit_gemm<4, kFilterColumns, kAddCounts, true>(fn, p, stream)
                                 : launch_bit_gemm<4, kFilterColumns, kStoreCounts, true>(fn, p, stream);
         return g.accumulate ? launch_bit_gemm<4, kFilterColumns, kAddCounts>(fn, p, stream)

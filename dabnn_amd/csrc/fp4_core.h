@@ -82,17 +82,17 @@ __device__ __forceinline__ constexpr int fp4_row(int kb, int v) {
 
 // N dwords through a buffer descriptor / from LDS
 template <int N>
-__device__ __forceinline__ void load_dwords(uint32_t (&d)[N], __amdgpu_buffer_rsrc_t r, int off) {
+__device__ __forceinline__ void load_dwords(uint32_t (&d)[N], __amdgpu_buffer_rsrc_t r, int off, int scalar = 0) {
     static_assert(N == 1 || N == 2 || N % 4 == 0, "whole loads");
     if constexpr (N == 1) {
-        d[0] = __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, 0);
+        d[0] = __builtin_amdgcn_raw_buffer_load_b32(r, off, scalar, 0);
     } else if constexpr (N == 2) {
-        const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0);
+        const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(r, off, scalar, 0);
         d[0] = v.x, d[1] = v.y;
     } else {
 #pragma unroll
         for (int i = 0; i < N / 4; ++i) {
-            const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r, off, i * 16, 0);
+            const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r, off, scalar + i * 16, 0);
             d[4 * i] = v.x, d[4 * i + 1] = v.y, d[4 * i + 2] = v.z, d[4 * i + 3] = v.w;
         }
     }
