@@ -135,14 +135,14 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t tile_rsrc(const float *t, cons
 enum Epilogue { kStoreCounts, kAddCounts, kAffine, kAffineSign };
 
 // Few tiles, or a depth that does not fit LDS as filters: a block is one tile of 32 pixels x 32 * NT channels, its four
-// waves take every fourth unit of the depth each and load their operands straight from memory, kUnitsAhead units at a time; the
-// partial sums meet in LDS.  Both operands +-1 (fp4_core.h).  m512 k72 n3136, accumulating: 7.8 us against 16.2 for the
-// xor/popcount kernel before.
+// (eight) waves take every fourth (eighth) unit of the depth each and load their operands straight from memory, kUnitsAhead units while
+// as many are multiplied; the partial sums meet in LDS.  Both operands +-1 (fp4_core.h).  Bound by their expansion: m512 k72 n3136,
+// accumulating, 8.7 us (9.8 with three units asked for at a time and none while they were multiplied).
 constexpr int kUnitsAhead = 2;
-template <int CC, FilterLayout L, int E, int NT, bool LONG>
-__global__ __launch_bounds__(256, 4) void bit_gemm_split_kernel(const BitGemmArgs p) {
+template <int CC, FilterLayout L, int E, int NT, int WAVES, bool LONG>
+__global__ __launch_bounds__(64 * WAVES, 4) void bit_gemm_split_kernel(const BitGemmArgs p) {
     constexpr int CH = 32 * NT, LD = CH + 1;
-    __shared__ float part[4][32 * LD];
+    __shared__ float part[WAVES][32 * LD];
     const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5, l32 = lane & 31;
     const int wib = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t block_tile = p.div_col_tiles.div(blockIdx.x);
@@ -153,7 +153,7 @@ __global__ __launch_bounds__(256, 4) void bit_gemm_split_kernel(const BitGemmArg
     px.start(p, row0, l32, half);
 
     // this thread's outputs: channel tid % CH of pixels tid / CH + i * (256 / CH)
-    constexpr int RPI = 256 / CH, ROWS = 32 / RPI;
+    constexpr int RPI = 64 * WAVES / CH, ROWS = 32 / RPI;
     const int ch = ch0 + tid % CH, r0 = tid / CH;
     const bool ch_ok = ch < p.g.cols;
     float old[ROWS], ea = 0.f, eb = 0.f;
@@ -167,10 +167,10 @@ __global__ __launch_bounds__(256, 4) void bit_gemm_split_kernel(const BitGemmArg
     auto fetch = [&](int slot, int u0) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < kUnitsAhead; ++i)
-            if (u0 + 4 * i < p.units) {
-                px.load(a[slot][i], p, u0 + 4 * i, half);
+            if (u0 + WAVES * i < p.units) {
+                px.load(a[slot][i], p, u0 + WAVES * i, half);
 #pragma unroll
-                for (int n = 0; n < NT; ++n) load_filter<CC, L, LONG>(w[slot][i][n], p, rw, ch0 + n * 32 + l32, u0 + 4 * i, half);
+                for (int n = 0; n < NT; ++n) load_filter<CC, L, LONG>(w[slot][i][n], p, rw, ch0 + n * 32 + l32, u0 + WAVES * i, half);
             }
     };
     fetch(0, wib);
@@ -194,7 +194,7 @@ __global__ __launch_bounds__(256, 4) void bit_gemm_split_kernel(const BitGemmArg
     auto multiply = [&](int slot, int u0) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < kUnitsAhead; ++i)
-            if (u0 + 4 * i < p.units) {
+            if (u0 + WAVES * i < p.units) {
 #pragma unroll
                 for (int c = 0; c < CC; ++c) {
                     const i32x8 av = bitspm1(a[slot][i][c]);
@@ -203,11 +203,11 @@ __global__ __launch_bounds__(256, 4) void bit_gemm_split_kernel(const BitGemmArg
                 }
             }
     };
-    for (int u0 = wib; u0 < p.units; u0 += 8 * kUnitsAhead) {
-        fetch(1, u0 + 4 * kUnitsAhead);
+    for (int u0 = wib; u0 < p.units; u0 += 2 * WAVES * kUnitsAhead) {
+        fetch(1, u0 + WAVES * kUnitsAhead);
         multiply(0, u0);
-        fetch(0, u0 + 8 * kUnitsAhead);
-        multiply(1, u0 + 4 * kUnitsAhead);
+        fetch(0, u0 + 2 * WAVES * kUnitsAhead);
+        multiply(1, u0 + WAVES * kUnitsAhead);
     }
 #pragma unroll
     for (int n = 0; n < NT; ++n)
@@ -222,7 +222,9 @@ __global__ __launch_bounds__(256, 4) void bit_gemm_split_kernel(const BitGemmArg
         const int row = r0 + i * RPI;
         const long long r = row0 + row;
         const int o = row * LD + tid % CH;
-        float v = half_depth - 0.5f * ((part[0][o] + part[1][o]) + (part[2][o] + part[3][o])) + (float)extra;
+        float sum = (part[0][o] + part[1][o]) + (part[2][o] + part[3][o]);
+        if constexpr (WAVES == 8) sum = sum + ((part[4][o] + part[5][o]) + (part[6][o] + part[7][o]));
+        float v = half_depth - 0.5f * sum + (float)extra;
         if constexpr (E == kAddCounts) v = old[i] + v;
         if constexpr (E == kAffine || E == kAffineSign) {
 #pragma clang fp contract(off)
@@ -516,14 +518,20 @@ static int launch_bit_gemm(const char *fn, BitGemmArgs &p, hipStream_t s) {
         p.div_col_tiles = FastDiv((uint32_t)p.col_tiles);
         const long long blocks = p.row_tiles * p.col_tiles;
         if (blocks >= (1ll << 31)) return fail(DAB_EUNSUPPORTED, "%s: too many work units", fn);
+        // Eight waves where they have depth for it and a CU no more than two blocks: 200 x 1000 x 150 5.5 -> 5.0 us, 300 x 300 x 100 4.5 ->
+        // 4.2, 1 x 14 x 14 x 256 -> 256, 5 x 5, 4.1 -> 3.7, at 8 images 5.3 -> 5.1; 64 x 12000 x 50 (750 blocks) 5.0 -> 5.1, 60 x 14 x 14 x
+        // 256 -> 40, 5 x 5 (736) 6.1 -> 6.3, 4 x 28 x 28 x 192 -> 192, 3 x 3 (nine units) 4.1 -> 4.2.
+        const bool eight = p.units >= 12 && blocks <= simd_count() / 2;
         const long long most = kMostBlocks / p.col_tiles > 1 ? kMostBlocks / p.col_tiles : 1;  // row tiles of a launch
         for (p.first_tile = 0; p.first_tile < p.row_tiles; p.first_tile += most) {
             const long long tiles = p.row_tiles - p.first_tile < most ? p.row_tiles - p.first_tile : most;
             const dim3 grid((unsigned)(tiles * p.col_tiles));
             if (split_ch == 64)
-                hipLaunchKernelGGL((bit_gemm_split_kernel<CC, L, E, 2, LONG>), grid, dim3(256), 0, s, p);
+                hipLaunchKernelGGL((bit_gemm_split_kernel<CC, L, E, 2, 4, LONG>), grid, dim3(256), 0, s, p);
+            else if (eight)
+                hipLaunchKernelGGL((bit_gemm_split_kernel<CC, L, E, 1, 8, LONG>), grid, dim3(512), 0, s, p);
             else
-                hipLaunchKernelGGL((bit_gemm_split_kernel<CC, L, E, 1, LONG>), grid, dim3(256), 0, s, p);
+                hipLaunchKernelGGL((bit_gemm_split_kernel<CC, L, E, 1, 4, LONG>), grid, dim3(256), 0, s, p);
         }
     }
     DAB_LAUNCH_CHECK();
