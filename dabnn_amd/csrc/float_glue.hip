@@ -393,6 +393,144 @@ __global__ __launch_bounds__(256) void fconv_kernel(const FconvArgs p) {
     }
 }
 
+// 3x3 windows over three-channel images to up to 64 channels (a first layer): 27 depths, too few to stage.  Bound by what it writes:
+// a wave takes 32 pixels x all channels, its filters stay in registers and each lane fetches five taps of its pixel with one 12-byte load each
+// -- the lower half of the lanes taps 0..4, the upper half 5..8 and 4 -- while the tile before is multiplied, fourteen instructions of two depths
+// per 32 channels.  us, the tile kernel / this one: 3 -> 64 over 32 x 32, 128 images, with PRelu and sign bits,
+// into slices 15.2 / 12.2; 3 -> 32, stride 2, over 224 x 224, 1 / 6 / 20 / 100 / 256 images 4.7 / 4.1, 6.7 / 6.3, 14.0 / 10.8, 51 / 42, 145 / 99.
+// Every second (fourth) step has a sum of its own, so that the error against 64 bits is no larger than the tile kernels', which split the
+// depth of small problems over four waves.
+template <int NT, bool STREAM>
+__global__ __launch_bounds__(256, NT == 2 ? 3 : 4) void fconv_rgb3x3_kernel(const FconvArgs p) {
+    constexpr int STEPS = 14, SUMS = NT == 1 ? 4 : 2;
+    typedef float f32x3 __attribute__((ext_vector_type(3)));
+    const int lane = threadIdx.x & 63, half = lane >> 5, l32 = lane & 31;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int tiles = (p.M + 31) / 32, step = (int)gridDim.x * 4;
+    __shared__ float filters[NT * 32 * 27];
+    auto tap_of = [&](int j) { return half == 0 ? j : j < 4 ? 5 + j : 4; };
+
+    f32x3 x[5], next[5];
+    auto fetch = [&](f32x3 (&v)[5], int tile) __attribute__((always_inline)) {
+        const int m0 = tile * 32, img0 = (int)p.div_oh.div(p.div_ow.div((uint32_t)m0)), img_elems = p.h * p.wd * 3;
+        const long long left = (long long)(p.n - img0) * img_elems * 4;
+        const auto x_rsrc = make_rsrc(p.x + (size_t)img0 * img_elems, (uint32_t)(left < kOobRow ? left : kOobRow));
+        const int pix = m0 + l32 < p.M ? m0 + l32 : p.M - 1;
+        const uint32_t t0 = p.div_ow.div((uint32_t)pix);
+        const int ox = pix - (int)t0 * p.ow, img = (int)p.div_oh.div(t0), oy = (int)t0 - img * p.oh;
+        const int y0 = oy * p.stride_h - p.pad_h, x0 = ox * p.stride_w - p.pad_w;
+        const int base = ((img - img0) * p.h + y0) * p.wd + x0;
+#pragma unroll
+        for (int j = 0; j < 5; ++j) {
+            const int tap = tap_of(j), ty = (tap * 11) >> 5, dy = ty * p.dil_h, dx = (tap - 3 * ty) * p.dil_w;
+            const bool ok = (unsigned)(y0 + dy) < (unsigned)p.h && (unsigned)(x0 + dx) < (unsigned)p.wd;
+            v[j] = __builtin_bit_cast(f32x3, __builtin_amdgcn_raw_buffer_load_b96(x_rsrc, ok ? (base + dy * p.wd + dx) * 12 : (int)kOob, 0, 0));
+        }
+    };
+    int tile = (int)blockIdx.x * 4 + wave;
+    const bool any = tile < tiles;
+    if (any) fetch(x, tile);
+    for (int i = threadIdx.x; i < NT * 32 * 27; i += 256) filters[i] = i < p.cout * 27 ? p.w[i] : 0.f;
+    __syncthreads();
+    if (!any) return;
+
+    // the filters in the order of the taps: element c of load j, then what load 4 leaves for the two halves (elements 0, 1 and 2)
+    float w[STEPS][NT], bias[NT], fa[NT], fb[NT], slope[NT];
+    int out_lane[NT];
+#pragma unroll
+    for (int n = 0; n < NT; ++n) {
+        const int co = n * 32 + l32;
+        const bool ok = co < p.cout;
+#pragma unroll
+        for (int s = 0; s < STEPS; ++s) {
+            const int place = s < 12 ? tap_of(s / 3) * 3 + s % 3 : s == 12 ? (half ? 14 : 12) : 13;
+            w[s][n] = s == 13 && half ? 0.f : filters[co * 27 + place];
+        }
+        bias[n] = ok && p.bias ? p.bias[co] : 0.f;
+        fa[n] = ok && p.aff_a ? p.aff_a[co] : 0.f, fb[n] = ok && p.aff_a ? p.aff_b[co] : 0.f;
+        slope[n] = ok && p.slope ? p.slope[p.slope_n == 1 ? 0 : co] : 0.f;
+        out_lane[n] = ok ? co * 4 + 4 * half * p.out_ld * 4 : (int)kOob;
+    }
+
+    using Prelu = std::integral_constant<int, 2>;
+    using T = std::true_type;
+    using F = std::false_type;
+    for (;; tile += step) {
+        const bool more = tile + step < tiles;
+        if (more) fetch(next, tile + step);
+        f32x16 acc[NT], part[SUMS][NT];
+#pragma unroll
+        for (int i = 0; i < SUMS; ++i)
+#pragma unroll
+            for (int n = 0; n < NT; ++n)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) part[i][n][e] = 0.f;
+#pragma unroll
+        for (int s = 0; s < STEPS; ++s) {
+            const float a = s < 12 ? x[s / 3][s % 3] : s == 12 ? (half ? x[4][2] : x[4][0]) : (half ? 0.f : x[4][1]);
+#pragma unroll
+            for (int n = 0; n < NT; ++n) part[s % SUMS][n] = __builtin_amdgcn_mfma_f32_32x32x2f32(a, w[s][n], part[s % SUMS][n], 0, 0, 0);
+        }
+#pragma unroll
+        for (int n = 0; n < NT; ++n)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                acc[n][e] = part[0][n][e] + part[1][n][e];
+                if constexpr (SUMS == 4) acc[n][e] = acc[n][e] + (part[2][n][e] + part[3][n][e]);
+            }
+        const int m0 = tile * 32, rows = p.M - m0 < 32 ? p.M - m0 : 32;
+        const auto o_rsrc = make_rsrc(p.out + (size_t)m0 * p.out_ld, (uint32_t)((rows - 1) * p.out_ld + p.cout) * 4u);
+        // accumulator element e of lane l: pixel 8 * (e / 4) + 4 * (l / 32) + e % 4, channel l % 32
+        auto emit = [&](auto has_bias, auto has_affine, auto act) __attribute__((always_inline)) {
+#pragma unroll
+            for (int n = 0; n < NT; ++n) {
+                uint32_t signs = 0;
+                int lane_off = out_lane[n];
+                asm volatile("" : "+v"(lane_off));  // sixteen offsets kept from tile to tile would not fit
+                static_for<16>([&](auto e_) {
+#pragma clang fp contract(off)
+                    constexpr int e = decltype(e_)::value, row = 8 * (e / 4) + e % 4;
+                    float v = acc[n][e];
+                    if constexpr (decltype(has_bias)::value) v = v + bias[n];
+                    if constexpr (decltype(has_affine)::value) {
+                        v = fa[n] * v;
+                        v = v + fb[n];
+                    }
+                    if constexpr (std::is_same<decltype(act), Prelu>::value)
+                        v = v < 0.f ? v * slope[n] : v;
+                    else if constexpr (decltype(act)::value)
+                        v = v < 0.f ? 0.f : v;  // std::max(v, 0.f): a NaN stays
+                    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), o_rsrc, lane_off + row * p.out_ld * 4, 0, STREAM ? kStoreStream : kStoreThrough);
+                    if constexpr (std::is_same<decltype(act), Prelu>::value) {
+                        const uint64_t mask = __ballot(v > 0.f);
+                        signs = dab_writelane((uint32_t)mask, row, signs);
+                        signs = dab_writelane((uint32_t)(mask >> 32), row + 4, signs);
+                    }
+                });
+                if constexpr (std::is_same<decltype(act), Prelu>::value)
+                    if (p.bits && half == 0 && l32 < rows && n * 32 < p.cout) p.bits[(size_t)(m0 + l32) * p.bits_ld + n] = signs;
+            }
+        };
+        auto emit_act = [&](auto act) __attribute__((always_inline)) {
+            switch ((p.bias ? 2 : 0) | (p.aff_a ? 1 : 0)) {
+                case 0: emit(F{}, F{}, act); break;
+                case 1: emit(F{}, T{}, act); break;
+                case 2: emit(T{}, F{}, act); break;
+                default: emit(T{}, T{}, act); break;
+            }
+        };
+        if (p.slope)
+            emit_act(Prelu{});
+        else if (p.relu)
+            emit_act(T{});
+        else
+            emit_act(F{});
+        if (!more) break;
+#pragma unroll
+        for (int j = 0; j < 5; ++j) x[j] = next[j];
+    }
+}
+
 // AvePool 2x2 stride 2 + 1x1 convolution over K input channels (a multiple of 64; built for 64) when the launch is
 // bound by the input it reads.  fconv_kernel<..., POOL> pools a tile's pixels once per column tile and fetches a
 // pixel's channels slice by slice.  Here a block pools its BM pixels once, whole pixels at a time (4K contiguous bytes
@@ -1010,6 +1148,25 @@ static int fconv_impl(const char *fn, const float *x, int n, int h, int w, int c
     if (slice == nullptr && M <= 8 && kh == 1 && kw == 1 && pad_h == 0 && pad_w == 0 && stride_h == 1 && stride_w == 1 && vec4 && cout >= 64) {
         // a matrix-vector product (the classifier at small batch): one wave per output channel
         hipLaunchKernelGGL(fconv_gemv_kernel, dim3((unsigned)((cout + 3) / 4)), dim3(256), 0, s, a);
+    } else if (c == 3 && kh == 3 && kw == 3 && cout <= 64 && M >= (cout <= 32 ? 8192 : 10000)) {
+        // (below, the split depth of the small tiles: 8192 pixels 3 -> 64 5.0 us against 5.6, 16 384 7.9 against 5.7.)  Two waves a SIMD, equal shares; results of
+        // 256 MB and more, which nothing holds for their reader, stream past the caches (411 MB: 99 us against 115 written through; 160 MB
+        // 42 either way, 33 MB in slices 13.0 against 12.2)
+        const long long tiles = (M + 31) / 32, most = 2ll * simd_count();
+        const long long rounds = (tiles + most - 1) / most;
+        const dim3 grid((unsigned)((tiles + 4 * rounds - 1) / (4 * rounds)));
+        const bool stream_out = M * cout * 4 >= (256ll << 20);
+        auto launch = [&](auto nt) {
+            constexpr int NT = decltype(nt)::value;
+            if (stream_out)
+                hipLaunchKernelGGL((fconv_rgb3x3_kernel<NT, true>), grid, dim3(256), 0, s, a);
+            else
+                hipLaunchKernelGGL((fconv_rgb3x3_kernel<NT, false>), grid, dim3(256), 0, s, a);
+        };
+        if (cout <= 32)
+            launch(std::integral_constant<int, 1>{});
+        else
+            launch(std::integral_constant<int, 2>{});
     } else if (big_tiles < simd_count() / 4 && vec3 && (M + 63) / 64 >= simd_count() / 8) {
         // a three-channel image too small for 128-pixel tiles (the stem at batch 1): 64-pixel tiles keep the
         // one-load-per-tap loader and still give most CUs a block
