@@ -472,9 +472,14 @@ static int launch_bit_gemm(const char *fn, BitGemmArgs &p, hipStream_t s) {
         const int cus = simd_count() / 4, by_registers = ch == 64 ? 3 : 4, by_lds = (int)(160 * 1024 / (w.lds + 1024));
         const long long most = (long long)cus * (by_lds < by_registers ? by_lds : by_registers) / w.col_tiles, want = (p.row_tiles + 3) / 4;
         w.groups = want < most ? want : most < 1 ? 1 : most;
-        const long long per_wave = (p.row_tiles + w.groups * 4 - 1) / (w.groups * 4);
-        w.groups = (p.row_tiles + 4 * per_wave - 1) / (4 * per_wave);
-        w.rounds = (w.groups * w.col_tiles + cus - 1) / cus * per_wave;
+        // Equal shares, on as few blocks as that takes -- but for windows whose fullest CU would then walk a sixteenth more tiles than the
+        // average one, where all resident blocks share them out: 64 x 28 x 28 x 192 -> 192, 3 x 3, 17.4 -> 15.2 us (12 tiles against 9.2),
+        // 50 x 30 x 30 x 256 -> 256, 5 x 5, 49 -> 44 (12 / 11), 256 x 32 x 32 x 128 -> 64 into slices 23.3 -> 21.3 (9 / 8); with 128 images,
+        // 4 tiles either way, 13.5 -> 15.  40 random layers 1.05 times as fast, 0.98 to 1.2; with one to three words a filter, bound by
+        // the stores, 0.96 to 1.  (Plain matrices 0.9 to 1.2 times as fast: they keep equal shares.)
+        const long long per_wave = (p.row_tiles + w.groups * 4 - 1) / (w.groups * 4), equal = (p.row_tiles + 4 * per_wave - 1) / (4 * per_wave);
+        w.rounds = (equal * w.col_tiles + cus - 1) / cus * per_wave;
+        if (L == kFilterColumns || p.g.words < 4 || w.rounds * 64 * cus < 17 * p.row_tiles * w.col_tiles) w.groups = equal;
         return w;
     };
     // 64 channels a wave for plain matrices (m128 k18 n50176: 12.6 us against 16.4).  For windows, whose lanes spend more on addresses
