@@ -67,6 +67,8 @@ SIGNATURES = {
     "dab_ave_pool2_fconv1x1": (_i, [_vp, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _i, _i, _vp, _vp, _vp]),
     "dab_max_pool2_fconv1x1": (_i, [_vp] + [_i] * 4 + [_vp] * 4 + [_i, _vp, _i, _i, _vp, _i64, _vp, _i64, _vp]),
     "dab_max_pool2_fconv1x1_takes": (_i, [_i] * 5),
+    "dab_fconv_affine_relu_copy": (_i, [_vp, _i, _i, _i, _i, _vp, _vp, _vp, _vp] + [_i] * 10 + [_vp, _vp, _vp]),
+    "dab_global_ave_pool_fconv1x1_copy": (_i, [_vp, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _i, _i, _vp, _vp, _vp, _vp]),
     "dab_global_ave_pool_fconv1x1": (_i, [_vp, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _i, _i, _vp, _vp, _vp]),
     "dab_global_ave_pool_fconv1x1_takes": (_i, [_i] * 5),
     "dab_fconv_maxpool": (_i, [_vp, _i, _i, _i, _i, _vp, _vp, _vp, _vp] + [_i] * 10 + [_vp, _vp, _vp, _vp]),

@@ -47,6 +47,7 @@ struct FconvArgs {
     const float *aff_b;
     float *out;
     float *pooled;  // averages: the pooled input, written as a side product
+    float *copy = nullptr;  // the result a second time (pinned host memory), by the kernels at the end of a net; null: not
     int n, h, wd, c;
     int kw, dil_h, dil_w;
     int pad_h, pad_w, stride_h, stride_w;
@@ -105,6 +106,7 @@ __global__ __launch_bounds__(256) void fconv_kernel(const FconvArgs p) {
     const int rows_n = p.cout - n0 < BN ? p.cout - n0 : BN, rows_m = p.M - m0 < BM ? p.M - m0 : BM;
     const auto w_rsrc = make_rsrc(p.w + (size_t)n0 * p.K, (uint32_t)rows_n * p.K * 4u);
     const auto o_rsrc = make_rsrc(p.out + (size_t)m0 * p.out_ld, (uint32_t)((rows_m - 1) * p.out_ld + p.cout) * 4u);
+    const auto c_rsrc = make_rsrc(p.copy + (p.copy ? (size_t)m0 * p.out_ld : 0), p.copy ? (uint32_t)((rows_m - 1) * p.out_ld + p.cout) * 4u : 0u);
 
     // loader: depth l_k of the slice, tile rows l_r + RP*i
     const int l_k = tid % LK, l_r = tid / LK;
@@ -299,6 +301,8 @@ __global__ __launch_bounds__(256) void fconv_kernel(const FconvArgs p) {
         else if constexpr (decltype(act)::value)
             v = v < 0.f ? 0.f : v;  // std::max(v, 0.f): a NaN stays
         __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), o_rsrc, (int)off, 0, 0);
+        if constexpr (KSPLIT > 1 && POOL == Pool2::none)
+            if (p.copy) __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), c_rsrc, (int)off, 0, 0);
         return v;
     };
     // The sign bits of a 32 x 32 tile: element e of all lanes is channels 0..31 of two rows, a dword of each, which is
@@ -824,6 +828,7 @@ __global__ __launch_bounds__(256) void global_avepool_gemv_kernel(const FconvArg
             }
             if (p.relu) v = v < 0.f ? 0.f : v;
             p.out[(size_t)img * p.cout + co] = v;
+            if (p.copy) p.copy[(size_t)img * p.cout + co] = v;
         }
     }
 }
@@ -1081,7 +1086,7 @@ struct PreluSlice {
 
 static int fconv_impl(const char *fn, const float *x, int n, int h, int w, int c, const float *wgt, const float *bias,
                       const float *aff_a, const float *aff_b, int relu, int kh, int kw, int pad_h, int pad_w, int stride_h,
-                      int stride_w, int dil_h, int dil_w, int cout, float *out, dab_stream_t stream, const PreluSlice *slice = nullptr) {
+                      int stride_w, int dil_h, int dil_w, int cout, float *out, dab_stream_t stream, const PreluSlice *slice = nullptr, float *copy = nullptr) {
     using namespace dab;
     DAB_REQUIRE(x && wgt && out, "%s: null pointer", fn);
     DAB_REQUIRE(n > 0 && h > 0 && w > 0 && c > 0 && kh > 0 && kw > 0 && cout > 0, "%s: non-positive dimension", fn);
@@ -1124,8 +1129,12 @@ static int fconv_impl(const char *fn, const float *x, int n, int h, int w, int c
     } else {
         const int rc = fconv_c32_try(x, n, h, w, c, wgt, bias, aff_a, aff_b, relu, kh, kw, pad_h, pad_w, stride_h, stride_w,
                                      dil_h, dil_w, cout, a.oh, a.ow, out, s);
-        if (rc != 0) return rc < 0 ? rc : DAB_OK;
+        if (rc < 0) return rc;
+        if (rc != 0) return copy ? dab_copy_f32(copy, out, M * cout, stream) : DAB_OK;
     }
+    // the copy by the kernel itself, where that is the one for few tiles; up to eight pixels, where other kernels run too, by a launch
+    bool copied = false;
+    a.copy = M > 8 ? copy : nullptr;
     // without padding every tap of every window is inside the image and the bounds test is dropped
     const bool padded = pad_h != 0 || pad_w != 0 || (a.oh - 1) * stride_h + (kh - 1) * dil_h >= h ||
                         (a.ow - 1) * stride_w + (kw - 1) * dil_w >= w;
@@ -1133,6 +1142,7 @@ static int fconv_impl(const char *fn, const float *x, int n, int h, int w, int c
     const long long big_tiles = ((M + 127) / 128) * ((cout + bn - 1) / bn);
 #define DAB_FCONV_LAUNCH(BM, BN, SK, KSPLIT, CV)                                                         \
     do {                                                                                                 \
+        copied = KSPLIT > 1 && a.copy != nullptr;                                                        \
         const dim3 grid((unsigned)((M + BM - 1) / BM), (unsigned)((cout + BN - 1) / BN));                \
         if (padded)                                                                                      \
             hipLaunchKernelGGL((fconv_kernel<BM, BN, SK, KSPLIT, true, CV>), grid, dim3(256), 0, s, a);  \
@@ -1209,6 +1219,7 @@ static int fconv_impl(const char *fn, const float *x, int n, int h, int w, int c
     }
 #undef DAB_FCONV_LAUNCH
     DAB_LAUNCH_CHECK();
+    if (copy && !copied) return dab_copy_f32(copy, out, M * cout, stream);
     return DAB_OK;
 }
 
@@ -1221,11 +1232,10 @@ extern "C" int dab_global_ave_pool_fconv1x1_takes(int n, int h, int w, int c, in
            c / 4 <= kGlobalPoolDepth4 && cout >= 64;
 }
 
-extern "C" int dab_global_ave_pool_fconv1x1(const float *x, int n, int h, int w, int c, const float *wgt, const float *bias,
-                                            const float *aff_a, const float *aff_b, int relu, int cout, float *pooled,
-                                            float *out, dab_stream_t stream) {
+static int global_ave_pool_fconv1x1(const char *fn, const float *x, int n, int h, int w, int c, const float *wgt, const float *bias,
+                                    const float *aff_a, const float *aff_b, int relu, int cout, float *pooled, float *out, float *copy,
+                                    dab_stream_t stream) {
     using namespace dab;
-    const char *fn = "dab_global_ave_pool_fconv1x1";
     DAB_REQUIRE(x && wgt && pooled && out, "%s: null pointer", fn);
     DAB_REQUIRE(n > 0 && h > 0 && w > 0 && c > 0 && cout > 0, "%s: non-positive dimension", fn);
     DAB_REQUIRE((aff_a == nullptr) == (aff_b == nullptr), "%s: affine needs both coefficient vectors", fn);
@@ -1234,7 +1244,7 @@ extern "C" int dab_global_ave_pool_fconv1x1(const float *x, int n, int h, int w,
         return fail(DAB_EUNSUPPORTED, "%s: needs n <= 8, h * w <= %d, c %% 4 == 0, c <= %d, cout >= 64 and 16-byte aligned buffers", fn,
                     kGlobalPoolTaps, 4 * kGlobalPoolDepth4);
     FconvArgs a = {};
-    a.x = x, a.w = wgt, a.bias = bias, a.aff_a = aff_a, a.aff_b = aff_b, a.relu = relu, a.out = out, a.pooled = pooled;
+    a.x = x, a.w = wgt, a.bias = bias, a.aff_a = aff_a, a.aff_b = aff_b, a.relu = relu, a.out = out, a.pooled = pooled, a.copy = copy;
     a.n = n, a.h = h, a.wd = w, a.c = c, a.cout = cout, a.K = c, a.M = n;
     const unsigned blocks = (unsigned)((cout + 4 * kGlobalPoolChannels - 1) / (4 * kGlobalPoolChannels));
     const dim3 grid(blocks, (unsigned)n);
@@ -1247,6 +1257,19 @@ extern "C" int dab_global_ave_pool_fconv1x1(const float *x, int n, int h, int w,
         hipLaunchKernelGGL((global_avepool_gemv_kernel<4, 32>), grid, dim3(256), 0, s, a);
     DAB_LAUNCH_CHECK();
     return DAB_OK;
+}
+
+extern "C" int dab_global_ave_pool_fconv1x1(const float *x, int n, int h, int w, int c, const float *wgt, const float *bias,
+                                            const float *aff_a, const float *aff_b, int relu, int cout, float *pooled,
+                                            float *out, dab_stream_t stream) {
+    return global_ave_pool_fconv1x1("dab_global_ave_pool_fconv1x1", x, n, h, w, c, wgt, bias, aff_a, aff_b, relu, cout, pooled, out, nullptr, stream);
+}
+
+extern "C" int dab_global_ave_pool_fconv1x1_copy(const float *x, int n, int h, int w, int c, const float *wgt, const float *bias,
+                                                 const float *aff_a, const float *aff_b, int relu, int cout, float *pooled,
+                                                 float *out, float *copy, dab_stream_t stream) {
+    DAB_REQUIRE(copy, "dab_global_ave_pool_fconv1x1_copy: null pointer");
+    return global_ave_pool_fconv1x1("dab_global_ave_pool_fconv1x1_copy", x, n, h, w, c, wgt, bias, aff_a, aff_b, relu, cout, pooled, out, copy, stream);
 }
 
 extern "C" int dab_max_pool2_fconv1x1_takes(int n, int h, int w, int c, int cout) {
@@ -1396,6 +1419,15 @@ extern "C" int dab_fconv_affine_relu(const float *x, int n, int h, int w, int c,
                                      dab_stream_t stream) {
     return fconv_impl("dab_fconv_affine_relu", x, n, h, w, c, wgt, bias, a, b, relu, kh, kw, pad_h, pad_w, stride_h,
                       stride_w, dil_h, dil_w, cout, out, stream);
+}
+
+extern "C" int dab_fconv_affine_relu_copy(const float *x, int n, int h, int w, int c, const float *wgt, const float *bias,
+                                     const float *a, const float *b, int relu, int kh, int kw, int pad_h, int pad_w,
+                                     int stride_h, int stride_w, int dil_h, int dil_w, int cout, float *out, float *copy,
+                                     dab_stream_t stream) {
+    DAB_REQUIRE(copy, "dab_fconv_affine_relu_copy: null pointer");
+    return fconv_impl("dab_fconv_affine_relu_copy", x, n, h, w, c, wgt, bias, a, b, relu, kh, kw, pad_h, pad_w, stride_h,
+                      stride_w, dil_h, dil_w, cout, out, stream, nullptr, copy);
 }
 
 extern "C" int dab_fconv_affine_prelu(const float *x, int n, int h, int w, int c, const float *wgt, const float *bias,

@@ -321,6 +321,15 @@ void FloatConv::forward_impl() const {
             fused_sign_out ? (fused_sign_out->ld ? fused_sign_out->ld : fused_sign_out->c) : 0, stream()));
         return;
     }
+    if (fused_pool_global && copy_to) {
+        const Mat &in = *fused_pool_input;
+        dab_check(dab_global_ave_pool_fconv1x1_copy(
+            static_cast<const float *>(in.dev), in.n, in.h, in.w, in.c, static_cast<const float *>(weight_mat->dev),
+            bias_mat ? static_cast<const float *>(bias_mat->dev) : nullptr, fused_a ? static_cast<const float *>(fused_a->dev) : nullptr,
+            fused_b ? static_cast<const float *>(fused_b->dev) : nullptr, fused_relu ? 1 : 0, output_mat->c, static_cast<float *>(input_mat->dev),
+            static_cast<float *>(output_mat->dev), copy_to, stream()));
+        return;
+    }
     if (fused_pool_input) {
         dab_check((fused_pool_global ? dab_global_ave_pool_fconv1x1 : dab_ave_pool2_fconv1x1)(
             static_cast<const float *>(fused_pool_input->dev), fused_pool_input->n, fused_pool_input->h, fused_pool_input->w,
@@ -354,13 +363,17 @@ void FloatConv::forward_impl() const {
             fused_sign_out ? (fused_sign_out->ld ? fused_sign_out->ld : fused_sign_out->c) : 0, stream()));
         return;
     }
-    dab_check(dab_fconv_affine_relu(
-        static_cast<const float *>(input_mat->dev), input_mat->n, input_mat->h, input_mat->w, input_mat->c,
-        static_cast<const float *>(weight_mat->dev), bias_mat ? static_cast<const float *>(bias_mat->dev) : nullptr,
-        fused_a ? static_cast<const float *>(fused_a->dev) : nullptr,
-        fused_b ? static_cast<const float *>(fused_b->dev) : nullptr, fused_relu ? 1 : 0, weight_mat->h, weight_mat->w,
-        pad_h, pad_w, stride_h, stride_w, dilation, dilation, output_mat->c, static_cast<float *>(output_mat->dev),
-        stream()));
+    const auto *x = static_cast<const float *>(input_mat->dev), *w = static_cast<const float *>(weight_mat->dev);
+    auto floats = [](const MatP &m) { return m ? static_cast<const float *>(m->dev) : nullptr; };
+    auto *out = static_cast<float *>(output_mat->dev);
+    const Mat &in = *input_mat;
+    const int kh = weight_mat->h, kw = weight_mat->w, relu = fused_relu ? 1 : 0, cout = output_mat->c;
+    if (copy_to)
+        dab_check(dab_fconv_affine_relu_copy(x, in.n, in.h, in.w, in.c, w, floats(bias_mat), floats(fused_a), floats(fused_b), relu, kh, kw, pad_h, pad_w,
+                                             stride_h, stride_w, dilation, dilation, cout, out, copy_to, stream()));
+    else
+        dab_check(dab_fconv_affine_relu(x, in.n, in.h, in.w, in.c, w, floats(bias_mat), floats(fused_a), floats(fused_b), relu, kh, kw, pad_h, pad_w,
+                                        stride_h, stride_w, dilation, dilation, cout, out, stream()));
 }
 
 std::string FloatConv::to_str() const {

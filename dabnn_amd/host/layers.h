@@ -94,6 +94,9 @@ class BNN_API FloatConv : public Layer {
     // makes output_mat, which must have memory, for who asks for it after a run.
     const BinConv *inside_block = nullptr;
     void forward_alone() const override;
+    // Whether forward() can write the result a second time, and where to; set by the net for the launches it enqueues.
+    bool can_copy() const { return output_mat && !output_mat->ld && !fused_pool_max && !fused_slope && !inside_block && (!fused_pool_input || fused_pool_global); }
+    float *copy_to = nullptr;
     const int pad_h, pad_w, stride_h, stride_w, dilation;
     FloatConv(NetCP net, css name, css input, css weight, css bias, css output, int pad_h, int pad_w, int stride_h,
               int stride_w, int dilation);

@@ -428,7 +428,8 @@ bool Net::layers_write_input() {
 // takes 20 to 100 us of a call (from the device to pageable memory, and a second synchronisation); behind the layers it
 // takes 2 (4 KB) to 20 us (1 MB: 66 us of a call before).  Above that size the link would hold up callers who ask for another blob.
 // Who never asks should not pay it either (batch 1 from device memory 96 -> 101 us, batch 256 20 of 1030): a blob that nobody asked for
-// after the first two runs, which are not captured, is left out until somebody does.
+// after the first two runs, which are not captured, is left out until somebody does.  A FloatConv that makes such a blob writes the copy
+// itself (batch 1 and 6: 3 us of a run less, a launch; batch 256, whose megabyte then leaves while the classifier runs: 10).
 void Net::plan_mirrors() {
     constexpr size_t kMost = 2u << 20;
     std::vector<const Mat *> rd, wr;
@@ -446,7 +447,13 @@ void Net::plan_mirrors() {
         if (known || m->data_type != DataType::Float || m->ld || !m->dev || !written.count(m.get()) || read.count(m.get()) ||
             m->bytes() == 0 || total + m->bytes() > kMost)
             continue;
-        mirrors_.emplace_back(Mirror{m, nullptr});
+        std::shared_ptr<FloatConv> writer;
+        for (const auto &l : layers) {
+            layer_io(l, rd, wr);
+            if (std::find(wr.begin(), wr.end(), m.get()) != wr.end()) writer = std::dynamic_pointer_cast<FloatConv>(l);
+        }
+        if (writer && (writer->output_mat != m || !writer->can_copy())) writer = nullptr;
+        mirrors_.emplace_back(Mirror{m, nullptr, writer});
         total += (m->bytes() + 255) / 256 * 256;
     }
     if (mirrors_.empty()) return;
@@ -990,9 +997,11 @@ void Net::enqueue_layers(bool staged_input) {
         const auto in = blob(input_name_);
         dab_check(dab_copy_f32(static_cast<float *>(in->dev), reinterpret_cast<const float *>(staging_->memory()), (int64_t)in->total(), stream_));
     }
+    for (const Mirror &m : mirrors_)
+        if (m.writer) m.writer->copy_to = m.copied ? m.host : nullptr;
     for (const auto &layer : layers) layer->forward();
     for (const Mirror &m : mirrors_)
-        if (m.copied) dab_check(dab_copy_f32(m.host, static_cast<const float *>(m.mat->dev), (int64_t)m.mat->total(), stream_));
+        if (m.copied && !m.writer) dab_check(dab_copy_f32(m.host, static_cast<const float *>(m.mat->dev), (int64_t)m.mat->total(), stream_));
 }
 
 void Net::launch_layers(bool staged_input) {

@@ -23,6 +23,8 @@ namespace bnn {
 class BinConv;
 class Staging;
 
+class FloatConv;
+
 class BNN_API Net : public std::enable_shared_from_this<Net> {
    public:
     static std::shared_ptr<Net> create();
@@ -125,6 +127,7 @@ class BNN_API Net : public std::enable_shared_from_this<Net> {
     struct Mirror {
         std::shared_ptr<Mat> mat;
         float *host;
+        std::shared_ptr<FloatConv> writer;  // the layer that writes it last, where that can write the copy too
         bool asked = false;
         bool copied = false;  // by the run at hand
         bool valid = false;   // holds what the last run left

@@ -282,6 +282,11 @@ DAB_API int dab_fconv_affine_relu(const float *x, int n, int h, int w, int c, co
                                   const float *a, const float *b, int relu, int kh, int kw, int pad_h, int pad_w,
                                   int stride_h, int stride_w, int dil_h, int dil_w, int cout, float *out,
                                   dab_stream_t stream);
+/* The same, and the result a second time at `copy`, which may be pinned host memory: in the same launch for 9 to a few hundred pixels. */
+DAB_API int dab_fconv_affine_relu_copy(const float *x, int n, int h, int w, int c, const float *wgt, const float *bias,
+                                  const float *a, const float *b, int relu, int kh, int kw, int pad_h, int pad_w,
+                                  int stride_h, int stride_w, int dil_h, int dil_w, int cout, float *out, float *copy,
+                                  dab_stream_t stream);
 
 /*
  * dab_fconv_affine_relu with a PRelu (dabnn/layers/PRelu.cpp:6-30, slope_n = 1 or cout slopes) in the Relu's place, whose
@@ -333,6 +338,10 @@ DAB_API int dab_max_pool2_fconv1x1_takes(int n, int h, int w, int c, int cout);
  */
 DAB_API int dab_global_ave_pool_fconv1x1(const float *x, int n, int h, int w, int c, const float *wgt, const float *bias,
                                          const float *a, const float *b, int relu, int cout, float *pooled, float *out,
+                                         dab_stream_t stream);
+/* The same, and out a second time at `copy`, which may be pinned host memory. */
+DAB_API int dab_global_ave_pool_fconv1x1_copy(const float *x, int n, int h, int w, int c, const float *wgt, const float *bias,
+                                         const float *a, const float *b, int relu, int cout, float *pooled, float *out, float *copy,
                                          dab_stream_t stream);
 
 /*

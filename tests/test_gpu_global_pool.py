@@ -21,3 +21,29 @@ def test_average_over_the_whole_image(n, h, w, c):
     got = dab.ave_pool(torch.from_numpy(x).cuda(), h, w, 0, 0, 3, 2).cpu().numpy()
     sample = sorted({0, n // 2, n - 1})
     np.testing.assert_array_equal(got[sample], np.stack([orc.ave_pool(x[i], h, w, 0, 0, 3, 2) for i in sample]))
+
+
+@pytest.mark.parametrize("m,cout", [(1, 70), (8, 64), (9, 33), (40, 1000), (256, 1000), (300, 31), (70000, 8)])
+def test_a_second_copy_of_the_result(m, cout):
+    """dab_fconv_affine_relu_copy: the result and what pinned memory holds are the plain call's, whichever kernel runs; nothing is written past them."""
+    import ctypes
+    import torch
+    from dabnn_amd import capi
+    g = torch.Generator(device="cuda").manual_seed(m)
+    x, w = torch.randn((m, 1, 1, 64), device="cuda", generator=g), torch.randn((cout, 64), device="cuda", generator=g)
+    s = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    args = (x.data_ptr(), m, 1, 1, 64, w.data_ptr(), None, None, None, 1, 1, 1, 0, 0, 1, 1, 1, 1, cout)
+    want, out = torch.empty((m, cout), device="cuda"), torch.empty((m, cout), device="cuda")
+    host = torch.full((m * cout + 8,), -3.0).pin_memory()
+    assert capi.lib.dab_fconv_affine_relu(*args, want.data_ptr(), s) == 0
+    assert capi.lib.dab_fconv_affine_relu_copy(*args, out.data_ptr(), host.data_ptr(), s) == 0
+    torch.cuda.synchronize()
+    assert torch.equal(out, want) and torch.equal(host[:-8].view(m, cout), want.cpu()) and bool((host[-8:] == -3).all())
+    if m <= 8:
+        y = torch.randn((m, 7, 7, 64), device="cuda", generator=g)
+        pooled = torch.empty((m, 64), device="cuda")
+        gap = (y.data_ptr(), m, 7, 7, 64, w.data_ptr(), None, None, None, 0, cout, pooled.data_ptr())
+        assert capi.lib.dab_global_ave_pool_fconv1x1(*gap, want.data_ptr(), s) == 0
+        assert capi.lib.dab_global_ave_pool_fconv1x1_copy(*gap, out.data_ptr(), host.data_ptr(), s) == 0
+        torch.cuda.synchronize()
+        assert torch.equal(out, want) and torch.equal(host[:-8].view(m, cout), want.cpu())
