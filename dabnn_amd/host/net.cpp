@@ -76,6 +76,9 @@ Net::~Net() {
     mat_map_.clear();
     staging_.reset();
     if (mirror_memory_) (void)hipHostFree(mirror_memory_);
+    for (void *e : arrivals_) (void)hipEventDestroy(static_cast<hipEvent_t>(e));
+    for (void *up : upload_streams_)
+        if (up) (void)hipStreamDestroy(static_cast<hipStream_t>(up));
     if (stream_) (void)hipStreamDestroy(static_cast<hipStream_t>(stream_));
 }
 
@@ -335,6 +338,7 @@ void Net::prepare(const void *buf, size_t len) {
     allocate_blobs();
     // an in-place layer on the input blob would write into a caller's buffer that is read in place
     copy_input_ = layers_write_input();
+    find_head();
     staging_ = std::make_unique<Staging>(blob(input_name_)->bytes());
     plan_mirrors();
     hip_check(hipStreamSynchronize(static_cast<hipStream_t>(stream_)), "hipStreamSynchronize");
@@ -945,7 +949,14 @@ void Net::run(const void *host_input) {
     else
         (void)hipGetLastError();
     const bool staged = pageable && in->bytes() <= (1u << 20);  // (staging_ holds that much)
-    bind_input(nullptr, staged);
+    if (!staged && head_ && !profile && (!pageable || uploaded_)) {
+        BNN_ASSERT(!(strict && !run_fconv), "fconv must be run in strict mode");
+        bind_input(nullptr, kBehindHead);
+        upload_and_run_head(host_input, pageable);
+        launch_layers(kBehindHead);
+        return;
+    }
+    bind_input(nullptr, staged ? kStagedLayers : kLayers);
     if (staged)
         std::memcpy(staging_->memory(), host_input, in->bytes());
     else if (pageable && uploaded_) {
@@ -958,22 +969,140 @@ void Net::run(const void *host_input) {
         hip_check(hipMemcpyAsync(in->dev, host_input, in->bytes(), hipMemcpyHostToDevice, static_cast<hipStream_t>(stream_)),
                   "hipMemcpyAsync");
     uploaded_ = uploaded_ || (pageable && !staged);
-    launch_layers(staged);
+    launch_layers(staged ? kStagedLayers : kLayers);
+}
+
+// A large host input goes to the device in shares of this many bytes or more, and the head follows each.
+static constexpr size_t kShare = 8u << 20;
+
+// The layers at the front that can run on some of the images: a stem that is one pass with its MaxPool over three channels, and the binary
+// convolutions behind it that read nothing else.  Their results do not depend on how many images a launch has (the float
+// layers' other kernels are chosen by that, and add in another order).
+void Net::find_head() {
+    auto stem = layers.empty() ? nullptr : std::dynamic_pointer_cast<FloatConv>(layers[0]);
+    if (copy_input_ || blob(input_name_)->bytes() < 2 * kShare || !stem || !stem->fused_maxpool_out || stem->input_mat != stored_blob(input_name_) || stem->input_mat->c != 3) return;
+    std::vector<const Mat *> rd, wr;
+    std::set<const Mat *> made = {stem->input_mat.get()};
+    for (size_t i = 0; i < layers.size(); ++i) {
+        auto bc = std::dynamic_pointer_cast<BinConv>(layers[i]);
+        if (bc && bc->inside_pass) {
+            head_ = i + 1;
+            continue;
+        }
+        if (i > 0 && (!bc || bc->method() != BinConv::DIRECT_CONV || bc->branch || bc->has_slices())) return;
+        layer_io(layers[i], rd, wr);
+        if (bc && bc->fused_sign_out) wr.push_back(bc->fused_sign_out.get());
+        for (const Mat *m : rd)
+            if (!made.count(m)) return;
+        for (const auto *list : {&rd, &wr})
+            for (const Mat *m : *list)
+                if (m->n != batch_ || m->bytes() / batch_ % 16 != 0) return;  // (the kernels want aligned images)
+        made.insert(wr.begin(), wr.end());
+        head_ = i + 1;
+    }
+}
+
+// The head's launches on images first .. first + count - 1: its blobs stand for those alone while they are made.
+void Net::run_head(int first, int count) {
+    std::vector<const Mat *> rd, wr;
+    std::set<const Mat *> blobs;
+    for (size_t i = 0; i < head_; ++i) {
+        layer_io(layers[i], rd, wr);
+        blobs.insert(rd.begin(), rd.end());
+        blobs.insert(wr.begin(), wr.end());
+        auto bc = std::dynamic_pointer_cast<BinConv>(layers[i]);
+        if (bc && !bc->inside_pass && !bc->next_in_pass && bc->fused_sign_out) blobs.insert(bc->fused_sign_out.get());
+    }
+    struct View {
+        Mat *m;
+        void *dev;
+        int n;
+        View(Mat *m_, int first, int count) : m(m_), dev(m_->dev), n(m_->n) {
+            m->dev = static_cast<unsigned char *>(dev) + m->bytes() / n * first;
+            m->n = count;
+        }
+        ~View() { m->dev = dev, m->n = n; }
+        View(const View &) = delete;
+    };
+    std::vector<std::unique_ptr<View>> views;
+    for (const Mat *m : blobs)
+        if (m->dev) views.push_back(std::make_unique<View>(const_cast<Mat *>(m), first, count));
+    for (size_t i = 0; i < head_; ++i) layers[i]->forward();
+}
+
+// Behind each share the head's launches on the images that are whole by then, so that only the last share's are left when the input is
+// there.  A share's event holds up what follows it on its stream by about 20 us, so the next share takes the other stream.  bireal18
+// from pageable memory, us, before, in shares of 4 MB and of 8: 16 images 494 / 469 / 519, 40 867 / 831 / 802, 64 1268 / 1235 / 1159,
+// 100 1908 / 1766 / 1755, 256 4196 / 3794 / 3643; all shares on one stream: 40 811, 100 1814, 256 3830.  From pinned memory: 40 722 ->
+// 673, 100 1613 -> 1484.
+void Net::upload_and_run_head(const void *host_input, bool pageable) {
+    auto in = blob(input_name_);
+    const size_t image = in->bytes() / batch_;
+    hipStream_t s = static_cast<hipStream_t>(stream_);
+    hip_check(hipStreamSynchronize(s), "hipStreamSynchronize");  // (a run that failed may have left kernels that read the input)
+    for (void *&up : upload_streams_) {
+        if (up) continue;
+        std::lock_guard<std::mutex> lock(capture_mutex());
+        hipStream_t made;
+        hip_check(hipStreamCreateWithFlags(&made, hipStreamNonBlocking), "hipStreamCreate");
+        up = made;
+    }
+    int done = 0;
+    size_t share = 0;
+    auto arriving = [&](size_t bytes) -> void * {
+        const int there = (int)(bytes / image);
+        if (there < batch_ && (size_t)(there - done) * image < kShare) return upload_streams_[share % 2];
+        if (share == arrivals_.size()) {
+            std::lock_guard<std::mutex> lock(capture_mutex());
+            hipEvent_t e;
+            hip_check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate");
+            arrivals_.push_back(e);
+        }
+        hipEvent_t e = static_cast<hipEvent_t>(arrivals_[share]);
+        hip_check(hipEventRecord(e, static_cast<hipStream_t>(upload_streams_[share % 2])), "hipEventRecord");
+        hip_check(hipStreamWaitEvent(s, e, 0), "hipStreamWaitEvent");
+        run_head(done, there - done);
+        done = there;
+        return upload_streams_[++share % 2];
+    };
+    try {
+        void *up = upload_streams_[0];
+        if (pageable) {
+            {
+                std::lock_guard<std::mutex> lock(capture_mutex());
+                staging_->grow(in->bytes());
+            }
+            staging_->upload(in->dev, host_input, in->bytes(), up, arriving);
+        } else {
+            for (size_t at = 0; at < in->bytes();) {
+                const size_t n = std::min(kShare + image, in->bytes() - at);  // (with kShare of whole images)
+                hip_check(hipMemcpyAsync(static_cast<unsigned char *>(in->dev) + at, static_cast<const unsigned char *>(host_input) + at, n,
+                                         hipMemcpyHostToDevice, static_cast<hipStream_t>(up)),
+                          "hipMemcpyAsync");
+                at += n;
+                up = arriving(at);
+            }
+        }
+    } catch (...) {
+        for (void *up : upload_streams_) (void)hipStreamSynchronize(static_cast<hipStream_t>(up));
+        (void)hipStreamSynchronize(s);
+        throw;
+    }
 }
 
 void Net::run_device(const void *device_input) {
     BNN_ASSERT(prepared_, "run before read");
-    bind_input(device_input, false);
-    launch_layers(false);
+    bind_input(device_input, kLayers);
+    launch_layers(kLayers);
 }
 
 // Points the input blob at the memory this run reads: the caller's device buffer in place, or the blob's own
 // allocation (host inputs, unaligned buffers, callers whose buffers keep changing), filled here from device_input.
-void Net::bind_input(const void *device_input, bool staged_input) {
+void Net::bind_input(const void *device_input, Kind kind) {
     auto in = blob(input_name_);
     const bool in_place = device_input != nullptr && !copy_input_ && reinterpret_cast<uintptr_t>(device_input) % 256 == 0;
     void *want = in_place ? const_cast<void *>(device_input) : input_own_dev_;
-    Graph &graph = graphs_[staged_input];
+    Graph &graph = graphs_[kind];
     if (graph.exec && graph.input != want) {
         // the graph's kernels hold the address they were captured with
         if (in_place && ++input_rebinds_ >= 3) {
@@ -992,22 +1121,22 @@ void Net::bind_input(const void *device_input, bool staged_input) {
                   "hipMemcpyAsync");
 }
 
-void Net::enqueue_layers(bool staged_input) {
-    if (staged_input) {
+void Net::enqueue_layers(Kind kind) {
+    if (kind == kStagedLayers) {
         const auto in = blob(input_name_);
         dab_check(dab_copy_f32(static_cast<float *>(in->dev), reinterpret_cast<const float *>(staging_->memory()), (int64_t)in->total(), stream_));
     }
     for (const Mirror &m : mirrors_)
         if (m.writer) m.writer->copy_to = m.copied ? m.host : nullptr;
-    for (const auto &layer : layers) layer->forward();
+    for (size_t i = kind == kBehindHead ? head_ : 0; i < layers.size(); ++i) layers[i]->forward();
     for (const Mirror &m : mirrors_)
         if (m.copied && !m.writer) dab_check(dab_copy_f32(m.host, static_cast<const float *>(m.mat->dev), (int64_t)m.mat->total(), stream_));
 }
 
-void Net::launch_layers(bool staged_input) {
+void Net::launch_layers(Kind kind) {
     BNN_ASSERT(!(strict && !run_fconv), "fconv must be run in strict mode");
     hipStream_t s = static_cast<hipStream_t>(stream_);
-    Graph &graph = graphs_[staged_input];
+    Graph &graph = graphs_[kind];
     int copies = 0;
     for (Mirror &m : mirrors_) {
         m.valid = false;
@@ -1020,7 +1149,7 @@ void Net::launch_layers(bool staged_input) {
         graph.exec = nullptr;
     }
     if (profile || !use_graph) {
-        enqueue_layers(staged_input);
+        enqueue_layers(kind);
     } else if (graph.exec) {
         hip_check(hipGraphLaunch(static_cast<hipGraphExec_t>(graph.exec), s), "hipGraphLaunch");
     } else if (runs_ >= 2) {
@@ -1029,7 +1158,7 @@ void Net::launch_layers(bool staged_input) {
         hipGraph_t captured = nullptr;
         hip_check(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture");
         try {
-            enqueue_layers(staged_input);
+            enqueue_layers(kind);
         } catch (...) {
             (void)hipStreamEndCapture(s, &captured);
             if (captured) (void)hipGraphDestroy(captured);
@@ -1044,7 +1173,7 @@ void Net::launch_layers(bool staged_input) {
         graph.copies = copies;
         hip_check(hipGraphLaunch(exec, s), "hipGraphLaunch");
     } else {
-        enqueue_layers(staged_input);
+        enqueue_layers(kind);
     }
     for (const auto &kv : contiguous_) kv.first->gather_to(kv.second->dev, s);
     for (const auto &l : alone_) l->forward_alone();

@@ -106,20 +106,29 @@ class BNN_API Net : public std::enable_shared_from_this<Net> {
     std::vector<std::shared_ptr<const BinConv>> columns_;  // layers whose column matrix somebody asked for
     std::vector<std::shared_ptr<const Layer>> alone_;      // and those inside another's pass whose own results somebody did
     int runs_ = 0;
-    // The captured layers and the input address that their kernels hold: [1] begins with the copy of a small host input
-    // from staging_.
+    // The captured layers and the input address that their kernels hold: all of them, all of them behind the copy of a small host
+    // input from staging_, or those behind the head.
+    enum Kind { kLayers, kStagedLayers, kBehindHead, kKinds };
     struct Graph {
         void *exec = nullptr;
         const void *input = nullptr;
         int copies = 0;  // of mirrors
-    } graphs_[2];
+    } graphs_[kKinds];
     void *input_own_dev_ = nullptr;       // the input blob's own allocation
     int input_rebinds_ = 0;               // captures thrown away because the caller's buffer changed
     bool copy_input_ = false;             // the caller's buffers keep changing: copy into the own blob
-    void bind_input(const void *device_input, bool staged_input);
+    void bind_input(const void *device_input, Kind kind);
     bool layers_write_input();
-    void launch_layers(bool staged_input);
-    void enqueue_layers(bool staged_input);
+    void launch_layers(Kind kind);
+    void enqueue_layers(Kind kind);
+    // How many layers at the front run on the first images of a large host input while the others are still on their way, the
+    // streams that bring its shares in turn, and an event for each share.
+    size_t head_ = 0;
+    void *upload_streams_[2] = {};
+    std::vector<void *> arrivals_;
+    void find_head();
+    void run_head(int first, int count);
+    void upload_and_run_head(const void *host_input, bool pageable);
     std::unique_ptr<Staging> staging_;    // pinned memory for inputs, and for blobs that are asked for
     bool uploaded_ = false;               // a large input from pageable memory
     // Small blobs that no layer reads are copied to pinned memory behind the layers of the first two runs, and of every run once they

@@ -125,7 +125,7 @@ void Staging::start_helpers() {
     }
 }
 
-void Staging::upload(void *dst, const void *src, size_t bytes, void *stream) {
+void Staging::upload(void *dst, const void *src, size_t bytes, void *stream, const std::function<void *(size_t)> &arriving) {
     if (bytes == 0) return;
     std::lock_guard<std::mutex> one(use_);
     hipStream_t s = static_cast<hipStream_t>(stream);
@@ -161,6 +161,7 @@ void Staging::upload(void *dst, const void *src, size_t bytes, void *stream) {
             hip_check(hipMemcpyAsync(dst_ + at, memory_ + (transfers_[t].first % ring_) * kBlock, n, hipMemcpyHostToDevice, s), "hipMemcpyAsync");
             if (ring_ < blocks_) hip_check(hipEventRecord(static_cast<hipEvent_t>(events_[t % kEvents]), s), "hipEventRecord");
             issued_.store(t + 1, std::memory_order_release);
+            if (arriving) s = static_cast<hipStream_t>(arriving(at + n));
         }
         if (failed_.load(std::memory_order_relaxed)) throw std::runtime_error("the input's copy failed");
     };

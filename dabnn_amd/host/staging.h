@@ -14,6 +14,7 @@
 #include <atomic>
 #include <condition_variable>
 #include <cstddef>
+#include <functional>
 #include <mutex>
 #include <thread>
 #include <vector>
@@ -42,8 +43,9 @@ class Staging {
     size_t bytes() const { return bytes_; }
 
     // Copies host memory to the device on `stream`; `src` may change once the call returns.  The caller synchronises the
-    // stream before the next call (a Net's runs do).
-    void upload(void *dst, const void *src, size_t bytes, void *stream);
+    // stream before the next call (a Net's runs do).  `arriving`, if given, is told how many bytes have been asked for, from the
+    // front on, each time that grows, and says which stream brings the next (the caller synchronises all of them).
+    void upload(void *dst, const void *src, size_t bytes, void *stream, const std::function<void *(size_t)> &arriving = nullptr);
     // Copies device memory to the host and waits, over the copy stream of the device that the Staging's events are of: the runtime
     // records no event of one device on a stream of another.
     void download(void *dst, const void *src, size_t bytes);
