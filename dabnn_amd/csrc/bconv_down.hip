@@ -12,7 +12,7 @@
 //   tile    a block is 32 pixels x 128 channels, a wave 32 channels
 //   walk    many pieces, 64 and 128 input channels: a wave keeps the filters of 32 channels, blocks walk over pixel tiles
 // One Bi-Real-18 pass, the three layers as two launches each / in one (us, in a graph): batch 1 5.9 + 6.9 + 8.1 / 3.8 + 3.7 + 4.0, batch
-// 6 9.4 + 9.0 + 9.0 / 5.7 + 5.7 + 5.8, batch 40 22 + 18 + 20 / 13.6 + 12.0 + 11.3, batch 256 100 + 68 / 61 + 43 (the third stays two).
+// 6 9.4 + 9.0 + 9.0 / 5.7 + 5.7 + 5.8, batch 40 22 + 18 + 20 / 13.6 + 12.0 + 10.4, batch 256 100 + 68 + 59 / 61 + 43 + 54.
 #include "fp4_core.h"
 
 namespace dab {
@@ -260,11 +260,16 @@ __global__ __launch_bounds__(512) void bconv3x3_down_staged_kernel(const BconvDo
 
 // ---------------------------------------------------------------- between
 // A wave counts, the block pools its pixels into LDS, the wave multiplies on the fp32 matrix instruction -- 32 of 64 cycles per 64
-// channels of depth, which is what bounds the kernel: 40 images of 28 x 28 x 128 to 256 take 12.0 us.
+// channels of depth, which is what bounds the kernel: 40 images of 28 x 28 x 128 to 256 take 12.0 us.  Two blocks share a CU, one
+// multiplying while the other waits for its floats: with 256 input channels a thread's 32 taps take 128 registers, so half of them are
+// asked for when the bits have been counted, into their registers.  14 x 14 x 256 to 512, us, all at once and one block a CU / so: 40
+// images 11.1 / 10.4, 60 20.1 / 17.0, 100 29.6 / 23.6, 256 70.5 / 53.4; a block of eight waves, the floats read half as often, 65.5 there, and
+// three blocks a CU, with spills, 72.5.
 template <int CW, int WAVES, bool POOLED>
-__global__ __launch_bounds__(WAVES * 64) void bconv3x3_down_tile_kernel(const BconvDownArgs p) {
+__global__ __launch_bounds__(WAVES * 64, 2) void bconv3x3_down_tile_kernel(const BconvDownArgs p) {
     constexpr int C = CW * 64, AS = C + 4, CH = 32 * WAVES, THREADS = 64 * WAVES;  // AS: rows 4 floats off a multiple of 64 banks
     constexpr int PIECES = 32 * (C / 4) / THREADS;  // 16-byte pieces of the pooled tile per thread
+    constexpr int EARLY = !POOLED && PIECES > 4 ? PIECES / 2 : PIECES;  // of those: asked for before anything is counted
     constexpr int CHUNK = 8, CHUNKS = C / 8 / CHUNK;  // a wave's filters in steps of 8 depths, asked for CHUNK steps at a time
     __shared__ __attribute__((aligned(16))) float pooled[32][AS];
     const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5, l32 = lane & 31;
@@ -291,11 +296,15 @@ __global__ __launch_bounds__(WAVES * 64) void bconv3x3_down_tile_kernel(const Bc
         for (int t = 0; t < 9; ++t) load_dwords<CW>(wt[t], rw, ch_ok ? ch * (CW * 72) + t * (CW * 8) + half * (CW * 4) : kDownOutside);
     }
     DownPiece<POOLED> x[PIECES];
+    auto fetch_floats = [&](int from, int to) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < PIECES; ++i) {
-        const int piece = tid + THREADS * i, pix = m0 + piece / (C / 4);
-        x[i].fetch(p, pix < p.total ? pix : p.total - 1, (piece % (C / 4)) * 4, C);
-    }
+        for (int i = 0; i < PIECES; ++i) {
+            if (i < from || i >= to) continue;
+            const int piece = tid + THREADS * i, pix = m0 + piece / (C / 4);
+            x[i].fetch(p, pix < p.total ? pix : p.total - 1, (piece % (C / 4)) * 4, C);
+        }
+    };
+    fetch_floats(0, EARLY);
     const float *filter = p.sw + (size_t)(ch_ok ? ch : 0) * C + half * 4;
     f32x4m f[CHUNKS > 1 ? 2 : 1][CHUNK];
     auto fetch_filters = [&](int chunk) {
@@ -317,6 +326,11 @@ __global__ __launch_bounds__(WAVES * 64) void bconv3x3_down_tile_kernel(const Bc
     for (int t = 0; t < 9; ++t)
 #pragma unroll
         for (int c = 0; c < CW; ++c) mfma_fp4<32>(cnt, bitspm1(act[t][c]), bitspm1(wt[t][c]));
+    if constexpr (EARLY < PIECES) {
+        __builtin_amdgcn_sched_barrier(0);
+        fetch_floats(EARLY, PIECES);  // into the registers of the bits
+        __builtin_amdgcn_sched_barrier(0);
+    }
 #pragma unroll
     for (int i = 0; i < PIECES; ++i) {
         const int piece = tid + THREADS * i;
@@ -363,7 +377,7 @@ __global__ __launch_bounds__(WAVES * 64) void bconv3x3_down_tile_kernel(const Bc
 // value too small for the split is made on the fp32 matrix instruction.  With 64 input channels bound by memory: 256 images of
 // 56 x 56 x 64 to 128 move 315 MB in 61 us, 5.2 TB/s, the rate of a copy (tile kernel 75, two launches 100).  With 128 a block has eight
 // waves, so that the floats are read once: 28 x 28 at 256 images 43 us (tile 63, two launches 68; four waves 63).  256 input
-// channels, whose filters take 192 registers, were no faster (64 us, two launches 59).
+// channels, whose filters take 192 registers, were slower (14 x 14 at 256 images 64 us, tile kernel 53).
 template <int CW, int WAVES, bool POOLED>
 __global__ __launch_bounds__(WAVES * 64, 2) void bconv3x3_down_walk_kernel(const BconvDownArgs p) {
     constexpr int C = CW * 64, CH = 32 * WAVES, THREADS = 64 * WAVES;

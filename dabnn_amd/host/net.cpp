@@ -868,8 +868,7 @@ void Net::pair_residual_layers() {
 // The shortcut branch of a down-sampling block -- AvePool 2x2 inside a 1x1 FloatConv (+ Affine) that reads what the block's first
 // BinConv reads and whose result only that layer adds -- runs in the BinConv's pass, which keeps the branch's result on the chip; who
 // asks for its blob has the pass run again with that output.  So nothing may rewrite, later, what the pass reads or writes, nor read
-// or write the branch's blob.  Two launches / one: bconv_down.hip; 256 input channels only up to 4 000 pieces of 32 pixels x 32
-// channels (14 x 14 x 256 to 512: 100 images, 2 464 pieces, 35.6 / 29.8 us, 256 images, 6 272 pieces, 59 / 71).
+// or write the branch's blob.  Two launches against one: bconv_down.hip.
 void Net::branches_inside_binconvs() {
     std::vector<const Mat *> rd, wr;
     for (size_t i = 1; i < layers.size(); ++i) {
@@ -879,8 +878,7 @@ void Net::branches_inside_binconvs() {
             continue;
         const Mat &in = *bc->input_mat;
         const int cout = bc->weight_mat->n;
-        const long long pieces = ((long long)in.n * (in.h / 2) * (in.w / 2) + 31) / 32 * (cout / 32);
-        if (!dab_bconv3x3_down_takes(in.n, in.h, in.w, in.elem_c, cout) || (in.elem_c == 256 && pieces > 4000)) continue;
+        if (!dab_bconv3x3_down_takes(in.n, in.h, in.w, in.elem_c, cout)) continue;
         std::shared_ptr<FloatConv> branch;
         size_t at = 0;
         for (size_t j = 0; j < i; ++j) {

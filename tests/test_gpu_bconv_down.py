@@ -183,7 +183,7 @@ def block_net(models, n_in, cout, hw, seed=0, relu=False, second_reader=False):
 
 
 @pytest.mark.parametrize("cin,cout,hw,batch,inside", [(64, 128, 16, 1, True), (128, 256, 12, 3, True), (64, 128, 56, 20, True), (256, 192, 14, 33, True),
-                                                      (128, 128, 28, 60, True), (256, 512, 14, 190, False), (64, 64, 4, 1, False)])
+                                                      (128, 128, 28, 60, True), (256, 512, 14, 190, True), (64, 64, 4, 1, False)])
 def test_net_every_blob_on_every_run(cin, cout, hw, batch, inside):
     from dabnn_amd import dab_format, models, net
     from oracle import net as orc_net
