@@ -138,8 +138,10 @@ enum Epilogue { kStoreCounts, kAddCounts, kAffine, kAffineSign };
 // (eight) waves take every fourth (eighth) unit of the depth each and load their operands straight from memory, kUnitsAhead units while
 // as many are multiplied; the partial sums meet in LDS.  Both operands +-1 (fp4_core.h).  Bound by their expansion: m512 k72 n3136,
 // accumulating, 8.7 us (9.8 with three units asked for at a time and none while they were multiplied).
-constexpr int kUnitsAhead = 2;
-template <int CC, FilterLayout L, int E, int NT, int WAVES, bool LONG>
+// SHALLOW: up to kUnitsAtOnce units a wave, all asked for at once, without the loop, whose length alone costs a launch of 2 to 3 us
+// 0.1 to 0.2 (116 x 405 x 14 2.44 -> 2.29 us, 94 x 23 x 17 2.54 -> 2.36, 88 x 300 x 40 2.84 -> 2.67).
+constexpr int kUnitsAhead = 2, kUnitsAtOnce = 3;
+template <int CC, FilterLayout L, int E, int NT, int WAVES, bool LONG, bool SHALLOW = false>
 __global__ __launch_bounds__(64 * WAVES, 4) void bit_gemm_split_kernel(const BitGemmArgs p) {
     constexpr int CH = 32 * NT, LD = CH + 1;
     __shared__ float part[WAVES][32 * LD];
@@ -163,10 +165,11 @@ __global__ __launch_bounds__(64 * WAVES, 4) void bit_gemm_split_kernel(const Bit
         if (ch_ok) ea = p.g.a[ch], eb = p.g.b[ch];
     const int out_off = ch_ok ? (r0 * (int)p.g.out_ld + ch) * 4 : kBeyond, out_step = RPI * (int)p.g.out_ld * 4;
     auto element = [&](int i) { return p.g.out + (row0 + r0 + i * RPI) * p.g.out_ld + ch; };  // LONG: output i
-    uint32_t a[2][kUnitsAhead][CC], w[2][kUnitsAhead][NT][CC];
+    constexpr int SLOTS = SHALLOW ? 1 : 2, AHEAD = SHALLOW ? kUnitsAtOnce : kUnitsAhead;
+    uint32_t a[SLOTS][AHEAD][CC], w[SLOTS][AHEAD][NT][CC];
     auto fetch = [&](int slot, int u0) __attribute__((always_inline)) {
 #pragma unroll
-        for (int i = 0; i < kUnitsAhead; ++i)
+        for (int i = 0; i < AHEAD; ++i)
             if (u0 + WAVES * i < p.units) {
                 px.load(a[slot][i], p, u0 + WAVES * i, half);
 #pragma unroll
@@ -193,7 +196,7 @@ __global__ __launch_bounds__(64 * WAVES, 4) void bit_gemm_split_kernel(const Bit
         for (int v = 0; v < 16; ++v) acc[n][v] = 0.f;
     auto multiply = [&](int slot, int u0) __attribute__((always_inline)) {
 #pragma unroll
-        for (int i = 0; i < kUnitsAhead; ++i)
+        for (int i = 0; i < AHEAD; ++i)
             if (u0 + WAVES * i < p.units) {
 #pragma unroll
                 for (int c = 0; c < CC; ++c) {
@@ -203,11 +206,15 @@ __global__ __launch_bounds__(64 * WAVES, 4) void bit_gemm_split_kernel(const Bit
                 }
             }
     };
-    for (int u0 = wib; u0 < p.units; u0 += 2 * WAVES * kUnitsAhead) {
-        fetch(1, u0 + WAVES * kUnitsAhead);
-        multiply(0, u0);
-        fetch(0, u0 + 2 * WAVES * kUnitsAhead);
-        multiply(1, u0 + WAVES * kUnitsAhead);
+    if constexpr (SHALLOW) {
+        multiply(0, wib);
+    } else {
+        for (int u0 = wib; u0 < p.units; u0 += 2 * WAVES * AHEAD) {
+            fetch(1, u0 + WAVES * AHEAD);
+            multiply(0, u0);
+            fetch(0, u0 + 2 * WAVES * AHEAD);
+            multiply(1, u0 + WAVES * AHEAD);
+        }
     }
 #pragma unroll
     for (int n = 0; n < NT; ++n)
@@ -535,6 +542,8 @@ static int launch_bit_gemm(const char *fn, BitGemmArgs &p, hipStream_t s) {
                 hipLaunchKernelGGL((bit_gemm_split_kernel<CC, L, E, 2, 4, LONG>), grid, dim3(256), 0, s, p);
             else if (eight)
                 hipLaunchKernelGGL((bit_gemm_split_kernel<CC, L, E, 1, 8, LONG>), grid, dim3(512), 0, s, p);
+            else if (!LONG && p.units <= 4 * kUnitsAtOnce)
+                hipLaunchKernelGGL((bit_gemm_split_kernel<CC, L, E, 1, 4, LONG, !LONG>), grid, dim3(256), 0, s, p);
             else
                 hipLaunchKernelGGL((bit_gemm_split_kernel<CC, L, E, 1, 4, LONG>), grid, dim3(256), 0, s, p);
         }

@@ -37,7 +37,7 @@ def check(m, n, k, lda, ldb, g):
 
 
 @pytest.mark.parametrize("m,n,k", [(40, 33, k) for k in (13, 16, 17, 31, 32, 33, 44, 45, 47, 48, 49, 63, 64, 65, 96, 97, 128, 129, 160)] +
-                         [(32, 512 * 32, 48), (32, 513 * 32, 48), (32, 512 * 32 - 5, 45), (200, 1000, 150), (512, 1024, 72), (510, 1023, 71)])
+                         [(32, 512 * 32, 48), (32, 513 * 32, 48), (32, 513 * 32, 49), (32, 513 * 32, 33), (32, 512 * 32 - 5, 45), (200, 1000, 150), (512, 1024, 72), (510, 1023, 71)])
 def test_waves_and_units(m, n, k):
     g = torch.Generator(device="cuda").manual_seed(m + n + k)
     check(m, n, k, m + 1, k + 3, g)
