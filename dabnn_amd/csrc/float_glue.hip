@@ -1208,9 +1208,9 @@ static int fconv_impl(const char *fn, const float *x, int n, int h, int w, int c
     } else if (vec3) {
         DAB_FCONV_LAUNCH(128, 64, 24, 1, 3);
     } else if (c == 3 && bn == 32) {
-        // few output channels: the launch is bound by its loads and stores, and one 12-byte load per tap beats three
-        // 4-byte ones even where two slices of eight taps hold only nine (3x3 stride 2, 3 -> 32 at 224 x 224, batch
-        // 256: 162 against 178 us)
+        // few output channels, windows other than 3x3: the launch is bound by its loads and stores, and one 12-byte load per tap beats
+        // three 4-byte ones even where slices of eight taps are not full (3x3 stride 2, 3 -> 32 at 224 x 224, batch 256, before it had a
+        // kernel of its own: 162 against 178 us)
         DAB_FCONV_LAUNCH(128, 32, 24, 1, 3);
     } else if (bn == 32) {
         if (vec4)
