@@ -830,8 +830,8 @@ void Net::pool_inside_convs() {
 // Two residual layers over 64 channels that follow each other (BinConv + Affine + Add of its own input, at stride 1) run as one
 // pass that keeps the blob between them on the chip, where that blob and its packed copy have no other reader and nothing
 // rewrites what the first layer reads (who asks for them has that layer run again).  Pays from 48 000 pixels on, where the
-// layers are bound by memory, two launches / one pass: 56 x 56 at 12 images 11.4 / 11.5 us, 16 12.2 / 11.5, 24 20.5 / 13.7, 64
-// 43 / 25, 256 156 / 88; 28 x 28 at 40 images 9.6 / 11.9, 64 12.1 / 9.6.  Up to 64 columns: a strip of wider rows is so low
+// layers are bound by memory, two launches / one pass: 56 x 56 at 12 images 12.0 / 11.3 us, 16 12.5 / 11.5, 24 20.8 / 13.4, 64
+// 43 / 21, 256 158 / 90; 28 x 28 at 40 images 9.7 / 12.1, 64 12.2 / 9.8.  Up to 64 columns: a strip of wider rows is so low
 // that its neighbours' rows are most of the work.
 void Net::pair_residual_layers() {
     std::vector<const Mat *> rd, wr;
@@ -868,7 +868,8 @@ void Net::pair_residual_layers() {
 // The shortcut branch of a down-sampling block -- AvePool 2x2 inside a 1x1 FloatConv (+ Affine) that reads what the block's first
 // BinConv reads and whose result only that layer adds -- runs in the BinConv's pass, which keeps the branch's result on the chip; who
 // asks for its blob has the pass run again with that output.  So nothing may rewrite, later, what the pass reads or writes, nor read
-// or write the branch's blob.  Two launches against one: bconv_down.hip.
+// or write the branch's blob.  Two launches against one: bconv_down.hip; 256 input channels gain least in large nets, whose clock is lower
+// (Bi-Real-18, a run with that block in two / one: 100 images 549 / 539 us, 200 916 / 904, 256 1108 / 1107, 300 1273 / 1278).
 void Net::branches_inside_binconvs() {
     std::vector<const Mat *> rd, wr;
     for (size_t i = 1; i < layers.size(); ++i) {
