@@ -8,11 +8,12 @@
 // written for who asks for them (`sc_out`).
 //
 // Three kernels, chosen by the number of 32-pixel x 32-channel pieces of the output (pick_down has both sides of its lines):
-//   staged  few pieces: a block is one tile, all its operands are asked for at once, eight waves share the branch's depth
+//   staged  few pieces: a block is one tile, all its operands are asked for at once, four or eight waves share the branch's depth
 //   tile    a block is 32 pixels x 128 channels, a wave 32 channels
 //   walk    many pieces, 64 and 128 input channels: a wave keeps the filters of 32 channels, blocks walk over pixel tiles
-// One Bi-Real-18 pass, the three layers as two launches each / in one (us, in a graph): batch 1 5.9 + 6.9 + 8.1 / 3.8 + 3.7 + 4.0, batch
-// 6 9.4 + 9.0 + 9.0 / 5.7 + 5.7 + 5.8, batch 40 22 + 18 + 20 / 13.6 + 12.0 + 10.4, batch 256 100 + 68 + 59 / 61 + 43 + 54.
+// All of them add the branch's products in dab_ave_pool2_fconv1x1's order, so its values are that call's to the bit.
+// One Bi-Real-18 pass, the three layers as two launches each / in one (us, in a graph): batch 1 5.9 + 6.9 + 8.1 / 3.7 + 3.5 + 4.0, batch
+// 6 9.1 + 8.9 + 9.0 / 5.6 + 5.8 + 5.7, batch 40 21 + 18 + 21 / 14.1 + 11.8 + 10.5, batch 256 96 + 67 + 59 / 61 + 55 + 53.
 #include "fp4_core.h"
 
 namespace dab {
@@ -99,6 +100,9 @@ __device__ __forceinline__ float down_value(float cnt, float ea, float eb, float
 // block's floats and filters in whole lines, which meet in LDS; then the waves take 16 pixels and a part of the branch's depth each, and
 // the partial sums meet in LDS too.  (Floats fetched by each lane for its own pixel and depths, without the staging: a load then
 // touches 16 or 32 lines, and 256 input channels took 5.3 to 9 us instead of 4.0 to 5.8.)
+// The branch's four parts are those of dab_ave_pool2_fconv1x1, and so is the order in each: 0, 4, 1, 5 of eight depths in one
+// instruction, 2, 6, 3, 7 in the next (the hardware rounds behind every product, in the order of the depth slots).  LDS holds a
+// part's 16 depths as the four lanes of a row want them: 0 2 8 10, 4 6 12 14, 1 3 9 11, 5 7 13 15.
 template <int CW, int T, int NT>
 __global__ __launch_bounds__(512) void bconv3x3_down_staged_kernel(const BconvDownArgs p) {
     constexpr int C = CW * 64, CH = 16 * NT, LD = CH + 4, AS = C + 4, THREADS = 512;
@@ -106,7 +110,7 @@ __global__ __launch_bounds__(512) void bconv3x3_down_staged_kernel(const BconvDo
     constexpr bool kPair = 2 * CW < KB;
     constexpr int STEPS = kPair ? 2 : 3;
     constexpr int XP = T * (C / 4) / THREADS < 1 ? 1 : T * (C / 4) / THREADS, FP = CH * (C / 4) / THREADS < 1 ? 1 : CH * (C / 4) / THREADS;
-    constexpr int PXG = T / 16, DG = 8 / PXG, DEPTH = C / DG;  // the branch: PXG groups of 16 pixels, DG parts of the depth
+    constexpr int PXG = T / 16, DG = 4;  // the branch: PXG groups of 16 pixels, DG parts of the depth
     __shared__ __attribute__((aligned(16))) float pooled[T][AS];
     __shared__ __attribute__((aligned(16))) float filt[CH][AS];
     __shared__ __attribute__((aligned(16))) float part[3 + DG][T * LD];
@@ -179,43 +183,40 @@ __global__ __launch_bounds__(512) void bconv3x3_down_staged_kernel(const BconvDo
 #pragma unroll
             for (int v = 0; v < Fp4Acc<T>::regs; ++v) part[r][fp4_row<T>(kb, v) * LD + n * T + lr] = acc[n][v];
     }
+    // depths 4 q .. 4 q + 3 of their 16: two places of two
+    auto put = [](float *row, int q, f32x4m v) __attribute__((always_inline)) {
+        typedef float f32x2m __attribute__((ext_vector_type(2)));
+        float *to = row + (q & ~3) * 4 + (q & 1) * 4 + (q & 2);
+        *reinterpret_cast<f32x2m *>(to) = f32x2m{v[0], v[2]};
+        *reinterpret_cast<f32x2m *>(to + 8) = f32x2m{v[1], v[3]};
+    };
 #pragma unroll
     for (int i = 0; i < XP; ++i) {
         const int piece = tid + THREADS * i;
-        if (piece < T * (C / 4)) *reinterpret_cast<f32x4m *>(&pooled[piece / (C / 4)][(piece % (C / 4)) * 4]) = x[i].value();
+        if (piece < T * (C / 4)) put(pooled[piece / (C / 4)], piece % (C / 4), x[i].value());
     }
 #pragma unroll
     for (int i = 0; i < FP; ++i) {
         const int piece = tid + THREADS * i;
-        if (piece < CH * (C / 4)) *reinterpret_cast<f32x4m *>(&filt[piece / (C / 4)][(piece % (C / 4)) * 4]) = f[i];
+        if (piece < CH * (C / 4)) put(filt[piece / (C / 4)], piece % (C / 4), f[i]);
     }
     __syncthreads();
-    {
+    if (r < PXG * DG) {
         const int l16 = lane & 15, k4 = lane >> 4, px = r % PXG, dg = r / PXG;
         f32x4m acc[NT];
 #pragma unroll
         for (int n = 0; n < NT; ++n) acc[n] = zero;
-        if constexpr (DEPTH >= 16) {
 #pragma unroll
-            for (int d = 0; d < DEPTH; d += 16) {
-                const int k = dg * DEPTH + d + 4 * k4;
-                const f32x4m a = *reinterpret_cast<const f32x4m *>(&pooled[px * 16 + l16][k]);
-                f32x4m b[NT];
+        for (int d = 0; d < C; d += 64) {
+            const int k = d + dg * 16 + 4 * k4;
+            const f32x4m a = *reinterpret_cast<const f32x4m *>(&pooled[px * 16 + l16][k]);
+            f32x4m b[NT];
 #pragma unroll
-                for (int n = 0; n < NT; ++n) b[n] = *reinterpret_cast<const f32x4m *>(&filt[n * 16 + l16][k]);
+            for (int n = 0; n < NT; ++n) b[n] = *reinterpret_cast<const f32x4m *>(&filt[n * 16 + l16][k]);
 #pragma unroll
-                for (int e = 0; e < 4; ++e)
+            for (int e = 0; e < 4; ++e)
 #pragma unroll
-                    for (int n = 0; n < NT; ++n) acc[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], b[n][e], acc[n], 0, 0, 0);
-            }
-        } else {
-#pragma unroll
-            for (int d = 0; d < DEPTH; d += 4) {
-                const int k = dg * DEPTH + d + k4;
-                const float a = pooled[px * 16 + l16][k];
-#pragma unroll
-                for (int n = 0; n < NT; ++n) acc[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, filt[n * 16 + l16][k], acc[n], 0, 0, 0);
-            }
+                for (int n = 0; n < NT; ++n) acc[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], b[n][e], acc[n], 0, 0, 0);
         }
 #pragma unroll
         for (int n = 0; n < NT; ++n)
@@ -232,8 +233,7 @@ __global__ __launch_bounds__(512) void bconv3x3_down_staged_kernel(const BconvDo
     for (int i = 0; i < 3 + DG; ++i) s[i] = *reinterpret_cast<f32x4m *>(&part[i][o]);
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-        float t = (s[3][e] + s[4][e]) + (s[5][e] + s[6][e]);
-        if constexpr (DG == 8) t = t + ((s[7][e] + s[8][e]) + (s[9][e] + s[10][e]));
+        const float t = ((s[3][e] + s[4][e]) + s[5][e]) + s[6][e];
         sc[e] = branch_value(t, p.bias != nullptr, bias[e], p.sa != nullptr, sa[e], sb[e]);
         v[e] = down_value(kHalfDepth - 0.5f * (s[0][e] + s[1][e] + s[2][e]), ea[e], eb[e], sc[e]);
     }
@@ -265,7 +265,8 @@ __global__ __launch_bounds__(512) void bconv3x3_down_staged_kernel(const BconvDo
 // asked for when the bits have been counted, into their registers.  14 x 14 x 256 to 512, us, all at once and one block a CU / so: 40
 // images 11.1 / 10.4, 60 20.1 / 17.0, 100 29.6 / 23.6, 256 70.5 / 53.4; a block of eight waves, the floats read half as often, 65.5 there, and
 // three blocks a CU, with spills, 72.5.
-template <int CW, int WAVES, bool POOLED>
+// SPLIT: four sums of a quarter of the depth each, one behind the other, as dab_ave_pool2_fconv1x1 has them for problems this small.
+template <int CW, int WAVES, bool POOLED, bool SPLIT>
 __global__ __launch_bounds__(WAVES * 64, 2) void bconv3x3_down_tile_kernel(const BconvDownArgs p) {
     constexpr int C = CW * 64, AS = C + 4, CH = 32 * WAVES, THREADS = 64 * WAVES;  // AS: rows 4 floats off a multiple of 64 banks
     constexpr int PIECES = 32 * (C / 4) / THREADS;  // 16-byte pieces of the pooled tile per thread
@@ -307,9 +308,12 @@ __global__ __launch_bounds__(WAVES * 64, 2) void bconv3x3_down_tile_kernel(const
     fetch_floats(0, EARLY);
     const float *filter = p.sw + (size_t)(ch_ok ? ch : 0) * C + half * 4;
     f32x4m f[CHUNKS > 1 ? 2 : 1][CHUNK];
+    // the first depth of step i, of C / 8: in order, or all 16-deep pieces of a part and then the next part's
+    constexpr int PART = C / 32;  // steps
+    auto depth_of = [](int i) { return SPLIT ? (i % PART) / 2 * 64 + i / PART * 16 + i % 2 * 8 : i * 8; };
     auto fetch_filters = [&](int chunk) {
 #pragma unroll
-        for (int s = 0; s < CHUNK; ++s) f[chunk & 1][s] = *reinterpret_cast<const f32x4m *>(filter + (chunk * CHUNK + s) * 8);
+        for (int s = 0; s < CHUNK; ++s) f[chunk & 1][s] = *reinterpret_cast<const f32x4m *>(filter + depth_of(chunk * CHUNK + s));
     };
     fetch_filters(0);
     float ea = 0.f, eb = 0.f, bias = 0.f, sa = 0.f, sb = 0.f;
@@ -319,9 +323,9 @@ __global__ __launch_bounds__(WAVES * 64, 2) void bconv3x3_down_tile_kernel(const
         if (p.sa) sa = p.sa[ch], sb = p.sb[ch];
     }
 
-    f32x16m cnt, sum;
+    f32x16m cnt, sum, parts;
 #pragma unroll
-    for (int v = 0; v < 16; ++v) cnt[v] = 0.f, sum[v] = 0.f;
+    for (int v = 0; v < 16; ++v) cnt[v] = 0.f, sum[v] = 0.f, parts[v] = 0.f;
 #pragma unroll
     for (int t = 0; t < 9; ++t)
 #pragma unroll
@@ -343,10 +347,19 @@ __global__ __launch_bounds__(WAVES * 64, 2) void bconv3x3_down_tile_kernel(const
         if (chunk + 1 < CHUNKS) fetch_filters(chunk + 1);
 #pragma unroll
         for (int s = 0; s < CHUNK; ++s) {
-            const f32x4m a = *reinterpret_cast<const f32x4m *>(&pooled[l32][(chunk * CHUNK + s) * 8 + half * 4]);
+            const int step = chunk * CHUNK + s;
+            if (SPLIT && step > 0 && step % PART == 0) {
+#pragma unroll
+                for (int v = 0; v < 16; ++v) parts[v] = step == PART ? sum[v] : parts[v] + sum[v], sum[v] = 0.f;
+            }
+            const f32x4m a = *reinterpret_cast<const f32x4m *>(&pooled[l32][depth_of(step) + half * 4]);
 #pragma unroll
             for (int e = 0; e < 4; ++e) sum = __builtin_amdgcn_mfma_f32_32x32x2f32(a[e], f[chunk & 1][s][e], sum, 0, 0, 0);
         }
+    }
+    if constexpr (SPLIT) {
+#pragma unroll
+        for (int v = 0; v < 16; ++v) sum[v] = parts[v] + sum[v];
     }
 
     constexpr float kHalfDepth = 0.5f * 9 * C;
@@ -371,20 +384,17 @@ __global__ __launch_bounds__(WAVES * 64, 2) void bconv3x3_down_tile_kernel(const
 }
 
 // ---------------------------------------------------------------- many pieces: blocks that walk over pixel tiles
-// A wave keeps the filters of 32 channels for its lifetime, the branch's as three planes of bf16 (common.h: six products per 16
-// depths, fp32 accuracy, the cross terms in a sum of their own), and a block walks over tiles of 32 pixels: it pools and splits a
-// tile into LDS while the next one's floats and bits are on their way.  A tile (or a wave's filters) with an infinity, a NaN or a
-// value too small for the split is made on the fp32 matrix instruction.  With 64 input channels bound by memory: 256 images of
-// 56 x 56 x 64 to 128 move 315 MB in 61 us, 5.2 TB/s, the rate of a copy (tile kernel 75, two launches 100).  With 128 a block has eight
-// waves, so that the floats are read once: 28 x 28 at 256 images 43 us (tile 63, two launches 68; four waves 63).  256 input
-// channels, whose filters take 192 registers, were slower (14 x 14 at 256 images 64 us, tile kernel 53).
+// A wave keeps the filters of 32 channels for its lifetime, and a block walks over tiles of 32 pixels: it pools a tile into LDS while
+// the next one's floats and bits are on their way.  Bound by its instructions, of which vector and matrix ones do not overlap here: 256
+// images of 56 x 56 x 64 to 128 take 61 us (two launches 96, the tile kernel 66), 51 from the pooled tensor (tile kernel 57) -- of 125 000
+// cycles, the fp32 matrix instructions of a SIMD have 50 000, counting 7 000, the vector instructions 31 000 and more.  With 128 input channels a
+// block has eight waves, so that the floats are read once: 28 x 28 at 256 images 55 us (two launches 67, tile kernel 57).  (The same with the
+// products on the bf16 matrix instruction, in three parts each: 60, 47 and 43 us, but not the separate launch's sums to the last bit.)
 template <int CW, int WAVES, bool POOLED>
-__global__ __launch_bounds__(WAVES * 64, 2) void bconv3x3_down_walk_kernel(const BconvDownArgs p) {
+__global__ __launch_bounds__(WAVES * 64, CW == 1 ? 3 : 2) void bconv3x3_down_walk_kernel(const BconvDownArgs p) {
     constexpr int C = CW * 64, CH = 32 * WAVES, THREADS = 64 * WAVES;
-    constexpr int PIECES = 32 * (C / 4) / THREADS, GROUPS = C / 16;
-    constexpr int ROW = C + 8, PLANE = 32 * ROW;  // bf16 elements; rows 4 dwords off a multiple of 32: a quarter wave's reads hit all banks
-    extern __shared__ __attribute__((aligned(16))) uint16_t planes[];  // [buffer][plane][pixel][depth]
-    __shared__ int special_tile[2];
+    constexpr int PIECES = 32 * (C / 4) / THREADS, AS = C + 4;  // AS: rows 4 floats off a multiple of 64 banks
+    __shared__ __attribute__((aligned(16))) float pooled[2][32][AS];
     const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5, l32 = lane & 31;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int group = (int)p.div_cols.div(blockIdx.x), groups = (int)p.div_cols.div(gridDim.x);
@@ -392,7 +402,6 @@ __global__ __launch_bounds__(WAVES * 64, 2) void bconv3x3_down_walk_kernel(const
     const bool ch_ok = ch0 < p.cout;  // (32 channels are all there or none)
     const int tiles = (p.total + 31) / 32;
     const __amdgpu_buffer_rsrc_t rx = make_rsrc(p.x, p.x_bytes), rw = make_rsrc(p.w, p.w_bytes);
-    typedef SplitFrag8::u4 u4;
 
     DownPiece<POOLED> x[PIECES];
     uint32_t act[9][CW];
@@ -419,22 +428,10 @@ __global__ __launch_bounds__(WAVES * 64, 2) void bconv3x3_down_walk_kernel(const
     uint32_t wt[9][CW];
 #pragma unroll
     for (int t = 0; t < 9; ++t) load_dwords<CW>(wt[t], rw, ch_ok ? ch * (CW * 72) + t * (CW * 8) + half * (CW * 4) : kDownOutside);
-    const float *filter = p.sw + (size_t)(ch_ok ? ch : 0) * C;
-    u4 fhi[GROUPS], fmid[GROUPS], flo[GROUPS];
-    uint32_t fsmall = ~0u, ftop = 0;
+    const float *filter = p.sw + (size_t)(ch_ok ? ch : 0) * C + half * 4;
+    f32x4m f[C / 8];
 #pragma unroll
-    for (int g = 0; g < GROUPS; ++g) {
-        const f32x4m v0 = *reinterpret_cast<const f32x4m *>(filter + g * 16 + half * 8), v1 = *reinterpret_cast<const f32x4m *>(filter + g * 16 + half * 8 + 4);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const float a = e < 2 ? v0[2 * e] : v1[2 * e - 4], b = e < 2 ? v0[2 * e + 1] : v1[2 * e - 3];
-            fsmall = smallest_magnitude(fsmall, a, b);
-            const SplitPair sp = split_pair_finite(a, b);
-            ftop = bf16_pair_max(ftop, sp.hi);
-            fhi[g][e] = sp.hi, fmid[g][e] = sp.mid, flo[g][e] = sp.lo;
-        }
-    }
-    const bool filter_special = __builtin_amdgcn_ballot_w64(loses_bits_when_split(fsmall) || !bf16_pairs_finite(ftop)) != 0;
+    for (int i = 0; i < C / 8; ++i) f[i] = *reinterpret_cast<const f32x4m *>(filter + i * 8);
     uint32_t set = 0;
 #pragma unroll
     for (int t = 0; t < 9; ++t)
@@ -448,61 +445,30 @@ __global__ __launch_bounds__(WAVES * 64, 2) void bconv3x3_down_walk_kernel(const
         if (p.bias) bias = p.bias[ch];
         if (p.sa) sa = p.sa[ch], sb = p.sb[ch];
     }
-    if (tid < 2) special_tile[tid] = -1;
-    __syncthreads();
+
+    // here, and not at their first use inside the loop: there the wait would be for the next tile's floats as well
+#pragma unroll
+    for (int i = 0; i < C / 8; ++i) asm volatile("" : "+v"(f[i]));
+    asm volatile("" : "+v"(ea), "+v"(eb), "+v"(bias), "+v"(sa), "+v"(sb));
 
     for (int buf = 0; tile < tiles; tile += groups, buf ^= 1) {
-        uint16_t *const out_planes = planes + buf * 3 * PLANE;
-        uint32_t small = ~0u, top = 0;
 #pragma unroll
         for (int i = 0; i < PIECES; ++i) {
             const int piece = tid + THREADS * i;
-            const f32x4m v = x[i].value();
-            small = smallest_magnitude(smallest_magnitude(small, v[0], v[1]), v[2], v[3]);
-            const SplitPair s0 = split_pair_finite(v[0], v[1]), s1 = split_pair_finite(v[2], v[3]);
-            top = bf16_pair_max(bf16_pair_max(top, s0.hi), s1.hi);
-            uint16_t *d = out_planes + (piece / (C / 4)) * ROW + (piece % (C / 4)) * 4;
-            *reinterpret_cast<u32x2 *>(d) = u32x2{s0.hi, s1.hi};
-            *reinterpret_cast<u32x2 *>(d + PLANE) = u32x2{s0.mid, s1.mid};
-            *reinterpret_cast<u32x2 *>(d + 2 * PLANE) = u32x2{s0.lo, s1.lo};
+            *reinterpret_cast<f32x4m *>(&pooled[buf][piece / (C / 4)][(piece % (C / 4)) * 4]) = x[i].value();
         }
-        if (loses_bits_when_split(small) || !bf16_pairs_finite(top)) special_tile[buf] = tile;
         const bool more = tile + groups < tiles;
         if (more) fetch_floats(tile + groups);
         __syncthreads();
         f32x16m sum;
 #pragma unroll
         for (int v = 0; v < 16; ++v) sum[v] = 0.f;
-        if (!filter_special && special_tile[buf] != tile) {
-            f32x16m cross = sum;
-            const uint16_t *src = out_planes + l32 * ROW + half * 8;
-            auto v = [](u4 w) { return __builtin_bit_cast(bf16x8, w); };
 #pragma unroll
-            for (int g = 0; g < GROUPS; ++g) {
-                const u4 hi = *reinterpret_cast<const u4 *>(src + g * 16), mid = *reinterpret_cast<const u4 *>(src + g * 16 + PLANE),
-                         lo = *reinterpret_cast<const u4 *>(src + g * 16 + 2 * PLANE);
-                cross = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v(lo), v(fhi[g]), cross, 0, 0, 0);
-                sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v(hi), v(fhi[g]), sum, 0, 0, 0);
-                cross = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v(hi), v(flo[g]), cross, 0, 0, 0);
-                cross = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v(mid), v(fmid[g]), cross, 0, 0, 0);
-                cross = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v(mid), v(fhi[g]), cross, 0, 0, 0);
-                cross = __builtin_amdgcn_mfma_f32_32x32x16_bf16(v(hi), v(fmid[g]), cross, 0, 0, 0);
-            }
+        for (int i = 0; i < C / 8; ++i) {
+            const f32x4m a = *reinterpret_cast<const f32x4m *>(&pooled[buf][l32][i * 8 + half * 4]);
 #pragma unroll
-            for (int e = 0; e < 16; ++e) sum[e] = sum[e] + cross[e];
-        } else {
-            const int pix = tile * 32 + l32 < p.total ? tile * 32 + l32 : p.total - 1;
-#pragma unroll 1
-            for (int d = half * 4; d < C; d += 8) {
-                DownPiece<POOLED> again;
-                again.fetch(p, pix, d, C);
-                const f32x4m a = again.value(), b = *reinterpret_cast<const f32x4m *>(filter + d);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) sum = __builtin_amdgcn_mfma_f32_32x32x2f32(a[e], b[e], sum, 0, 0, 0);
-            }
+            for (int e = 0; e < 4; ++e) sum = __builtin_amdgcn_mfma_f32_32x32x2f32(a[e], f[i][e], sum, 0, 0, 0);
         }
-#pragma unroll
-        for (int v = 0; v < 16; ++v) sum[v] = branch_value(sum[v], p.bias != nullptr, bias, p.sa != nullptr, sa, sb);
         f32x16m cnt;
 #pragma unroll
         for (int v = 0; v < 16; ++v) cnt[v] = init;
@@ -519,19 +485,26 @@ __global__ __launch_bounds__(WAVES * 64, 2) void bconv3x3_down_walk_kernel(const
         const int rows = p.total - tile * 32 < 32 ? p.total - tile * 32 : 32;
         const __amdgpu_buffer_rsrc_t ro = make_rsrc(p.out + base, (uint32_t)rows * p.cout * 4u);
         const __amdgpu_buffer_rsrc_t rs = make_rsrc(p.sc_out + (p.sc_out ? base : 0), p.sc_out ? (uint32_t)rows * p.cout * 4u : 0u);
-        int lane_off = ch_ok ? (half * 4 * p.cout + ch) * 4 : kDownOutside;
-        asm volatile("" : "+v"(lane_off));  // sixteen offsets kept from tile to tile would not fit
+        const int lane_off = ch_ok ? (half * 4 * p.cout + ch) * 4 : kDownOutside;
         uint32_t word = 0;
+        auto finish = [&](auto usual) __attribute__((always_inline)) {  // a converter's block: an Affine and no bias, the branch's blob not wanted
+            constexpr bool U = decltype(usual)::value;
 #pragma unroll
-        for (int v = 0; v < 16; ++v) {
-            const int row = 8 * (v / 4) + v % 4;
-            const float sc = sum[v], r = down_value(cnt[v], ea, eb, sc);
-            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, r), ro, lane_off + row * p.cout * 4, 0, kStoreStream);
-            if (p.sc_out) __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, sc), rs, lane_off + row * p.cout * 4, 0, 0);
-            const uint64_t mask = __ballot(r > 0.f);
-            word = dab_writelane((uint32_t)mask, row, word);
-            word = dab_writelane((uint32_t)(mask >> 32), row + 4, word);
-        }
+            for (int v = 0; v < 16; ++v) {
+                const int row = 8 * (v / 4) + v % 4;
+                const float sc = U ? branch_value(sum[v], false, 0.f, true, sa, sb) : branch_value(sum[v], p.bias != nullptr, bias, p.sa != nullptr, sa, sb);
+                const float r = down_value(cnt[v], ea, eb, sc);
+                __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, r), ro, lane_off, row * p.cout * 4, kStoreStream);
+                if (!U && p.sc_out) __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, sc), rs, lane_off, row * p.cout * 4, 0);
+                const uint64_t mask = __ballot(r > 0.f);
+                word = dab_writelane((uint32_t)mask, row, word);
+                word = dab_writelane((uint32_t)(mask >> 32), row + 4, word);
+            }
+        };
+        if (p.sa && !p.bias && !p.sc_out)
+            finish(std::true_type{});
+        else
+            finish(std::false_type{});
         if (p.bits && half == 0 && l32 < rows && ch_ok) p.bits[((size_t)tile * 32 + l32) * (p.cout / 32) + ch0 / 32] = word;
     }
 }
@@ -548,20 +521,21 @@ static bool down_geometry(BconvDownArgs &a, int n, int h, int w, int cin, int co
     return true;
 }
 
-enum class Down { staged16, staged32, tile, walk };
-// By 32-pixel x 32-channel pieces, us:
-//   16 x 16 tiles up to 128 pieces of 128 and 256 input channels: 28 x 28 x 128 at batch 1 (56 pieces) 3.7 against 4.2, at batch 4
-//   (200) 6.1 against 4.5; 14 x 14 x 256 at batch 2 (64) 4.1 against 5.6, at batch 6 (160) 6.8 against 5.8
-//   32 x 32 tiles up to 700 pieces (64 input channels) and 512: 56 x 56 x 64 at batch 6 (588) 5.7 against the tile kernel's 6.4, at
-//   batch 9 (884) 7.5 against 6.5; 28 x 28 x 128 at batch 9 (448) 6.0 against 7.5, at batch 16 (784) 12.4 against 7.7; 14 x 14 x 256 at
-//   batch 16 (400) 9.7 against 10.8
-//   walking from 2600 pieces: 56 x 56 x 64 at batch 16 (1568) 9.3 against the tile kernel's 9.1, at batch 40 (3920) 13.6 against 15.5;
-//   28 x 28 x 128 at batch 40 (1960) 13.8 against 12.0, at batch 100 (4904) 23 against 27
+enum class Down { staged16, staged32, tile_split, tile, walk };
+// The branch's sums are dab_ave_pool2_fconv1x1's to the bit, so it follows from that call's rule whether the depth is split: for problems
+// of up to about 768 pieces of 32 pixels x 32 channels (512 with 64 output channels).  us:
+//   16 x 16 tiles up to 128 pieces of 128 and 256 input channels: 28 x 28 x 128 at batch 1 (56 pieces) 3.5 against 4.2, at batch 4
+//   (200) 6.1 against 4.5; 14 x 14 x 256 at batch 2 (64) 4.0 against 5.6, at batch 6 (160) 6.8 against 5.7
+//   32 x 32 tiles up to 700 pieces (64 input channels) and 512: 56 x 56 x 64 at batch 6 (588) 5.6 against the tile kernel's 6.4; 28 x 28 x
+//   128 at batch 9 (448) 6.0 against 7.5; 14 x 14 x 256 at batch 16 (400) 9.7 against 10.8
+// and in one sum, for which a block needs whole depths:
+//   walking from 780 tiles of 32 pixels: 56 x 56 x 64 to 128 at batch 30 (735) 11.7 against the tile kernel's 11.4, at 40 14.1 / 14.5, at
+//   100 28.9 / 29.8; 28 x 28 x 128 to 256 at batch 100 (613) 26.7 / 25.1, at 150 (919) 35.4 / 37.3; 64 to 256 channels at 735 20.6 / 18.4
 static Down pick_down(long long total, int cin, int cout) {
-    const long long pieces = (total + 31) / 32 * (cout / 32);
+    const long long tiles = (total + 31) / 32, pieces = tiles * (cout / 32);
+    if (!pool2_fconv1x1_splits_depth(total, cout)) return cin <= 128 && tiles >= 780 ? Down::walk : Down::tile;
     if (cin >= 128 && pieces <= 128) return Down::staged16;
-    if (pieces <= (cin == 64 ? 700 : 512)) return Down::staged32;
-    return cin <= 128 && pieces >= 2600 ? Down::walk : Down::tile;
+    return pieces <= (cin == 64 ? 700 : 512) ? Down::staged32 : Down::tile_split;
 }
 
 template <class Kernel>
@@ -578,24 +552,17 @@ static int launch_down(Kernel kernel, BconvDownArgs &a, int px, int ch, int thre
 template <int CW, int WAVES, bool POOLED>
 static int launch_down_walk(BconvDownArgs &a, hipStream_t s) {
     constexpr int CH = 32 * WAVES;
-    constexpr size_t lds = 2 * 3 * 32 * (CW * 64 + 8) * 2;
     auto kernel = bconv3x3_down_walk_kernel<CW, WAVES, POOLED>;
     a.cols = (a.cout + CH - 1) / CH;
     a.div_cols = FastDiv((uint32_t)a.cols);
-    if (lds > 64 * 1024) {
-        const int rc = allow_dynamic_lds<bconv3x3_down_walk_kernel<CW, WAVES, POOLED>>("dab_bconv3x3_down", lds);
-        if (rc != DAB_OK) return rc;
-    }
     static const int per_cu = [&] {
         int blocks = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, kernel, WAVES * 64, lds) != hipSuccess || blocks < 1) blocks = 1;
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&blocks, kernel, WAVES * 64, 0) != hipSuccess || blocks < 1) blocks = 1;
         return blocks;
     }();
     const int tiles = (int)(((long long)a.total + 31) / 32), most = simd_count() / 4 * per_cu / a.cols;
-    int groups = tiles < most ? tiles : most < 1 ? 1 : most;
-    const int per_block = (tiles + groups - 1) / groups;
-    groups = (tiles + per_block - 1) / per_block;
-    hipLaunchKernelGGL(kernel, dim3((unsigned)(groups * a.cols)), dim3(WAVES * 64), lds, s, a);
+    const int groups = tiles < most ? tiles : most < 1 ? 1 : most;  // (equal shares on fewer blocks: 64 images 25.7 us instead of 22.3, 256 64 instead of 61)
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(groups * a.cols)), dim3(WAVES * 64), 0, s, a);
     DAB_LAUNCH_CHECK();
     return DAB_OK;
 }
@@ -609,7 +576,8 @@ static int launch_bconv_down(BconvDownArgs &a, hipStream_t s) {
         if (kernel == Down::staged32) return launch_down(bconv3x3_down_staged_kernel<CW, 32, 2>, a, 32, 32, 512, s);
     if constexpr (CW <= 2)
         if (kernel == Down::walk) return launch_down_walk<CW, 4 * CW, POOLED>(a, s);
-    return launch_down(bconv3x3_down_tile_kernel<CW, 4, POOLED>, a, 32, 128, 256, s);
+    if (kernel != Down::tile) return launch_down(bconv3x3_down_tile_kernel<CW, 4, POOLED, true>, a, 32, 128, 256, s);
+    return launch_down(bconv3x3_down_tile_kernel<CW, 4, POOLED, false>, a, 32, 128, 256, s);
 }
 
 }  // namespace dab

@@ -66,6 +66,10 @@ int fconv_c32_pool_run(const float *x, int n, int h, int w, const float *wgt, co
                        const float *aff_b, int relu, int pad_h, int pad_w, int cout, int oh, int ow, float *pooled,
                        uint64_t *pooled_packed, float *work, hipStream_t s);
 
+// Whether dab_ave_pool2_fconv1x1 adds the sums of so many pooled pixels (more than eight) in four parts -- part i the depths 16 i to
+// 16 i + 15 of every 64, the parts then in order -- or in one: eight depths at a time, d and d + 4 one behind the other.
+bool pool2_fconv1x1_splits_depth(long long pixels, int cout);
+
 // A launch has fewer than 2^32 threads (hipLaunchKernel refuses more): grids that grow with the problem are launched in
 // pieces of this many blocks of up to 256 threads.
 constexpr long long kMostBlocks = 1ll << 23;

@@ -1068,6 +1068,13 @@ static int small_1x1_tiles(int taps, long long M, int cout) {
     return 3;
 }
 
+bool dab::pool2_fconv1x1_splits_depth(long long M, int cout) {
+    const int bn = cout <= 32 ? 32 : cout <= 64 ? 64 : 128;
+    if (((M + 127) / 128) * ((cout + bn - 1) / bn) >= simd_count() / 4) return false;
+    const int small = small_1x1_tiles(1, M, cout);
+    return small == 3 || (small == 0 && ((M + 63) / 64) * ((cout + 63) / 64) < simd_count() / 8);
+}
+
 // Whether a 1x1 convolution to more than 64 channels takes 64 x 64 tiles in 32-deep slices: from three quarters of the CUs
 // on.  Four blocks of a CU cover each other's loads, and the last round of blocks is a shorter one than with 128 x 128 tiles
 // in 16-deep slices (16 x 16 x 256 -> 128, 128 images: 22.1 us against 25.4; 14 x 14 x 512 -> 256, 256 images: 116 against
@@ -1378,10 +1385,7 @@ extern "C" int dab_ave_pool2_fconv1x1(const float *x, int n, int h, int w, int c
     // Bit for bit the 1x1 convolution of the pooled tensor: a tile's sums run over the depth in order, whatever the tile and
     // its slices, but where the depth is split over the waves -- that is done here for the problems for which
     // dab_fconv_affine_relu does it
-    const bool few = big_tiles < simd_count() / 4;
-    const int small = few ? small_1x1_tiles(1, M, cout) : 0;
-    const bool depth_split = few && (small == 3 || (small == 0 && ((M + 63) / 64) * ((cout + 63) / 64) < simd_count() / 8));
-    if (c == 64 && cout > 64 && !depth_split && (long long)cout * c * 4 < (1ll << 30))
+    if (c == 64 && cout > 64 && !pool2_fconv1x1_splits_depth(M, cout) && (long long)cout * c * 4 < (1ll << 30))
         // 64 input channels: the launch is bound by the input it reads, and the kernel that pools whole pixels once
         // into LDS reads it at the rate of a copy (256 x 56 x 56 x 64 -> 128: 66 us against 85, 58 without the pooled
         // tensor; batch 8: 5.2 against 6.1).  With 128 and 256 channels the two forms take the same time at batch

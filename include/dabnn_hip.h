@@ -208,8 +208,8 @@ DAB_API int dab_bconv3x3_pair_pool_takes(int n, int h, int w);
  *   out = a * bconv3x3(x_packed, stride 2, pad 1) + b + (sc_a * (conv1x1(avepool2x2(x)) + sc_bias) + sc_b)
  * x [n][h][w][cin] floats with x_packed = pack_mat(x), or, with x_pooled, avepool2x2(x) [n][h/2][w/2][cin] in its place; wgt as dab_bconv3x3, sc_wgt [cout][cin]; sc_bias, and sc_a with sc_b, may be NULL.
  * out [n][h/2][w/2][cout]; out_packed = pack_mat(out) and shortcut (what the branch adds) are written unless NULL.  No
- * result may overlap an input.  Every operation behind the sums is rounded by itself, as in the separate layers; the branch's fp32
- * sums may be added in another order than dab_ave_pool2_fconv1x1's.  Buffers 16-byte aligned (wgt and out_packed 8).
+ * result may overlap an input.  Every operation behind the sums is rounded by itself, as in the separate layers; beyond
+ * eight output pixels the branch's fp32 sums are dab_ave_pool2_fconv1x1's to the bit.  Buffers 16-byte aligned (wgt and out_packed 8).
  * DAB_EUNSUPPORTED for shapes that dab_bconv3x3_down_takes answers with 0: it takes 64, 128 and 256 input channels, multiples of 64
  * output channels and even h and w, within 32-bit pixel numbers.
  */

@@ -142,6 +142,45 @@ def test_no_further_from_64_bits_than_the_separate_launch(gpu, n, h, cin, cout):
     assert rel <= 1.02 * before
 
 
+# more than eight pooled pixels (fewer go to a matrix-vector kernel in the separate launch), and the sizes around which that launch
+# splits the depth over its waves and those at which this one changes its tiles
+BRANCH_SHAPES = [s for s in SHAPES if s[0] * s[1] * s[2] > 32] + [
+    (3, 2, 6, 64, 64), (11, 28, 28, 128, 256), (15, 28, 28, 128, 256), (21, 14, 14, 256, 512), (30, 14, 14, 256, 512), (7, 56, 56, 64, 128), (10, 48, 48, 64, 128),
+    (1, 128, 190, 64, 128), (1, 156, 156, 64, 128), (1, 128, 254, 64, 64), (1, 144, 226, 64, 64), (1, 126, 128, 128, 192), (1, 128, 128, 128, 192),
+    (1, 8, 8, 64, 12288), (1, 8, 8, 256, 12224), (256, 14, 14, 256, 512)]
+# blocks that walk over pixel tiles, from 780 tiles on: either side of that, last tiles of 1 to 31 pixels, channel blocks that are not full
+WALK_SHAPES = [(1, 312, 320, 64, 64), (1, 310, 320, 64, 64), (45, 50, 46, 64, 192), (33, 56, 56, 64, 320), (1, 2, 50562, 64, 128), (1, 320, 312, 128, 64),
+               (131, 30, 26, 128, 320), (128, 28, 28, 128, 256), (515, 14, 14, 128, 448)]
+BRANCH_SHAPES += WALK_SHAPES
+
+
+@pytest.mark.parametrize("n,h,w,cin,cout", WALK_SHAPES)
+@pytest.mark.parametrize("with_bias,with_affine", [(False, True), (True, True), (False, False)])
+def test_walking_blocks(gpu, n, h, w, cin, cout, with_bias, with_affine):
+    x, wt, v, sw = problem(gpu, n, h, w, cin, cout, n + cout)
+    r = np.random.default_rng(n)
+    for value in (float("inf"), -float("inf"), float("nan")):
+        x[int(r.integers(n)), int(r.integers(h)), int(r.integers(w)), int(r.integers(cin))] = value
+    check(gpu, x, wt, v, sw, cout, with_bias, with_affine, special=True)
+
+
+@pytest.mark.parametrize("n,h,w,cin,cout", BRANCH_SHAPES)
+def test_branch_is_the_separate_launchs_to_the_bit(gpu, n, h, w, cin, cout):
+    """The sums of dab_ave_pool2_fconv1x1, in its order, from the whole and from the pooled tensor."""
+    torch, dab, capi = gpu
+    x, wt, v, sw = problem(gpu, n, h, w, cin, cout, n + h + cin)
+    packed = dab.pack_mat(x)
+    pooled, want = torch.empty((n, h // 2, w // 2, cin), device="cuda"), torch.empty((n, h // 2, w // 2, cout), device="cuda")
+    for bias, branch in ((v[4], (v[2], v[3])), (None, (None, None))):
+        rc = capi.lib.dab_ave_pool2_fconv1x1(ptr(x), n, h, w, cin, ptr(sw), ptr(bias), ptr(branch[0]), ptr(branch[1]), 0, cout, ptr(pooled), ptr(want),
+                                             ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+        assert rc == 0, capi.lib.dab_last_error()
+        for given in (None, pooled):
+            _, got, _ = down(gpu, x, packed, wt, v, sw, bias, branch, cout, pooled=given)
+            differ = (got.view(torch.int32) != want.view(torch.int32)).float().mean().item()
+            assert differ == 0, "%.3g of the values differ, %s" % (differ, "pooled" if given is not None else "whole")
+
+
 def block_net(models, n_in, cout, hw, seed=0, relu=False, second_reader=False):
     """1x1 convolution to n_in channels -> down-sampling block -> binary convolution -> classifier."""
     r = np.random.default_rng(seed)
