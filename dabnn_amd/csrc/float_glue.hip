@@ -399,20 +399,20 @@ __global__ __launch_bounds__(256) void fconv_kernel(const FconvArgs p) {
 
 // 3x3 windows over three-channel images to up to 64 channels (a first layer): 27 depths, too few to stage.  Bound by what it writes:
 // a wave takes 32 pixels x all channels, its filters stay in registers and each lane fetches five taps of its pixel with one 12-byte load each
-// -- the lower half of the lanes taps 0..4, the upper half 5..8 and 4 -- while the tile before is multiplied, fourteen instructions of two depths
-// per 32 channels.  us, the tile kernel / this one: 3 -> 64 over 32 x 32, 128 images, with PRelu and sign bits,
-// into slices 15.2 / 12.2; 3 -> 32, stride 2, over 224 x 224, 1 / 6 / 20 / 100 / 256 images 4.7 / 4.1, 6.7 / 6.3, 14.0 / 10.8, 51 / 42, 145 / 99.
-// Every second (fourth) step has a sum of its own, so that the error against 64 bits is no larger than the tile kernels', which split the
-// depth of small problems over four waves.
-template <int NT, bool STREAM>
+// -- the lower half of the lanes taps 0..4, the upper half 5..8 and 7 -- while the tile before is multiplied, fifteen instructions of two depths
+// per 32 channels.  us, the tile kernel / this one: 3 -> 64 over 32 x 32, 128 images, with PRelu and sign bits, into slices 14.6 / 11.9;
+// 3 -> 32, stride 2, over 224 x 224, 1 / 6 / 20 / 100 / 256 images 4.6 / 3.9, 6.8 / 6.2, 14.0 / 10.8, 50 / 43, 143 / 97.
+// The sums are fconv_kernel's to the bit: eight depths at a time, d and d + 4 in one instruction, for which the halves of the lanes
+// exchange what they have fetched; SPLIT, where that kernel splits the depth over its waves (64 at a time: 0..15 and 16..26 here), in two parts.
+template <int NT, bool STREAM, bool SPLIT>
 __global__ __launch_bounds__(256, NT == 2 ? 3 : 4) void fconv_rgb3x3_kernel(const FconvArgs p) {
-    constexpr int STEPS = 14, SUMS = NT == 1 ? 4 : 2;
+    constexpr int STEPS = 15, PARTS = SPLIT ? 2 : 1;
     typedef float f32x3 __attribute__((ext_vector_type(3)));
     const int lane = threadIdx.x & 63, half = lane >> 5, l32 = lane & 31;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int tiles = (p.M + 31) / 32, step = (int)gridDim.x * 4;
     __shared__ float filters[NT * 32 * 27];
-    auto tap_of = [&](int j) { return half == 0 ? j : j < 4 ? 5 + j : 4; };
+    auto tap_of = [&](int j) { return half == 0 ? j : j < 4 ? 5 + j : 7; };
 
     f32x3 x[5], next[5];
     auto fetch = [&](f32x3 (&v)[5], int tile) __attribute__((always_inline)) {
@@ -438,7 +438,7 @@ __global__ __launch_bounds__(256, NT == 2 ? 3 : 4) void fconv_rgb3x3_kernel(cons
     __syncthreads();
     if (!any) return;
 
-    // the filters in the order of the taps: element c of load j, then what load 4 leaves for the two halves (elements 0, 1 and 2)
+    // step s: depths 8 (s / 4) + s % 4 and, but for the last three, 4 more
     float w[STEPS][NT], bias[NT], fa[NT], fb[NT], slope[NT];
     int out_lane[NT];
 #pragma unroll
@@ -447,8 +447,8 @@ __global__ __launch_bounds__(256, NT == 2 ? 3 : 4) void fconv_rgb3x3_kernel(cons
         const bool ok = co < p.cout;
 #pragma unroll
         for (int s = 0; s < STEPS; ++s) {
-            const int place = s < 12 ? tap_of(s / 3) * 3 + s % 3 : s == 12 ? (half ? 14 : 12) : 13;
-            w[s][n] = s == 13 && half ? 0.f : filters[co * 27 + place];
+            const float v = filters[co * 27 + (s / 4) * 8 + s % 4 + (s < 12 ? 4 * half : 0)];
+            w[s][n] = s >= 12 && half ? 0.f : v;
         }
         bias[n] = ok && p.bias ? p.bias[co] : 0.f;
         fa[n] = ok && p.aff_a ? p.aff_a[co] : 0.f, fb[n] = ok && p.aff_a ? p.aff_b[co] : 0.f;
@@ -462,26 +462,41 @@ __global__ __launch_bounds__(256, NT == 2 ? 3 : 4) void fconv_rgb3x3_kernel(cons
     for (;; tile += step) {
         const bool more = tile + step < tiles;
         if (more) fetch(next, tile + step);
-        f32x16 acc[NT], part[SUMS][NT];
+        // a[i]: depth i in the lower lanes and 15 + i (the last three: 21, 22, 23) in the upper ones, exchanged into the steps' pairs
+        float a[STEPS], step[STEPS];
 #pragma unroll
-        for (int i = 0; i < SUMS; ++i)
+        for (int i = 0; i < STEPS; ++i) a[i] = x[i / 3][i % 3];
+        auto swap = [](float &u, float &v) __attribute__((always_inline)) {  // the upper lanes of u and the lower ones of v
+            const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, u), __builtin_bit_cast(uint32_t, v), false, false);
+            const uint32_t first = r[0], second = r[1];  // (a bit cast of an element itself would take the first)
+            u = __builtin_bit_cast(float, first), v = __builtin_bit_cast(float, second);
+        };
+        swap(a[0], a[4]), swap(a[1], a[5]), swap(a[2], a[6]), swap(a[3], a[7]);  // 0 4, 1 5, 2 6, 3 7 and 15 19, 16 20, 17 21, 18 22
+        swap(a[8], a[12]), swap(a[9], a[13]), swap(a[10], a[14]);                // 8 12, 9 13, 10 14 and 23 21, 24 22, 25 23
+        swap(a[11], a[4]);                                                        // 11 15 and 26 19
+        step[12] = half ? 0.f : a[13], step[13] = half ? 0.f : a[14], step[14] = half ? 0.f : a[4];
+        swap(a[4], a[14]);  // 26 25 and 19 23
+#pragma unroll
+        for (int i = 0; i < 4; ++i) step[i] = a[i], step[4 + i] = a[8 + i];
+        step[8] = a[5], step[9] = a[6], step[10] = a[7], step[11] = a[14];
+        f32x16 acc[NT], part[PARTS][NT];
+#pragma unroll
+        for (int i = 0; i < PARTS; ++i)
 #pragma unroll
             for (int n = 0; n < NT; ++n)
 #pragma unroll
                 for (int e = 0; e < 16; ++e) part[i][n][e] = 0.f;
 #pragma unroll
-        for (int s = 0; s < STEPS; ++s) {
-            const float a = s < 12 ? x[s / 3][s % 3] : s == 12 ? (half ? x[4][2] : x[4][0]) : (half ? 0.f : x[4][1]);
+        for (int s = 0; s < STEPS; ++s)
 #pragma unroll
-            for (int n = 0; n < NT; ++n) part[s % SUMS][n] = __builtin_amdgcn_mfma_f32_32x32x2f32(a, w[s][n], part[s % SUMS][n], 0, 0, 0);
-        }
+            for (int n = 0; n < NT; ++n) {
+                f32x16 &sum = part[SPLIT && s >= 8][n];
+                sum = __builtin_amdgcn_mfma_f32_32x32x2f32(step[s], w[s][n], sum, 0, 0, 0);
+            }
 #pragma unroll
         for (int n = 0; n < NT; ++n)
 #pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                acc[n][e] = part[0][n][e] + part[1][n][e];
-                if constexpr (SUMS == 4) acc[n][e] = acc[n][e] + (part[2][n][e] + part[3][n][e]);
-            }
+            for (int e = 0; e < 16; ++e) acc[n][e] = SPLIT ? part[0][n][e] + part[PARTS - 1][n][e] : part[0][n][e];
         const int m0 = tile * 32, rows = p.M - m0 < 32 ? p.M - m0 : 32;
         const auto o_rsrc = make_rsrc(p.out + (size_t)m0 * p.out_ld, (uint32_t)((rows - 1) * p.out_ld + p.cout) * 4u);
         // accumulator element e of lane l: pixel 8 * (e / 4) + 4 * (l / 32) + e % 4, channel l % 32
@@ -1186,10 +1201,12 @@ static int fconv_impl(const char *fn, const float *x, int n, int h, int w, int c
         const bool stream_out = M * cout * 4 >= (256ll << 20);
         auto launch = [&](auto nt) {
             constexpr int NT = decltype(nt)::value;
-            if (stream_out)
-                hipLaunchKernelGGL((fconv_rgb3x3_kernel<NT, true>), grid, dim3(256), 0, s, a);
+            if (big_tiles < simd_count() / 4)  // where the tile kernel splits the depth
+                hipLaunchKernelGGL((fconv_rgb3x3_kernel<NT, false, true>), grid, dim3(256), 0, s, a);
+            else if (stream_out)
+                hipLaunchKernelGGL((fconv_rgb3x3_kernel<NT, true, false>), grid, dim3(256), 0, s, a);
             else
-                hipLaunchKernelGGL((fconv_rgb3x3_kernel<NT, false>), grid, dim3(256), 0, s, a);
+                hipLaunchKernelGGL((fconv_rgb3x3_kernel<NT, false, false>), grid, dim3(256), 0, s, a);
         };
         if (cout <= 32)
             launch(std::integral_constant<int, 1>{});

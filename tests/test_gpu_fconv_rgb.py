@@ -78,3 +78,21 @@ def test_infinities_and_nans(cout):
     assert torch.equal(out.isnan(), want.isnan()) and torch.equal(out.isinf(), want.isinf())
     inf = want.isinf()
     assert torch.equal(out[inf], want[inf])
+
+
+@pytest.mark.parametrize("n,h,w,cout,stride,pad,dil", [
+    (1, 90, 92, 32, 1, 1, 1), (1, 100, 100, 64, 1, 1, 1), (1, 128, 128, 64, 1, 1, 1), (6, 112, 112, 32, 2, 1, 1), (1, 181, 181, 64, 1, 1, 1), (1, 181, 182, 33, 1, 1, 1),
+    (256, 9, 17, 17, 2, 3, 1), (32, 32, 32, 64, 1, 1, 1), (33, 32, 32, 64, 1, 1, 1), (5, 99, 130, 48, 1, 2, 2), (64, 32, 31, 1, 1, 0, 1), (128, 32, 32, 64, 1, 1, 1),
+    (90, 224, 224, 32, 2, 1, 1), (180, 112, 112, 64, 1, 1, 1)])
+def test_sums_are_the_tile_kernels_to_the_bit(n, h, w, cout, stride, pad, dil):
+    """With the filters of 96 channels (zeros behind the first) the tile kernels run, below 256 tiles of 128 pixels with the depth split over
+    waves: the same sums in the same order."""
+    g = torch.Generator(device="cuda").manual_seed(n + w)
+    x, wt = torch.randn((n, h, w, 3), device="cuda", generator=g), torch.zeros((96, 3, 3, 3), device="cuda")
+    wt[:cout] = torch.randn((cout, 3, 3, 3), device="cuda", generator=g)
+    oh, ow = (h + 2 * pad - 2 * dil - 1) // stride + 1, (w + 2 * pad - 2 * dil - 1) // stride + 1
+    got, want = (torch.full((n, oh, ow, c), 9.0, device="cuda") for c in (cout, 96))
+    for c, out in ((cout, got), (96, want)):
+        assert capi.lib.dab_fconv_affine_relu(p(x), n, h, w, 3, p(wt), None, None, None, 0, 3, 3, pad, pad, stride, stride, dil, dil, c, p(out), stream()) == 0, capi.last_error()
+    differ = (got != want[..., :cout]).float().mean().item()
+    assert differ == 0, "%.3g of the values differ" % differ
