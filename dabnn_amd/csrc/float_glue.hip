@@ -73,7 +73,8 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 constexpr uint32_t kOob = 0x80000000u;     // descriptors here are shorter than 2^30 bytes
 constexpr uint32_t kOobRow = 0x40000000u;  // kOobRow + kOob and kOobRow + (anything < 2^30) stay out of range
 
-template <int BM, int BN, int SK, int KSPLIT, bool PADDED, int CV = 1, Pool2 POOL = Pool2::none>
+// COPY: the result goes to p.copy too (a form of its own: the test alone cost every small convolution 0.1 to 0.15 us of 3 to 5).
+template <int BM, int BN, int SK, int KSPLIT, bool PADDED, int CV = 1, Pool2 POOL = Pool2::none, bool COPY = false>
 __global__ __launch_bounds__(256) void fconv_kernel(const FconvArgs p) {
     constexpr int WAVES_MN = 4 / KSPLIT;
     constexpr int WAVES_N = (WAVES_MN >= 2 && BN >= 64) ? 2 : 1, WAVES_M = WAVES_MN / WAVES_N;
@@ -106,7 +107,6 @@ __global__ __launch_bounds__(256) void fconv_kernel(const FconvArgs p) {
     const int rows_n = p.cout - n0 < BN ? p.cout - n0 : BN, rows_m = p.M - m0 < BM ? p.M - m0 : BM;
     const auto w_rsrc = make_rsrc(p.w + (size_t)n0 * p.K, (uint32_t)rows_n * p.K * 4u);
     const auto o_rsrc = make_rsrc(p.out + (size_t)m0 * p.out_ld, (uint32_t)((rows_m - 1) * p.out_ld + p.cout) * 4u);
-    const auto c_rsrc = make_rsrc(p.copy + (p.copy ? (size_t)m0 * p.out_ld : 0), p.copy ? (uint32_t)((rows_m - 1) * p.out_ld + p.cout) * 4u : 0u);
 
     // loader: depth l_k of the slice, tile rows l_r + RP*i
     const int l_k = tid % LK, l_r = tid / LK;
@@ -301,8 +301,10 @@ __global__ __launch_bounds__(256) void fconv_kernel(const FconvArgs p) {
         else if constexpr (decltype(act)::value)
             v = v < 0.f ? 0.f : v;  // std::max(v, 0.f): a NaN stays
         __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), o_rsrc, (int)off, 0, 0);
-        if constexpr (KSPLIT > 1 && POOL == Pool2::none)
-            if (p.copy) __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), c_rsrc, (int)off, 0, 0);
+        if constexpr (COPY) {
+            const auto c_rsrc = make_rsrc(p.copy + (size_t)m0 * p.out_ld, (uint32_t)((rows_m - 1) * p.out_ld + p.cout) * 4u);
+            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), c_rsrc, (int)off, 0, 0);
+        }
         return v;
     };
     // The sign bits of a 32 x 32 tile: element e of all lanes is channels 0..31 of two rows, a dword of each, which is
@@ -1175,12 +1177,18 @@ static int fconv_impl(const char *fn, const float *x, int n, int h, int w, int c
     const long long big_tiles = ((M + 127) / 128) * ((cout + bn - 1) / bn);
 #define DAB_FCONV_LAUNCH(BM, BN, SK, KSPLIT, CV)                                                         \
     do {                                                                                                 \
-        copied = KSPLIT > 1 && a.copy != nullptr;                                                        \
+        constexpr bool kCopies = KSPLIT > 1;                                                             \
+        copied = kCopies && a.copy != nullptr;                                                           \
         const dim3 grid((unsigned)((M + BM - 1) / BM), (unsigned)((cout + BN - 1) / BN));                \
-        if (padded)                                                                                      \
-            hipLaunchKernelGGL((fconv_kernel<BM, BN, SK, KSPLIT, true, CV>), grid, dim3(256), 0, s, a);  \
+        auto launch = [&](auto pad_, auto copy_) {                                                       \
+            constexpr bool PAD = decltype(pad_)::value, COPY = decltype(copy_)::value;                   \
+            hipLaunchKernelGGL((fconv_kernel<BM, BN, SK, KSPLIT, PAD, CV, Pool2::none, COPY>), grid, dim3(256), 0, s, a); \
+        };                                                                                               \
+        using Copies = std::integral_constant<bool, kCopies>;                                            \
+        if (copied)                                                                                      \
+            padded ? launch(std::true_type{}, Copies{}) : launch(std::false_type{}, Copies{});           \
         else                                                                                             \
-            hipLaunchKernelGGL((fconv_kernel<BM, BN, SK, KSPLIT, false, CV>), grid, dim3(256), 0, s, a); \
+            padded ? launch(std::true_type{}, std::false_type{}) : launch(std::false_type{}, std::false_type{}); \
     } while (0)
     // Loader: 16-byte loads of four channels when the channel count allows it; for three-channel images one 12-byte
     // load per tap if the window has enough taps that slices of eight taps waste little (7x7: 56 for 49); else

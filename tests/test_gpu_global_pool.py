@@ -47,3 +47,20 @@ def test_a_second_copy_of_the_result(m, cout):
         assert capi.lib.dab_global_ave_pool_fconv1x1_copy(*gap, out.data_ptr(), host.data_ptr(), s) == 0
         torch.cuda.synchronize()
         assert torch.equal(out, want) and torch.equal(host[:-8].view(m, cout), want.cpu())
+
+
+@pytest.mark.parametrize("n,h,c,cout,k,pad", [(3, 5, 64, 40, 3, 1), (2, 9, 20, 33, 1, 0), (5, 6, 3, 70, 5, 2), (4, 7, 65, 31, 3, 0), (1, 12, 7, 100, 2, 1), (9, 40, 64, 64, 3, 1)])
+def test_a_second_copy_of_windows(n, h, c, cout, k, pad):
+    """The copying forms of the kernel that splits the depth: padded and not, four channels a load and one; and a larger problem, copied by a launch."""
+    import ctypes
+    from dabnn_amd import capi
+    g = torch.Generator(device="cuda").manual_seed(n + c)
+    x, w, b = (torch.randn(s, device="cuda", generator=g) for s in ((n, h, h, c), (cout, k, k, c), (cout,)))
+    s, o = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream), h + 2 * pad - k + 1
+    args = (x.data_ptr(), n, h, h, c, w.data_ptr(), b.data_ptr(), None, None, 0, k, k, pad, pad, 1, 1, 1, 1, cout)
+    want, out = torch.empty((n, o, o, cout), device="cuda"), torch.empty((n, o, o, cout), device="cuda")
+    host = torch.full((want.numel() + 8,), -3.0).pin_memory()
+    assert capi.lib.dab_fconv_affine_relu(*args, want.data_ptr(), s) == 0
+    assert capi.lib.dab_fconv_affine_relu_copy(*args, out.data_ptr(), host.data_ptr(), s) == 0
+    torch.cuda.synchronize()
+    assert torch.equal(out, want) and torch.equal(host[:-8].view_as(want), want.cpu()) and bool((host[-8:] == -3).all())
