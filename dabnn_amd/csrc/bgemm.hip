@@ -278,7 +278,8 @@ __global__ __launch_bounds__(256, NT == 2 ? 3 : 4) void bit_gemm_stream_kernel(c
             const int s = s0 + j * 256;
             int u, c, h;
             if constexpr (L == kFilterColumns) {
-                c = s % CH, h = (s / CH) & 1, u = s / (2 * CH);
+                // (the same unit in all lanes of a wave, whose 64 pieces never straddle 2 * CH)
+                c = s % CH, h = (s / CH) & 1, u = __builtin_amdgcn_readfirstlane(s / (2 * CH));
             } else {
                 c = (int)p.div_row_pieces.div((uint32_t)s);
                 const int r = s - c * p.units * 2;

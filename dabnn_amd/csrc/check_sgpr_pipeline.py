@@ -13,6 +13,10 @@ it has issued.  The compiler inserts the wait states behind the stores it emits 
 inline-asm statement, where the next vector instruction may overwrite the data: such a store must be followed, inside
 its own statement, by `s_nop 1` or more.
 
+A third rule is about time: where the scalar offset of a buffer load is a value that the compiler cannot prove equal in all
+lanes, it wraps the load in a loop over the values that occur (v_readfirstlane, v_cmp_eq, s_and_saveexec), so that loads
+meant to be asked for together wait for each other's branches.  The kernels here pass wave-uniform offsets only.
+
 usage: check_sgpr_pipeline.py file.s [file.s ...]
 """
 import re
@@ -97,14 +101,36 @@ def check(path):
     return problems
 
 
+def lane_loops(path):
+    """Loops over the values that a scalar operand takes in the lanes."""
+    problems = []
+    kernel = None
+    recent = []  # the last instructions, for the pattern at a loop's head
+    for no, line in enumerate(open(path), 1):
+        text = line.rstrip("\n")
+        if LABEL.match(text):
+            if not text.startswith(".L"):
+                kernel = text.rstrip(":")
+            recent = []
+            continue
+        op = text.split(";")[0].strip().split(None, 1)
+        if not op or op[0].startswith("."):
+            continue
+        if op[0].startswith("s_and_saveexec") and any(o.startswith("v_cmp_eq_u32") for o in recent) and "v_readfirstlane_b32" in recent:
+            problems.append("%s:%d: a loop over the lanes' values of a scalar operand (kernel %s)" % (path, no, kernel))
+        recent = (recent + [op[0]])[-8:]
+    return problems
+
+
 def main():
     bad = []
     for path in sys.argv[1:]:
         bad += check(path)
+        bad += lane_loops(path)
     for p in bad[:40]:
         print(p, file=sys.stderr)
     if bad:
-        print("check_sgpr_pipeline: %d instruction(s) touch scalar-load destinations before their wait" % len(bad), file=sys.stderr)
+        print("check_sgpr_pipeline: %d problem(s)" % len(bad), file=sys.stderr)
         return 1
     print("check_sgpr_pipeline: ok (%s)" % ", ".join(sys.argv[1:]))
     return 0

@@ -88,3 +88,43 @@ _Z6kernelv:
         bad.write_text("_Z6kernelv:\n\t;;#ASMSTART\n\t" + body + "\t;;#ASMEND\n\tv_mov_b32 v144, 1\n\ts_endpgm\n")
         problems = chk.check(str(bad))
         assert len(problems) == 1 and "more than 8 bytes" in problems[0], (body, problems)
+
+
+def test_checker_flags_a_loop_over_the_lanes_values_of_a_scalar_offset(tmp_path):
+    """What the compiler makes of a buffer load whose scalar offset it cannot prove uniform; a uniform one is a plain load."""
+    chk = load_checker()
+    loop, plain = tmp_path / "loop.s", tmp_path / "plain.s"
+    loop.write_text("""
+_Z6kernelv:
+	s_mov_b64 s[2:3], exec
+.LBB0_2:
+	v_readfirstlane_b32 s4, v9
+	v_cmp_eq_u32_e32 vcc, s4, v9
+	s_and_saveexec_b64 vcc, vcc
+	buffer_load_dwordx2 v[4:5], v3, s[8:11], s4 offen
+	s_xor_b64 exec, exec, vcc
+	s_cbranch_execnz .LBB0_2
+	s_endpgm
+""")
+    plain.write_text("""
+_Z6kernelv:
+	v_readfirstlane_b32 s4, v9
+	s_mul_i32 s4, s4, s5
+	buffer_load_dwordx2 v[4:5], v3, s[8:11], s4 offen
+	v_cmp_gt_i32_e32 vcc, s6, v9
+	s_and_saveexec_b64 s[2:3], vcc
+	s_endpgm
+""")
+    assert chk.lane_loops(str(plain)) == []
+    problems = chk.lane_loops(str(loop))
+    assert len(problems) == 1 and "_Z6kernelv" in problems[0], problems
+
+
+def test_the_kernels_assembly_holds_no_such_loop():
+    """Of the sources whose assembly the build leaves behind; built libraries may come without it."""
+    temps = os.path.join(ROOT, "dabnn_amd", "csrc", "build", "temps")
+    chk = load_checker()
+    for name in ("bgemm", "bconv3x3"):
+        path = os.path.join(temps, name + "-hip-amdgcn-amd-amdhsa-gfx950.s")
+        if os.path.exists(path):
+            assert chk.lane_loops(path) == []
