@@ -75,10 +75,8 @@ Net::~Net() {
     mirrors_.clear();
     mat_map_.clear();
     staging_.reset();
+    shares_.reset();
     if (mirror_memory_) (void)hipHostFree(mirror_memory_);
-    for (void *e : arrivals_) (void)hipEventDestroy(static_cast<hipEvent_t>(e));
-    for (void *up : upload_streams_)
-        if (up) (void)hipStreamDestroy(static_cast<hipStream_t>(up));
     if (stream_) (void)hipStreamDestroy(static_cast<hipStream_t>(stream_));
 }
 
@@ -340,6 +338,7 @@ void Net::prepare(const void *buf, size_t len) {
     copy_input_ = layers_write_input();
     find_head();
     staging_ = std::make_unique<Staging>(blob(input_name_)->bytes());
+    if (head_) shares_ = std::make_unique<ShareStreams>(staging_->device());
     plan_mirrors();
     hip_check(hipStreamSynchronize(static_cast<hipStream_t>(stream_)), "hipStreamSynchronize");
     prepared_ = true;
@@ -1039,33 +1038,21 @@ void Net::upload_and_run_head(const void *host_input, bool pageable) {
     const size_t image = in->bytes() / batch_;
     hipStream_t s = static_cast<hipStream_t>(stream_);
     hip_check(hipStreamSynchronize(s), "hipStreamSynchronize");  // (a run that failed may have left kernels that read the input)
-    for (void *&up : upload_streams_) {
-        if (up) continue;
+    void *up = nullptr;
+    {
         std::lock_guard<std::mutex> lock(capture_mutex());
-        hipStream_t made;
-        hip_check(hipStreamCreateWithFlags(&made, hipStreamNonBlocking), "hipStreamCreate");
-        up = made;
+        up = shares_->begin(in->bytes() / kShare + 1);  // (all but the last are of kShare or more)
     }
     int done = 0;
-    size_t share = 0;
     auto arriving = [&](size_t bytes) -> void * {
         const int there = (int)(bytes / image);
-        if (there < batch_ && (size_t)(there - done) * image < kShare) return upload_streams_[share % 2];
-        if (share == arrivals_.size()) {
-            std::lock_guard<std::mutex> lock(capture_mutex());
-            hipEvent_t e;
-            hip_check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate");
-            arrivals_.push_back(e);
-        }
-        hipEvent_t e = static_cast<hipEvent_t>(arrivals_[share]);
-        hip_check(hipEventRecord(e, static_cast<hipStream_t>(upload_streams_[share % 2])), "hipEventRecord");
-        hip_check(hipStreamWaitEvent(s, e, 0), "hipStreamWaitEvent");
+        if (there < batch_ && (size_t)(there - done) * image < kShare) return shares_->at_hand();
+        void *next = shares_->pass(s);
         run_head(done, there - done);
         done = there;
-        return upload_streams_[++share % 2];
+        return next;
     };
     try {
-        void *up = upload_streams_[0];
         if (pageable) {
             {
                 std::lock_guard<std::mutex> lock(capture_mutex());
@@ -1083,7 +1070,7 @@ void Net::upload_and_run_head(const void *host_input, bool pageable) {
             }
         }
     } catch (...) {
-        for (void *up : upload_streams_) (void)hipStreamSynchronize(static_cast<hipStream_t>(up));
+        shares_->synchronize();
         (void)hipStreamSynchronize(s);
         throw;
     }

@@ -22,6 +22,7 @@ namespace bnn {
 
 class BinConv;
 class Staging;
+class ShareStreams;
 
 class FloatConv;
 
@@ -121,11 +122,10 @@ class BNN_API Net : public std::enable_shared_from_this<Net> {
     bool layers_write_input();
     void launch_layers(Kind kind);
     void enqueue_layers(Kind kind);
-    // How many layers at the front run on the first images of a large host input while the others are still on their way, the
-    // streams that bring its shares in turn, and an event for each share.
+    // How many layers at the front run on the first images of a large host input while the others are still on their way, and the
+    // streams that bring its shares.
     size_t head_ = 0;
-    void *upload_streams_[2] = {};
-    std::vector<void *> arrivals_;
+    std::unique_ptr<ShareStreams> shares_;
     void find_head();
     void run_head(int first, int count);
     void upload_and_run_head(const void *host_input, bool pageable);

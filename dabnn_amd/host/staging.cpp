@@ -14,20 +14,74 @@ static void hip_check(hipError_t e, const char *what) {
     if (e != hipSuccess) throw std::runtime_error(std::string(what) + ": " + hipGetErrorString(e));
 }
 
+namespace {
+// Another device is the calling thread's current one for a while.
+class OnDevice {
+   public:
+    explicit OnDevice(int device) {
+        hip_check(hipGetDevice(&before_), "hipGetDevice");
+        if (before_ == device) return;
+        hip_check(hipSetDevice(device), "hipSetDevice");
+        changed_ = true;
+    }
+    ~OnDevice() {
+        if (changed_) (void)hipSetDevice(before_);
+    }
+    OnDevice(const OnDevice &) = delete;
+    OnDevice &operator=(const OnDevice &) = delete;
+
+   private:
+    int before_ = 0;
+    bool changed_ = false;
+};
+}  // namespace
+
 void *copy_stream(int device) {
     static std::mutex mutex;
     static auto &streams = *new std::map<int, hipStream_t>;  // never destroyed: a blob may be read while the process ends
     std::lock_guard<std::mutex> lock(mutex);
     hipStream_t &s = streams[device];
     if (!s) {
-        int current = 0;
-        hip_check(hipGetDevice(&current), "hipGetDevice");
-        if (current != device) hip_check(hipSetDevice(device), "hipSetDevice");
-        const hipError_t e = hipStreamCreateWithFlags(&s, hipStreamNonBlocking);
-        if (current != device) hip_check(hipSetDevice(current), "hipSetDevice");
-        hip_check(e, "hipStreamCreate");
+        const OnDevice on(device);
+        hip_check(hipStreamCreateWithFlags(&s, hipStreamNonBlocking), "hipStreamCreate");
     }
     return s;
+}
+
+void *ShareStreams::begin(size_t most) {
+    share_ = 0;
+    const OnDevice on(device_);
+    for (void *&s : streams_) {
+        if (s) continue;
+        hipStream_t made;
+        hip_check(hipStreamCreateWithFlags(&made, hipStreamNonBlocking), "hipStreamCreate");
+        s = made;
+    }
+    while (events_.size() < most) {
+        hipEvent_t e;
+        hip_check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate");
+        events_.push_back(e);
+    }
+    return at_hand();
+}
+
+void *ShareStreams::pass(void *behind) {
+    hipEvent_t e = static_cast<hipEvent_t>(events_.at(share_));
+    hip_check(hipEventRecord(e, static_cast<hipStream_t>(at_hand())), "hipEventRecord");
+    hip_check(hipStreamWaitEvent(static_cast<hipStream_t>(behind), e, 0), "hipStreamWaitEvent");
+    ++share_;
+    return at_hand();
+}
+
+void ShareStreams::synchronize() {
+    for (void *s : streams_)
+        if (s) (void)hipStreamSynchronize(static_cast<hipStream_t>(s));
+}
+
+ShareStreams::~ShareStreams() {
+    for (void *e : events_) (void)hipEventDestroy(static_cast<hipEvent_t>(e));
+    for (void *s : streams_)
+        if (s) (void)hipStreamDestroy(static_cast<hipStream_t>(s));
 }
 
 Staging::Staging(size_t bytes) {

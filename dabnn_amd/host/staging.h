@@ -41,6 +41,7 @@ class Staging {
 
     unsigned char *memory() const { return memory_; }
     size_t bytes() const { return bytes_; }
+    int device() const { return device_; }
 
     // Copies host memory to the device on `stream`; `src` may change once the call returns.  The caller synchronises the
     // stream before the next call (a Net's runs do).  `arriving`, if given, is told how many bytes have been asked for, from the
@@ -84,6 +85,29 @@ class Staging {
     int busy_ = 0;       // and has this many
     bool stop_ = false;
     std::mutex use_;  // one upload or download at a time
+};
+
+// The streams that bring the shares of an input in turn, and an event for each share, on a device of the caller's choice -- that of the
+// stream behind them -- whichever is current for the calling thread: the runtime records no event of one device on a stream of another.
+class ShareStreams {
+   public:
+    explicit ShareStreams(int device) : device_(device) {}
+    ~ShareStreams();
+    ShareStreams(const ShareStreams &) = delete;
+    ShareStreams &operator=(const ShareStreams &) = delete;
+
+    // The stream of the first of at most so many shares; what that takes and is not there yet is made here.
+    void *begin(size_t most);
+    // `behind` waits for what the share's stream has been given; the next share's stream.
+    void *pass(void *behind);
+    void *at_hand() const { return streams_[share_ % 2]; }
+    void synchronize();
+
+   private:
+    int device_;
+    void *streams_[2] = {};
+    std::vector<void *> events_;
+    size_t share_ = 0;
 };
 
 }  // namespace bnn

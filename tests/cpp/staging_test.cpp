@@ -31,6 +31,7 @@ hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) { return ++events, *e = reinterpret_cast<hipEvent_t>(new Owned{current}), hipSuccess; }
 hipError_t hipEventDestroy(hipEvent_t e) { return --events, delete reinterpret_cast<Owned *>(e), hipSuccess; }
 hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) { return device_of(e) == device_of(s) ? hipSuccess : hipErrorInvalidHandle; }
+hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuccess; }  // (of any device)
 hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
 hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipStream_t) { return memcpy(d, s, n), hipSuccess; }
 hipError_t hipMemcpy2DAsync(void *d, size_t dp, const void *s, size_t sp, size_t w, size_t h, hipMemcpyKind, hipStream_t) {
@@ -59,6 +60,37 @@ static int round_trip(bnn::Staging &staging, int device, size_t floats) {
     (void)hipStreamDestroy(s);
     m->download(out.data(), floats * 4, &staging);
     CHECK(out == in);
+    return 0;
+}
+
+// An input in shares, as a net takes a large one: the streams and events are of the net's device, whichever is current for the thread
+// that runs it.
+static int shares_of_an_input(int device, size_t floats) {
+    current = device;
+    bnn::Staging staging(floats * 4);
+    staging.grow(floats * 4);
+    bnn::ShareStreams shares(staging.device());
+    hipStream_t behind;
+    (void)hipStreamCreateWithFlags(&behind, 0);
+    current = 1 - device;
+    const int events_before = events;
+    for (int run = 0; run < 3; ++run) {
+        std::vector<float> in(floats), out(floats, -1.f);
+        for (size_t i = 0; i < floats; ++i) in[i] = (float)((i + run) % 1000003);
+        size_t done = 0, told = 0;
+        staging.upload(out.data(), in.data(), floats * 4, shares.begin(floats * 4 / (8u << 20) + 1), [&](size_t bytes) -> void * {
+            told = bytes;
+            if (bytes < floats * 4 && bytes - done < (8u << 20)) return shares.at_hand();
+            done = bytes;
+            void *before = shares.at_hand(), *next = shares.pass(behind);
+            if (next == before) throw std::runtime_error("the next share is on the same stream");
+            return next;
+        });
+        shares.synchronize();
+        CHECK(out == in && told == floats * 4 && current == 1 - device);
+    }
+    CHECK(events - events_before == (int)(floats * 4 / (8u << 20) + 1));  // made once
+    (void)hipStreamDestroy(behind);
     return 0;
 }
 
@@ -91,6 +123,8 @@ int main() {
             staging.download(out.data(), in.data(), in.size() * 4);
             CHECK(out == in && current == 1 - device);
         }
+        for (int device : {0, 1})
+            for (size_t floats : {4500000, 12000000, 30000000}) CHECK(shares_of_an_input(device, floats) == 0);  // below and above the pinned memory's 32 MB
         CHECK(pinned == 0 && events == 0 && streams == 2);  // one copy stream per device
     } catch (const std::exception &e) {
         printf("exception: %s\n", e.what());
