@@ -129,7 +129,7 @@ void Staging::wait_for_room(size_t block) {
         if (failed_.load(std::memory_order_relaxed)) return;
         std::this_thread::yield();
     }
-    // (the event may be that of a later transfer by now: of the same stream, so over after this one)
+    // (the event may be that of a later transfer by now, which took it over when this one had ended)
     hip_check(hipEventSynchronize(static_cast<hipEvent_t>(events_[transfer % kEvents])), "hipEventSynchronize");
 }
 
@@ -213,7 +213,12 @@ void Staging::upload(void *dst, const void *src, size_t bytes, void *stream, con
         for (; t < transfers_.size() && transfers_[t].first + transfers_[t].blocks <= ready; ++t) {
             const size_t at = transfers_[t].first * kBlock, n = std::min(transfers_[t].blocks * kBlock, size_ - at);
             hip_check(hipMemcpyAsync(dst_ + at, memory_ + (transfers_[t].first % ring_) * kBlock, n, hipMemcpyHostToDevice, s), "hipMemcpyAsync");
-            if (ring_ < blocks_) hip_check(hipEventRecord(static_cast<hipEvent_t>(events_[t % kEvents]), s), "hipEventRecord");
+            if (ring_ < blocks_) {
+                hipEvent_t e = static_cast<hipEvent_t>(events_[t % kEvents]);
+                // whoever waits for the transfer that had it before -- of another stream, perhaps -- may find this one's record
+                if (t >= kEvents) hip_check(hipEventSynchronize(e), "hipEventSynchronize");
+                hip_check(hipEventRecord(e, s), "hipEventRecord");
+            }
             issued_.store(t + 1, std::memory_order_release);
             if (arriving) s = static_cast<hipStream_t>(arriving(at + n));
         }

@@ -1,10 +1,14 @@
 // Staging and Mat's copies through it over a runtime of two devices that lives in host memory: what the real one refuses -- an event
-// of one device on a stream of another -- is refused here too.  Run by tests/test_staging.py, without a GPU.
+// of one device on a stream of another -- is refused here too, and a stream does its copies as late as it may, when somebody waits for
+// it or for an event behind them.  Run by tests/test_staging.py, without a GPU.
 #include <hip/hip_runtime_api.h>
 
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <deque>
+#include <functional>
+#include <mutex>
 #include <vector>
 
 #include "../../dabnn_amd/host/mat.h"
@@ -12,10 +16,27 @@
 
 static thread_local int current = 0;
 static int pinned = 0, streams = 0, events = 0;  // alive
-struct Owned {
+struct Stream {
     int device;
+    std::deque<std::function<void()>> waiting;
+    size_t asked = 0, done = 0;
+    void run_until(size_t n) {
+        for (; done < n; ++done) waiting.front()(), waiting.pop_front();
+    }
 };
-static int device_of(const void *p) { return static_cast<const Owned *>(p)->device; }
+struct Event {
+    int device;
+    Stream *stream = nullptr;
+    size_t behind = 0;  // so many operations of the stream
+};
+static std::mutex runtime;  // copies of several threads
+static Stream &of(hipStream_t s) { return *reinterpret_cast<Stream *>(s); }
+static Event &of(hipEvent_t e) { return *reinterpret_cast<Event *>(e); }
+static hipError_t ask(hipStream_t s, std::function<void()> operation) {
+    std::lock_guard<std::mutex> lock(runtime);
+    of(s).waiting.push_back(std::move(operation)), ++of(s).asked;
+    return hipSuccess;
+}
 
 extern "C" {
 const char *hipGetErrorString(hipError_t e) { return e == hipSuccess ? "success" : "refused"; }
@@ -25,18 +46,32 @@ hipError_t hipMalloc(void **p, size_t n) { return *p = malloc(n), hipSuccess; }
 hipError_t hipFree(void *p) { return free(p), hipSuccess; }
 hipError_t hipHostMalloc(void **p, size_t n, unsigned) { return ++pinned, *p = malloc(n), hipSuccess; }
 hipError_t hipHostFree(void *p) { return --pinned, free(p), hipSuccess; }
-hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) { return ++streams, *s = reinterpret_cast<hipStream_t>(new Owned{current}), hipSuccess; }
-hipError_t hipStreamDestroy(hipStream_t s) { return --streams, delete reinterpret_cast<Owned *>(s), hipSuccess; }
-hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
-hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) { return ++events, *e = reinterpret_cast<hipEvent_t>(new Owned{current}), hipSuccess; }
-hipError_t hipEventDestroy(hipEvent_t e) { return --events, delete reinterpret_cast<Owned *>(e), hipSuccess; }
-hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) { return device_of(e) == device_of(s) ? hipSuccess : hipErrorInvalidHandle; }
+hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) { return ++streams, *s = reinterpret_cast<hipStream_t>(new Stream{current, {}}), hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t s) {
+    std::lock_guard<std::mutex> lock(runtime);
+    return of(s).run_until(of(s).asked), hipSuccess;
+}
+hipError_t hipStreamDestroy(hipStream_t s) { return hipStreamSynchronize(s), --streams, delete &of(s), hipSuccess; }
+hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) { return ++events, *e = reinterpret_cast<hipEvent_t>(new Event{current}), hipSuccess; }
+hipError_t hipEventDestroy(hipEvent_t e) { return --events, delete &of(e), hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) {
+    std::lock_guard<std::mutex> lock(runtime);
+    if (of(e).device != of(s).device) return hipErrorInvalidHandle;
+    return of(e).stream = &of(s), of(e).behind = of(s).asked, hipSuccess;
+}
 hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuccess; }  // (of any device)
-hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
-hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipStream_t) { return memcpy(d, s, n), hipSuccess; }
-hipError_t hipMemcpy2DAsync(void *d, size_t dp, const void *s, size_t sp, size_t w, size_t h, hipMemcpyKind, hipStream_t) {
-    for (size_t y = 0; y < h; ++y) memcpy(static_cast<char *>(d) + y * dp, static_cast<const char *>(s) + y * sp, w);
+hipError_t hipEventSynchronize(hipEvent_t e) {
+    std::lock_guard<std::mutex> lock(runtime);
+    if (of(e).stream) of(e).stream->run_until(of(e).behind);
     return hipSuccess;
+}
+hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipStream_t stream) {
+    return ask(stream, [=] { memcpy(d, s, n); });
+}
+hipError_t hipMemcpy2DAsync(void *d, size_t dp, const void *s, size_t sp, size_t w, size_t h, hipMemcpyKind, hipStream_t stream) {
+    return ask(stream, [=] {
+        for (size_t y = 0; y < h; ++y) memcpy(static_cast<char *>(d) + y * dp, static_cast<const char *>(s) + y * sp, w);
+    });
 }
 }
 
