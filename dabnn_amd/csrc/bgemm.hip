@@ -135,12 +135,14 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t tile_rsrc(const float *t, cons
 enum Epilogue { kStoreCounts, kAddCounts, kAffine, kAffineSign };
 
 // Few tiles, or a depth that does not fit LDS as filters: a block is one tile of 32 pixels x 32 * NT channels, its four
-// (eight) waves take every fourth (eighth) unit of the depth each and load their operands straight from memory, kUnitsAhead units while
-// as many are multiplied; the partial sums meet in LDS.  Both operands +-1 (fp4_core.h).  Bound by their expansion: m512 k72 n3136,
-// accumulating, 8.7 us (9.8 with three units asked for at a time and none while they were multiplied).
-// SHALLOW: up to kUnitsAtOnce units a wave, all asked for at once, without the loop, whose length alone costs a launch of 2 to 3 us
-// 0.1 to 0.2 (116 x 405 x 14 2.44 -> 2.29 us, 94 x 23 x 17 2.54 -> 2.36, 88 x 300 x 40 2.84 -> 2.67).
-constexpr int kUnitsAhead = 2, kUnitsAtOnce = 3;
+// (eight) waves take every fourth (eighth) unit of the depth each and load their operands straight from memory, kUnitsAtOnce units at a
+// time; the partial sums meet in LDS.  Both operands +-1 (fp4_core.h).  Bound by their expansion: m512 k72 n3136, accumulating, 7.9 us.
+// (Two units asked for while two are multiplied: 8.0 there, 900 x 1000 x 50 6.3 instead of 5.8, 7 x 47 x 47 x 192 -> 120, 3 x 3, 5.5 instead of 5.1.)
+// SHALLOW: up to kUnitsAtOnce units a wave, without the loop, and what C holds is asked for before them: behind them its wait shows in
+// launches this short (189 x 26 x 13, accumulating, 2.52 us instead of 2.75, 300 x 300 x 40 3.03 instead of 3.19), while deeper ones begin with the
+// units (m512 k72 n3136 8.4 the other way round; 1 x 14 x 14 x 256 -> 256, 5 x 5, 3.60 instead of 3.69) -- but for windows with 64 channels a
+// block, whose loop is a shorter one without units in front of it (3 x 49 x 49 x 256 -> 208, 5 x 5, 9.0 us instead of 9.4).
+constexpr int kUnitsAtOnce = 3;
 template <int CC, FilterLayout L, int E, int NT, int WAVES, bool LONG, bool SHALLOW = false>
 __global__ __launch_bounds__(64 * WAVES, 4) void bit_gemm_split_kernel(const BitGemmArgs p) {
     constexpr int CH = 32 * NT, LD = CH + 1;
@@ -165,18 +167,18 @@ __global__ __launch_bounds__(64 * WAVES, 4) void bit_gemm_split_kernel(const Bit
         if (ch_ok) ea = p.g.a[ch], eb = p.g.b[ch];
     const int out_off = ch_ok ? (r0 * (int)p.g.out_ld + ch) * 4 : kBeyond, out_step = RPI * (int)p.g.out_ld * 4;
     auto element = [&](int i) { return p.g.out + (row0 + r0 + i * RPI) * p.g.out_ld + ch; };  // LONG: output i
-    constexpr int SLOTS = SHALLOW ? 1 : 2, AHEAD = SHALLOW ? kUnitsAtOnce : kUnitsAhead;
-    uint32_t a[SLOTS][AHEAD][CC], w[SLOTS][AHEAD][NT][CC];
-    auto fetch = [&](int slot, int u0) __attribute__((always_inline)) {
+    uint32_t a[kUnitsAtOnce][CC], w[kUnitsAtOnce][NT][CC];
+    auto fetch = [&](int u0) __attribute__((always_inline)) {
 #pragma unroll
-        for (int i = 0; i < AHEAD; ++i)
+        for (int i = 0; i < kUnitsAtOnce; ++i)
             if (u0 + WAVES * i < p.units) {
-                px.load(a[slot][i], p, u0 + WAVES * i, half);
+                px.load(a[i], p, u0 + WAVES * i, half);
 #pragma unroll
-                for (int n = 0; n < NT; ++n) load_filter<CC, L, LONG>(w[slot][i][n], p, rw, ch0 + n * 32 + l32, u0 + WAVES * i, half);
+                for (int n = 0; n < NT; ++n) load_filter<CC, L, LONG>(w[i][n], p, rw, ch0 + n * 32 + l32, u0 + WAVES * i, half);
             }
     };
-    fetch(0, wib);
+    constexpr bool kFirst = !SHALLOW && (L == kFilterColumns || NT == 1);
+    if constexpr (kFirst) fetch(wib);
     const float *second = E == kAddCounts ? p.g.out : p.g.shortcut;
     if constexpr (LONG) {
         static_assert(L == kFilterColumns, "a plain matrix");
@@ -189,31 +191,30 @@ __global__ __launch_bounds__(64 * WAVES, 4) void bit_gemm_split_kernel(const Bit
 #pragma unroll
         for (int i = 0; i < ROWS; ++i) old[i] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, out_off, i * out_step, 0));
     }
+    if constexpr (SHALLOW) fetch(wib);
     f32x16m acc[NT];
 #pragma unroll
     for (int n = 0; n < NT; ++n)
 #pragma unroll
         for (int v = 0; v < 16; ++v) acc[n][v] = 0.f;
-    auto multiply = [&](int slot, int u0) __attribute__((always_inline)) {
+    auto multiply = [&](int u0) __attribute__((always_inline)) {
 #pragma unroll
-        for (int i = 0; i < AHEAD; ++i)
+        for (int i = 0; i < kUnitsAtOnce; ++i)
             if (u0 + WAVES * i < p.units) {
 #pragma unroll
                 for (int c = 0; c < CC; ++c) {
-                    const i32x8 av = bitspm1(a[slot][i][c]);
+                    const i32x8 av = bitspm1(a[i][c]);
 #pragma unroll
-                    for (int n = 0; n < NT; ++n) mfma_fp4<32>(acc[n], av, bitspm1(w[slot][i][n][c]));
+                    for (int n = 0; n < NT; ++n) mfma_fp4<32>(acc[n], av, bitspm1(w[i][n][c]));
                 }
             }
     };
     if constexpr (SHALLOW) {
-        multiply(0, wib);
+        multiply(wib);
     } else {
-        for (int u0 = wib; u0 < p.units; u0 += 2 * WAVES * AHEAD) {
-            fetch(1, u0 + WAVES * AHEAD);
-            multiply(0, u0);
-            fetch(0, u0 + 2 * WAVES * AHEAD);
-            multiply(1, u0 + WAVES * AHEAD);
+        for (int u0 = wib; u0 < p.units; u0 += WAVES * kUnitsAtOnce) {
+            if (!kFirst || u0 != wib) fetch(u0);
+            multiply(u0);
         }
     }
 #pragma unroll
