@@ -32,8 +32,9 @@ constexpr int kPairFilterBytes = 9 * 2 * 64 * 16;
 
 // The packed rows of a strip and the filters of both layers, which LDS holds before anything is counted.  They are asked for
 // before the floats: loads come back in the order they were asked for, and the floats are only wanted behind the first tile's counts.
-// (The floats first: 56 x 56 at 256 images 89 us instead of 75, the pooled form 77 instead of 65.  The results are written through
-// the L2: the pass behind this one reads them, and both together take 2 to 4 % less than with streaming stores.)
+// (The floats first, us in a graph by itself: 56 x 56 at 40 images 18.1 instead of 17.6, at 100 43 / 38, at 256 90 either way; the pooled form at
+// 256 77 instead of 66.  The results are written through the L2: the pass behind this one reads them, and both together take 2 to 4 % less
+// than with streaming stores.)
 struct PairStage {
     // (at most 800 words: five rows of 160)
     uint64_t rows[4], filters[5];
@@ -223,7 +224,8 @@ static int pair_bands(int n, int h, int w) {
 // eight 2x2 windows, in the order of the pooled tensor, one window the four registers of an accumulator quad, so that pooling
 // takes no exchange.  A strip has an even number of rows; the rows above and below it, of which only the sign bits are wanted, are a
 // fifth tile of each wave that no register outlives, so that a strip has eight rows of 56 where the kernel above has seven.
-// 56 x 56 at batch 256, with the block's first layer behind it (bconv_down.hip): 89 + 61 us (one behind the other 164) as it was, 65 + 46 (118) now.
+// 56 x 56 at batch 256, and the block's first layer behind it (bconv_down.hip), us in a graph: the pass 66 (unpooled 90 to 93), that layer 51
+// (62), one behind the other 125 (159).
 struct BconvPairPoolArgs {
     const uint64_t *x;
     const float *shortcut;

@@ -160,9 +160,11 @@ void BinConv::forward_with_branch(float *branch_out) const {
     auto *packed = static_cast<uint64_t *>(binarized_mat->dev);
     const int n = input_mat->n, h = input_mat->h, w = input_mat->w, c = input_mat->elem_c;
     if (!input_prepacked) dab_check(dab_bitpack_nhwc(x, packed, (int64_t)n * h * w, c, stream()));
-    dab_check(dab_bconv3x3_down(packed, branch_pooled ? floats(branch_pooled) : x, branch_pooled ? 1 : 0, n, h, w, c, static_cast<const uint64_t *>(weight_mat->dev), floats(fused_a), floats(fused_b), weight_mat->n,
+    auto *sign = fused_sign_out ? static_cast<uint64_t *>(fused_sign_out->dev) : nullptr;
+    dab_check(dab_bconv3x3_down(packed, branch_pooled ? floats(branch_pooled) : x, branch_pooled ? 1 : 0, n, h, w, c,
+                                static_cast<const uint64_t *>(weight_mat->dev), floats(fused_a), floats(fused_b), weight_mat->n,
                                 floats(branch->weight_mat), floats(branch->bias_mat), floats(branch->fused_a), floats(branch->fused_b), branch_out,
-                                static_cast<float *>(output_mat->dev), fused_sign_out ? static_cast<uint64_t *>(fused_sign_out->dev) : nullptr, stream()));
+                                static_cast<float *>(output_mat->dev), sign, stream()));
 }
 
 void BinConv::forward_alone() const {

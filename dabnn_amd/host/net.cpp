@@ -829,7 +829,7 @@ void Net::pool_inside_convs() {
 // Two residual layers over 64 channels that follow each other (BinConv + Affine + Add of its own input, at stride 1) run as one
 // pass that keeps the blob between them on the chip, where that blob and its packed copy have no other reader and nothing
 // rewrites what the first layer reads (who asks for them has that layer run again).  Pays from 48 000 pixels on, where the
-// layers are bound by memory, two launches / one pass: 56 x 56 at 12 images 12.0 / 11.3 us, 16 12.5 / 11.5, 24 20.8 / 13.4, 64
+// layers are bound by memory, two launches / one pass, by themselves in a graph: 56 x 56 at 12 images 12.0 / 11.3 us, 16 12.5 / 11.5, 24 20.8 / 13.4, 64
 // 43 / 21, 256 158 / 90; 28 x 28 at 40 images 9.7 / 12.1, 64 12.2 / 9.8.  Up to 64 columns: a strip of wider rows is so low
 // that its neighbours' rows are most of the work.
 void Net::pair_residual_layers() {
@@ -910,8 +910,8 @@ void Net::branches_inside_binconvs() {
 
 // Two residual layers in one pass, in front of a down-sampling block whose branch runs in its BinConv's pass: where nobody else reads
 // the second layer's result, the pass writes it pooled (and its sign bits), a quarter of the bytes, and the block's pass reads that; who
-// asks for the result has the unpooled pass run.  56 x 56, the two passes together, us: 17 images 21.5 -> 18.8, 40 34 -> 33, 100 70 ->
-// 60, 256 164 -> 131.
+// asks for the result has the unpooled pass run.  56 x 56, the two passes one behind the other in a graph, us: 17 images 21.0 -> 18.7, 40
+// 33.5 -> 32.0, 100 65.6 -> 56.2, 256 159 -> 125.
 void Net::pool_inside_pairs() {
     std::vector<const Mat *> rd, wr;
     for (const auto &l : layers) {

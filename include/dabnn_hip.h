@@ -206,7 +206,9 @@ DAB_API int dab_bconv3x3_pair_pool_takes(int n, int h, int w);
 /*
  * The first layer of a down-sampling block and its shortcut branch in one pass (BinConv, Affine, AvePool 2x2, FloatConv 1x1, Affine, Add):
  *   out = a * bconv3x3(x_packed, stride 2, pad 1) + b + (sc_a * (conv1x1(avepool2x2(x)) + sc_bias) + sc_b)
- * x [n][h][w][cin] floats with x_packed = pack_mat(x), or, with x_pooled, avepool2x2(x) [n][h/2][w/2][cin] in its place; wgt as dab_bconv3x3, sc_wgt [cout][cin]; sc_bias, and sc_a with sc_b, may be NULL.
+ * x [n][h][w][cin] floats with x_packed = pack_mat(x), or, with x_pooled, avepool2x2(x) [n][h/2][w/2][cin] in its place (a Net has that
+ * for 64 input channels, from dab_bconv3x3_pair_pool; 128 and 256 are there for direct callers); wgt as dab_bconv3x3, sc_wgt
+ * [cout][cin]; sc_bias, and sc_a with sc_b, may be NULL.
  * out [n][h/2][w/2][cout]; out_packed = pack_mat(out) and shortcut (what the branch adds) are written unless NULL.  No
  * result may overlap an input.  Every operation behind the sums is rounded by itself, as in the separate layers; beyond
  * eight output pixels the branch's fp32 sums are dab_ave_pool2_fconv1x1's to the bit.  Buffers 16-byte aligned (wgt and out_packed 8).

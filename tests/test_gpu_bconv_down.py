@@ -1,5 +1,6 @@
 """dab_bconv3x3_down: the first layer of a down-sampling block with its shortcut branch in one launch.  Given the branch's values, counts,
-Affine, Add and sign bits are bit for bit the separate calls'; the branch's fp32 sums are compared with 64-bit ones."""
+Affine, Add and sign bits are bit for bit the separate calls'; the branch's fp32 sums are compared with 64-bit ones and, bit for bit, with
+dab_ave_pool2_fconv1x1's."""
 import ctypes
 
 import numpy as np

@@ -1,5 +1,5 @@
-"""The GEMM kernel that splits the depth over a block's waves: four and eight of them, depths that end inside a unit and inside a pipelined
-pair of units, both sides of the switch, and matrices that are addressed by pointer because a row, or the filters, are too long for 32 bits."""
+"""The GEMM kernel that splits the depth over a block's waves: four and eight of them, depths that end inside a unit and inside a batch
+of units, both sides of the switch, and matrices that are addressed by pointer because a row, or the filters, are too long for 32 bits."""
 import pytest
 import torch
 
