@@ -1134,7 +1134,7 @@ void Net::launch_layers(Kind kind) {
         (void)hipGraphExecDestroy(static_cast<hipGraphExec_t>(graph.exec));
         graph.exec = nullptr;
     }
-    if (profile || !use_graph) {
+    if (profile || !use_graph || (kind == kBehindHead && head_ == layers.size())) {  // (no layer behind the head: nothing to capture)
         enqueue_layers(kind);
     } else if (graph.exec) {
         hip_check(hipGraphLaunch(static_cast<hipGraphExec_t>(graph.exec), s), "hipGraphLaunch");

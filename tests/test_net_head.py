@@ -69,7 +69,7 @@ def test_two_nets_on_threads(model):
         assert len(g) == 8 and all(np.array_equal(v, w) for v in g)
 
 
-def headed_net(blocks, hw, seed=0, width=64):
+def headed_net(blocks, hw, seed=0, width=64, classifier=True):
     """7x7 stem and MaxPool -> binary layers, each (output channels, stride, residual, Affine) -> classifier; and the names of all blobs."""
     from dabnn_amd import models
     r = np.random.default_rng(seed)
@@ -103,6 +103,8 @@ def headed_net(blocks, hw, seed=0, width=64):
         if residual:
             out = add("Add", p + "_add", p + "_out", input1=out, input2=cur)
         cur, cin, size = out, cout, (size - 1) // stride + 1
+    if not classifier:
+        return (layers, inits, [("data", [1, hw, hw, 3])]), names
     cur = add("AvePool", "gap", "gap_out", input=cur, kernel_shape=[size, size], pads=[0] * 4, strides=[1, 1])
     add("FpConv2D", "fc", "logits", input=cur, weight=tensor("fc_w", (r.standard_normal((10, 1, 1, cin)) / 8).astype(np.float32)), pads=[0] * 4, strides=[1, 1], dilations=[1, 1])
     return (layers, inits, [("data", [1, hw, hw, 3])]), names
@@ -155,3 +157,21 @@ def test_heads_of_other_nets(kind):
             assert np.array_equal(got[name], want[name]), (run, name)
     a.close()
     b.close()
+
+
+@pytest.mark.parametrize("blocks", [[(64, 1, True, True)], [(64, 1, True, True)] * 2, [(64, 1, False, True), (64, 1, True, True), (128, 2, False, True)]])
+def test_nets_that_end_with_their_head(blocks):
+    """No layer is left behind it; results too large to be copied for who asks, and (64 x 7 x 7) small enough."""
+    from dabnn_amd import dab_format, net
+    for blocks in (blocks, blocks + [(64, 2, False, True)] * 2):
+        model, names = headed_net(blocks, 224, classifier=False)
+        data = dab_format.write_model(*model)
+        a, b = (net.Net(batch=30).read_buf(data) for _ in range(2))
+        r = np.random.default_rng(len(blocks))
+        for run in range(6):
+            x = r.standard_normal((30, 224, 224, 3)).astype(np.float32)
+            a.run(torch.from_numpy(x).pin_memory().numpy() if run % 2 else x)
+            b.run(torch.from_numpy(x).cuda())
+            assert np.array_equal(a.get_blob(names[-1]), b.get_blob(names[-1])), run
+        a.close()
+        b.close()
